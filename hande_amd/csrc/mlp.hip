@@ -175,19 +175,51 @@ __global__ void k_mlp_feat(int64_t ns, int nb, int d_in, const uint64_t* __restr
   x[t] = occ ? (c < nb ? 1.0f : static_cast<float>(eps[o])) : 0.0f;
 }
 
-// C[M][N] = op(A)[M][K] op(B)[K][N] (+ bias[N]); op(A)[i][k] = ta ? A[k][i] : A[i][k],
-// on fp32 matrix cores: a 64x64 tile of C per block, each
-// of its four waves a 32x32 quarter as 2x2 tiles of v_mfma_f32_16x16x4_f32
-// (lane l feeds A[row l%16][k l/16] and B[k l/16][col l%16] and holds
-// D[rows 4(l/16)..+3][col l%16]); K in slabs of 16 staged through LDS with
-// the transposes applied on load.  The accumulation order is fixed by the
-// tile shape, so results are deterministic.
-constexpr int kGemmTile = 64, kGemmSlab = 16;
+// C[M][N] = A[M][K] op(B)[K][N] on fp32 matrix cores, op(B)[k][j] = TB ?
+// B[j][k] : B[k][j].  A block makes a 64x64 tile of C, each of its four waves a
+// 32x32 quarter as 2x2 tiles of v_mfma_f32_16x16x4_f32 (lane l feeds
+// A[row l%16][k l/16] and B[k l/16][col l%16] and holds D[rows 4(l/16)..+3]
+// [col l%16]).  K goes in slabs of 32 staged through LDS, the next slab's
+// loads in flight while a slab is multiplied (a slab's 32 MFMAs take ~1000
+// cycles, about one trip to L2).  Rows of Bs are 80 floats apart, so the four
+// k groups of a fragment read 4 x 16 different banks.  The accumulation order
+// is fixed by the tile shape, so results are deterministic.
+// The epilogue is fused (kEpiBias: C = acc + bias; kEpiGelu: Z = acc + bias,
+// C = gelu(Z); kEpiGeluBwd: C = acc * gelu'(Z)), which saves each hidden
+// layer's separate pass over its 16384 x 256 activations.  At 16384 samples
+// and nbasis 80 a product takes 31-36 us (43-60 TFLOP/s), bound by the LDS
+// staging between barriers at 4 waves a block.
+constexpr int kGemmTile = 64, kGemmSlab = 32;
+constexpr int kGemmPer = kGemmTile * kGemmSlab / kBlock;  // elements of each operand a thread stages per slab
+enum GemmEpilogue { kEpiBias, kEpiGelu, kEpiGeluBwd };
+
+struct GemmTiles {
+  float As[kGemmTile][kGemmSlab + 1];
+  float Bs[kGemmSlab][kGemmTile + 16];
+};
+// acc += the staged slab's product for this wave's quarter (wr, wc).
+__device__ __forceinline__ void gemm_slab(const GemmTiles& t, int lane, int wr, int wc, f32x4 (&acc)[2][2]) {
+#pragma unroll
+  for (int kk = 0; kk < kGemmSlab; kk += 4) {
+    const int kq = kk + (lane >> 4);
+    float av[2], bv[2];
+#pragma unroll
+    for (int a = 0; a < 2; ++a) av[a] = t.As[wr + a * 16 + (lane & 15)][kq];
+#pragma unroll
+    for (int b = 0; b < 2; ++b) bv[b] = t.Bs[kq][wc + b * 16 + (lane & 15)];
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[a], bv[b], acc[a][b], 0, 0, 0);
+  }
+}
+
+template <bool TB, GemmEpilogue E>
 __global__ __launch_bounds__(kBlock) void k_gemm_mfma(int M, int N, int K, const float* __restrict__ A, int lda,
-                                                      int ta, const float* __restrict__ B, int ldb, int tb,
-                                                      const float* __restrict__ bias, float* __restrict__ C, int ldc) {
-  __shared__ float As[kGemmTile][kGemmSlab + 1];
-  __shared__ float Bs[kGemmSlab][kGemmTile + 1];
+                                                      const float* __restrict__ B, int ldb,
+                                                      const float* __restrict__ bias, float* __restrict__ Z,
+                                                      float* __restrict__ C, int ldc) {
+  __shared__ GemmTiles sm;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int i0 = blockIdx.y * kGemmTile, j0 = blockIdx.x * kGemmTile;
   const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
@@ -196,41 +228,34 @@ __global__ __launch_bounds__(kBlock) void k_gemm_mfma(int M, int N, int K, const
   for (int a = 0; a < 2; ++a)
 #pragma unroll
     for (int b = 0; b < 2; ++b) acc[a][b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  for (int k0 = 0; k0 < K; k0 += kGemmSlab) {
-    // 64 x 16 of op(A) and 16 x 64 of op(B): 1024 elements each, 4 per thread
+  float ra[kGemmPer], rb[kGemmPer];
+  auto fetch = [&](int k0) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
+    for (int q = 0; q < kGemmPer; ++q) {
       const int e = q * kBlock + tid;
-      {  // A: consecutive threads along k (row-major A) or along i (transposed A)
-        const int r = ta ? (e & 63) : (e >> 4), kk = ta ? (e >> 6) : (e & 15);
-        const int gi = i0 + r, gk = k0 + kk;
-        As[r][kk] = (gi < M && gk < K)
-                        ? (ta ? A[static_cast<int64_t>(gk) * lda + gi] : A[static_cast<int64_t>(gi) * lda + gk])
-                        : 0.0f;
-      }
-      {  // B: along j (row-major B) or along k (transposed B)
-        const int cidx = tb ? (e >> 4) : (e & 63), kk = tb ? (e & 15) : (e >> 6);
-        const int gj = j0 + cidx, gk = k0 + kk;
-        Bs[kk][cidx] = (gj < N && gk < K)
-                           ? (tb ? B[static_cast<int64_t>(gj) * ldb + gk] : B[static_cast<int64_t>(gk) * ldb + gj])
-                           : 0.0f;
-      }
+      const int r = e >> 5, ka = k0 + (e & 31);  // consecutive threads along k
+      ra[q] = (i0 + r < M && ka < K) ? A[static_cast<int64_t>(i0 + r) * lda + ka] : 0.0f;
+      const int c = TB ? (e >> 5) : (e & 63), kb = k0 + (TB ? (e & 31) : (e >> 6));
+      rb[q] = (j0 + c < N && kb < K)
+                  ? (TB ? B[static_cast<int64_t>(j0 + c) * ldb + kb] : B[static_cast<int64_t>(kb) * ldb + j0 + c])
+                  : 0.0f;
+    }
+  };
+  fetch(0);
+  for (int k0 = 0; k0 < K; k0 += kGemmSlab) {
+    __syncthreads();  // the previous slab has been read
+#pragma unroll
+    for (int q = 0; q < kGemmPer; ++q) {
+      const int e = q * kBlock + tid;
+      sm.As[e >> 5][e & 31] = ra[q];
+      if (TB)
+        sm.Bs[e & 31][e >> 5] = rb[q];
+      else
+        sm.Bs[e >> 6][e & 63] = rb[q];
     }
     __syncthreads();
-#pragma unroll
-    for (int kk = 0; kk < kGemmSlab; kk += 4) {
-      const int kq = kk + (lane >> 4);
-      float av[2], bv[2];
-#pragma unroll
-      for (int a = 0; a < 2; ++a) av[a] = As[wr + a * 16 + (lane & 15)][kq];
-#pragma unroll
-      for (int b = 0; b < 2; ++b) bv[b] = Bs[kq][wc + b * 16 + (lane & 15)];
-#pragma unroll
-      for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[a], bv[b], acc[a][b], 0, 0, 0);
-    }
-    __syncthreads();
+    if (k0 + kGemmSlab < K) fetch(k0 + kGemmSlab);
+    gemm_slab(sm, lane, wr, wc, acc);
   }
 #pragma unroll
   for (int a = 0; a < 2; ++a)
@@ -239,25 +264,110 @@ __global__ __launch_bounds__(kBlock) void k_gemm_mfma(int M, int N, int K, const
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int gi = i0 + wr + a * 16 + (lane >> 4) * 4 + r, gj = j0 + wc + b * 16 + (lane & 15);
-        if (gi < M && gj < N) C[static_cast<int64_t>(gi) * ldc + gj] = acc[a][b][r] + (bias ? bias[gj] : 0.0f);
+        if (gi >= M || gj >= N) continue;
+        const int64_t o = static_cast<int64_t>(gi) * ldc + gj;
+        if constexpr (E == kEpiGeluBwd) {
+          C[o] = acc[a][b][r] * gelu_g(Z[o]);
+        } else {
+          const float z = acc[a][b][r] + bias[gj];
+          if constexpr (E == kEpiGelu) {
+            Z[o] = z;
+            C[o] = gelu_f(z);
+          } else {
+            C[o] = z;
+          }
+        }
       }
 }
 
-__global__ void k_gelu_fwd(int64_t n, const float* __restrict__ z, float* __restrict__ a) {
-  const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t < n) a[t] = gelu_f(z[t]);
+// The three weight gradients act^T D (act [B][M], D [B][N], B samples) and bias
+// gradients (column sums of D) in one launch: a block takes one 64x64 tile of
+// one gradient over one chunk of the samples and writes it to that chunk's
+// copy of the parameter vector; k_sum_splits adds the chunks in order.
+// The gradients have only 12 + 16 + 12 tiles (nbasis 80), which without the
+// split left 216 of the 256 CUs idle behind 1024 serial slabs: at 16384
+// samples the three products and the column sums (then a kernel of one thread
+// per column) took 18.4 of a training step's 19.5 ms, with 32 chunks 80 us
+// (65 TFLOP/s; a large fp32 product reaches 153 here).
+// Bias sums come from the D values the first row of tiles stages anyway.
+struct WGrad {
+  const float* act;
+  const float* d;
+  int M, N;
+  int64_t o_w, o_b;  // offsets of the gradient and the bias gradient in the parameter vector
+  int first;         // first tile of this gradient (tiles are numbered over all three)
+};
+struct WGrads {
+  WGrad g[3];
+  int tiles;
+};
+__global__ __launch_bounds__(kBlock) void k_wgrad(WGrads w, int64_t ns, int64_t chunk, int64_t stride,
+                                                  float* __restrict__ part) {
+  __shared__ GemmTiles sm;
+  __shared__ float cs[kBlock];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tile = blockIdx.x;
+  const WGrad g = tile >= w.g[2].first ? w.g[2] : tile >= w.g[1].first ? w.g[1] : w.g[0];
+  const int tn = (g.N + kGemmTile - 1) / kGemmTile, t = tile - g.first;
+  const int i0 = (t / tn) * kGemmTile, j0 = (t % tn) * kGemmTile;
+  const int64_t s0 = blockIdx.y * chunk, s1 = s0 + chunk < ns ? s0 + chunk : ns;
+  float* out = part + static_cast<int64_t>(blockIdx.y) * stride;
+  const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
+  f32x4 acc[2][2];
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b) acc[a][b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  float ra[kGemmPer], rb[kGemmPer], csum = 0.0f;
+  const int c = tid & 63;  // this thread's row of act^T and column of D
+  auto fetch = [&](int64_t k0) {
+#pragma unroll
+    for (int q = 0; q < kGemmPer; ++q) {
+      const int64_t k = k0 + q * (kBlock / 64) + wave;
+      ra[q] = (i0 + c < g.M && k < s1) ? g.act[k * g.M + i0 + c] : 0.0f;
+      rb[q] = (j0 + c < g.N && k < s1) ? g.d[k * g.N + j0 + c] : 0.0f;
+    }
+  };
+  fetch(s0);
+  for (int64_t k0 = s0; k0 < s1; k0 += kGemmSlab) {
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < kGemmPer; ++q) {
+      const int kk = q * (kBlock / 64) + wave;
+      sm.As[c][kk] = ra[q];
+      sm.Bs[kk][c] = rb[q];
+      csum += rb[q];
+    }
+    __syncthreads();
+    if (k0 + kGemmSlab < s1) fetch(k0 + kGemmSlab);
+    gemm_slab(sm, lane, wr, wc, acc);
+  }
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int gi = i0 + wr + a * 16 + (lane >> 4) * 4 + r, gj = j0 + wc + b * 16 + (lane & 15);
+        if (gi < g.M && gj < g.N) out[g.o_w + static_cast<int64_t>(gi) * g.N + gj] = acc[a][b][r];
+      }
+  if (i0 == 0) {  // block-uniform
+    cs[tid] = csum;
+    __syncthreads();
+    if (wave == 0 && j0 + c < g.N) out[g.o_b + j0 + c] = (cs[c] + cs[64 + c]) + (cs[128 + c] + cs[192 + c]);
+  }
 }
-__global__ void k_gelu_bwd(int64_t n, const float* __restrict__ z, float* __restrict__ d) {
-  const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t < n) d[t] = d[t] * gelu_g(z[t]);
-}
-// out[j] = sum_i D[i][j], rows in order (one thread per column).
-__global__ void k_colsum(int M, int N, const float* __restrict__ D, int ldd, float* __restrict__ out) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= N) return;
+// The gradient of parameter t: its chunks' partial sums in order.
+__device__ __forceinline__ float sum_splits(const float* __restrict__ part, int64_t t, int64_t stride, int nsplit) {
   float acc = 0.0f;
-  for (int i = 0; i < M; ++i) acc = acc + D[static_cast<int64_t>(i) * ldd + j];
-  out[j] = acc;
+#pragma unroll 8
+  for (int z = 0; z < nsplit; ++z) acc += part[z * stride + t];
+  return acc;
+}
+__global__ void k_sum_splits(int64_t n, int64_t stride, int nsplit, const float* __restrict__ part,
+                             float* __restrict__ g) {
+  const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (t < n) g[t] = sum_splits(part, t, stride, nsplit);
 }
 // Fixed-order sum of n doubles on one block.
 __global__ void k_dsum(int64_t n, const double* __restrict__ x, double* __restrict__ out) {
@@ -461,11 +571,13 @@ __global__ void k_aff_table(int64_t n, const float* __restrict__ th, float* __re
   if (k < n) aff[k] = static_cast<float>(exp(static_cast<double>(fminf(fmaxf(th[k], -kClip), kClip))));
 }
 
-__global__ void k_adam(int64_t n, float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m,
-                       float* __restrict__ v, float lr, float c1, float c2) {
+// Adam over all parameters; those from o_th on (the affinity) with their own rate.
+__global__ void k_adam(int64_t n, int64_t o_th, float* __restrict__ p, const float* __restrict__ g,
+                       float* __restrict__ m, float* __restrict__ v, float lr_net, float lr_aff, float c1, float c2) {
   const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (t >= n) return;
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
+  const float lr = t < o_th ? lr_net : lr_aff;
   const float gt = g[t];
   const float mt = b1 * m[t] + (1.0f - b1) * gt;
   const float vt = b2 * v[t] + (1.0f - b2) * gt * gt;
@@ -538,11 +650,12 @@ void dfree(T*& p) {
   p = nullptr;
 }
 
-void gemm(int M, int N, int K, const float* A, int lda, int ta, const float* B, int ldb, int tb, const float* bias,
+template <bool TB, GemmEpilogue E>
+void gemm(int M, int N, int K, const float* A, int lda, const float* B, int ldb, const float* bias, float* Z,
           float* C, int ldc, hipStream_t st) {
-  hipLaunchKernelGGL(k_gemm_mfma, dim3(static_cast<unsigned>(ceil_div(N, kGemmTile)),
-                                      static_cast<unsigned>(ceil_div(M, kGemmTile))),
-                     dim3(kBlock), 0, st, M, N, K, A, lda, ta, B, ldb, tb, bias, C, ldc);
+  hipLaunchKernelGGL((k_gemm_mfma<TB, E>), dim3(static_cast<unsigned>(ceil_div(N, kGemmTile)),
+                                               static_cast<unsigned>(ceil_div(M, kGemmTile))),
+                     dim3(kBlock), 0, st, M, N, K, A, lda, B, ldb, bias, Z, C, ldc);
 }
 
 // splitmix64 -> standard normal (Box--Muller) for parameter initialisation.
@@ -603,6 +716,7 @@ int mlp_alloc(Mlp& m, int nb, int W, int64_t bcap) {
   rc |= dalloc(&m.aff, static_cast<int64_t>(nb) * nb);
   rc |= dalloc(&m.dth, bcap * 2 * nb);
   rc |= dalloc(&m.aff_part, static_cast<int64_t>(m.nchunk) * nb * nb);
+  rc |= dalloc(&m.gpart, static_cast<int64_t>(kGradSplits) * m.o_th);
   return rc == FQ_OK ? FQ_OK : FQ_ERR_NOMEM;
 }
 
@@ -640,6 +754,7 @@ void mlp_free(Mlp& m) {
   dfree(m.ck);
   dfree(m.dth);
   dfree(m.aff_part);
+  dfree(m.gpart);
   dfree(m.scum);
   dfree(m.swts);
   m.scum_cap = 0;
@@ -719,11 +834,9 @@ int mlp_train_step(Mlp& m, const fqd::Sys& s, int64_t ns, double lr, bool apply,
   const int H = kHidden, di = m.d_in, dout = m.d_out, B = static_cast<int>(ns);
   hipLaunchKernelGGL(k_mlp_feat, dim3(blocks(ns * di)), dim3(kBlock), 0, st, ns, m.nb, di, m.sdet, m.bcap,
                      s.sp_eigv, m.x);
-  gemm(B, H, di, m.x, di, 0, m.p + m.o_w1, H, 0, m.p + m.o_b1, m.z1, H, st);
-  hipLaunchKernelGGL(k_gelu_fwd, dim3(blocks(ns * H)), dim3(kBlock), 0, st, ns * H, m.z1, m.a1);
-  gemm(B, H, H, m.a1, H, 0, m.p + m.o_w2, H, 0, m.p + m.o_b2, m.z2, H, st);
-  hipLaunchKernelGGL(k_gelu_fwd, dim3(blocks(ns * H)), dim3(kBlock), 0, st, ns * H, m.z2, m.a2);
-  gemm(B, dout, H, m.a2, H, 0, m.p + m.o_w3, dout, 0, m.p + m.o_b3, m.z3, dout, st);
+  gemm<false, kEpiGelu>(B, H, di, m.x, di, m.p + m.o_w1, H, m.p + m.o_b1, m.z1, m.a1, H, st);
+  gemm<false, kEpiGelu>(B, H, H, m.a1, H, m.p + m.o_w2, H, m.p + m.o_b2, m.z2, m.a2, H, st);
+  gemm<false, kEpiBias>(B, dout, H, m.a2, H, m.p + m.o_w3, dout, m.p + m.o_b3, nullptr, m.z3, dout, st);
   hipLaunchKernelGGL(k_dsum, dim3(1), dim3(kBlock), 0, st, ns, m.sw, m.dsum);
   hipLaunchKernelGGL(k_mlp_loss_grad, dim3(blocks(ns)), dim3(kBlock), 0, st, s, ns, m.nb, dout, m.sdet, m.bcap,
                      m.sexc, m.sw, m.sflat, m.dsum, m.z3, m.p + m.o_th, m.d3, m.dth, m.sloss, m.sh, m.objective);
@@ -736,26 +849,30 @@ int mlp_train_step(Mlp& m, const fqd::Sys& s, int64_t ns, double lr, bool apply,
   hipLaunchKernelGGL(k_aff_grad_sum, dim3(blocks(na)), dim3(kBlock), 0, st, m.nb, nchunk, m.aff_part,
                      m.g + m.o_th);
   // backward
-  gemm(H, dout, B, m.a2, H, 1, m.d3, dout, 0, nullptr, m.g + m.o_w3, dout, st);
-  hipLaunchKernelGGL(k_colsum, dim3(blocks(dout)), dim3(kBlock), 0, st, B, dout, m.d3, dout, m.g + m.o_b3);
-  gemm(B, H, dout, m.d3, dout, 0, m.p + m.o_w3, dout, 1, nullptr, m.d2, H, st);
-  hipLaunchKernelGGL(k_gelu_bwd, dim3(blocks(ns * H)), dim3(kBlock), 0, st, ns * H, m.z2, m.d2);
-  gemm(H, H, B, m.a1, H, 1, m.d2, H, 0, nullptr, m.g + m.o_w2, H, st);
-  hipLaunchKernelGGL(k_colsum, dim3(blocks(H)), dim3(kBlock), 0, st, B, H, m.d2, H, m.g + m.o_b2);
-  gemm(B, H, H, m.d2, H, 0, m.p + m.o_w2, H, 1, nullptr, m.d1, H, st);
-  hipLaunchKernelGGL(k_gelu_bwd, dim3(blocks(ns * H)), dim3(kBlock), 0, st, ns * H, m.z1, m.d1);
-  gemm(di, H, B, m.x, di, 1, m.d1, H, 0, nullptr, m.g + m.o_w1, H, st);
-  hipLaunchKernelGGL(k_colsum, dim3(blocks(H)), dim3(kBlock), 0, st, B, H, m.d1, H, m.g + m.o_b1);
+  gemm<true, kEpiGeluBwd>(B, H, dout, m.d3, dout, m.p + m.o_w3, dout, nullptr, m.z2, m.d2, H, st);
+  gemm<true, kEpiGeluBwd>(B, H, H, m.d2, H, m.p + m.o_w2, H, nullptr, m.z1, m.d1, H, st);
+  // weight and bias gradients: chunks of at least 4 slabs of samples, at most kGradSplits of them
+  const int64_t chunk = std::max<int64_t>(4 * kGemmSlab, ceil_div(ceil_div(ns, kGradSplits), kGemmSlab) * kGemmSlab);
+  const int nsplit = static_cast<int>(ceil_div(ns, chunk));
+  WGrads wg;
+  wg.g[0] = WGrad{m.x, m.d1, di, H, m.o_w1, m.o_b1, 0};
+  wg.g[1] = WGrad{m.a1, m.d2, H, H, m.o_w2, m.o_b2, 0};
+  wg.g[2] = WGrad{m.a2, m.d3, H, dout, m.o_w3, m.o_b3, 0};
+  wg.tiles = 0;
+  for (auto& g : wg.g) {
+    g.first = wg.tiles;
+    wg.tiles += static_cast<int>(ceil_div(g.M, kGemmTile) * ceil_div(g.N, kGemmTile));
+  }
+  hipLaunchKernelGGL(k_wgrad, dim3(static_cast<unsigned>(wg.tiles), static_cast<unsigned>(nsplit)), dim3(kBlock), 0, st,
+                     wg, ns, chunk, m.o_th, m.gpart);
+  hipLaunchKernelGGL(k_sum_splits, dim3(blocks(m.o_th)), dim3(kBlock), 0, st, m.o_th, m.o_th, nsplit, m.gpart, m.g);
   MLP_HIP(hipGetLastError());
   if (apply) {
     m.adam_t += 1;
     const float c1 = static_cast<float>(1.0 - std::pow(0.9, static_cast<double>(m.adam_t)));
     const float c2 = static_cast<float>(1.0 - std::pow(0.999, static_cast<double>(m.adam_t)));
-    hipLaunchKernelGGL(k_adam, dim3(blocks(m.o_th)), dim3(kBlock), 0, st, m.o_th, m.p, m.g, m.m, m.v,
-                       static_cast<float>(lr), c1, c2);
-    const int64_t na = m.nparams - m.o_th;
-    hipLaunchKernelGGL(k_adam, dim3(blocks(na)), dim3(kBlock), 0, st, na, m.p + m.o_th, m.g + m.o_th,
-                       m.m + m.o_th, m.v + m.o_th, static_cast<float>(lr * kAffLrScale), c1, c2);
+    hipLaunchKernelGGL(k_adam, dim3(blocks(m.nparams)), dim3(kBlock), 0, st, m.nparams, m.o_th, m.p, m.g, m.m, m.v,
+                       static_cast<float>(lr), static_cast<float>(lr * kAffLrScale), c1, c2);
     MLP_HIP(hipGetLastError());
     return mlp_refresh(m, st);
   }

@@ -24,6 +24,7 @@ namespace fqm {
 constexpr int kHidden = 256;
 constexpr float kClip = 60.0f;
 constexpr int kAffChunk = 512;        // samples per block of the affinity-gradient reduction
+constexpr int64_t kGradSplits = 32;   // most sample chunks of a weight-gradient product
 constexpr double kAffLrScale = 10.0;  // Adam step of theta relative to the network's
 
 struct Mlp {
@@ -57,6 +58,7 @@ struct Mlp {
   float* dth = nullptr;       // [bcap][2][nb]: per-sample gradients of the affinity rows of holes i, j
   float* aff_part = nullptr;  // [nchunk][nb][nb]: chunk sums of dth
   int nchunk = 0;
+  float* gpart = nullptr;     // [kGradSplits][o_th]: weight-gradient sums of the sample chunks
   uint64_t* sdet = nullptr;  // [W][bcap]
   int32_t* sexc = nullptr;   // [bcap][4]: i, j, a, b (i<j, a<b)
   double* sw = nullptr;      // sample weights
