@@ -369,14 +369,17 @@ __global__ void k_sum_splits(int64_t n, int64_t stride, int nsplit, const float*
   const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (t < n) g[t] = sum_splits(part, t, stride, nsplit);
 }
-// Fixed-order sum of n doubles on one block.
-__global__ void k_dsum(int64_t n, const double* __restrict__ x, double* __restrict__ out) {
-  __shared__ double sh[kBlock];
+// Fixed-order sum of n doubles on one block (kSumBlock threads: 16384 values
+// are 16 loads a thread, all in flight; 16.6 us with 256 threads, 4.7 now).
+constexpr int kSumBlock = 1024;
+__global__ __launch_bounds__(kSumBlock) void k_dsum(int64_t n, const double* __restrict__ x, double* __restrict__ out) {
+  __shared__ double sh[kSumBlock];
   double acc = 0.0;
-  for (int64_t i = threadIdx.x; i < n; i += kBlock) acc = acc + x[i];
+#pragma unroll 8
+  for (int64_t i = threadIdx.x; i < n; i += kSumBlock) acc = acc + x[i];
   sh[threadIdx.x] = acc;
   __syncthreads();
-  for (int k = kBlock / 2; k > 0; k >>= 1) {
+  for (int k = kSumBlock / 2; k > 0; k >>= 1) {
     if (threadIdx.x < k) sh[threadIdx.x] = sh[threadIdx.x] + sh[threadIdx.x + k];
     __syncthreads();
   }
@@ -385,190 +388,296 @@ __global__ void k_dsum(int64_t n, const double* __restrict__ x, double* __restri
 
 // Weighted NLL of each sample's double under the network distribution and its
 // gradient with respect to the logits (d3) and to the affinity rows of the
-// sample's two holes (dth: row i then row j, nb each), one thread per sample.
+// sample's two holes (dth: row i then row j, nb each), one wavefront per sample.
 // The network component sums four paths (h1, h2, p1, p2): the first particle
 // p1 is drawn with h1's affinity over the unoccupied orbitals (normaliser
 // Z1(h1)), its partner p2 with h2's affinity over p1's partner class (Z2).
 // A sample flagged flat (sflat, may be null) is scored as a determinant the
 // network does not run on: hole and particle weights 1 (logits 0), so only the
 // affinity receives its gradient.
-__global__ void k_mlp_loss_grad(fqd::Sys s, int64_t ns, int nb, int d_out, const uint64_t* __restrict__ sdet,
-                                int64_t bcap, const int32_t* __restrict__ sexc, const double* __restrict__ sw,
-                                const int32_t* __restrict__ sflat, const double* __restrict__ wsum,
-                                const float* __restrict__ z3, const float* __restrict__ th, float* __restrict__ d3,
-                                float* __restrict__ dth, double* __restrict__ sloss, const double* __restrict__ sh,
-                                int variance) {
-  const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t >= ns) return;
+// Lane l holds orbitals l + 1 and l + 65 (nbasis <= 128): the rows of logits
+// and affinities are read and the gradients written coalesced, each exponential
+// is evaluated once, and 16384 samples are 16384 wavefronts.  (One thread per
+// sample walked its rows twice at one wavefront per CU: 190 -> 21 us at 16384
+// samples and nbasis 80, 142 -> 13 us at 4096 and 52.)
+constexpr int kLossOrbs = 2;  // orbitals per lane
+__device__ __forceinline__ double wave_dsum(double x) {
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) x = x + __shfl_xor(x, d, 64);
+  return x;
+}
+__global__ __launch_bounds__(kBlock) void k_mlp_loss_grad(
+    fqd::Sys s, int64_t ns, int nb, int d_out, const uint64_t* __restrict__ sdet, int64_t bcap,
+    const int32_t* __restrict__ sexc, const double* __restrict__ sw, const int32_t* __restrict__ sflat,
+    const double* __restrict__ wsum, const float* __restrict__ z3, const float* __restrict__ th,
+    float* __restrict__ d3, float* __restrict__ dth, double* __restrict__ sloss, const double* __restrict__ sh,
+    int variance) {
+  const int lane = threadIdx.x & 63;
+  const int64_t t = static_cast<int64_t>(blockIdx.x) * (kBlock / 64) + (threadIdx.x >> 6);
+  if (t >= ns) return;  // whole wavefront
   const float* z = z3 + t * d_out;
   float* d = d3 + t * d_out;
   float* gth = dth + t * 2 * nb;
-  const double wt = sw[t] / *wsum;
   if (!(sw[t] > 0.0)) {
-    for (int c = 0; c < d_out; ++c) d[c] = 0.0f;
-    for (int c = 0; c < 2 * nb; ++c) gth[c] = 0.0f;
-    sloss[t] = 0.0;
+    for (int c = lane; c < d_out; c += 64) d[c] = 0.0f;
+    for (int c = lane; c < 2 * nb; c += 64) gth[c] = 0.0f;
+    if (lane == 0) sloss[t] = 0.0;
     return;
   }
+  const double wt = sw[t] / *wsum;
   uint64_t f[FQ_MAX_WORDS] = {0, 0};
   for (int w = 0; w < s.W; ++w) f[w] = sdet[static_cast<int64_t>(w) * bcap + t];
   const int i = sexc[4 * t], j = sexc[4 * t + 1], a = sexc[4 * t + 2], b = sexc[4 * t + 3];
   const bool flat = sflat && sflat[t];
-  auto ew = [&](int o) { return flat ? 1.0 : exp(static_cast<double>(fminf(fmaxf(z[o - 1], -kClip), kClip))); };
-  auto fw = [&](int o) { return flat ? 1.0 : exp(static_cast<double>(fminf(fmaxf(z[nb + o - 1], -kClip), kClip))); };
-  auto aff = [&](int hole, int o) {
-    return exp(static_cast<double>(fminf(fmaxf(th[(hole - 1) * nb + o - 1], -kClip), kClip)));
-  };
+  auto clip = [](float x) { return static_cast<double>(fminf(fmaxf(x, -kClip), kClip)); };
   const fqd::PartnerClass cb = fqd::partner_class(s, i, j, a), ca = fqd::partner_class(s, i, j, b);
   auto in_class = [&](const fqd::PartnerClass& c, int o, int x) {
-    return c.ok && o != x && !fqd::btest(f, o) && fqd::ims_of(o) == c.ims && s.orb_sym[o - 1] == c.sym;
+    return c.ok && o != x && fqd::ims_of(o) == c.ims && s.orb_sym[o - 1] == c.sym;
   };
+  // e: hole weight of an occupied orbital; wi, wj: f_o A[i][o], f_o A[j][o] of an unoccupied one
+  double e[kLossOrbs], wi[kLossOrbs], wj[kLossOrbs];
+  float zh_[kLossOrbs], zp_[kLossOrbs], ti[kLossOrbs], tj[kLossOrbs];
+  bool occ[kLossOrbs], inb[kLossOrbs], ina[kLossOrbs];
   // Z1(i), Z1(j); Z2 of holes i, j over b's class given a first (zbi, zbj) and a's given b (zai, zaj)
   double zh = 0.0, z1i = 0.0, z1j = 0.0, zbi = 0.0, zbj = 0.0, zai = 0.0, zaj = 0.0;
-  for (int o = 1; o <= nb; ++o) {
-    if (fqd::btest(f, o)) {
-      zh = zh + ew(o);
-    } else {
-      const double v = fw(o), wi = v * aff(i, o), wj = v * aff(j, o);
-      z1i = z1i + wi;
-      z1j = z1j + wj;
-      if (in_class(cb, o, a)) {
-        zbi = zbi + wi;
-        zbj = zbj + wj;
-      }
-      if (in_class(ca, o, b)) {
-        zai = zai + wi;
-        zaj = zaj + wj;
+#pragma unroll
+  for (int k = 0; k < kLossOrbs; ++k) {
+    const int o = lane + 1 + 64 * k;
+    e[k] = wi[k] = wj[k] = 0.0;
+    zh_[k] = zp_[k] = ti[k] = tj[k] = 0.0f;
+    occ[k] = inb[k] = ina[k] = false;
+    if (o <= nb) {
+      zh_[k] = z[o - 1];
+      zp_[k] = z[nb + o - 1];
+      ti[k] = th[(i - 1) * nb + o - 1];
+      tj[k] = th[(j - 1) * nb + o - 1];
+      occ[k] = (f[k] >> lane) & 1;
+      if (occ[k]) {
+        e[k] = flat ? 1.0 : exp(clip(zh_[k]));
+      } else {
+        const double v = flat ? 1.0 : exp(clip(zp_[k]));
+        wi[k] = v * exp(clip(ti[k]));
+        wj[k] = v * exp(clip(tj[k]));
+        inb[k] = in_class(cb, o, a);
+        ina[k] = in_class(ca, o, b);
       }
     }
+    zh = zh + e[k];
+    z1i = z1i + wi[k];
+    z1j = z1j + wj[k];
+    zbi = zbi + (inb[k] ? wi[k] : 0.0);
+    zbj = zbj + (inb[k] ? wj[k] : 0.0);
+    zai = zai + (ina[k] ? wi[k] : 0.0);
+    zaj = zaj + (ina[k] ? wj[k] : 0.0);
   }
-  const double ei = ew(i), ej = ew(j), fa = fw(a), fb = fw(b);
-  const double aia = aff(i, a), aib = aff(i, b), aja = aff(j, a), ajb = aff(j, b);
+  zh = wave_dsum(zh);
+  z1i = wave_dsum(z1i);
+  z1j = wave_dsum(z1j);
+  zbi = wave_dsum(zbi);
+  zbj = wave_dsum(zbj);
+  zai = wave_dsum(zai);
+  zaj = wave_dsum(zaj);
+  static_assert(kLossOrbs == 2, "an orbital's value is in one of two registers");
+  auto at = [](const double(&v)[kLossOrbs], int o) { return __shfl(o > 64 ? v[1] : v[0], (o - 1) & 63, 64); };
+  const double ei = at(e, i), ej = at(e, j);
+  const double wia = at(wi, a), wib = at(wi, b), wja = at(wj, a), wjb = at(wj, b);
   const double pij = ei / zh * ej / (zh - ei), pji = ej / zh * ei / (zh - ej);
-  const double t1 = pij * (fa * aia / z1i) * (fb * ajb / zbj);  // (i, j, a, b)
-  const double t2 = pij * (fb * aib / z1i) * (fa * aja / zaj);  // (i, j, b, a)
-  const double t3 = pji * (fa * aja / z1j) * (fb * aib / zbi);  // (j, i, a, b)
-  const double t4 = pji * (fb * ajb / z1j) * (fa * aia / zai);  // (j, i, b, a)
+  const double t1 = pij * (wia / z1i) * (wjb / zbj);  // (i, j, a, b)
+  const double t2 = pij * (wib / z1i) * (wja / zaj);  // (i, j, b, a)
+  const double t3 = pji * (wja / z1j) * (wib / zbi);  // (j, i, a, b)
+  const double t4 = pji * (wjb / z1j) * (wia / zai);  // (j, i, b, a)
   const double q = t1 + t2 + t3 + t4;
   const double r1 = t1 / q, r2 = t2 / q, r3 = t3 / q, r4 = t4 / q;
   // the sample's loss and the factor of its -log q gradient: the NLL weighted
   // by wt, or the spawning-variance term wt |H| / q, whose gradient is the NLL
   // gradient weighted by that term
   const double c = variance ? wt * sh[t] / q : wt;
-  sloss[t] = variance ? c : wt * -log(q);
-  for (int o = 1; o <= nb; ++o) {
+  if (lane == 0) sloss[t] = variance ? c : wt * -log(q);
+#pragma unroll
+  for (int k = 0; k < kLossOrbs; ++k) {
+    const int o = lane + 1 + 64 * k;
+    if (o > nb) continue;
     double gu = 0.0, gi = 0.0, gj = 0.0;
-    if (fqd::btest(f, o)) {
-      const double e = ew(o);
-      double gij = -e / zh - (o != i ? e / (zh - ei) : 0.0);
-      double gji = -e / zh - (o != j ? e / (zh - ej) : 0.0);
+    if (occ[k]) {
+      double gij = -e[k] / zh - (o != i ? e[k] / (zh - ei) : 0.0);
+      double gji = -e[k] / zh - (o != j ? e[k] / (zh - ej) : 0.0);
       if (o == i || o == j) {
         gij += 1.0;
         gji += 1.0;
       }
       gu = (r1 + r2) * gij + (r3 + r4) * gji;
     } else {
-      const double v = fw(o), wi = v * aff(i, o), wj = v * aff(j, o);
       const double da = o == a ? 1.0 : 0.0, db = o == b ? 1.0 : 0.0;
-      const bool inb = in_class(cb, o, a), ina = in_class(ca, o, b);
-      gi = r1 * (da - wi / z1i) + r2 * (db - wi / z1i) + r3 * (db - (inb ? wi / zbi : 0.0)) +
-           r4 * (da - (ina ? wi / zai : 0.0));
-      gj = r1 * (db - (inb ? wj / zbj : 0.0)) + r2 * (da - (ina ? wj / zaj : 0.0)) + r3 * (da - wj / z1j) +
-           r4 * (db - wj / z1j);
+      gi = r1 * (da - wi[k] / z1i) + r2 * (db - wi[k] / z1i) + r3 * (db - (inb[k] ? wi[k] / zbi : 0.0)) +
+           r4 * (da - (ina[k] ? wi[k] / zai : 0.0));
+      gj = r1 * (db - (inb[k] ? wj[k] / zbj : 0.0)) + r2 * (da - (ina[k] ? wj[k] / zaj : 0.0)) +
+           r3 * (da - wj[k] / z1j) + r4 * (db - wj[k] / z1j);
     }
-    const bool in_h = !flat && fabsf(z[o - 1]) < kClip, in_p = !flat && fabsf(z[nb + o - 1]) < kClip;
+    const bool in_h = !flat && fabsf(zh_[k]) < kClip, in_p = !flat && fabsf(zp_[k]) < kClip;
     d[o - 1] = in_h ? static_cast<float>(-c * gu) : 0.0f;
     d[nb + o - 1] = in_p ? static_cast<float>(-c * (gi + gj)) : 0.0f;
-    gth[o - 1] = fabsf(th[(i - 1) * nb + o - 1]) < kClip ? static_cast<float>(-c * gi) : 0.0f;
-    gth[nb + o - 1] = fabsf(th[(j - 1) * nb + o - 1]) < kClip ? static_cast<float>(-c * gj) : 0.0f;
+    gth[o - 1] = fabsf(ti[k]) < kClip ? static_cast<float>(-c * gi) : 0.0f;
+    gth[nb + o - 1] = fabsf(tj[k]) < kClip ? static_cast<float>(-c * gj) : 0.0f;
   }
-  for (int k = 2 * nb; k < d_out; ++k) d[k] = 0.0f;
+  for (int k = 2 * nb + lane; k < d_out; k += 64) d[k] = 0.0f;
 }
 
-// Affinity gradient, deterministic: block (h, c) sums, in sample order, the
-// row gradients of the samples [c*chunk, (c+1)*chunk) whose hole i or j is
-// h + 1 into part[c][h][.]; k_aff_grad_sum adds the chunks in order.
-__global__ void k_aff_grad_part(int64_t ns, int nb, int64_t chunk, const int32_t* __restrict__ sexc,
-                                const double* __restrict__ sw, const float* __restrict__ dth,
-                                float* __restrict__ part) {
-  const int h = blockIdx.x + 1, c = blockIdx.y, o = threadIdx.x;
-  if (o >= nb) return;
-  const int64_t s0 = c * chunk, s1 = s0 + chunk < ns ? s0 + chunk : ns;
-  float acc = 0.0f;
-  for (int64_t t = s0; t < s1; ++t) {
-    if (!(sw[t] > 0.0)) continue;
-    if (sexc[4 * t] == h) acc += dth[t * 2 * nb + o];
-    if (sexc[4 * t + 1] == h) acc += dth[t * 2 * nb + nb + o];
-  }
-  part[(static_cast<int64_t>(c) * nb + (h - 1)) * nb + o] = acc;
-}
-
-__global__ void k_aff_grad_sum(int nb, int nchunk, const float* __restrict__ part, float* __restrict__ g) {
-  const int64_t k = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int64_t n = static_cast<int64_t>(nb) * nb;
-  if (k >= n) return;
-  float acc = 0.0f;
-  for (int c = 0; c < nchunk; ++c) acc += part[c * n + k];
-  g[k] = acc;
-}
-
-// Row sums of the stored affinity (one thread per hole h, orbital order) and
-// per spin/irrep class (members in the class table's order); thread 0 also
-// writes the class bit masks.
-__global__ void k_aff_sums(int nb, const float* __restrict__ aff, const int* __restrict__ nbss,
-                           const int* __restrict__ ssbf, int nsym_pg, int max_sym_spin, double* __restrict__ rs,
-                           double* __restrict__ crs, uint64_t* __restrict__ cmask) {
-  const int h = static_cast<int>(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int ncls = 2 * nsym_pg;
-  if (h == 0)
-    for (int c = 0; c < ncls; ++c) {
-      uint64_t mw[FQ_MAX_WORDS] = {0, 0};
-      for (int k = 0; k < nbss[c]; ++k) {
-        const int o = ssbf[c * max_sym_spin + k] - 1;
-        mw[o >> 6] |= uint64_t{1} << (o & 63);
+// Affinity gradient, deterministic: block c adds, in sample order, the row
+// gradients of the samples [c*chunk, (c+1)*chunk) to its copy of the table in
+// LDS (thread o owns column o of every row) and writes it to part[c];
+// k_aff_grad_sum adds the chunks in order.  Each sample's rows are read once,
+// eight samples' loads in flight.  (A block per (hole, chunk) read every sample
+// once per hole: 80 -> 18 us at 16384 samples and nbasis 80, 102 -> 22 us at
+// 4096 and 52.)
+constexpr int kAffAhead = 8;
+__global__ __launch_bounds__(kHidden / 2) void k_aff_grad_part(int64_t ns, int nb, int64_t chunk,
+                                                               const int32_t* __restrict__ sexc,
+                                                               const double* __restrict__ sw,
+                                                               const float* __restrict__ dth,
+                                                               float* __restrict__ part) {
+  extern __shared__ float tab[];  // nb x nb
+  const int o = threadIdx.x;
+  const int64_t s0 = blockIdx.x * chunk, s1 = s0 + chunk < ns ? s0 + chunk : ns;
+  if (o < nb) {  // no barrier: a thread touches its own column only
+    for (int h = 0; h < nb; ++h) tab[h * nb + o] = 0.0f;
+    for (int64_t t0 = s0; t0 < s1; t0 += kAffAhead) {
+      int hi[kAffAhead], hj[kAffAhead];  // 0: sample not used
+      float gi[kAffAhead], gj[kAffAhead];
+#pragma unroll
+      for (int u = 0; u < kAffAhead; ++u) {
+        const int64_t t = t0 + u < s1 ? t0 + u : s1 - 1;
+        const bool use = t0 + u < s1 && sw[t] > 0.0;
+        hi[u] = use ? sexc[4 * t] : 0;
+        hj[u] = use ? sexc[4 * t + 1] : 0;
+        gi[u] = dth[t * 2 * nb + o];
+        gj[u] = dth[t * 2 * nb + nb + o];
       }
-      for (int w = 0; w < FQ_MAX_WORDS; ++w) cmask[c * FQ_MAX_WORDS + w] = mw[w];
+#pragma unroll
+      for (int u = 0; u < kAffAhead; ++u) {
+        if (hi[u]) {
+          tab[(hi[u] - 1) * nb + o] += gi[u];
+          tab[(hj[u] - 1) * nb + o] += gj[u];
+        }
+      }
     }
-  if (h >= nb) return;
-  const float* row = aff + static_cast<int64_t>(h) * nb;
-  double z = 0.0;
-  for (int p = 0; p < nb; ++p) z = z + static_cast<double>(row[p]);
-  rs[h] = z;
-  for (int c = 0; c < ncls; ++c) {
-    double zc = 0.0;
-    for (int k = 0; k < nbss[c]; ++k) zc = zc + static_cast<double>(row[ssbf[c * max_sym_spin + k] - 1]);
-    crs[h * ncls + c] = zc;
+    float* out = part + static_cast<int64_t>(blockIdx.x) * nb * nb;
+    for (int h = 0; h < nb; ++h) out[h * nb + o] = tab[h * nb + o];
   }
 }
 
-// Alias tables of the affinity rows (one thread per (hole, table): table 0 the
-// whole row, table 1 + c class c's members), after k_aff_sums.
-__global__ void k_aff_alias(int nb, const float* __restrict__ aff, const int* __restrict__ nbss,
-                            const int* __restrict__ ssbf, int nsym_pg, int max_sym_spin,
-                            const double* __restrict__ rs, const double* __restrict__ crs, double* __restrict__ au,
-                            int* __restrict__ ak, double* __restrict__ cu, int* __restrict__ ck) {
-  const int ncls = 2 * nsym_pg;
-  const int t = static_cast<int>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t >= nb * (1 + ncls)) return;
-  const int h = t / (1 + ncls), c = t % (1 + ncls) - 1;
-  const float* row = aff + static_cast<int64_t>(h) * nb;
-  double w[128];
-  if (c < 0) {
-    for (int p = 0; p < nb; ++p) w[p] = static_cast<double>(row[p]);
-    fqd::build_alias(nb, w, rs[h], au + static_cast<int64_t>(h) * nb, ak + static_cast<int64_t>(h) * nb);
-  } else {
-    const int n = nbss[c];
-    if (n == 0) return;
-    for (int q = 0; q < n; ++q) w[q] = static_cast<double>(row[ssbf[c * max_sym_spin + q] - 1]);
-    const int64_t o = (static_cast<int64_t>(h) * ncls + c) * max_sym_spin;
-    fqd::build_alias(n, w, crs[h * ncls + c], cu + o, ck + o);
+// 64 elements a block, its four wavefronts each adding a quarter of the chunks in order.
+__global__ __launch_bounds__(kBlock) void k_aff_grad_sum(int nb, int nchunk, const float* __restrict__ part,
+                                                         float* __restrict__ g) {
+  __shared__ float sh[kBlock];
+  const int64_t n = static_cast<int64_t>(nb) * nb;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t k = static_cast<int64_t>(blockIdx.x) * 64 + lane;
+  const int per = (nchunk + 3) / 4, c0 = wave * per, c1 = c0 + per < nchunk ? c0 + per : nchunk;
+  float acc = 0.0f;
+  if (k < n) {
+#pragma unroll 8
+    for (int c = c0; c < c1; ++c) acc += part[c * n + k];
   }
+  sh[threadIdx.x] = acc;
+  __syncthreads();
+  if (wave == 0 && k < n) g[k] = (sh[lane] + sh[64 + lane]) + (sh[128 + lane] + sh[192 + lane]);
 }
 
-// The stored affinity table: exp(clamp(theta, -60, 60)) rounded to float.
-__global__ void k_aff_table(int64_t n, const float* __restrict__ th, float* __restrict__ aff) {
-  const int64_t k = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (k < n) aff[k] = static_cast<float>(exp(static_cast<double>(fminf(fmaxf(th[k], -kClip), kClip))));
+// Everything the generator reads of the affinity, one wavefront per (hole h,
+// table): table 0 the whole row, table 1 + c the members of spin/irrep class c
+// (in the class table's order).  The stored affinity is exp(clamp(theta, -60,
+// 60)) rounded to float; its sums (rs, crs) are taken in row or member order,
+// and the alias tables repeat generate_alias_tables' steps (fqd::build_alias)
+// with the weights and its two stacks in LDS and the current top of "over" in
+// a register.  Block 0 also writes the class bit masks.  (Table, sums and alias
+// tables as three kernels, one thread per row or table with the stacks in
+// scratch memory, took 142 us at nbasis 80; this takes 17.)
+constexpr int kMaxAlias = 128;
+__global__ __launch_bounds__(64) void k_aff_tables(int nb, const float* __restrict__ th, float* __restrict__ aff,
+                                                   const int* __restrict__ nbss, const int* __restrict__ ssbf,
+                                                   int nsym_pg, int max_sym_spin, double* __restrict__ rs,
+                                                   double* __restrict__ crs, uint64_t* __restrict__ cmask,
+                                                   double* __restrict__ au, int* __restrict__ ak,
+                                                   double* __restrict__ cu, int* __restrict__ ck) {
+  __shared__ double u[kMaxAlias];
+  __shared__ int alias[kMaxAlias];
+  __shared__ uint8_t under[kMaxAlias], over[kMaxAlias];
+  const int ncls = 2 * nsym_pg, lane = threadIdx.x;
+  const int h = blockIdx.x / (1 + ncls), c = blockIdx.x % (1 + ncls) - 1;
+  if (blockIdx.x == 0 && lane < ncls) {
+    uint64_t mw[FQ_MAX_WORDS] = {0, 0};
+    for (int k = 0; k < nbss[lane]; ++k) {
+      const int o = ssbf[lane * max_sym_spin + k] - 1;
+      if (o < 64)
+        mw[0] |= uint64_t{1} << o;
+      else
+        mw[1] |= uint64_t{1} << (o - 64);
+    }
+    for (int w = 0; w < FQ_MAX_WORDS; ++w) cmask[lane * FQ_MAX_WORDS + w] = mw[w];
+  }
+  const int n = c < 0 ? nb : nbss[c];
+  for (int q = lane; q < n; q += 64) {
+    const int o = c < 0 ? q : ssbf[c * max_sym_spin + q] - 1;
+    const float a = static_cast<float>(exp(static_cast<double>(fminf(fmaxf(th[h * nb + o], -kClip), kClip))));
+    u[q] = static_cast<double>(a);
+    if (c < 0) aff[h * nb + q] = a;
+  }
+  __syncthreads();
+  double tot = 0.0;
+  for (int q = 0; q < n; ++q) tot = tot + u[q];
+  if (lane == 0) {
+    if (c < 0)
+      rs[h] = tot;
+    else
+      crs[h * ncls + c] = tot;
+  }
+  if (n == 0) return;  // whole block
+  __syncthreads();
+  const double scale = static_cast<double>(n) / tot;
+  int nunder = 0, nover = 0;  // the same in every lane
+  for (int q0 = 0; q0 < n; q0 += 64) {
+    const int q = q0 + lane;
+    bool lo = false;
+    if (q < n) {
+      u[q] = u[q] * scale;
+      lo = u[q] <= 1.0;
+      alias[q] = q + 1;
+    }
+    const unsigned long long bl = __ballot(q < n && lo), bh = __ballot(q < n && !lo), below = (1ull << lane) - 1;
+    if (q < n) {
+      if (lo)
+        under[nunder + __popcll(bl & below)] = static_cast<uint8_t>(q + 1);
+      else
+        over[nover + __popcll(bh & below)] = static_cast<uint8_t>(q + 1);
+    }
+    nunder += __popcll(bl);
+    nover += __popcll(bh);
+  }
+  __syncthreads();
+  if (lane == 0 && nover > 0) {
+    int ov = over[nover - 1];
+    double uo = u[ov - 1];
+    while (nover > 0 && nunder > 0) {
+      const int un = under[--nunder];
+      alias[un - 1] = ov;
+      uo = uo - (1.0 - u[un - 1]);
+      if (uo < 1.0) {
+        u[ov - 1] = uo;
+        under[nunder++] = static_cast<uint8_t>(ov);
+        if (--nover > 0) {
+          ov = over[nover - 1];
+          uo = u[ov - 1];
+        }
+      }
+    }
+    if (nover > 0) u[ov - 1] = uo;
+  }
+  __syncthreads();
+  const int64_t o0 = c < 0 ? static_cast<int64_t>(h) * nb : (static_cast<int64_t>(h) * ncls + c) * max_sym_spin;
+  for (int q = lane; q < n; q += 64) {
+    (c < 0 ? au : cu)[o0 + q] = u[q];
+    (c < 0 ? ak : ck)[o0 + q] = alias[q];
+  }
 }
 
 // Adam over all parameters; those from o_th on (the affinity) with their own rate.
@@ -601,12 +710,17 @@ __global__ void k_det_weight(int64_t n, int64_t cap, int S, const int64_t* __res
 
 // One heat-bath training sample per thread; its determinant is flagged flat
 // when even rounded up it makes fewer than min_att attempts (the network does
-// not run on it in production).
-__global__ void k_hb_sample(fqd::Sys s, const uint64_t* __restrict__ det, int64_t cap, int64_t n,
+// not run on it in production).  Blocks of one wavefront, the generator's nel
+// on-the-fly weights in a column of LDS each: 16384 samples are one wavefront
+// per CU, so the chain of dependent reads (the search of the list, the tables)
+// sets the time: 60 us, 82 with the weights in scratch memory.
+constexpr int kSampleBlock = 64;
+__global__ __launch_bounds__(kSampleBlock) void k_hb_sample(fqd::Sys s, const uint64_t* __restrict__ det, int64_t cap, int64_t n,
                             const int64_t* __restrict__ cum, const int64_t* __restrict__ dw, int64_t min_att,
                             int64_t ns, uint64_t seed, uint32_t step, uint64_t* __restrict__ sdet, int64_t bcap,
                             int32_t* __restrict__ sexc, double* __restrict__ sw, int32_t* __restrict__ sflat,
                             double* __restrict__ sh) {
+  extern __shared__ double hb_lds[];
   const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (t >= ns) return;
   fqd::Philox rng(seed, static_cast<uint32_t>(t), static_cast<uint32_t>(t >> 32), step ^ (fqd::kDrawTrain << 24));
@@ -624,8 +738,7 @@ __global__ void k_hb_sample(fqd::Sys s, const uint64_t* __restrict__ det, int64_
   FQ_FOR_WORDS(w, s.W) f[w] = det[static_cast<int64_t>(w) * cap + lo];
   fqd::Excit conn;
   double h = 0.0, pgen = 1.0;
-  double wloc[fqd::kHbMaxNel];
-  fqd::gen_heat_bath(s, rng, f, conn, h, pgen, fqd::HbBuf{wloc, 1});
+  fqd::gen_heat_bath(s, rng, f, conn, h, pgen, fqd::HbBuf{hb_lds + threadIdx.x, kSampleBlock});
   FQ_FOR_WORDS(w, s.W) sdet[static_cast<int64_t>(w) * bcap + t] = f[w];
   const bool use = conn.nexcit == 2 && h != 0.0;
   sexc[4 * t] = conn.from[0];
@@ -765,15 +878,10 @@ int mlp_refresh(Mlp& m, hipStream_t st) {
                         static_cast<int64_t>(m.n3) * kHidden;
   hipLaunchKernelGGL(k_mlp_pack, dim3(blocks(total)), dim3(kBlock), 0, st, m.d_in, m.k1, m.d_out, m.n3, m.p, m.o_w1,
                      m.o_w2, m.o_w3, m.w1t, m.w2t, m.w3t);
-  const int64_t na = static_cast<int64_t>(m.nb) * m.nb;
-  hipLaunchKernelGGL(k_aff_table, dim3(blocks(na)), dim3(kBlock), 0, st, na, m.p + m.o_th, m.aff);
-  if (m.nbss) {
-    hipLaunchKernelGGL(k_aff_sums, dim3(blocks(m.nb)), dim3(kBlock), 0, st, m.nb, m.aff, m.nbss, m.ssbf, m.nsym_pg,
-                       m.max_sym_spin, m.rs, m.crs, m.cmask);
-    const int ntab = m.nb * (1 + 2 * m.nsym_pg);
-    hipLaunchKernelGGL(k_aff_alias, dim3(blocks(ntab)), dim3(kBlock), 0, st, m.nb, m.aff, m.nbss, m.ssbf,
-                       m.nsym_pg, m.max_sym_spin, m.rs, m.crs, m.au, m.ak, m.cu, m.ck);
-  }
+  if (m.nbss)
+    hipLaunchKernelGGL(k_aff_tables, dim3(static_cast<unsigned>(m.nb * (1 + 2 * m.nsym_pg))), dim3(64), 0, st, m.nb,
+                       m.p + m.o_th, m.aff, m.nbss, m.ssbf, m.nsym_pg, m.max_sym_spin, m.rs, m.crs, m.cmask, m.au,
+                       m.ak, m.cu, m.ck);
   MLP_HIP(hipGetLastError());
   return FQ_OK;
 }
@@ -837,17 +945,17 @@ int mlp_train_step(Mlp& m, const fqd::Sys& s, int64_t ns, double lr, bool apply,
   gemm<false, kEpiGelu>(B, H, di, m.x, di, m.p + m.o_w1, H, m.p + m.o_b1, m.z1, m.a1, H, st);
   gemm<false, kEpiGelu>(B, H, H, m.a1, H, m.p + m.o_w2, H, m.p + m.o_b2, m.z2, m.a2, H, st);
   gemm<false, kEpiBias>(B, dout, H, m.a2, H, m.p + m.o_w3, dout, m.p + m.o_b3, nullptr, m.z3, dout, st);
-  hipLaunchKernelGGL(k_dsum, dim3(1), dim3(kBlock), 0, st, ns, m.sw, m.dsum);
-  hipLaunchKernelGGL(k_mlp_loss_grad, dim3(blocks(ns)), dim3(kBlock), 0, st, s, ns, m.nb, dout, m.sdet, m.bcap,
+  hipLaunchKernelGGL(k_dsum, dim3(1), dim3(kSumBlock), 0, st, ns, m.sw, m.dsum);
+  hipLaunchKernelGGL(k_mlp_loss_grad, dim3(blocks(ns * 64)), dim3(kBlock), 0, st, s, ns, m.nb, dout, m.sdet, m.bcap,
                      m.sexc, m.sw, m.sflat, m.dsum, m.z3, m.p + m.o_th, m.d3, m.dth, m.sloss, m.sh, m.objective);
-  hipLaunchKernelGGL(k_dsum, dim3(1), dim3(kBlock), 0, st, ns, m.sloss, m.dsum + 1);
+  hipLaunchKernelGGL(k_dsum, dim3(1), dim3(kSumBlock), 0, st, ns, m.sloss, m.dsum + 1);
   const int nchunk = static_cast<int>(ceil_div(ns, kAffChunk));
-  hipLaunchKernelGGL(k_aff_grad_part, dim3(static_cast<unsigned>(m.nb), static_cast<unsigned>(nchunk)),
-                     dim3(kHidden / 2), 0, st, ns, m.nb, static_cast<int64_t>(kAffChunk), m.sexc, m.sw, m.dth,
-                     m.aff_part);
   const int64_t na = static_cast<int64_t>(m.nb) * m.nb;
-  hipLaunchKernelGGL(k_aff_grad_sum, dim3(blocks(na)), dim3(kBlock), 0, st, m.nb, nchunk, m.aff_part,
-                     m.g + m.o_th);
+  hipLaunchKernelGGL(k_aff_grad_part, dim3(static_cast<unsigned>(nchunk)), dim3(kHidden / 2),
+                     sizeof(float) * static_cast<size_t>(na), st, ns, m.nb, static_cast<int64_t>(kAffChunk), m.sexc,
+                     m.sw, m.dth, m.aff_part);
+  hipLaunchKernelGGL(k_aff_grad_sum, dim3(static_cast<unsigned>(ceil_div(na, 64))), dim3(kBlock), 0, st, m.nb, nchunk,
+                     m.aff_part, m.g + m.o_th);
   // backward
   gemm<true, kEpiGeluBwd>(B, H, dout, m.d3, dout, m.p + m.o_w3, dout, nullptr, m.z2, m.d2, H, st);
   gemm<true, kEpiGeluBwd>(B, H, H, m.d2, H, m.p + m.o_w2, H, nullptr, m.z1, m.d1, H, st);
@@ -896,7 +1004,8 @@ int mlp_sample(Mlp& m, const fqd::Sys& s, const uint64_t* det, const int64_t* po
   hipLaunchKernelGGL(k_det_weight, dim3(blocks(n)), dim3(kBlock), 0, st, n, cap, s.S, pop, shift, m.swts);
   int rc = scan(scan_ctx, m.swts, m.scum, n);
   if (rc != FQ_OK) return rc;
-  hipLaunchKernelGGL(k_hb_sample, dim3(blocks(ns)), dim3(kBlock), 0, st, s, det, cap, n, m.scum, m.swts, min_att,
+  hipLaunchKernelGGL(k_hb_sample, dim3(static_cast<unsigned>(ceil_div(ns, kSampleBlock))), dim3(kSampleBlock),
+                     sizeof(double) * static_cast<size_t>(s.nel) * kSampleBlock, st, s, det, cap, n, m.scum, m.swts, min_att,
                      ns, seed, step, m.sdet, m.bcap, m.sexc, m.sw, m.sflat, m.sh);
   MLP_HIP(hipGetLastError());
   return FQ_OK;

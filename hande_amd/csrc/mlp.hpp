@@ -23,7 +23,7 @@ namespace fqm {
 
 constexpr int kHidden = 256;
 constexpr float kClip = 60.0f;
-constexpr int kAffChunk = 512;        // samples per block of the affinity-gradient reduction
+constexpr int kAffChunk = 64;         // samples per block of the affinity-gradient reduction
 constexpr int64_t kGradSplits = 32;   // most sample chunks of a weight-gradient product
 constexpr double kAffLrScale = 10.0;  // Adam step of theta relative to the network's
 
