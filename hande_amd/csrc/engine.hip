@@ -2123,28 +2123,72 @@ __global__ __launch_bounds__(kBlock) void k_determ_fill(Sys s, int transp, const
   }
 }
 
-// Production deterministic projection, one thread per core determinant and
+// sum + a term of each stored element of row `row` in order, the terms being
+// scale * H * v (separate) or H * v (combined), by one wavefront: its lanes
+// evaluate 64 terms at a time (coalesced reads of the row, the next chunk's in
+// flight) and park them in LDS, and every lane then adds them in the row's
+// order, so the sum is the one thread's sum bit for bit.
+__device__ __forceinline__ double determ_row_sum(const DetermDev& dd, int S, int64_t row, int sp, double sum,
+                                                 bool scaled, double scale, int lane, double* __restrict__ term) {
+  const int64_t k0 = dd.row[row], k1 = dd.row[row + 1];
+  auto value = [&](int64_t k) {
+    if (k >= k1) return 0.0;
+    const double m = dd.mat[k], v = dd.vec[dd.col[k] * S + sp];
+    return scaled ? scale * m * v : m * v;
+  };
+  double next = value(k0 + lane);
+  for (int64_t k = k0; k < k1; k += 64) {
+    __builtin_amdgcn_wave_barrier();  // the previous chunk's reads come first (LDS is in order within a wavefront)
+    term[lane] = next;
+    __builtin_amdgcn_wave_barrier();
+    next = value(k + 64 + lane);
+    if (k1 - k >= 64) {
+#pragma unroll 16
+      for (int q = 0; q < 64; ++q) sum = sum + term[q];
+    } else {
+      for (int q = 0; q < static_cast<int>(k1 - k); ++q) sum = sum + term[q];
+    }
+  }
+  return sum;
+}
+
+// Production deterministic projection, one wavefront per core determinant and
 // space, each with its own draw keyed (row, space, cycle).  Combined
 // annihilation writes the encoded amplitude to the spawned list after the
 // stochastic spawns (key and payload, as an initiator's spawn; the count is
 // added by k_add_nspawn); separate annihilation adds it to the core
-// determinant's post-death population.
+// determinant's post-death population.  (One thread per row read its row
+// uncoalesced, one element per trip to memory: 239 us with a 1000-determinant
+// core of a 26-orbital molecule, 13 now.)
 __global__ __launch_bounds__(kBlock) void k_determ_proj(Sys s, KeyPlan kp, DetermDev dd, double tau, double sh0,
                                                         double sh1, double e0, double e1, uint64_t seed, uint32_t cyc,
                                                         int64_t cap, int64_t* __restrict__ pop_new,
                                                         uint64_t* __restrict__ keys, int64_t* __restrict__ pay,
                                                         int64_t scap, Stats* __restrict__ st) {
-  const int64_t t = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
-  if (t >= dd.nd * s.S) return;
+  __shared__ double term[kBlock / 64][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t t = static_cast<int64_t>(blockIdx.x) * (kBlock / 64) + wave;
+  if (t >= dd.nd * s.S) return;  // whole wavefront; no block barriers below
   const int64_t row = t / s.S;
   const int sp = static_cast<int>(t - row * s.S);
   const double shift = sp == 0 ? sh0 : sh1, eold = sp == 0 ? e0 : e1;
-  fqd::Philox rng(seed, static_cast<uint32_t>(row), static_cast<uint32_t>(sp) << 28, cyc ^ (fqd::kDrawDeterm << 24));
+  const double v = dd.vec[row * s.S + sp];
+  // the expressions of determ_separate and determ_combined
+  double amp;
   if (dd.separate) {
-    pop_new[sp * cap + dd.pos[row]] += fqd::stoch_encode(rng, determ_separate(dd, s.S, row, sp, tau, shift, eold), s.rf);
+    amp = determ_row_sum(dd, s.S, row, sp, -(tau * (eold * (1.0 - 1.0) - shift * 1.0)) * v, true, -1.0 * tau, lane,
+                         term[wave]);
+  } else {
+    const double out = determ_row_sum(dd, s.S, row, sp, 0.0, false, 0.0, lane, term[wave]);
+    amp = -tau * (out + (eold * (1.0 - 1.0) - 1.0 * shift) * v);
+  }
+  if (lane != 0) return;
+  fqd::Philox rng(seed, static_cast<uint32_t>(row), static_cast<uint32_t>(sp) << 28, cyc ^ (fqd::kDrawDeterm << 24));
+  const int64_t k = fqd::stoch_encode(rng, amp, s.rf);
+  if (dd.separate) {
+    pop_new[sp * cap + dd.pos[row]] += k;
     return;
   }
-  const int64_t k = fqd::stoch_encode(rng, determ_combined(dd, s.S, row, sp, tau, shift, eold), s.rf);
   const int64_t slot = st->nspawn + t;
   if (slot >= scap) {
     st->spawn_overflow = 1;
@@ -3768,7 +3812,7 @@ static int cycle_body(fq_engine* e, const double* shift, const double* eproj_old
     int64_t ndet_entries = 0;  // the deterministic projection's spawned entries (combined annihilation)
     if (e->ndeterm > 0) {
       const int64_t m = e->ndeterm * e->S;
-      hipLaunchKernelGGL(k_determ_proj, dim3(grid_for(m)), dim3(kBlock), 0, st, e->sys, key_plan(e), determ_dev(e),
+      hipLaunchKernelGGL(k_determ_proj, dim3(grid_for(m, kBlock / 64)), dim3(kBlock), 0, st, e->sys, key_plan(e), determ_dev(e),
                          tau, shift[0], sh1, eproj_old[0], e1, e->par.philox_seed, cyc, cap, e->pop_new,
                          e->kbuf[0], e->pbuf[0], e->scap, e->d_stats);
       if (!e->determ_separate) {
