@@ -14,7 +14,6 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kBlock = 256;
-constexpr int kInferRows = 64;  // determinants per inference block: 4 waves x 16 rows
 
 #define MLP_HIP(call)                                                                                   \
   do {                                                                                                  \
@@ -43,39 +42,51 @@ __device__ inline float gelu_g(float z) {
 }
 
 // ---- inference ---------------------------------------------------------------
-// Rows [row, row+16) of the block's tile times W (stored transposed [N][K]):
-// acc[t] is the 16x16 output tile t (v_mfma_f32_16x16x32_bf16: lane l feeds
-// A[row l%16][k 8(l/16)..+7] and B[k 8(l/16)..+7][col l%16] and holds
-// D[rows 4(l/16)..+3][col l%16]).  Each 32-wide slab of K of W is staged once
-// per block in LDS (slab: the activation buffer this layer does not use),
-// so the block's four waves share one read of the weights; every thread of
-// the block calls this.
-constexpr int kSlabLd = 40;  // slab row stride (bf16): 32 + 8 keeps 16-byte rows and spreads banks
-template <int NT>
-__device__ inline void mfma_rows16(const uint16_t* A, int lda, int K, const uint16_t* __restrict__ Wt, int ntiles,
-                                   f32x4 (&acc)[NT], int row, int kq, int cl, uint16_t* slab) {
+// A block takes 16 RT determinants through the three layers; its four wavefronts
+// split the output columns (column tile t of 16 to wavefront t % 4), so every
+// weight is read by one wavefront of the block, straight from L2 into the
+// operand registers of v_mfma_f32_16x16x32_bf16 (lane l feeds A[row l%16]
+// [k 8(l/16)..+7] and B[k 8(l/16)..+7][col l%16], the weights being stored
+// transposed, [N][K], and holds D[rows 4(l/16)..+3][col l%16]).  The
+// activations (bf16) sit in one LDS buffer that a layer reads, barrier,
+// overwrites; rows are 264 apart so that a fragment's 16 rows spread over the
+// banks.  Every output accumulates its K slabs in order, whatever RT, so both
+// instances give the same bits.  RT = 1 for lists of at most kFewRows, which
+// fill at most two blocks per CU and are bound by the latency of the weights;
+// RT = 4 reads them once per 64 rows.  (Staging every weight slab in LDS between
+// two barriers took 79 us for a list of a few determinants at nbasis 80; 20 us
+// now.  65536 determinants: 288 -> 117 us, 145 TFLOP/s.)
+constexpr int kActLd = kHidden + 8;
+constexpr int64_t kFewRows = 8192;
+constexpr int kColTiles = kHidden / 16 / 4;  // column tiles of a wavefront
+
+// acc[r][c]: rows 16 r.. times column tile 4 c + wave of the layer.
+template <int RT>
+__device__ __forceinline__ void layer_mfma(const uint16_t* act, int K, const uint16_t* __restrict__ Wt, int ntiles,
+                                           f32x4 (&acc)[RT][kColTiles], int wave, int lane) {
+  const int kq = (lane >> 4) * 8, cl = lane & 15;
 #pragma unroll
-  for (int t = 0; t < NT; ++t) acc[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  const int ncols = ntiles * 16;
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int c = 0; c < kColTiles; ++c) acc[r][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 8
   for (int k0 = 0; k0 < K; k0 += 32) {
-    for (int e = threadIdx.x; e < ncols * 4; e += blockDim.x) {  // 4 x 8 bf16 per row
-      const int n = e >> 2, part = (e & 3) * 8;
-      *reinterpret_cast<bf16x8*>(slab + n * kSlabLd + part) =
-          *reinterpret_cast<const bf16x8*>(Wt + static_cast<int64_t>(n) * K + k0 + part);
-    }
-    __syncthreads();
-    const bf16x8 a = *reinterpret_cast<const bf16x8*>(A + row * lda + k0 + kq);
+    bf16x8 b[kColTiles];
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      if (t < ntiles) {
-        const bf16x8 b = *reinterpret_cast<const bf16x8*>(slab + (t * 16 + cl) * kSlabLd + kq);
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[t], 0, 0, 0);
-      }
+    for (int c = 0; c < kColTiles; ++c) {
+      const int t = 4 * c + wave < ntiles ? 4 * c + wave : 0;
+      b[c] = *reinterpret_cast<const bf16x8*>(Wt + static_cast<int64_t>(t * 16 + cl) * K + k0 + kq);
     }
-    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+      const bf16x8 a = *reinterpret_cast<const bf16x8*>(act + (r * 16 + cl) * kActLd + k0 + kq);
+#pragma unroll
+      for (int c = 0; c < kColTiles; ++c) acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[c], acc[r][c], 0, 0, 0);
+    }
   }
 }
 
+template <int RT>
 __global__ __launch_bounds__(kBlock) void k_mlp_infer(int nb, int k1, int n3, int d_out,
                                                       const uint64_t* __restrict__ det, int64_t cap, int64_t n,
                                                       const int64_t* __restrict__ idx,
@@ -84,10 +95,10 @@ __global__ __launch_bounds__(kBlock) void k_mlp_infer(int nb, int k1, int n3, in
                                                       const uint16_t* __restrict__ w2t, const float* __restrict__ b2,
                                                       const uint16_t* __restrict__ w3t, const float* __restrict__ b3,
                                                       float* __restrict__ tab, int64_t ld) {
-  __shared__ __attribute__((aligned(16))) uint16_t bufA[kInferRows * kHidden];
-  __shared__ __attribute__((aligned(16))) uint16_t bufB[kInferRows * kHidden];
-  const int64_t row0 = static_cast<int64_t>(blockIdx.x) * kInferRows;
-  for (int el = threadIdx.x; el < kInferRows * k1; el += blockDim.x) {
+  constexpr int R = 16 * RT;
+  __shared__ __attribute__((aligned(16))) uint16_t act[R * kActLd];
+  const int64_t row0 = static_cast<int64_t>(blockIdx.x) * R;
+  for (int el = threadIdx.x; el < R * k1; el += blockDim.x) {
     const int r = el / k1, c = el - r * k1;
     const int64_t d = row0 + r;
     float x = 0.0f;
@@ -97,48 +108,45 @@ __global__ __launch_bounds__(kBlock) void k_mlp_infer(int nb, int k1, int n3, in
       const bool occ = (det[static_cast<int64_t>(o >> 6) * cap + src] >> (o & 63)) & 1;
       x = occ ? (c < nb ? 1.0f : static_cast<float>(eps[o])) : 0.0f;
     }
-    bufA[r * k1 + c] = f2bf(x);
+    act[r * kActLd + c] = f2bf(x);
   }
   __syncthreads();
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int row = wave * 16 + (lane & 15), kq = (lane >> 4) * 8, cl = lane & 15;
-  const int orow = wave * 16 + (lane >> 4) * 4;
-  f32x4 acc[16];
-  static_assert(kHidden * kSlabLd <= kInferRows * kHidden, "a weight slab fits the idle activation buffer");
-  mfma_rows16<16>(bufA, k1, k1, w1t, 16, acc, row, kq, cl, bufB);
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, cl = lane & 15, orow = (lane >> 4) * 4;
+  f32x4 acc[RT][kColTiles];
+  auto hidden = [&](const float* __restrict__ bias) {  // GELU of the layer's output into the buffer it was read from
+    __syncthreads();
 #pragma unroll
-  for (int t = 0; t < 16; ++t)
+    for (int r = 0; r < RT; ++r)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int col = t * 16 + cl;
-      bufB[(orow + r) * kHidden + col] = f2bf(gelu_f(acc[t][r] + b1[col]));
-    }
-  __syncthreads();
-  mfma_rows16<16>(bufB, kHidden, kHidden, w2t, 16, acc, row, kq, cl, bufA);
-  __syncthreads();
+      for (int c = 0; c < kColTiles; ++c) {
+        const int col = (4 * c + wave) * 16 + cl;
 #pragma unroll
-  for (int t = 0; t < 16; ++t)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int col = t * 16 + cl;
-      bufA[(orow + r) * kHidden + col] = f2bf(gelu_f(acc[t][r] + b2[col]));
-    }
-  __syncthreads();
+        for (int q = 0; q < 4; ++q)
+          act[(r * 16 + orow + q) * kActLd + col] = f2bf(gelu_f(acc[r][c][q] + bias[col]));
+      }
+    __syncthreads();
+  };
+  layer_mfma<RT>(act, k1, w1t, kHidden / 16, acc, wave, lane);
+  hidden(b1);
+  layer_mfma<RT>(act, kHidden, w2t, kHidden / 16, acc, wave, lane);
+  hidden(b2);
   const int nt3 = n3 / 16;
-  mfma_rows16<16>(bufA, kHidden, kHidden, w3t, nt3, acc, row, kq, cl, bufB);
+  layer_mfma<RT>(act, kHidden, w3t, nt3, acc, wave, lane);
 #pragma unroll
-  for (int t = 0; t < 16; ++t) {
-    if (t >= nt3) break;
+  for (int r = 0; r < RT; ++r)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int col = t * 16 + cl;
-      const int64_t d = row0 + orow + r;
-      if (d < n && col < d_out) {
-        const float z = acc[t][r] + b3[col];
-        tab[d * ld + col] = expf(fminf(fmaxf(z, -kClip), kClip));
+    for (int c = 0; c < kColTiles; ++c) {
+      const int t = 4 * c + wave, col = t * 16 + cl;
+      if (t >= nt3 || col >= d_out) continue;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int64_t d = row0 + r * 16 + orow + q;
+        if (d < n) {
+          const float z = acc[r][c][q] + b3[col];
+          tab[d * ld + col] = expf(fminf(fmaxf(z, -kClip), kClip));
+        }
       }
     }
-  }
 }
 
 // bf16 inference copies: w1t[n][k] = W1[k][n] (k < d_in, else 0), w2t[n][k] =
@@ -928,11 +936,10 @@ int mlp_init(Mlp& m, uint64_t seed, hipStream_t st) {
 int mlp_infer(const Mlp& m, const fqd::Sys& s, const uint64_t* det, int64_t cap, int64_t n, float* tab,
               hipStream_t st, const int64_t* idx) {
   if (n <= 0) return FQ_OK;
-  const unsigned g = static_cast<unsigned>(ceil_div(n, kInferRows));
-  hipLaunchKernelGGL(k_mlp_infer, dim3(g), dim3(kBlock), 0, st, m.nb, m.k1, m.n3, m.d_out, det, cap, n, idx,
-                     s.sp_eigv,
-                     m.w1t, m.p + m.o_b1, m.w2t, m.p + m.o_b2, m.w3t, m.p + m.o_b3, tab,
-                     static_cast<int64_t>(m.d_out));
+  const int rt = n <= kFewRows ? 1 : 4;
+  hipLaunchKernelGGL(rt == 1 ? k_mlp_infer<1> : k_mlp_infer<4>, dim3(static_cast<unsigned>(ceil_div(n, 16 * rt))),
+                     dim3(kBlock), 0, st, m.nb, m.k1, m.n3, m.d_out, det, cap, n, idx, s.sp_eigv, m.w1t, m.p + m.o_b1,
+                     m.w2t, m.p + m.o_b2, m.w3t, m.p + m.o_b3, tab, static_cast<int64_t>(m.d_out));
   MLP_HIP(hipGetLastError());
   return FQ_OK;
 }
