@@ -19,14 +19,14 @@
 //                         their bit strings do in fewer bits.
 //                         replay: the reference's quicksort (src/sort.f90:213-396)
 //                         on one thread, so equal keys keep its order.
-//   self-annihilation     k_reduce_runs: one thread per run of equal keys,
-//                         plain and initiator rules (src/spawn_data.F90:859-1101).
-//   merge with main list  k_merge_runs: per block, the main-list window of its
-//                         runs' key range, then a search within that window
-//                         (src/annihilation.f90:294-486).
-//   rounding, compaction  k_round_main / k_round_new: stochastic rounding of small
-//                         real populations (src/annihilation.f90:537-675), draws
-//                         from Philox or from the replay stream at scan offsets.
+//   self-annihilation,    k_run_count / k_runs: one thread per run of equal keys,
+//   merge, rounding of    plain and initiator rules (src/spawn_data.F90:859-1101);
+//   new determinants      the run's sort value looked up in the tile's window of
+//                         the main list's values (src/annihilation.f90:294-486);
+//                         new determinants rounded and listed.
+//   rounding, compaction  k_round: stochastic rounding of small real populations
+//                         (src/annihilation.f90:537-675), draws from Philox or from
+//                         the replay stream at scan offsets.
 //   insertion             k_scatter_main / k_scatter_new: merge-path placement
 //                         of surviving main entries and new determinants into the
 //                         other buffer, new K_ii from the Slater--Condon diagonal
@@ -84,8 +84,12 @@ constexpr int kBlock = 256;
 constexpr int kInstShift = 48;
 constexpr uint64_t kOrbMask = (uint64_t{1} << kInstShift) - 1;
 constexpr int kMaxInst = 1 << 16;
-constexpr int kRunTile = 4 * kBlock;  // sorted entries per run-detection tile
-constexpr int kMergeWin = 1024;       // main-list window entries a merge block stages in LDS
+constexpr int kRunTile = 4 * kBlock;   // sorted entries per run tile
+constexpr int kMainTile = 4 * kBlock;  // main-list entries per rounding and insertion tile
+// Counts of up to this many tiles are prefixed by every block that needs them
+// (its threads add the counts before its tile: 16384 counts are 64 KB from L2);
+// longer ones are scanned first.
+constexpr int64_t kPrefixMax = 16384;
 // Words per spawned-list record (populations, flag), padded to 16-byte
 // alignment so one record is one aligned read after the sort's permutation.
 __host__ __device__ constexpr int rec_stride(int S) { return S == 1 ? 2 : 4; }
@@ -115,6 +119,8 @@ struct Stats {
   int64_t spawn_overflow;
   int64_t total_attempts;
   int64_t nruns;
+  int64_t nnew;            // surviving new determinants
+  int64_t nmain;           // surviving main-list entries
   int64_t new_n;
   int64_t main_overflow;
   int64_t rng_pos;
@@ -189,7 +195,8 @@ __device__ __forceinline__ int64_t list_len(const int64_t* __restrict__ pn, int6
 // The cycle index: read on the device in graph-captured cycles.
 __device__ __forceinline__ uint32_t cycle_of(const uint32_t* __restrict__ pc, uint32_t cyc) { return pc ? *pc : cyc; }
 
-__global__ __launch_bounds__(kBlock) void k_tile_sums(const int64_t* __restrict__ in, int64_t n,
+template <class T>
+__global__ __launch_bounds__(kBlock) void k_tile_sums(const T* __restrict__ in, int64_t n,
                                                       int64_t* __restrict__ sums) {
   __shared__ int64_t wsh[kBlock / 64];
   const int64_t base = static_cast<int64_t>(blockIdx.x) * kScanTile;
@@ -216,7 +223,8 @@ __device__ __forceinline__ void block_inclusive_scan(int64_t* sh) {
 // the tile's offset: with prefix, the sum of part[0..tile) (part: tile sums);
 // otherwise part[tile] (part: exclusive tile offsets).  The tile holding
 // element n-1 also writes out[n] = total.
-__global__ __launch_bounds__(kBlock) void k_tile_scan(const int64_t* __restrict__ in, int64_t n,
+template <class T>
+__global__ __launch_bounds__(kBlock) void k_tile_scan(const T* __restrict__ in, int64_t n,
                                                       const int64_t* __restrict__ part, int prefix,
                                                       int64_t* __restrict__ out) {
   __shared__ int64_t wsh[kBlock / 64];
@@ -255,7 +263,8 @@ __global__ __launch_bounds__(kBlock) void k_tile_scan(const int64_t* __restrict_
 // Exclusive scan of n entries on one block of kSmallBlock threads: chunks of
 // kSmallBlock * kSmallItems with a running carry (one chunk for the small
 // scans; many for the tile sums of a very long array).
-__global__ __launch_bounds__(kSmallBlock) void k_scan_small(const int64_t* __restrict__ in, int64_t n,
+template <class T>
+__global__ __launch_bounds__(kSmallBlock) void k_scan_small(const T* __restrict__ in, int64_t n,
                                                             int64_t* __restrict__ out) {
   __shared__ int64_t wsh[kSmallBlock / 64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -380,10 +389,10 @@ struct fq_engine {
   fqm::Mlp mlp;
   float* mlp_tab = nullptr;  // rows x 2*nbasis, one row per determinant the network runs on
   float* mlp_flat = nullptr;  // 2*nbasis ones: weights of determinants without a row
-  const int64_t* p_nruns = nullptr;  // device address of this cycle's run count
   int64_t att_bound = -1;            // bound of the next cycle's attempts (-1: unknown)
   bool keys_ready = false;           // the spawning pass made this cycle's sort keys
-  int64_t run_bound = 0;             // host bound of it (the count itself in replay mode)
+  int new_src = 0;                   // the sort's idle buffers after this cycle's passes
+  int64_t run_tiles = 0;             // run tiles of this cycle's spawned list (a bound of it while captured)
   int64_t mlp_tab_rows = 0;
   int64_t* mlp_on = nullptr;   // [cap] network runs on this determinant this cycle
   int64_t* mlp_row = nullptr;  // [cap + 1] exclusive prefix of mlp_on
@@ -398,9 +407,11 @@ struct fq_engine {
   int64_t* nat = nullptr;       // S*cap attempts per (det, space), then scanned
   int64_t* att_off = nullptr;   // S*cap+1
   int64_t* flags = nullptr;     // cap parent initiator flags
-  uint64_t* mmask = nullptr;    // cap/64+2: surviving main entries, one bit each
-  int64_t* mcnt = nullptr;      // survivors per 64-entry word
-  int64_t* moff = nullptr;      // their exclusive prefix
+  uint64_t* mrank[2] = {nullptr, nullptr};  // sort_kw*cap: the entries' sort values (ranks), as the list's buffers
+  uint64_t* mmask = nullptr;    // surviving main entries, one bit each, by tiles of kMainTile
+  uint16_t* mpre = nullptr;     // per word of mmask: survivors of its tile before it
+  int32_t* mcnt = nullptr;      // survivors per tile
+  int64_t* moff = nullptr;      // survivors before each tile; [tiles] = their number
   int64_t* mdraw = nullptr;     // cap+1 (replay rounding draws)
   int64_t* mdraw_off = nullptr;
   double* part_d = nullptr;     // 4 * (cap/256+1) block partials
@@ -424,23 +435,20 @@ struct fq_engine {
   uint32_t* perm = nullptr;                // scap: replay quicksort order
   int64_t* pass_cnt = nullptr;             // 512 * kSortBlocks digit counts of a pass's blocks
   int64_t* pass_off = nullptr;             // their exclusive prefix (+ total)
-  int64_t* run_tcnt = nullptr;             // run heads per run tile
-  int64_t* run_toff = nullptr;             // their exclusive prefix; [ntiles] = the run count
-  int64_t* run_tfirst = nullptr;           // first head of each run tile (-1: none)
+  int32_t* run_tcnt = nullptr;             // run heads per run tile
+  int64_t* run_toff = nullptr;             // their exclusive prefix (lists of more than kPrefixMax tiles)
+  int32_t* run_tfirst = nullptr;           // first head of each run tile (-1: none)
   int64_t* run_tpre = nullptr;             // sums of each run tile's entries before its first head
-  uint64_t* rdet = nullptr;      // W*scap
-  int64_t* rpop = nullptr;       // S*scap
-  int64_t* rflag = nullptr;      // scap
-  int64_t* rpos = nullptr;       // scap
-  int64_t* rstate = nullptr;     // scap: 0 dead, 1 hit, 2 new candidate
-  int64_t* nlist = nullptr;      // scap: surviving new runs in order
-  int64_t* nrpos = nullptr;      // scap: their insertion positions (non-decreasing)
-  int64_t* bstart = nullptr;     // cap/256 + 2: new runs before each 256-entry block of the main list
-  int64_t* mwin = nullptr;       // main-list bounds of each merge block's first and last run
-  uint64_t* nmask = nullptr;     // scap/64+2: surviving new runs, one bit each
-  int64_t* ncnt = nullptr;       // survivors per 64-run word
-  int64_t* noff = nullptr;       // their exclusive prefix
-  int64_t* ndraw = nullptr;      // scap+1
+  int64_t* run_win = nullptr;              // main-list position of each run tile's first value; then the end
+  // new determinants: per run tile (values and populations in the sort's idle
+  // buffers, positions in new_pos[0]), then in one list
+  int32_t* new_cnt = nullptr;    // per run tile
+  int64_t* new_off = nullptr;    // their exclusive prefix (lists of more than kPrefixMax tiles)
+  int32_t* new_pos[2] = {nullptr, nullptr};  // scap: insertion positions (non-decreasing): staged, listed
+  uint64_t* new_val = nullptr;   // sort_kw*scap: sort values of the new determinants
+  int64_t* new_pop = nullptr;    // S*scap: their populations
+  int64_t* abs_part = nullptr;   // |N| sums of the insertion's blocks
+  int64_t* ndraw = nullptr;      // replay: rounding draws of each run tile's candidates
   int64_t* ndraw_off = nullptr;
   // scan scratch
   std::vector<int64_t*> scan_tmp;
@@ -560,28 +568,29 @@ int64_t* scan_scratch(fq_engine* e, int slot, int64_t need) {
 }
 
 // Exclusive scan: out[0..n] with out[n] = total (in and out distinct).
-int scan_exclusive(fq_engine* e, const int64_t* in, int64_t* out, int64_t n) {
+template <class T>
+int scan_exclusive(fq_engine* e, const T* in, int64_t* out, int64_t n) {
   if (n == 0) {
     hipLaunchKernelGGL(k_set_zero_total, dim3(1), dim3(1), 0, e->stream, out);
     return FQ_OK;
   }
   if (n <= kSmallScanMax) {
-    hipLaunchKernelGGL(k_scan_small, dim3(1), dim3(kSmallBlock), 0, e->stream, in, n, out);
+    hipLaunchKernelGGL(k_scan_small<T>, dim3(1), dim3(kSmallBlock), 0, e->stream, in, n, out);
     return FQ_OK;
   }
   const int64_t nb = ceil_div(n, kScanTile);
   int64_t* sums = scan_scratch(e, 0, nb);
   if (!sums) return FQ_ERR_NOMEM;
-  hipLaunchKernelGGL(k_tile_sums, dim3(static_cast<unsigned>(nb)), dim3(kBlock), 0, e->stream, in, n, sums);
+  hipLaunchKernelGGL(k_tile_sums<T>, dim3(static_cast<unsigned>(nb)), dim3(kBlock), 0, e->stream, in, n, sums);
   if (nb <= kPrefixTiles) {
-    hipLaunchKernelGGL(k_tile_scan, dim3(static_cast<unsigned>(nb)), dim3(kBlock), 0, e->stream, in, n, sums, 1,
+    hipLaunchKernelGGL(k_tile_scan<T>, dim3(static_cast<unsigned>(nb)), dim3(kBlock), 0, e->stream, in, n, sums, 1,
                        out);
     return FQ_OK;
   }
   int64_t* offs = scan_scratch(e, 1, nb + 1);
   if (!offs) return FQ_ERR_NOMEM;
-  hipLaunchKernelGGL(k_scan_small, dim3(1), dim3(kSmallBlock), 0, e->stream, sums, nb, offs);
-  hipLaunchKernelGGL(k_tile_scan, dim3(static_cast<unsigned>(nb)), dim3(kBlock), 0, e->stream, in, n, offs, 0, out);
+  hipLaunchKernelGGL(k_scan_small<int64_t>, dim3(1), dim3(kSmallBlock), 0, e->stream, sums, nb, offs);
+  hipLaunchKernelGGL(k_tile_scan<T>, dim3(static_cast<unsigned>(nb)), dim3(kBlock), 0, e->stream, in, n, offs, 0, out);
   return FQ_OK;
 }
 
@@ -1824,23 +1833,65 @@ __device__ __forceinline__ void entry_share(int64_t flags, const int64_t* pop, b
   }
 }
 
+// Sort values: one 64-bit word, or two as a 128-bit integer.
+template <int KW>
+using SortValue = typename std::conditional<KW == 1, uint64_t, unsigned __int128>::type;
+template <int KW>
+__device__ __forceinline__ SortValue<KW> load_value(const uint64_t* __restrict__ v, int64_t stride, int64_t i) {
+  if constexpr (KW == 1) return v[i];
+  else return (static_cast<unsigned __int128>(v[stride + i]) << 64) | v[i];
+}
+template <int KW>
+__device__ __forceinline__ uint64_t value_word(SortValue<KW> v, int w) {
+  if constexpr (KW == 1) return v;
+  else return static_cast<uint64_t>(v >> (64 * w));
+}
+// Lower bound of x among the sorted values [0, n) by one whole wavefront: 64
+// pivots a step (4 dependent reads for 10^7 values instead of 23).
+template <int KW>
+__device__ __forceinline__ int64_t wave_lower_bound(const uint64_t* __restrict__ v, int64_t stride, int64_t n,
+                                                    SortValue<KW> x, int lane) {
+  int64_t lo = 0, hi = n;  // the bound lies in [lo, hi]
+  while (hi - lo > 64) {
+    const int64_t step = (hi - lo + 63) / 64, q = lo + (lane + 1) * step - 1;
+    const int c = __popcll(__ballot(q < hi && load_value<KW>(v, stride, q) < x));  // the first c pivots are below x
+    const int64_t nlo = lo + c * step, nhi = lo + (c + 1) * step - 1;
+    lo = nlo < hi ? nlo : hi;
+    hi = nhi < hi ? nhi : hi;
+  }
+  return lo + __popcll(__ballot(lo + lane < hi && load_value<KW>(v, stride, lo + lane) < x));
+}
+
 // Per tile of kRunTile sorted keys: the number of run heads (first key, or
 // value differing from the previous key), the position of the first head (-1
-// if none), and the sums (entry_share) of the entries before it -- the part of
-// a run that began in an earlier tile.
+// if none), the sums (entry_share) of the entries before it -- the part of a
+// run that began in an earlier tile -- and the main-list position of the
+// tile's first value (mrank: the main list's n sort values), which with the
+// next tile's bounds the positions of the tile's runs; win[ntiles] is the end
+// of the last tile's.
 template <int KW, int S>
 __global__ __launch_bounds__(kBlock) void k_run_count(const uint64_t* __restrict__ keys,
                                                       const int64_t* __restrict__ pay, const int64_t* __restrict__ pn,
                                                       int64_t nsb, int64_t stride, int fb,
-                                                      int64_t* __restrict__ tcnt, int64_t* __restrict__ tfirst,
-                                                      int64_t* __restrict__ tpre) {
+                                                      const uint64_t* __restrict__ mrank, int64_t n, int64_t cap,
+                                                      const int64_t* __restrict__ pmain, int64_t ntiles,
+                                                      int32_t* __restrict__ tcnt, int32_t* __restrict__ tfirst,
+                                                      int64_t* __restrict__ tpre, int64_t* __restrict__ win) {
   constexpr int R = kRunTile / kBlock, NV = 3 * S;
   const int64_t ns = list_len(pn, nsb);
   __shared__ int64_t wsh[kBlock / 64];
   __shared__ int32_t wfirst[kBlock / 64];
   const int64_t tile = blockIdx.x, t0 = tile * kRunTile;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  int64_t c = 0;
+  if (t0 >= ns) {  // a grid sized by a bound: an empty tile
+    if (threadIdx.x == 0) {
+      tcnt[tile] = 0;
+      tfirst[tile] = -1;
+    }
+    return;
+  }
+  n = list_len(pmain, n);
+  int32_t c = 0;
   int first_here = kRunTile;  // this wavefront's first head in the tile
 #pragma unroll
   for (int r = 0; r < R; ++r) {
@@ -1860,6 +1911,15 @@ __global__ __launch_bounds__(kBlock) void k_run_count(const uint64_t* __restrict
     if (b && first_here == kRunTile) first_here = r * kBlock + wave * 64 + __builtin_ctzll(b);
   }
   if (lane == 0) wfirst[wave] = first_here;
+  if (wave == kBlock / 64 - 1) {
+    const int64_t lb = wave_lower_bound<KW>(mrank, cap, n, load_value<KW>(keys, stride, t0) >> fb, lane);
+    if (lane == 0) win[tile] = lb;
+  }
+  const bool last = t0 + kRunTile >= ns;
+  if (last && wave == 0) {  // one past the last value's position
+    const int64_t lb = wave_lower_bound<KW>(mrank, cap, n, load_value<KW>(keys, stride, ns - 1) >> fb, lane);
+    if (lane == 0) win[tile + 1] = lb;
+  }
   const int64_t t = block_sum(c, wsh);  // its barriers also publish wfirst
   int first = kRunTile;
 #pragma unroll
@@ -1886,11 +1946,20 @@ __global__ __launch_bounds__(kBlock) void k_run_count(const uint64_t* __restrict
     for (int k = 0; k < NV; ++k) acc[k] = block_sum(acc[k], wsh);
   }
   if (threadIdx.x == 0) {
-    tcnt[tile] = t;
+    tcnt[tile] = static_cast<int32_t>(t);
     tfirst[tile] = first < kRunTile ? first : -1;
 #pragma unroll
     for (int k = 0; k < NV; ++k) tpre[tile * NV + k] = acc[k];
   }
+}
+
+// Sum of cnt[0..b) (off, when given, holds it) for the whole block.
+__device__ __forceinline__ int64_t tiles_before(const int32_t* __restrict__ cnt, const int64_t* __restrict__ off,
+                                                int64_t b, int64_t* wsh) {
+  if (off) return off[b];
+  int64_t x = 0;
+  for (int64_t k = threadIdx.x; k < b; k += kBlock) x += cnt[k];
+  return block_sum(x, wsh);
 }
 
 // Runs longer than this are reduced by the whole block (a queue in LDS), so a
@@ -1898,52 +1967,88 @@ __global__ __launch_bounds__(kBlock) void k_run_count(const uint64_t* __restrict
 // its wavefront idles; shorter ones by one thread each.
 constexpr int kShortRun = 32;
 
-// annihilate_spawn_t(_initiator) (src/spawn_data.F90:859-1101) over the
-// sorted keys and populations, one block per tile of kRunTile keys.  The
-// tile's run heads are listed in order (wavefront ballots); thread h takes run
-// h, sums its entries' shares (entry_share) over consecutive keys and writes
-// the run -- its index is the tile's run offset (toff) + h, its determinant is
-// recovered from the key by unranking -- so every lane has a run whatever the
-// run lengths.  Runs longer than kShortRun are queued and reduced by the whole
-// block afterwards.  The tile's last run adds the head-free prefixes of the
-// following tiles (k_run_count) up to the next head.  The run's first entry
-// is its first in sorted order: the reference's quicksort order in replay
-// mode, the earliest spawned in production (the stable sort of an
-// attempt-ordered list).
-template <int KW, int S, bool WIDE>
-__global__ __launch_bounds__(kBlock) void k_runs(Sys s, KeyPlan kp, const uint64_t* __restrict__ keys,
-                                                 const int64_t* __restrict__ pay, int64_t ns, int64_t stride,
-                                                 const int64_t* __restrict__ toff, const int64_t* __restrict__ tfirst,
-                                                 const int64_t* __restrict__ tpre, int64_t ntiles,
-                                                 uint64_t* __restrict__ rdet, int64_t* __restrict__ rpop,
-                                                 int64_t* __restrict__ rflag, int64_t* __restrict__ rstate,
-                                                 const int64_t* __restrict__ pns) {
-  ns = list_len(pns, ns);
-  constexpr int R = kRunTile / kBlock, NV = 3 * S, NW = kBlock / 64;
+// Inputs and outputs of k_runs.
+struct RunArgs {
+  const uint64_t* keys;  // sorted keys and payload
+  const int64_t* pay;
+  int64_t ns;            // list length, or a bound of it with the length at pns
+  const int64_t* pns;
+  int64_t stride;
+  int fb;
+  const int32_t* tcnt;   // k_run_count's outputs; toff: exclusive prefix of tcnt, or null
+  const int64_t* toff;
+  const int32_t* tfirst;
+  const int64_t* tpre;
+  const int64_t* win;
+  int64_t ntiles;
+  const uint64_t* mrank;  // the main list's sort values, its length n (or a bound, the length at pmain)
+  int64_t n;
+  const int64_t* pmain;
+  int64_t cap;
+  int64_t* pop_new;
+  int initiator, real_amps, replay;
+  int64_t rf;
+  uint64_t seed;
+  uint32_t cyc;
+  const uint32_t* pcyc;
+  uint64_t* nval;  // new determinants of the tile, from slot tile * kRunTile: values, populations, positions
+  int64_t* npop;
+  int32_t* npos;
+  int32_t* ncnt;   // and their number
+  Stats* st;
+};
+constexpr int kRunWin = 2048;  // main-list values a tile stages in LDS (two-word values: half as many)
+
+// annihilate_spawn_t(_initiator), annihilate_main_list(_initiator) and
+// round_low_population_spawns (src/spawn_data.F90:859-1101,
+// src/annihilation.f90:294-486, 613-675) over the sorted keys and populations,
+// one block per tile of kRunTile keys.  The tile's run heads are listed in
+// order (wavefront ballots); thread h takes run h and sums its entries' shares
+// (entry_share), so every lane has a run whatever the run lengths.  Runs longer
+// than kShortRun are queued and reduced by the whole block afterwards.  The
+// tile's last run adds the head-free prefixes of the following tiles
+// (k_run_count) up to the next head.  The run's first entry is its first in
+// sorted order: the reference's quicksort order in replay mode, the earliest
+// spawned in production (the stable sort of an attempt-ordered list).
+// Run totals stay in LDS; each run's value is then looked up among the main
+// list's values between the tile's bounds (staged in LDS when they fit) -- a
+// hit adds to the post-death populations, a miss is a new determinant if it may
+// be one and its rounded populations do not vanish -- and the tile's new
+// determinants are listed in order.  Runs are compared by value, so only the
+// determinants that are inserted are ever unranked, by the insertion.
+// (Before, every run was unranked and written as a record that three further
+// kernels read: 253 us for 4.3e6 keys on 2.8e6 determinants (k_runs 165,
+// search bounds 26, merge 39, rounding of new 18, their list 5), 88 us now and
+// 20 for the ranks k_scatter_main moves and the unranking of the inserted.)
+template <int KW, int S>
+__global__ __launch_bounds__(kBlock) void k_runs(RunArgs g) {
+  using V = SortValue<KW>;
+  constexpr int R = kRunTile / kBlock, NV = 3 * S, NW = kBlock / 64, WIN = kRunWin / KW;
   __shared__ int32_t wcount[R][NW];
   __shared__ int32_t hpos[kRunTile + 1];  // tile-relative index of each head, in order; then the tile length
-  __shared__ int32_t longq[kRunTile];     // runs (by h) left to the whole block
+  __shared__ int16_t longq[kRunTile];     // runs (by h) left to the whole block
+  __shared__ uint8_t rflag[kRunTile];     // a run's flags, bit 7: some population is not zero
+  __shared__ int64_t rtot[S][kRunTile];   // a run's populations
+  __shared__ V wval[WIN];                 // the main-list values between the tile's bounds when they fit
   __shared__ int32_t nlong;
   __shared__ int64_t wsh[NW];
-  extern __shared__ uint64_t binom_lds[];
+  const int64_t ns = list_len(g.pns, g.ns);
+  const int64_t stride = g.stride;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int64_t tile = blockIdx.x, t0 = tile * kRunTile;
-  if (t0 >= ns) return;  // block-uniform
-  const bool staged = kp.rank && kp.binom_lds;
-  if (staged) {  // one-word ranks: the table saturated at 2^64 - 1, one word per entry
-    const int nv = kp.nbasis * kp.nel;
-    for (int k = tid; k < nv; k += kBlock) {
-      if constexpr (WIDE) {
-        binom_lds[2 * k] = kp.binom[2 * k];
-        binom_lds[2 * k + 1] = kp.binom[2 * k + 1];
-      } else {
-        binom_lds[k] = kp.binom[2 * k + 1] ? ~uint64_t{0} : kp.binom[2 * k];
-      }
-    }
+  if (t0 >= ns) {  // block-uniform
+    if (tid == 0) g.ncnt[tile] = 0;
+    return;
   }
   const int n = static_cast<int>(ns - t0 < kRunTile ? ns - t0 : kRunTile);
-  const int fb = kp.flag_bits;
+  const int fb = g.fb;
   const uint64_t fmask = (uint64_t{1} << fb) - 1;
+  // every value of the tile lies in [value(t0), value(t0 + n)], so its lower bound lies in [wlo, whi]
+  const int64_t nm = list_len(g.pmain, g.n);
+  const int64_t wlo = g.win[tile], wend = g.win[tile + 1] + 1, whi = wend < nm ? wend : nm;
+  const bool staged = whi - wlo <= WIN;
+  if (staged)
+    for (int64_t q = tid; q < whi - wlo; q += kBlock) wval[q] = load_value<KW>(g.mrank, g.cap, wlo + q);
   bool head[R];
 #pragma unroll
   for (int r = 0; r < R; ++r) {
@@ -1954,8 +2059,8 @@ __global__ __launch_bounds__(kBlock) void k_runs(Sys s, KeyPlan kp, const uint64
       uint64_t k[KW], prev[KW];
 #pragma unroll
       for (int w = 0; w < KW; ++w) {
-        k[w] = keys[w * stride + i];
-        prev[w] = i > 0 ? keys[w * stride + i - 1] : 0;
+        k[w] = g.keys[w * stride + i];
+        prev[w] = i > 0 ? g.keys[w * stride + i - 1] : 0;
       }
       head[r] = i == 0 || !same_value<KW>(k, prev, fb);
     }
@@ -1967,6 +2072,7 @@ __global__ __launch_bounds__(kBlock) void k_runs(Sys s, KeyPlan kp, const uint64
     if (lane == 0) wcount[r][wave] = __popcll(bal[r]);
   }
   if (tid == 0) nlong = 0;
+  const int64_t rbase = tiles_before(g.tcnt, g.toff, tile, wsh);
   __syncthreads();
   int32_t total = 0;
 #pragma unroll
@@ -1978,70 +2084,48 @@ __global__ __launch_bounds__(kBlock) void k_runs(Sys s, KeyPlan kp, const uint64
     }
     if (head[r]) hpos[p] = r * kBlock + tid;
   }
-  if (tid == 0) hpos[total] = n;
-  __syncthreads();  // also orders the table's staging
-  const int64_t rbase = toff[tile];
+  if (tid == 0) {
+    hpos[total] = n;
+    if (t0 + n >= ns) g.st->nruns = rbase + total;
+  }
+  __syncthreads();
   // the shares of run h's entries [a, b) of the tile, from index `from` (stride `step`)
   auto shares = [&](int a, int b, int from, int step, int64_t* acc) {
     for (int j = from; j < b; j += step) {
       int64_t pop[S], cv[NV];
 #pragma unroll
-      for (int q = 0; q < S; ++q) pop[q] = pay[q * stride + t0 + j];
-      entry_share<S>(static_cast<int64_t>(keys[t0 + j] & fmask), pop, j == a, cv);
+      for (int q = 0; q < S; ++q) pop[q] = g.pay[q * stride + t0 + j];
+      entry_share<S>(static_cast<int64_t>(g.keys[t0 + j] & fmask), pop, j == a, cv);
 #pragma unroll
       for (int k = 0; k < NV; ++k) acc[k] += cv[k];
     }
   };
-  // run h's totals complete: the continuation of the tile's last run, the
-  // initiator rules, and the run's record
+  // run h's totals complete: the continuation of the tile's last run and the initiator rules
   auto finish = [&](int h, int64_t* acc) {
-    if (h == total - 1 && t0 + n < ns && tfirst[tile + 1] != 0) {
-      for (int64_t u = tile + 1; u < ntiles; ++u) {
+    if (h == total - 1 && t0 + n < ns && g.tfirst[tile + 1] != 0) {
+      for (int64_t u = tile + 1; u < g.ntiles && u * kRunTile < ns; ++u) {
 #pragma unroll
-        for (int k = 0; k < NV; ++k) acc[k] += tpre[u * NV + k];
-        if (tfirst[u] >= 0) break;
+        for (int k = 0; k < NV; ++k) acc[k] += g.tpre[u * NV + k];
+        if (g.tfirst[u] >= 0) break;
       }
     }
-    const int64_t run = rbase + h;
-    int64_t fl = 0;
-    bool nz = false;
+    int fl = 0;
 #pragma unroll
     for (int sp = 0; sp < S; ++sp) {
       const int64_t tot = acc[sp], init = acc[S + sp], evs = acc[2 * S + sp];
-      nz = nz || tot != 0;
-      if (s.initiator) {
+      if (tot != 0) fl |= 0x80;
+      if (g.initiator) {
         const int st = tot >= 0 ? 1 : -1, si = init >= 0 ? 1 : -1;
-        if (init != 0 && st == si) {
-        } else if (evs > 1 || evs < -1) {
-        } else {
-          fl += int64_t{1} << sp;
-        }
+        if (!(init != 0 && st == si) && !(evs > 1 || evs < -1)) fl |= 1 << sp;
       }
-      rpop[sp * stride + run] = tot;
+      rtot[sp][h] = tot;
     }
-    rflag[run] = fl;
-    rstate[run] = nz ? 1 : 0;
-    const int64_t i = t0 + hpos[h];
-    uint64_t kk[KW];
-#pragma unroll
-    for (int w = 0; w < KW; ++w) kk[w] = keys[w * stride + i];
-    uint64_t d[2] = {0, 0};
-    const unsigned __int128 val =
-        (KW == 1 ? static_cast<unsigned __int128>(kk[0])
-                 : (static_cast<unsigned __int128>(kk[KW - 1]) << 64) | kk[0]) >> fb;
-    if (!kp.rank) {
-      d[0] = static_cast<uint64_t>(val);  // batched instances: the encoded word itself
-    } else if (staged) {
-      unrank<WIDE>(kp, binom_lds, !WIDE, val, d);
-    } else {
-      unrank<WIDE>(kp, kp.binom, false, val, d);
-    }
-    FQ_FOR_WORDS(w, s.W) rdet[w * stride + run] = d[w];
+    rflag[h] = static_cast<uint8_t>(fl);
   };
   for (int h = tid; h < total; h += kBlock) {
     const int a = hpos[h], b = hpos[h + 1];
     if (b - a > kShortRun) {
-      longq[atomicAdd(&nlong, 1)] = h;
+      longq[atomicAdd(&nlong, 1)] = static_cast<int16_t>(h);
       continue;
     }
     int64_t acc[NV];
@@ -2063,6 +2147,103 @@ __global__ __launch_bounds__(kBlock) void k_runs(Sys s, KeyPlan kp, const uint64
     for (int k = 0; k < NV; ++k) acc[k] = block_sum(acc[k], wsh);
     if (tid == 0) finish(h, acc);
   }
+  __syncthreads();
+  // merge with the main list and list the new determinants, kBlock runs at a time in order
+  const uint32_t cyc = cycle_of(g.pcyc, g.cyc);
+  int32_t nnew = 0;
+  for (int h0 = 0; h0 < total; h0 += kBlock) {  // block-uniform
+    const int h = h0 + tid;
+    bool isnew = false;
+    V val = 0;
+    int64_t pop[S], lo = 0;
+    if (h < total && (rflag[h] & 0x80)) {
+      const int fl = rflag[h] & 0x7f;
+      val = load_value<KW>(g.keys, stride, t0 + hpos[h]) >> fb;
+      bool hit;
+      if (staged) {
+        int a = 0, b = static_cast<int>(whi - wlo);
+        while (a < b) {
+          const int mid = (a + b) >> 1;
+          if (wval[mid] < val)
+            a = mid + 1;
+          else
+            b = mid;
+        }
+        lo = wlo + a;
+        hit = a < whi - wlo && wval[a] == val;
+      } else {
+        int64_t a = wlo, b = whi;
+        while (a < b) {
+          const int64_t mid = (a + b) >> 1;
+          if (load_value<KW>(g.mrank, g.cap, mid) < val)
+            a = mid + 1;
+          else
+            b = mid;
+        }
+        lo = a;
+        hit = lo < nm && load_value<KW>(g.mrank, g.cap, lo) == val;
+      }
+#pragma unroll
+      for (int sp = 0; sp < S; ++sp) pop[sp] = rtot[sp][h];
+      if (hit) {
+#pragma unroll
+        for (int sp = 0; sp < S; ++sp) {
+          int64_t& m = g.pop_new[sp * g.cap + lo];
+          if (!g.initiator)
+            m += pop[sp];
+          else if (m != 0)
+            m += pop[sp];
+          else if (!((fl >> sp) & 1))
+            m = pop[sp];
+        }
+      } else {
+        bool keep = !g.initiator;
+        if (g.initiator) {
+#pragma unroll
+          for (int sp = 0; sp < S; ++sp) {
+            if ((fl >> sp) & 1)
+              pop[sp] = 0;
+            else
+              keep = true;
+          }
+        }
+        if (keep) {
+          if (g.replay) {
+            isnew = true;  // the stream's rounding draws follow the main list's
+          } else {
+            if (g.real_amps) {
+              const int64_t r = rbase + h;
+              fqd::Philox rng(g.seed, static_cast<uint32_t>(r), static_cast<uint32_t>(r >> 32),
+                              cyc ^ (fqd::kDrawRoundSpawn << 24));
+#pragma unroll
+              for (int sp = 0; sp < S; ++sp) pop[sp] = fqd::stoch_round_pop(rng, pop[sp], g.rf);
+            }
+#pragma unroll
+            for (int sp = 0; sp < S; ++sp) isnew = isnew || pop[sp] != 0;
+          }
+        }
+      }
+    }
+    const unsigned long long bn = __ballot(isnew);
+    if (lane == 0) wcount[0][wave] = __popcll(bn);
+    __syncthreads();
+    int32_t k = nnew + __popcll(bn & ((1ull << lane) - 1));
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      if (w < wave) k += wcount[0][w];
+      nnew += wcount[0][w];
+    }
+    if (isnew) {
+      const int64_t slot = t0 + k;
+#pragma unroll
+      for (int w = 0; w < KW; ++w) g.nval[w * stride + slot] = value_word<KW>(val, w);
+#pragma unroll
+      for (int sp = 0; sp < S; ++sp) g.npop[sp * stride + slot] = pop[sp];
+      g.npos[slot] = static_cast<int32_t>(lo);
+    }
+    __syncthreads();  // wcount is rewritten by the next round
+  }
+  if (tid == 0) g.ncnt[tile] = nnew;
 }
 
 // ---------------------------------------------------------------------------
@@ -2207,141 +2388,6 @@ __global__ void k_add_nspawn(Stats* __restrict__ st, int64_t m) { st->nspawn += 
 // ---------------------------------------------------------------------------
 // Kernels: merge with the main list, rounding, insertion
 // ---------------------------------------------------------------------------
-// Per surviving run: binary search of its key in the (old) main list; a hit
-// adds into the post-death populations (annihilate_main_list(_initiator)), a
-// miss becomes a new-determinant candidate with flagged spaces cleared.
-// Lower bound of key k in the sorted main list positions [lo, hi).
-__device__ __forceinline__ int64_t main_lower_bound(const uint64_t* __restrict__ det, int64_t cap, int W,
-                                                    const uint64_t* k, int64_t lo, int64_t hi) {
-  while (lo < hi) {
-    const int64_t mid = (lo + hi) >> 1;
-    int c = 0;
-#pragma unroll
-    for (int w = FQ_MAX_WORDS - 1; w >= 0; --w)
-      if (w < W && c == 0) {
-        const uint64_t x = det[w * cap + mid];
-        c = (x < k[w]) ? -1 : (x > k[w] ? 1 : 0);
-      }
-    if (c < 0)
-      lo = mid + 1;
-    else
-      hi = mid;
-  }
-  return lo;
-}
-
-// Lower bounds in the main list of the first and last key of each merge
-// block's runs (one thread per block of kBlock runs).
-__global__ void k_merge_bounds(const int64_t* __restrict__ pnr, int64_t n, int64_t cap, int W,
-                               const uint64_t* __restrict__ det, const uint64_t* __restrict__ rdet, int64_t scap,
-                               int64_t* __restrict__ mwin, const int64_t* __restrict__ pn) {
-  const int64_t nruns = *pnr;
-  n = list_len(pn, n);
-  const int64_t b = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int64_t r0 = b * kBlock;
-  if (r0 >= nruns) return;
-  const int64_t r1 = (r0 + kBlock < nruns ? r0 + kBlock : nruns) - 1;
-  uint64_t k[FQ_MAX_WORDS] = {0, 0};
-  FQ_FOR_WORDS(w, W) k[w] = rdet[w * scap + r0];
-  const int64_t lo = main_lower_bound(det, cap, W, k, 0, n);
-  FQ_FOR_WORDS(w, W) k[w] = rdet[w * scap + r1];
-  mwin[2 * b] = lo;
-  mwin[2 * b + 1] = main_lower_bound(det, cap, W, k, lo, n);
-}
-
-// Runs are sorted, so a block's runs land between the lower bounds of its
-// first and last keys: two searches of the whole list per block, then each
-// thread searches only that window (merge-path partition of the two lists).
-__global__ __launch_bounds__(kBlock) void k_merge_runs(Sys s, const int64_t* __restrict__ pnr, int64_t n, int64_t cap,
-                                                       const uint64_t* __restrict__ det,
-                                                       int64_t* __restrict__ pop_new, const uint64_t* __restrict__ rdet,
-                                                       int64_t* __restrict__ rpop, const int64_t* __restrict__ rflag,
-                                                       int64_t scap, const int64_t* __restrict__ mwin,
-                                                       int64_t* __restrict__ rpos, int64_t* __restrict__ rstate,
-                                                       const int64_t* __restrict__ pn) {
-  const int64_t nruns = *pnr;
-  n = list_len(pn, n);
-  __shared__ uint64_t wdet[FQ_MAX_WORDS][kMergeWin];  // the window's determinants when it fits
-  const int64_t r0 = static_cast<int64_t>(blockIdx.x) * blockDim.x;
-  if (r0 >= nruns) return;  // whole block past the runs (the grid covers a bound); no window
-  // every key of the block lies in [key(r0), key(r1)], so its lower bound
-  // lies in [wlo, whi): whi = min(bound(r1) + 1, n)
-  const int64_t b0 = mwin[2 * blockIdx.x], b1 = mwin[2 * blockIdx.x + 1];
-  const int64_t wlo = b0, whi = b1 < n ? b1 + 1 : n;
-  const bool staged = whi - wlo <= kMergeWin;
-  if (staged)
-    for (int64_t q = threadIdx.x; q < whi - wlo; q += kBlock) FQ_FOR_WORDS(w, s.W) wdet[w][q] = det[w * cap + wlo + q];
-  __syncthreads();
-  const int64_t r = r0 + threadIdx.x;
-  if (r >= nruns) return;
-  if (rstate[r] == 0) {
-    rpos[r] = 0;
-    return;
-  }
-  uint64_t k[FQ_MAX_WORDS] = {0, 0};
-  FQ_FOR_WORDS(w, s.W) k[w] = rdet[w * scap + r];
-  int64_t lo;
-  bool hit = false;
-  if (staged) {
-    int a = 0, b = static_cast<int>(whi - wlo);
-    while (a < b) {
-      const int mid = (a + b) >> 1;
-      int c = 0;
-#pragma unroll
-      for (int w = FQ_MAX_WORDS - 1; w >= 0; --w)
-        if (w < s.W && c == 0) {
-          const uint64_t x = wdet[w][mid];
-          c = (x < k[w]) ? -1 : (x > k[w] ? 1 : 0);
-        }
-      if (c < 0)
-        a = mid + 1;
-      else
-        b = mid;
-    }
-    lo = wlo + a;
-    if (a < whi - wlo) {
-      hit = true;
-      FQ_FOR_WORDS(w, s.W) hit = hit && wdet[w][a] == k[w];
-    }
-  } else {
-    lo = main_lower_bound(det, cap, s.W, k, wlo, whi);
-    if (lo < n) {
-      hit = true;
-      FQ_FOR_WORDS(w, s.W) hit = hit && det[w * cap + lo] == k[w];
-    }
-  }
-  rpos[r] = lo;
-  const int64_t fl = rflag[r];
-  if (hit) {
-    for (int sp = 0; sp < s.S; ++sp) {
-      int64_t& m = pop_new[sp * cap + lo];
-      const int64_t v = rpop[sp * scap + r];
-      if (!s.initiator)
-        m += v;
-      else if (m != 0)
-        m += v;
-      else if (!((fl >> sp) & 1))
-        m = v;
-    }
-    rstate[r] = 3;  // annihilated into the main list
-  } else {
-    if (s.initiator) {
-      bool discard = true;
-      for (int sp = 0; sp < s.S; ++sp) {
-        if ((fl >> sp) & 1)
-          rpop[sp * scap + r] = 0;
-        else
-          discard = false;
-      }
-      if (discard) {
-        rstate[r] = 0;
-        return;
-      }
-    }
-    rstate[r] = 2;  // new determinant candidate
-  }
-}
-
 // Number of rounding draws an entry needs: spaces with 0 < |pop| < rf.
 __device__ __forceinline__ int round_draws(const int64_t* p, int64_t stride, int64_t i, int S, int64_t rf) {
   int c = 0;
@@ -2370,304 +2416,430 @@ __global__ void k_count_round_main(Sys s, int64_t n, int64_t cap, const int64_t*
   if (i >= n) return;
   mdraw[i] = (s.real_amps && !is_core_entry(s, det, cap, i)) ? round_draws(pop_new, cap, i, s.S, s.rf) : 0;
 }
-__global__ void k_count_round_new(Sys s, int64_t nruns, const int64_t* __restrict__ rpop,
-                                  const int64_t* __restrict__ rstate, int64_t scap, int64_t* __restrict__ ndraw) {
-  const int64_t r = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (r >= nruns) return;
-  ndraw[r] = (s.real_amps && rstate[r] == 2) ? round_draws(rpop, scap, r, s.S, s.rf) : 0;
+// Replay: rounding draws of a run tile's candidates, then (one block per tile)
+// the rounding itself at the tile's place in the stream, keeping the candidates
+// that survive at the front of the tile's slots.
+__global__ __launch_bounds__(kBlock) void k_count_round_new(Sys s, const int32_t* __restrict__ ncnt,
+                                                            const int64_t* __restrict__ npop, int64_t stride,
+                                                            int64_t* __restrict__ ndraw) {
+  __shared__ int64_t wsh[kBlock / 64];
+  const int64_t t0 = static_cast<int64_t>(blockIdx.x) * kRunTile;
+  const int cnt = ncnt[blockIdx.x];
+  int64_t c = 0;
+  if (s.real_amps)
+    for (int j = threadIdx.x; j < cnt; j += kBlock) c += round_draws(npop, stride, t0 + j, s.S, s.rf);
+  c = block_sum(c, wsh);
+  if (threadIdx.x == 0) ndraw[blockIdx.x] = c;
+}
+__global__ __launch_bounds__(kBlock) void k_replay_round_new(Sys s, int KW, int32_t* __restrict__ ncnt,
+                                                             uint64_t* __restrict__ nval, int64_t* __restrict__ npop,
+                                                             int32_t* __restrict__ npos, int64_t stride,
+                                                             const double* __restrict__ rbuf, int64_t rbase,
+                                                             const int64_t* __restrict__ ndraw_off) {
+  __shared__ uint32_t wsh[kBlock / 64];
+  const int64_t t0 = static_cast<int64_t>(blockIdx.x) * kRunTile;
+  const int cnt = ncnt[blockIdx.x];
+  int64_t drawn = ndraw_off[blockIdx.x];
+  uint32_t kept = 0;
+  for (int j0 = 0; j0 < cnt; j0 += kBlock) {  // block-uniform; slots before j0 are free to overwrite
+    const int j = j0 + static_cast<int>(threadIdx.x);
+    const bool in = j < cnt;
+    int64_t pop[FQ_MAX_SPACES] = {0, 0};
+    uint64_t val[2] = {0, 0};
+    int32_t pos = 0;
+    const uint32_t nd = in && s.real_amps ? round_draws(npop, stride, t0 + j, s.S, s.rf) : 0;
+    uint32_t all;
+    const int64_t at = rbase + drawn + block_exclusive_u32(nd, wsh, all);
+    bool alive = false;
+    if (in) {
+      fqd::ReplayRng rng{rbuf, at, at + nd, false};
+      for (int sp = 0; sp < s.S; ++sp) {
+        pop[sp] = npop[sp * stride + t0 + j];
+        if (s.real_amps) pop[sp] = fqd::stoch_round_pop(rng, pop[sp], s.rf);
+        alive = alive || pop[sp] != 0;
+      }
+      for (int w = 0; w < KW; ++w) val[w] = nval[w * stride + t0 + j];
+      pos = npos[t0 + j];
+    }
+    drawn += all;
+    const uint32_t k = kept + block_exclusive_u32(alive ? 1u : 0u, wsh, all);  // its barriers follow every read above
+    kept += all;
+    if (alive) {
+      for (int w = 0; w < KW; ++w) nval[w * stride + t0 + k] = val[w];
+      for (int sp = 0; sp < s.S; ++sp) npop[sp * stride + t0 + k] = pop[sp];
+      npos[t0 + k] = pos;
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) ncnt[blockIdx.x] = static_cast<int32_t>(kept);
 }
 
-// Survivor flags are kept as bits, one ballot word per 64 consecutive
-// entries, with each word's count; the rank of entry p among survivors is
-// off[p >> 6] + the word's bits below p (off: exclusive prefix of the counts).
-__device__ __forceinline__ bool bit_get(const uint64_t* __restrict__ mask, int64_t p) {
-  return (mask[p >> 6] >> (p & 63)) & 1;
+// Survivor flags are kept as bits, one ballot word per 64 consecutive entries,
+// with the survivors of its tile before each word (mpre) and per tile (mcnt,
+// prefixed in moff): an entry's rank among the survivors is moff + mpre + the
+// word's bits below it.
+//
+// Blocks [0, mtiles): remove_unoccupied_dets over a tile of the main list --
+// round small real populations, mark survivors.  The other blocks: run tile
+// b's new determinants go to their places in one list (a tile's place is the
+// count of those before it; noff, when given, holds it).  The two have nothing
+// to do with each other and share a launch.
+struct RoundArgs {
+  Sys s;
+  int64_t n;  // main-list length, or a bound of it with the length at pn
+  const int64_t* pn;
+  int64_t cap, mtiles;
+  const uint64_t* det;
+  int64_t* pop_new;
+  int replay;
+  const double* rbuf;
+  int64_t rbase;
+  const int64_t* mdraw_off;
+  uint64_t seed;
+  uint32_t cyc;
+  const uint32_t* pcyc;
+  uint64_t* mmask;
+  uint16_t* mpre;
+  int32_t* mcnt;
+  int KW;
+  int64_t scap, ntiles;
+  const int32_t* ncnt;
+  const int64_t* noff;
+  const uint64_t* nval;
+  const int64_t* npop;
+  const int32_t* npos;
+  uint64_t* lval;
+  int64_t* lpop;
+  int32_t* lpos;
+  Stats* st;
+};
+__global__ __launch_bounds__(kBlock) void k_round(RoundArgs g) {
+  constexpr int R = kMainTile / kBlock, NW = kBlock / 64;
+  __shared__ int64_t wsh[NW];
+  __shared__ int32_t wc[R * NW];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int S = g.s.S;
+  if (blockIdx.x >= g.mtiles) {
+    const int64_t b = blockIdx.x - g.mtiles;
+    const int32_t cnt = g.ncnt[b];
+    if (cnt == 0 && b != g.ntiles - 1) return;  // block-uniform
+    const int64_t k0 = tiles_before(g.ncnt, g.noff, b, wsh), t0 = b * kRunTile;
+    for (int j = tid; j < cnt; j += kBlock) {
+      for (int w = 0; w < g.KW; ++w) g.lval[w * g.scap + k0 + j] = g.nval[w * g.scap + t0 + j];
+      for (int sp = 0; sp < S; ++sp) g.lpop[sp * g.scap + k0 + j] = g.npop[sp * g.scap + t0 + j];
+      g.lpos[k0 + j] = g.npos[t0 + j];
+    }
+    if (tid == 0 && b == g.ntiles - 1) g.st->nnew = k0 + cnt;
+    return;
+  }
+  const int64_t t0 = static_cast<int64_t>(blockIdx.x) * kMainTile;
+  const int64_t nl = list_len(g.pn, g.n);  // entries past it (up to the bound n) are marked dead
+  const uint32_t cyc = cycle_of(g.pcyc, g.cyc);
+  unsigned long long bal[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int64_t i = t0 + r * kBlock + tid;
+    bool alive = false;
+    if (i < nl) {
+      if (is_core_entry(g.s, g.det, g.cap, i)) {
+        alive = true;
+      } else {
+        int64_t p[FQ_MAX_SPACES];
+#pragma unroll
+        for (int sp = 0; sp < FQ_MAX_SPACES; ++sp) p[sp] = sp < S ? g.pop_new[sp * g.cap + i] : 0;
+        if (g.s.real_amps) {
+          bool small = false;  // some population is rounded (draws only matter then)
+#pragma unroll
+          for (int sp = 0; sp < FQ_MAX_SPACES; ++sp) small = small || (p[sp] != 0 && p[sp] < g.s.rf && p[sp] > -g.s.rf);
+          if (small) {
+            if (g.replay) {
+              fqd::ReplayRng rng{g.rbuf, g.rbase + g.mdraw_off[i], g.rbase + g.mdraw_off[i + 1], false};
+              for (int sp = 0; sp < S; ++sp) p[sp] = fqd::stoch_round_pop(rng, p[sp], g.s.rf);
+            } else {
+              fqd::Philox rng(g.seed, static_cast<uint32_t>(i), static_cast<uint32_t>(i >> 32),
+                              cyc ^ (fqd::kDrawRoundMain << 24));
+              for (int sp = 0; sp < S; ++sp) p[sp] = fqd::stoch_round_pop(rng, p[sp], g.s.rf);
+            }
+            for (int sp = 0; sp < S; ++sp) g.pop_new[sp * g.cap + i] = p[sp];
+          }
+        }
+        alive = p[0] != 0 || p[1] != 0;
+      }
+    }
+    bal[r] = __ballot(alive);
+    if (lane == 0) wc[r * NW + wave] = __popcll(bal[r]);
+  }
+  __syncthreads();
+  int32_t before = 0;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      if (lane == 0 && w == wave) {
+        const int64_t word = (t0 >> 6) + r * NW + w;
+        g.mmask[word] = bal[r];
+        g.mpre[word] = static_cast<uint16_t>(before);
+      }
+      before += wc[r * NW + w];
+    }
+  }
+  if (tid == 0) g.mcnt[blockIdx.x] = before;
 }
-__device__ __forceinline__ int64_t bit_rank(const int64_t* __restrict__ off, const uint64_t* __restrict__ mask,
-                                            int64_t p) {
-  const int b = static_cast<int>(p & 63);
-  return off[p >> 6] + (b ? __popcll(mask[p >> 6] & ((1ull << b) - 1)) : 0);
+
+// Insertion of the surviving main entries.  An entry moves up by its rank among
+// the survivors plus the number of new determinants inserted at or before it:
+// lpos lists their positions, non-decreasing because the runs are sorted, so
+// each tile bounds its part of the list (two wavefronts' searches), stages it
+// in LDS when it fits and every thread searches only there.  Insertion is
+// skipped when the main list would overflow (insert_new_walkers' psip_list%error
+// path).  Also written: the survivors before each tile (moff), the new length,
+// and the tile's sums of |N|.
+struct InsertArgs {
+  Sys s;
+  int64_t n;
+  const int64_t* pn;
+  int64_t cap, mtiles;
+  const uint64_t* det;
+  const uint64_t* rank;  // the list's sort values (rank_words of them; 0: the determinant itself)
+  int rank_words;
+  const int64_t* pop_new;
+  const double* kii;
+  const uint64_t* mmask;
+  const uint16_t* mpre;
+  const int32_t* mcnt;
+  const int64_t* moff_in;  // exclusive prefix of mcnt, or null
+  int64_t* moff;
+  const int32_t* lpos;
+  const uint64_t* lval;
+  const int64_t* lpop;
+  int64_t scap;
+  Stats* st;
+  uint64_t* det_out;
+  uint64_t* rank_out;
+  int64_t* pop_out;
+  double* kii_out;
+  int64_t* abs_part;  // [S][abs_ld]: the tiles', then k_scatter_new's blocks'
+  int64_t abs_ld;
+};
+constexpr int kInsWin = 2048;
+// First k in [0, n) with v[k] >= x, by one wavefront.
+__device__ __forceinline__ int64_t wave_lower_bound32(const int32_t* __restrict__ v, int64_t n, int64_t x, int lane) {
+  int64_t lo = 0, hi = n;
+  while (hi - lo > 64) {
+    const int64_t step = (hi - lo + 63) / 64, q = lo + (lane + 1) * step - 1;
+    const int c = __popcll(__ballot(q < hi && v[q] < x));
+    const int64_t nlo = lo + c * step, nhi = lo + (c + 1) * step - 1;
+    lo = nlo < hi ? nlo : hi;
+    hi = nhi < hi ? nhi : hi;
+  }
+  return lo + __popcll(__ballot(lo + lane < hi && v[lo + lane] < x));
 }
-// All lanes of a wavefront call this; its 64 entries start at a multiple of 64.
-__device__ __forceinline__ void store_ballot(bool alive, int64_t i, int64_t n, uint64_t* __restrict__ mask,
-                                             int64_t* __restrict__ cnt) {
-  const unsigned long long bal = __ballot(alive);
-  if ((threadIdx.x & 63) == 0 && i < n) {
-    mask[i >> 6] = bal;
-    cnt[i >> 6] = __popcll(bal);
+__global__ __launch_bounds__(kBlock) void k_scatter_main(InsertArgs g) {
+  constexpr int R = kMainTile / kBlock, NW = kBlock / 64;
+  __shared__ int32_t win[kInsWin];
+  __shared__ int64_t wsh[NW], bounds[2];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int64_t n = list_len(g.pn, g.n), tile = blockIdx.x, t0 = tile * kMainTile;
+  const int64_t nnew = g.st->nnew;
+  // survivors before the tile, and of the whole list
+  int64_t off, total;
+  if (g.moff_in) {
+    off = g.moff_in[tile];
+    total = g.moff_in[g.mtiles];
+  } else {
+    int64_t pre = 0, all = 0;
+    for (int64_t k = tid; k < g.mtiles; k += kBlock) {
+      const int64_t c = g.mcnt[k];
+      all += c;
+      if (k < tile) pre += c;
+    }
+    off = block_sum(pre, wsh);
+    total = block_sum(all, wsh);
+  }
+  const bool ovf = total + nnew > g.cap;
+  if (tid == 0) {
+    g.moff[tile] = off;
+    if (tile == g.mtiles - 1) {
+      g.moff[g.mtiles] = total;
+      g.st->nmain = total;
+      g.st->main_overflow = ovf ? 1 : 0;
+      g.st->new_n = ovf ? total : total + nnew;
+    }
+  }
+  int64_t sum[FQ_MAX_SPACES] = {0, 0};
+  if (t0 < n) {  // block-uniform
+    if (wave < 2) {
+      const int64_t b = ovf ? 0 : wave_lower_bound32(g.lpos, nnew, wave == 0 ? t0 : t0 + kMainTile, lane);
+      if (lane == 0) bounds[wave] = b;
+    }
+    __syncthreads();
+    const int64_t c0 = bounds[0], c1 = bounds[1];
+    const bool staged = c1 - c0 <= kInsWin;
+    if (staged)
+      for (int64_t q = tid; q < c1 - c0; q += kBlock) win[q] = g.lpos[c0 + q];
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int64_t i = t0 + r * kBlock + tid;
+      const int64_t word = i >> 6;  // the wavefront's 64 entries
+      const uint64_t m = t0 + r * kBlock + wave * 64 < n ? g.mmask[word] : 0;
+      if (!((m >> lane) & 1)) continue;
+      int64_t shift;
+      if (staged) {
+        int a = 0, b = static_cast<int>(c1 - c0);
+        while (a < b) {
+          const int mid = (a + b) >> 1;
+          if (win[mid] <= i)
+            a = mid + 1;
+          else
+            b = mid;
+        }
+        shift = c0 + a;
+      } else {
+        int64_t a = c0, b = c1;
+        while (a < b) {
+          const int64_t mid = (a + b) >> 1;
+          if (g.lpos[mid] <= i)
+            a = mid + 1;
+          else
+            b = mid;
+        }
+        shift = a;
+      }
+      const int64_t o = off + g.mpre[word] + __popcll(m & ((1ull << lane) - 1)) + shift;
+      for (int w = 0; w < g.s.W; ++w) g.det_out[w * g.cap + o] = g.det[w * g.cap + i];
+      for (int w = 0; w < g.rank_words; ++w) g.rank_out[w * g.cap + o] = g.rank[w * g.cap + i];
+#pragma unroll
+      for (int sp = 0; sp < FQ_MAX_SPACES; ++sp)
+        if (sp < g.s.S) {
+          const int64_t p = g.pop_new[sp * g.cap + i];
+          g.pop_out[sp * g.cap + o] = p;
+          sum[sp] += p < 0 ? -p : p;
+        }
+      g.kii_out[o] = g.kii[i];
+    }
+  }
+  for (int sp = 0; sp < g.s.S; ++sp) {
+    const int64_t x = block_sum(sp == 0 ? sum[0] : sum[1], wsh);
+    if (tid == 0) g.abs_part[sp * g.abs_ld + tile] = x;
   }
 }
 
-// remove_unoccupied_dets: round small real populations, mark survivors.
-__global__ __launch_bounds__(kBlock) void k_round_main(Sys s, int64_t n, int64_t cap, int64_t* __restrict__ pop_new,
-                                                       int replay, const double* __restrict__ rbuf, int64_t rbase,
-                                                       const int64_t* __restrict__ mdraw_off, uint64_t seed,
-                                                       uint32_t cyc, uint64_t* __restrict__ mmask,
-                                                       int64_t* __restrict__ mcnt, const uint64_t* __restrict__ det,
-                                                       const int64_t* __restrict__ pn, const uint32_t* __restrict__ pcyc) {
+// Insertion of the new determinants (grid-stride, list order = rank order):
+// the determinant unranked from its sort value, K_ii from the diagonal rule.
+// A molecular system's dense pair tables (2 norb^2 doubles) and the binomial
+// table are staged in LDS when jk_lds / kp.binom_lds say so.
+template <bool WIDE>
+__global__ __launch_bounds__(kBlock) void k_scatter_new(InsertArgs g, KeyPlan kp, const Sys* __restrict__ sys_arr,
+                                                        int jk_lds) {
+  extern __shared__ double dyn[];
+  __shared__ int64_t wsh[kBlock / 64];
+  const Sys& s = g.s;
+  const int64_t nnew = g.st->main_overflow ? 0 : g.st->nnew;
+  const int64_t n = list_len(g.pn, g.n), nmain = g.st->nmain;
+  const int64_t k0 = static_cast<int64_t>(blockIdx.x) * kBlock;
+  int64_t sum[FQ_MAX_SPACES] = {0, 0};
+  if (k0 < nnew) {  // block-uniform
+    double* jk = dyn;
+    const int nn = s.norb * s.norb;
+    uint64_t* binom = reinterpret_cast<uint64_t*>(dyn + (jk_lds ? 2 * nn : 0));
+    if (jk_lds)
+      for (int q = threadIdx.x; q < nn; q += kBlock) {
+        jk[q] = s.jmat[q];
+        jk[nn + q] = s.kmat[q];
+      }
+    if (kp.rank && kp.binom_lds) {  // one-word ranks: the table saturated at 2^64 - 1, one word per entry
+      const int nv = kp.nbasis * kp.nel;
+      for (int k = threadIdx.x; k < nv; k += kBlock) {
+        if constexpr (WIDE) {
+          binom[2 * k] = kp.binom[2 * k];
+          binom[2 * k + 1] = kp.binom[2 * k + 1];
+        } else {
+          binom[k] = kp.binom[2 * k + 1] ? ~uint64_t{0} : kp.binom[2 * k];
+        }
+      }
+    }
+    __syncthreads();
+    for (int64_t k = k0 + threadIdx.x; k < nnew; k += static_cast<int64_t>(gridDim.x) * kBlock) {
+      const int64_t p = g.lpos[k];
+      int64_t o = k + nmain;
+      if (p < n) {  // survivors before entry p
+        const uint64_t m = g.mmask[p >> 6];
+        o = k + g.moff[p / kMainTile] + g.mpre[p >> 6] + __popcll(m & ((1ull << (p & 63)) - 1));
+      }
+      uint64_t f[FQ_MAX_WORDS] = {0, 0};
+      const uint64_t v0 = g.lval[k];
+      if (!kp.rank) {
+        f[0] = v0;  // batched instances: the encoded word itself
+      } else {
+        const unsigned __int128 v = WIDE ? (static_cast<unsigned __int128>(g.lval[g.scap + k]) << 64) | v0 : v0;
+        if (kp.binom_lds)
+          unrank<WIDE>(kp, binom, !WIDE, v, f);
+        else
+          unrank<WIDE>(kp, kp.binom, false, v, f);
+      }
+      FQ_FOR_WORDS(w, s.W) g.det_out[w * g.cap + o] = f[w];
+      for (int w = 0; w < g.rank_words; ++w) g.rank_out[w * g.cap + o] = g.lval[w * g.scap + k];
+#pragma unroll
+      for (int sp = 0; sp < FQ_MAX_SPACES; ++sp)
+        if (sp < s.S) {
+          const int64_t x = g.lpop[sp * g.scap + k];
+          g.pop_out[sp * g.cap + o] = x;
+          sum[sp] += x < 0 ? -x : x;
+        }
+      if (sys_arr) {  // batched: the instance's diagonal
+        const Sys& si = sys_arr[f[0] >> kInstShift];
+        f[0] &= kOrbMask;
+        g.kii_out[o] = fqd::diagonal(si, f) - si.H00;
+      } else if (jk_lds) {
+        g.kii_out[o] = fqd::diagonal_mol(s, f, jk, jk + nn) - s.H00;
+      } else {
+        g.kii_out[o] = fqd::diagonal(s, f) - s.H00;
+      }
+    }
+  }
+  for (int sp = 0; sp < s.S; ++sp) {
+    const int64_t x = block_sum(sp == 0 ? sum[0] : sum[1], wsh);
+    if (threadIdx.x == 0) g.abs_part[sp * g.abs_ld + g.mtiles + blockIdx.x] = x;
+  }
+}
+
+// Sum |N| over the new list from the insertion's block sums (exact integers:
+// any order gives the same totals).
+constexpr int kFinishBlock = 1024;
+__global__ __launch_bounds__(kFinishBlock) void k_sum_abs(const int64_t* __restrict__ part, int64_t ld, int64_t nb, int S,
+                                                          Stats* __restrict__ st) {
+  __shared__ int64_t sh[kFinishBlock / 64];
+  for (int sp = 0; sp < S; ++sp) {
+    int64_t x = 0;
+#pragma unroll 4
+    for (int64_t b = threadIdx.x; b < nb; b += kFinishBlock) x += part[sp * ld + b];
+    x = wave_sum(x);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = x;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      for (int w = 1; w < kFinishBlock / 64; ++w) x += sh[w];
+      st->abs_pop[sp] = static_cast<unsigned long long>(x);
+    }
+    __syncthreads();
+  }
+}
+
+// Sort values of the main list (a loaded list; the insertion keeps them up).
+__global__ void k_rank_list(KeyPlan kp, int W, int64_t n, int64_t cap, const uint64_t* __restrict__ det,
+                            uint64_t* __restrict__ rank) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int64_t nl = list_len(pn, n);  // entries past it (up to the bound n) are marked dead
-  cyc = cycle_of(pcyc, cyc);
-  bool alive = false;
-  if (i < nl && is_core_entry(s, det, cap, i)) {
-    alive = true;
-  } else if (i < nl) {
-    if (s.real_amps) {
-      if (replay) {
-        fqd::ReplayRng rng{rbuf, rbase + mdraw_off[i], rbase + mdraw_off[i + 1], false};
-        for (int sp = 0; sp < s.S; ++sp)
-          pop_new[sp * cap + i] = fqd::stoch_round_pop(rng, pop_new[sp * cap + i], s.rf);
-      } else {
-        fqd::Philox rng(seed, static_cast<uint32_t>(i), static_cast<uint32_t>(i >> 32),
-                        cyc ^ (fqd::kDrawRoundMain << 24));
-        for (int sp = 0; sp < s.S; ++sp)
-          pop_new[sp * cap + i] = fqd::stoch_round_pop(rng, pop_new[sp * cap + i], s.rf);
-      }
-    }
-    for (int sp = 0; sp < s.S; ++sp) alive = alive || pop_new[sp * cap + i] != 0;
-  }
-  store_ballot(alive, i, n, mmask, mcnt);
-}
-
-// round_low_population_spawns for new-determinant candidates.
-__global__ __launch_bounds__(kBlock) void k_round_new(Sys s, const int64_t* __restrict__ pnr, int64_t rb,
-                                                      int64_t* __restrict__ rpop,
-                                                      const int64_t* __restrict__ rstate, int64_t scap, int replay,
-                                                      const double* __restrict__ rbuf, int64_t rbase,
-                                                      const int64_t* __restrict__ ndraw_off, uint64_t seed,
-                                                      uint32_t cyc, uint64_t* __restrict__ nmask,
-                                                      int64_t* __restrict__ ncnt, const uint32_t* __restrict__ pcyc) {
-  const int64_t r = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  cyc = cycle_of(pcyc, cyc);
-  const int64_t nruns = *pnr;
-  bool alive = false;
-  if (r < nruns && rstate[r] == 2) {
-    if (s.real_amps) {
-      if (replay) {
-        fqd::ReplayRng rng{rbuf, rbase + ndraw_off[r], rbase + ndraw_off[r + 1], false};
-        for (int sp = 0; sp < s.S; ++sp) rpop[sp * scap + r] = fqd::stoch_round_pop(rng, rpop[sp * scap + r], s.rf);
-      } else {
-        fqd::Philox rng(seed, static_cast<uint32_t>(r), static_cast<uint32_t>(r >> 32),
-                        cyc ^ (fqd::kDrawRoundSpawn << 24));
-        for (int sp = 0; sp < s.S; ++sp) rpop[sp * scap + r] = fqd::stoch_round_pop(rng, rpop[sp * scap + r], s.rf);
-      }
-    }
-    for (int sp = 0; sp < s.S; ++sp) alive = alive || rpop[sp * scap + r] != 0;
-  }
-  store_ballot(alive, r, rb, nmask, ncnt);  // words up to the bound rb >= nruns (zero past nruns)
+  if (i >= n) return;
+  uint64_t f[FQ_MAX_WORDS] = {0, 0}, key[2];
+  FQ_FOR_WORDS(w, W) f[w] = det[w * cap + i];
+  kp.flag_bits = 0;
+  make_key(kp, f, W, 0, key);
+  for (int w = 0; w < kp.kw; ++w) rank[w * cap + i] = key[w];
 }
 
 __global__ void k_zero(int64_t* __restrict__ p, int64_t n) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i < n) p[i] = 0;
-}
-
-// Decide the new list length; insertion is skipped when the main list would
-// overflow (insert_new_walkers' psip_list%error path).
-// pnr: the number of spawned runs (nullptr: none); also recorded in the stats.
-__global__ void k_finalize_counts(int64_t n, const int64_t* __restrict__ pnr, const int64_t* __restrict__ moff,
-                                  const uint64_t* __restrict__ mmask, const int64_t* __restrict__ noff,
-                                  const uint64_t* __restrict__ nmask, int64_t cap, Stats* __restrict__ st,
-                                  const int64_t* __restrict__ pn) {
-  n = list_len(pn, n);
-  const int64_t nruns = pnr ? *pnr : 0;
-  st->nruns = nruns;
-  const int64_t nmain = bit_rank(moff, mmask, n), nnew = bit_rank(noff, nmask, nruns);
-  if (nmain + nnew > cap) {
-    st->main_overflow = 1;
-    st->new_n = nmain;
-  } else {
-    st->new_n = nmain + nnew;
-  }
-}
-
-// Surviving main entries move up by their rank among survivors plus the number
-// of surviving new runs inserted at or before them: nrpos lists those runs'
-// insertion positions in rank order, non-decreasing because the runs are
-// sorted, so the count is an upper-bound search.  Each block takes the counts
-// bounding its 256 entries from bstart (k_block_starts) and stages that window
-// of nrpos in LDS when it fits (dense insertion), so each thread searches only
-// there.
-constexpr int kInsWin = 1024;
-// bstart[b] = number of surviving new runs inserted before main entry 256 b
-// (nrpos < 256 b), b in [0, nblk]: thread k (k <= nnew) fills the blocks whose
-// first entry lies in (nrpos[k-1], nrpos[k]].
-__global__ void k_block_starts(const int64_t* __restrict__ nrpos, const Stats* __restrict__ st,
-                               const int64_t* __restrict__ moff, const uint64_t* __restrict__ mmask, int64_t n,
-                               int64_t bound, int64_t nblk, int64_t* __restrict__ bstart,
-                               const int64_t* __restrict__ pn) {
-  const int64_t k = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (k > bound) return;
-  if (pn) {  // the list's length and blocks on the device
-    n = list_len(pn, n);
-    nblk = (n + kBlock - 1) / kBlock;
-  }
-  const int64_t nnew = st->main_overflow ? 0 : st->new_n - bit_rank(moff, mmask, n);
-  if (k > nnew) return;
-  const int64_t prev = k == 0 ? -1 : nrpos[k - 1];
-  const int64_t b_lo = prev < 0 ? 0 : prev / kBlock + 1;
-  const int64_t b_hi = k == nnew ? nblk : (nrpos[k] / kBlock < nblk ? nrpos[k] / kBlock : nblk);
-  for (int64_t b = b_lo; b <= b_hi; ++b) bstart[b] = k;
-}
-__device__ __forceinline__ int64_t upper_bound_pos(const int64_t* __restrict__ v, int64_t lo, int64_t hi, int64_t x) {
-  while (lo < hi) {  // first k in [lo, hi) with v[k] > x
-    const int64_t mid = (lo + hi) >> 1;
-    if (v[mid] <= x)
-      lo = mid + 1;
-    else
-      hi = mid;
-  }
-  return lo;
-}
-__global__ __launch_bounds__(kBlock) void k_scatter_main(Sys s, int64_t n, int64_t cap,
-                                                         const uint64_t* __restrict__ det,
-                                                         const int64_t* __restrict__ pop_new,
-                                                         const double* __restrict__ kii,
-                                                         const uint64_t* __restrict__ mmask,
-                                                         const int64_t* __restrict__ moff,
-                                                         const int64_t* __restrict__ nrpos,
-                                                         const int64_t* __restrict__ bstart, const Stats* __restrict__ st,
-                                                         uint64_t* __restrict__ det_out, int64_t* __restrict__ pop_out,
-                                                         double* __restrict__ kii_out, const int64_t* __restrict__ pn) {
-  __shared__ int64_t win[kInsWin];
-  n = list_len(pn, n);
-  const int64_t i0 = static_cast<int64_t>(blockIdx.x) * blockDim.x;
-  if (i0 >= n) return;  // whole block
-  const bool ovf = st->main_overflow != 0;
-  // c0 = runs inserted before i0 exactly; c1 >= runs inserted at or before i1
-  const int64_t c0 = ovf ? 0 : bstart[blockIdx.x], c1 = ovf ? 0 : bstart[blockIdx.x + 1];
-  const bool staged = c1 - c0 <= kInsWin;
-  if (staged)
-    for (int64_t q = threadIdx.x; q < c1 - c0; q += kBlock) win[q] = nrpos[c0 + q];
-  __syncthreads();
-  const int64_t i = i0 + threadIdx.x;
-  if (i >= n || !bit_get(mmask, i)) return;
-  int64_t shift;
-  if (staged) {
-    int a = 0, b = static_cast<int>(c1 - c0);
-    while (a < b) {
-      const int mid = (a + b) >> 1;
-      if (win[mid] <= i)
-        a = mid + 1;
-      else
-        b = mid;
-    }
-    shift = c0 + a;
-  } else {
-    shift = upper_bound_pos(nrpos, c0, c1, i);
-  }
-  const int64_t o = bit_rank(moff, mmask, i) + shift;
-  for (int w = 0; w < s.W; ++w) det_out[w * cap + o] = det[w * cap + i];
-  for (int sp = 0; sp < s.S; ++sp) pop_out[sp * cap + o] = pop_new[sp * cap + i];
-  kii_out[o] = kii[i];
-}
-
-// Surviving new runs in order: list[rank among survivors] = run index.
-// The surviving new runs in rank order, with their insertion positions.
-__global__ void k_new_list(const int64_t* __restrict__ pnr, const uint64_t* __restrict__ nmask,
-                           const int64_t* __restrict__ noff, const int64_t* __restrict__ rpos,
-                           int64_t* __restrict__ list, int64_t* __restrict__ nrpos) {
-  const int64_t nruns = *pnr;
-  const int64_t r = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (r < nruns && bit_get(nmask, r)) {
-    const int64_t k = bit_rank(noff, nmask, r);
-    list[k] = r;
-    nrpos[k] = rpos[r];
-  }
-}
-
-// Insert the surviving new runs, one thread each (list order = rank order),
-// with K_ii from the diagonal rule; a molecular system's dense pair tables are
-// staged in LDS when jk_lds (2 * norb^2 doubles) is nonzero.
-__global__ __launch_bounds__(kBlock) void k_scatter_new(Sys s, const int64_t* __restrict__ pnr, int64_t cap,
-                                                        int64_t scap,
-                                                        const uint64_t* __restrict__ rdet,
-                                                        const int64_t* __restrict__ rpop,
-                                                        const int64_t* __restrict__ rpos,
-                                                        const uint64_t* __restrict__ nmask,
-                                                        const int64_t* __restrict__ noff,
-                                                        const int64_t* __restrict__ list,
-                                                        const uint64_t* __restrict__ mmask,
-                                                        const int64_t* __restrict__ moff,
-                                                        const Stats* __restrict__ st,
-                                                        uint64_t* __restrict__ det_out, int64_t* __restrict__ pop_out,
-                                                        double* __restrict__ kii_out, const Sys* __restrict__ sys_arr,
-                                                        int jk_lds) {
-  extern __shared__ double jk[];
-  const int64_t nruns = *pnr;
-  const int64_t nnew = bit_rank(noff, nmask, nruns);
-  const int64_t k0 = static_cast<int64_t>(blockIdx.x) * blockDim.x;
-  if (k0 >= nnew || st->main_overflow) return;  // whole block: no surviving run left
-  const int nn = s.norb * s.norb;
-  if (jk_lds) {
-    for (int q = threadIdx.x; q < nn; q += kBlock) {
-      jk[q] = s.jmat[q];
-      jk[nn + q] = s.kmat[q];
-    }
-    __syncthreads();
-  }
-  const int64_t k = k0 + threadIdx.x;
-  if (k >= nnew) return;
-  const int64_t r = list[k];
-  const int64_t o = k + bit_rank(moff, mmask, rpos[r]);
-  uint64_t f[FQ_MAX_WORDS] = {0, 0};
-  FQ_FOR_WORDS(w, s.W) {
-    f[w] = rdet[w * scap + r];
-    det_out[w * cap + o] = f[w];
-  }
-  for (int sp = 0; sp < s.S; ++sp) pop_out[sp * cap + o] = rpop[sp * scap + r];
-  if (sys_arr) {  // batched: the instance's diagonal
-    const Sys& si = sys_arr[f[0] >> kInstShift];
-    f[0] &= kOrbMask;
-    kii_out[o] = fqd::diagonal(si, f) - si.H00;
-  } else if (jk_lds) {
-    kii_out[o] = fqd::diagonal_mol(s, f, jk, jk + nn) - s.H00;
-  } else {
-    kii_out[o] = fqd::diagonal(s, f) - s.H00;
-  }
-}
-
-// Sums of |pop| over the new list (its length read from the stats the
-// insertion wrote); grid-stride.
-__global__ __launch_bounds__(kBlock) void k_abs_pop(const Stats* __restrict__ stn, int64_t cap, int S,
-                                                    const int64_t* __restrict__ pop, int64_t* __restrict__ part_i) {
-  __shared__ unsigned long long sh[FQ_MAX_SPACES][kBlock];
-  const int64_t n = stn->new_n;
-  // exact integer sums: any grid and order give the same totals
-  for (int sp = 0; sp < FQ_MAX_SPACES; ++sp) {
-    unsigned long long v = 0;
-    if (sp < S)
-      for (int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x; i < n;
-           i += static_cast<int64_t>(gridDim.x) * kBlock) {
-        const int64_t p = pop[sp * cap + i];
-        v += static_cast<unsigned long long>(p < 0 ? -p : p);
-      }
-    sh[sp][threadIdx.x] = v;
-  }
-  __syncthreads();
-  for (int k = kBlock / 2; k > 0; k >>= 1) {
-    if (threadIdx.x < k)
-      for (int sp = 0; sp < FQ_MAX_SPACES; ++sp) sh[sp][threadIdx.x] += sh[sp][threadIdx.x + k];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0)
-    for (int sp = 0; sp < FQ_MAX_SPACES; ++sp) part_i[sp * gridDim.x + blockIdx.x] = static_cast<int64_t>(sh[sp][0]);
-}
-
-__global__ __launch_bounds__(kBlock) void k_sum_abs(const int64_t* __restrict__ part_i, int nb, Stats* __restrict__ st) {
-  __shared__ unsigned long long sh[FQ_MAX_SPACES][kBlock];
-  unsigned long long acc[FQ_MAX_SPACES] = {0, 0};
-  for (int b = threadIdx.x; b < nb; b += kBlock)
-    for (int sp = 0; sp < FQ_MAX_SPACES; ++sp) acc[sp] += static_cast<unsigned long long>(part_i[sp * nb + b]);
-  for (int sp = 0; sp < FQ_MAX_SPACES; ++sp) sh[sp][threadIdx.x] = acc[sp];
-  __syncthreads();
-  for (int k = kBlock / 2; k > 0; k >>= 1) {
-    if (threadIdx.x < k)
-      for (int sp = 0; sp < FQ_MAX_SPACES; ++sp) sh[sp][threadIdx.x] += sh[sp][threadIdx.x + k];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0)
-    for (int sp = 0; sp < FQ_MAX_SPACES; ++sp) st->abs_pop[sp] = sh[sp][0];
 }
 
 // ---------------------------------------------------------------------------
@@ -2751,7 +2923,8 @@ int setup_sort(fq_engine* e) {
   // The spawned list as determinant words and records (sdet, srec) is only
   // read before the sort (replay walk, caller-supplied lists, rank exchange);
   // it shares the memory of the sort's second buffers.
-  if (kw != e->sort_kw || !e->kbuf[0]) {
+  const bool new_kw = kw != e->sort_kw || !e->kbuf[0];
+  if (new_kw) {
     for (int b = 0; b < 2; ++b) {
       dfree(e->kbuf[b]);
       rc |= dalloc(&e->kbuf[b], (b == 0 ? kw : std::max(kw, e->W)) * scap);
@@ -2765,10 +2938,26 @@ int setup_sort(fq_engine* e) {
   if (!e->perm && e->par.rng_mode == FQ_RNG_REPLAY) rc |= dalloc(&e->perm, scap);
   if (!e->pass_cnt) rc |= dalloc(&e->pass_cnt, 512 * kSortBlocks);
   if (!e->pass_off) rc |= dalloc(&e->pass_off, 512 * kSortBlocks + 1);
-  if (!e->run_tcnt) rc |= dalloc(&e->run_tcnt, ceil_div(scap, kRunTile) + 2);
-  if (!e->run_toff) rc |= dalloc(&e->run_toff, ceil_div(scap, kRunTile) + 2);
-  if (!e->run_tfirst) rc |= dalloc(&e->run_tfirst, ceil_div(scap, kRunTile) + 2);
-  if (!e->run_tpre) rc |= dalloc(&e->run_tpre, 3 * e->S * (ceil_div(scap, kRunTile) + 2));
+  const int64_t rtiles = ceil_div(scap, kRunTile) + 2;
+  if (!e->run_tcnt) rc |= dalloc(&e->run_tcnt, rtiles);
+  if (!e->run_toff) rc |= dalloc(&e->run_toff, rtiles);
+  if (!e->run_tfirst) rc |= dalloc(&e->run_tfirst, rtiles);
+  if (!e->run_tpre) rc |= dalloc(&e->run_tpre, 3 * e->S * rtiles);
+  if (!e->run_win) rc |= dalloc(&e->run_win, rtiles);
+  if (!e->new_cnt) rc |= dalloc(&e->new_cnt, rtiles);
+  if (!e->new_off) rc |= dalloc(&e->new_off, rtiles);
+  for (int b = 0; b < 2; ++b)
+    if (!e->new_pos[b]) rc |= dalloc(&e->new_pos[b], scap);
+  if (!e->new_pop) rc |= dalloc(&e->new_pop, e->S * scap);
+  if (new_kw) {
+    dfree(e->new_val);
+    rc |= dalloc(&e->new_val, kw * scap);
+  }
+  // the main list's sort values (a determinant that is its own value needs none)
+  if (new_kw || !e->rank_words)
+    for (int b = 0; b < 2; ++b) dfree(e->mrank[b]);
+  for (int b = 0; b < 2 && e->rank_words; ++b)
+    if (!e->mrank[b]) rc |= dalloc(&e->mrank[b], kw * e->cap);
   return rc == FQ_OK ? FQ_OK : FQ_ERR_NOMEM;
 }
 
@@ -2799,11 +2988,17 @@ int sort_pass_db(fq_engine* e, int src, int64_t ns, const int64_t* pns, int shif
   return db == 9 ? sort_pass<KW, S, 9>(e, src, ns, pns, shift) : sort_pass<KW, S, 8>(e, src, ns, pns, shift);
 }
 
-// Sort the spawned list and reduce runs; leaves the device address of the run
-// count in p_nruns and a host bound of it in run_bound.  The list holds ns
-// entries, or, when pns is given (production, no host wait for the length),
-// *pns entries with ns a bound of them.
-int sort_and_reduce(fq_engine* e, int64_t ns, const int64_t* pns, bool replay) {
+// The main list's sort values in buffer c.
+const uint64_t* main_values(const fq_engine* e, int c) { return e->rank_words ? e->mrank[c] : e->det[c]; }
+constexpr int64_t kNewBlocks = 1024;  // most blocks of the new determinants' insertion
+constexpr size_t kInsertLdsMax = 60 * 1024;  // their tables, beside the kernel's own LDS in the default 64 KB
+
+// Sort the spawned list, reduce its runs and merge them with the main list;
+// leaves the tiles' new determinants in the sort's idle buffers (new_src) and
+// the number of run tiles in run_tiles.  The list holds ns entries, or, when
+// pns is given (production, no host wait for the length), *pns entries with ns
+// a bound of them.
+int sort_and_reduce(fq_engine* e, int64_t ns, const int64_t* pns, bool replay, uint32_t cyc) {
   const bool keys_ready = e->keys_ready;  // made by the spawning pass for this spawned list
   e->keys_ready = false;
   const int64_t scap = e->scap;
@@ -2842,125 +3037,187 @@ int sort_and_reduce(fq_engine* e, int64_t ns, const int64_t* pns, bool replay) {
     pns = nullptr;
   }
   mark(e, e->pev[5]);
+  // Runs: totals, merge with the main list, the tiles' new determinants.
   const int64_t nt = ceil_div(ns, kRunTile);
-  int64_t* nruns = e->run_toff + nt;
+  e->run_tiles = nt;
+  e->new_src = 1 - src;
   if (ns > 0) {
+    const int64_t* dn = e->capturing ? e->dn : nullptr;
+    const uint64_t* mrank = main_values(e, e->cur);
     auto cnt = kw == 1 ? (S == 1 ? k_run_count<1, 1> : k_run_count<1, 2>)
                        : (S == 1 ? k_run_count<2, 1> : k_run_count<2, 2>);
-    hipLaunchKernelGGL(cnt, dim3(static_cast<unsigned>(nt)), dim3(kBlock), 0, st, e->kbuf[src], e->pbuf[src],
-                       pns, ns, scap, e->flag_bits, e->run_tcnt, e->run_tfirst, e->run_tpre);
-    const int rc = scan_exclusive(e, e->run_tcnt, e->run_toff, nt);
-    if (rc != FQ_OK) return rc;
-    KeyPlan kp = key_plan(e);
-    const size_t tab = binom_bytes(e);
-    kp.binom_lds = tab > 0 && tab <= kBinomLdsMax;
-    // one-word keys: 64-bit rank arithmetic
-    auto kern = kw == 1 ? (S == 1 ? k_runs<1, 1, false> : k_runs<1, 2, false>)
-                        : (S == 1 ? k_runs<2, 1, true> : k_runs<2, 2, true>);
-    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(nt)), dim3(kBlock), kp.binom_lds ? tab : 0, st, e->sys, kp,
-                       e->kbuf[src], e->pbuf[src], ns, scap, e->run_toff, e->run_tfirst, e->run_tpre, nt, e->rdet,
-                       e->rpop, e->rflag, e->rstate, pns);
-  }
-  // The number of runs stays on the device; kernels size their grids by a
-  // host bound: ns in production, the exact count in replay (read there
-  // anyway, for the rounding draws).
-  int64_t bound = 0;
-  e->p_nruns = nullptr;
-  if (ns > 0) {
-    e->p_nruns = nruns;
-    bound = ns;
-    if (replay) {
-      FQ_HIP(hipMemcpyAsync(&bound, nruns, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-      FQ_HIP(hipStreamSynchronize(st));
+    hipLaunchKernelGGL(cnt, dim3(static_cast<unsigned>(nt)), dim3(kBlock), 0, st, e->kbuf[src], e->pbuf[src], pns, ns,
+                       scap, e->flag_bits, mrank, e->n, e->cap, dn, nt, e->run_tcnt, e->run_tfirst, e->run_tpre,
+                       e->run_win);
+    if (nt > kPrefixMax) {
+      const int rc = scan_exclusive(e, e->run_tcnt, e->run_toff, nt);
+      if (rc != FQ_OK) return rc;
     }
+    RunArgs g{};
+    g.keys = e->kbuf[src];
+    g.pay = e->pbuf[src];
+    g.ns = ns;
+    g.pns = pns;
+    g.stride = scap;
+    g.fb = e->flag_bits;
+    g.tcnt = e->run_tcnt;
+    g.toff = nt > kPrefixMax ? e->run_toff : nullptr;
+    g.tfirst = e->run_tfirst;
+    g.tpre = e->run_tpre;
+    g.win = e->run_win;
+    g.ntiles = nt;
+    g.mrank = mrank;
+    g.n = e->n;
+    g.pmain = dn;
+    g.cap = e->cap;
+    g.pop_new = e->pop_new;
+    g.initiator = e->sys.initiator;
+    g.real_amps = e->sys.real_amps;
+    g.replay = replay ? 1 : 0;
+    g.rf = e->sys.rf;
+    g.seed = e->par.philox_seed;
+    g.cyc = cyc;
+    g.pcyc = e->capturing ? e->dcyc : nullptr;
+    g.nval = e->kbuf[1 - src];
+    g.npop = e->pbuf[1 - src];
+    g.npos = e->new_pos[0];
+    g.ncnt = e->new_cnt;
+    g.st = e->d_stats;
+    auto kern = kw == 1 ? (S == 1 ? k_runs<1, 1> : k_runs<1, 2>) : (S == 1 ? k_runs<2, 1> : k_runs<2, 2>);
+    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(nt)), dim3(kBlock), 0, st, g);
   }
   mark(e, e->pev[6]);
-  e->run_bound = bound;
   return FQ_OK;
 }
 
 // Annihilation proper: merge runs, round, compact, insert.  ns spawned
 // entries are in the spawned list; pop_new holds the post-death populations.
 int annihilate(fq_engine* e, int64_t ns, const int64_t* pns, bool replay, uint32_t cyc, int64_t& rng_pos) {
-  int rc = sort_and_reduce(e, ns, pns, replay);
+  int rc = sort_and_reduce(e, ns, pns, replay, cyc);
   if (rc != FQ_OK) return rc;
-  const int64_t nruns = e->run_bound;  // a bound in production, the count in replay
-  const int64_t* pnr = e->p_nruns;
+  const int64_t ntiles = e->run_tiles;
   // a graph-captured cycle: n is a bound of the list's length, read on the device from dn
   const int64_t n = e->n, cap = e->cap, scap = e->scap;
   const int64_t* dn = e->capturing ? e->dn : nullptr;
   const uint32_t* dcyc = e->capturing ? e->dcyc : nullptr;
-  const int c = e->cur;
+  const int c = e->cur, o = 1 - c, kw = e->sort_kw;
   hipStream_t st = e->stream;
+  uint64_t* nval = e->kbuf[e->new_src];
+  int64_t* npop = e->pbuf[e->new_src];
   mark(e, e->pev[7]);
-  if (nruns > 0) {
-    hipLaunchKernelGGL(k_merge_bounds, dim3(grid_for(grid_for(nruns))), dim3(kBlock), 0, st, pnr, n, cap, e->W,
-                       e->det[c], e->rdet, scap, e->mwin, dn);
-    hipLaunchKernelGGL(k_merge_runs, dim3(grid_for(nruns)), dim3(kBlock), 0, st, e->sys, pnr, n, cap, e->det[c],
-                       e->pop_new, e->rdet, e->rpop, e->rflag, scap, e->mwin, e->rpos, e->rstate, dn);
-  }
   // Rounding draws (replay: main list first, then new candidates, in order).
   int64_t main_draws = 0, new_draws = 0;
-  if (replay && e->sys.real_amps) {
-    hipLaunchKernelGGL(k_count_round_main, dim3(grid_for(n)), dim3(kBlock), 0, st, e->sys, n, cap, e->pop_new,
-                       e->det[c], e->mdraw);
-    rc = scan_exclusive(e, e->mdraw, e->mdraw_off, n);
-    if (rc != FQ_OK) return rc;
-    if (nruns > 0) {
-      hipLaunchKernelGGL(k_count_round_new, dim3(grid_for(nruns)), dim3(kBlock), 0, st, e->sys, nruns, e->rpop,
-                         e->rstate, scap, e->ndraw);
-      rc = scan_exclusive(e, e->ndraw, e->ndraw_off, nruns);
+  if (replay) {
+    if (e->sys.real_amps) {
+      hipLaunchKernelGGL(k_count_round_main, dim3(grid_for(n)), dim3(kBlock), 0, st, e->sys, n, cap, e->pop_new,
+                         e->det[c], e->mdraw);
+      rc = scan_exclusive(e, e->mdraw, e->mdraw_off, n);
       if (rc != FQ_OK) return rc;
     }
-    FQ_HIP(hipMemcpyAsync(&main_draws, e->mdraw_off + n, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-    if (nruns > 0) FQ_HIP(hipMemcpyAsync(&new_draws, e->ndraw_off + nruns, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-    FQ_HIP(hipStreamSynchronize(st));
-    if (rng_pos + main_draws + new_draws > e->rng_end) return FQ_ERR_RNG_EXHAUSTED;
+    if (ntiles > 0) {
+      hipLaunchKernelGGL(k_count_round_new, dim3(static_cast<unsigned>(ntiles)), dim3(kBlock), 0, st, e->sys,
+                         e->new_cnt, npop, scap, e->ndraw);
+      rc = scan_exclusive(e, e->ndraw, e->ndraw_off, ntiles);
+      if (rc != FQ_OK) return rc;
+    }
+    if (e->sys.real_amps) {
+      FQ_HIP(hipMemcpyAsync(&main_draws, e->mdraw_off + n, sizeof(int64_t), hipMemcpyDeviceToHost, st));
+      if (ntiles > 0)
+        FQ_HIP(hipMemcpyAsync(&new_draws, e->ndraw_off + ntiles, sizeof(int64_t), hipMemcpyDeviceToHost, st));
+      FQ_HIP(hipStreamSynchronize(st));
+      if (rng_pos + main_draws + new_draws > e->rng_end) return FQ_ERR_RNG_EXHAUSTED;
+    }
+    if (ntiles > 0)
+      hipLaunchKernelGGL(k_replay_round_new, dim3(static_cast<unsigned>(ntiles)), dim3(kBlock), 0, st, e->sys, kw,
+                         e->new_cnt, nval, npop, e->new_pos[0], scap, e->rng_buf, rng_pos + main_draws, e->ndraw_off);
   }
-  const uint64_t seed = e->par.philox_seed;
-  hipLaunchKernelGGL(k_round_main, dim3(grid_for(n)), dim3(kBlock), 0, st, e->sys, n, cap, e->pop_new,
-                     replay ? 1 : 0, e->rng_buf, rng_pos, e->mdraw_off, seed, cyc, e->mmask, e->mcnt, e->det[c], dn,
-                     dcyc);
-  if (nruns > 0)
-    hipLaunchKernelGGL(k_round_new, dim3(grid_for(nruns)), dim3(kBlock), 0, st, e->sys, pnr, nruns, e->rpop, e->rstate,
-                       scap, replay ? 1 : 0, e->rng_buf, rng_pos + main_draws, e->ndraw_off, seed, cyc, e->nmask,
-                       e->ncnt, dcyc);
-  rng_pos += main_draws + new_draws;
-  rc = scan_exclusive(e, e->mcnt, e->moff, ceil_div(n, 64));
-  if (rc != FQ_OK) return rc;
-  if (nruns > 0) {
-    rc = scan_exclusive(e, e->ncnt, e->noff, ceil_div(nruns, 64));
+  const int64_t mtiles = std::max<int64_t>(1, ceil_div(n, kMainTile));
+  if (ntiles > kPrefixMax) {
+    rc = scan_exclusive(e, e->new_cnt, e->new_off, ntiles);
     if (rc != FQ_OK) return rc;
-  } else {
-    hipLaunchKernelGGL(k_zero, dim3(1), dim3(kBlock), 0, st, e->noff, 1);
   }
-  if (nruns > 0)
-    hipLaunchKernelGGL(k_new_list, dim3(grid_for(nruns)), dim3(kBlock), 0, st, pnr, e->nmask, e->noff, e->rpos,
-                       e->nlist, e->nrpos);
-  hipLaunchKernelGGL(k_finalize_counts, dim3(1), dim3(1), 0, st, n, nruns > 0 ? pnr : nullptr, e->moff, e->mmask,
-                     e->noff, e->nmask, cap, e->d_stats, dn);
-  const int o = 1 - c;
-  const int64_t nblk = ceil_div(n, kBlock);
-  hipLaunchKernelGGL(k_block_starts, dim3(grid_for(nruns + 1)), dim3(kBlock), 0, st, e->nrpos, e->d_stats, e->moff,
-                     e->mmask, n, nruns, nblk, e->bstart, dn);
-  hipLaunchKernelGGL(k_scatter_main, dim3(grid_for(n)), dim3(kBlock), 0, st, e->sys, n, cap, e->det[c], e->pop_new,
-                     e->kii[c], e->mmask, e->moff, e->nrpos, e->bstart, e->d_stats, e->det[o], e->pop[o], e->kii[o],
-                     dn);
-  if (nruns > 0) {
-    // dense pair tables in LDS for the diagonal when they fit in 32 KB
+  RoundArgs r{};
+  r.s = e->sys;
+  r.n = n;
+  r.pn = dn;
+  r.cap = cap;
+  r.mtiles = mtiles;
+  r.det = e->det[c];
+  r.pop_new = e->pop_new;
+  r.replay = replay ? 1 : 0;
+  r.rbuf = e->rng_buf;
+  r.rbase = rng_pos;
+  r.mdraw_off = e->mdraw_off;
+  r.seed = e->par.philox_seed;
+  r.cyc = cyc;
+  r.pcyc = dcyc;
+  r.mmask = e->mmask;
+  r.mpre = e->mpre;
+  r.mcnt = e->mcnt;
+  r.KW = kw;
+  r.scap = scap;
+  r.ntiles = ntiles;
+  r.ncnt = e->new_cnt;
+  r.noff = ntiles > kPrefixMax ? e->new_off : nullptr;
+  r.nval = nval;
+  r.npop = npop;
+  r.npos = e->new_pos[0];
+  r.lval = e->new_val;
+  r.lpop = e->new_pop;
+  r.lpos = e->new_pos[1];
+  r.st = e->d_stats;
+  hipLaunchKernelGGL(k_round, dim3(static_cast<unsigned>(mtiles + ntiles)), dim3(kBlock), 0, st, r);
+  rng_pos += main_draws + new_draws;
+  if (mtiles > kPrefixMax) {  // offsets first: every tile's block would add too many counts
+    rc = scan_exclusive(e, e->mcnt, e->moff, mtiles);
+    if (rc != FQ_OK) return rc;
+  }
+  InsertArgs g{};
+  g.s = e->sys;
+  g.n = n;
+  g.pn = dn;
+  g.cap = cap;
+  g.mtiles = mtiles;
+  g.det = e->det[c];
+  g.rank = e->mrank[c];
+  g.rank_words = e->rank_words ? kw : 0;
+  g.pop_new = e->pop_new;
+  g.kii = e->kii[c];
+  g.mmask = e->mmask;
+  g.mpre = e->mpre;
+  g.mcnt = e->mcnt;
+  g.moff_in = mtiles > kPrefixMax ? e->moff : nullptr;
+  g.moff = e->moff;
+  g.lpos = e->new_pos[1];
+  g.lval = e->new_val;
+  g.lpop = e->new_pop;
+  g.scap = scap;
+  g.st = e->d_stats;
+  g.det_out = e->det[o];
+  g.rank_out = e->mrank[o];
+  g.pop_out = e->pop[o];
+  g.kii_out = e->kii[o];
+  g.abs_part = e->abs_part;
+  g.abs_ld = cap / kMainTile + 2 + kNewBlocks;
+  hipLaunchKernelGGL(k_scatter_main, dim3(static_cast<unsigned>(mtiles)), dim3(kBlock), 0, st, g);
+  int64_t nblk = mtiles;
+  if (ns > 0) {
+    // dense pair tables in LDS for the diagonal when they fit in 32 KB, the binomial table when it fits beside them
     const size_t jk = e->sys.system == FQ_SYS_READ_IN && !e->batched
                           ? 2 * sizeof(double) * static_cast<size_t>(e->sys.norb) * e->sys.norb
                           : 0;
-    const bool use_lds = jk > 0 && jk <= 32768;
-    hipLaunchKernelGGL(k_scatter_new, dim3(grid_for(nruns)), dim3(kBlock), use_lds ? jk : 0, st, e->sys, pnr, cap,
-                       scap, e->rdet, e->rpop, e->rpos, e->nmask, e->noff, e->nlist, e->mmask, e->moff, e->d_stats,
-                       e->det[o], e->pop[o], e->kii[o], e->batched ? e->d_sys_arr : nullptr, use_lds ? 1 : 0);
+    const bool use_jk = jk > 0 && jk <= 32768;
+    KeyPlan kp = key_plan(e);
+    const size_t tab = binom_bytes(e) / (kw == 1 ? 2 : 1);
+    kp.binom_lds = tab > 0 && tab + (use_jk ? jk : 0) <= kInsertLdsMax;
+    const unsigned nb = static_cast<unsigned>(std::min<int64_t>(ceil_div(ns, kBlock), kNewBlocks));
+    hipLaunchKernelGGL(kw == 1 ? k_scatter_new<false> : k_scatter_new<true>, dim3(nb), dim3(kBlock),
+                       (use_jk ? jk : 0) + (kp.binom_lds ? tab : 0), st, g, kp, e->batched ? e->d_sys_arr : nullptr,
+                       use_jk ? 1 : 0);
+    nblk += nb;
   }
   mark(e, e->pev[8]);
-  // the new list holds at most n + nruns entries
-  const unsigned nba = std::min<unsigned>(grid_for(std::min(n + nruns, cap)), 2048);
-  hipLaunchKernelGGL(k_abs_pop, dim3(nba), dim3(kBlock), 0, st, e->d_stats, cap, e->S, e->pop[o], e->part_i);
-  hipLaunchKernelGGL(k_sum_abs, dim3(1), dim3(kBlock), 0, st, e->part_i, static_cast<int>(nba), e->d_stats);
+  hipLaunchKernelGGL(k_sum_abs, dim3(1), dim3(kFinishBlock), 0, st, e->abs_part, g.abs_ld, nblk, e->S, e->d_stats);
   if (e->capturing) return FQ_OK;  // the caller reads the stats when the graph has run
   rc = sync_stats(e);
   if (rc != FQ_OK) return rc;
@@ -3128,6 +3385,8 @@ int build_heat_bath(fq_engine* e) {
 template <class T>
 int upload(T** dst, const T* src, int64_t count, hipStream_t st);
 
+constexpr int sort_passes(int bits) { return bits < 9 ? 1 : (bits + 8) / 9; }  // 8- or 9-bit digits
+
 // Binomial table and value width of the sort keys (combinatorial ranks).
 int setup_rank_keys(fq_engine* e) {
   const int nb = e->sys.nbasis, nel = e->sys.nel;
@@ -3150,6 +3409,11 @@ int setup_rank_keys(fq_engine* e) {
   unsigned __int128 top = row[nel] - 1;  // largest rank: C(nb, nel) - 1
   int bits = 1;
   while (bits < 128 && (top >> bits) != 0) ++bits;
+  // A one-word determinant that sorts in as many passes as its rank is its own
+  // sort value: no ranks are kept beside the main list and nothing is unranked.
+  // (18 electrons in 36 spin orbitals, 3e6 determinants: k_scatter_main 46 -> 38
+  // us without the 16 bytes of ranks per entry, k_scatter_new 26 -> 14 us.)
+  if (e->W == 1 && nb + e->S <= 64 && sort_passes(nb) <= sort_passes(bits)) return FQ_OK;
   e->rank_bits = bits;
   e->rank_words = bits > 64 ? 2 : 1;
   return upload(&e->d_binom, tab.data(), static_cast<int64_t>(tab.size()), e->stream);
@@ -3298,9 +3562,12 @@ int alloc_engine(fq_engine* e) {
   rc |= dalloc(&e->nat, S * cap + 1);  // det-major (det, space) entries
   rc |= dalloc(&e->att_off, S * cap + 1);
   rc |= dalloc(&e->flags, cap);
-  rc |= dalloc(&e->mmask, cap / 64 + 2);
-  rc |= dalloc(&e->mcnt, cap / 64 + 2);
-  rc |= dalloc(&e->moff, cap / 64 + 2);
+  const int64_t mtiles = cap / kMainTile + 2;
+  rc |= dalloc(&e->mmask, mtiles * (kMainTile / 64));
+  rc |= dalloc(&e->mpre, mtiles * (kMainTile / 64));
+  rc |= dalloc(&e->mcnt, mtiles);
+  rc |= dalloc(&e->moff, mtiles);
+  rc |= dalloc(&e->abs_part, S * (mtiles + kNewBlocks));
   const bool replay = e->par.rng_mode == FQ_RNG_REPLAY;
   if (replay) {  // rounding-draw counts of the replay stream
     rc |= dalloc(&e->mdraw, cap + 1);
@@ -3316,22 +3583,10 @@ int alloc_engine(fq_engine* e) {
   rc |= dalloc(&e->tile_cnt, e->bcap / kSpawnTile + 2);
   rc |= dalloc(&e->tile_off, e->bcap / kSpawnTile + 2);
   rc |= dalloc(&e->tile_win, 2 * (e->bcap / kSpawnTile + 2));
-  rc |= dalloc(&e->rdet, W * scap);
-  rc |= dalloc(&e->rpop, S * scap);
-  rc |= dalloc(&e->rflag, scap);
-  rc |= dalloc(&e->rpos, scap);
-  rc |= dalloc(&e->rstate, scap);
-  rc |= dalloc(&e->nlist, scap);
-  rc |= dalloc(&e->nrpos, scap);
-  rc |= dalloc(&e->bstart, cap / kBlock + 2);
   rc |= dalloc(&e->d_sysp, 1);
-  rc |= dalloc(&e->mwin, 2 * (scap / kBlock + 2));
-  rc |= dalloc(&e->nmask, scap / 64 + 2);
-  rc |= dalloc(&e->ncnt, scap / 64 + 2);
-  rc |= dalloc(&e->noff, scap / 64 + 2);
   if (replay) {
-    rc |= dalloc(&e->ndraw, scap + 1);
-    rc |= dalloc(&e->ndraw_off, scap + 1);
+    rc |= dalloc(&e->ndraw, scap / kRunTile + 2);
+    rc |= dalloc(&e->ndraw_off, scap / kRunTile + 2);
   }
   rc |= dalloc(&e->d_stats, 1);
   return rc == FQ_OK ? FQ_OK : FQ_ERR_NOMEM;
@@ -3557,6 +3812,9 @@ int fq_load(fq_engine* e, const uint64_t* states, const int64_t* pops, const dou
   for (int s = 0; s < S && n > 0; ++s)
     FQ_HIP(hipMemcpyAsync(e->pop[0] + s * e->cap, dp.data() + s * n, 8 * n, hipMemcpyHostToDevice, e->stream));
   if (n > 0) FQ_HIP(hipMemcpyAsync(e->kii[0], dat, 8 * n, hipMemcpyHostToDevice, e->stream));
+  if (n > 0 && e->rank_words)
+    hipLaunchKernelGGL(k_rank_list, dim3(grid_for(n)), dim3(kBlock), 0, e->stream, key_plan(e), W, n, e->cap,
+                       e->det[0], e->mrank[0]);
   FQ_HIP(hipStreamSynchronize(e->stream));
   e->n = n;
   e->att_bound = -1;
@@ -4788,6 +5046,8 @@ void fq_destroy(fq_engine* e) {
     dfree(e->pop[b]);
     dfree(e->kii[b]);
     dfree(e->kbuf[b]);
+    dfree(e->mrank[b]);
+    dfree(e->new_pos[b]);
   }
   dfree(e->pop_new);
   dfree(e->nat);
@@ -4795,6 +5055,13 @@ void fq_destroy(fq_engine* e) {
   dfree(e->flags);
   release_determ(e);
   dfree(e->mmask);
+  dfree(e->mpre);
+  dfree(e->abs_part);
+  dfree(e->run_win);
+  dfree(e->new_cnt);
+  dfree(e->new_off);
+  dfree(e->new_val);
+  dfree(e->new_pop);
   dfree(e->mcnt);
   dfree(e->moff);
   dfree(e->mdraw);
@@ -4818,19 +5085,7 @@ void fq_destroy(fq_engine* e) {
   dfree(e->run_toff);
   dfree(e->run_tfirst);
   dfree(e->run_tpre);
-  dfree(e->rdet);
-  dfree(e->rpop);
-  dfree(e->rflag);
-  dfree(e->rpos);
-  dfree(e->rstate);
-  dfree(e->nlist);
-  dfree(e->nrpos);
-  dfree(e->bstart);
   dfree(e->d_sysp);
-  dfree(e->mwin);
-  dfree(e->nmask);
-  dfree(e->ncnt);
-  dfree(e->noff);
   dfree(e->ndraw);
   dfree(e->ndraw_off);
   for (auto*& p : e->scan_tmp) dfree(p);
