@@ -334,8 +334,7 @@ struct fq_engine {
   bool graph_on = false;
   char* h_in = nullptr;       // pinned: [n][cycle index][tau, shift, E_proj per instance]
   char* d_in = nullptr;
-  Stats* h_gstats = nullptr;  // pinned copies the graph writes at its end
-  double* h_god = nullptr;
+  double* h_god = nullptr;    // pinned copies the graph writes at its end
   int64_t* h_goi = nullptr;
   struct GraphEntry {
     int c;
@@ -391,6 +390,7 @@ struct fq_engine {
   float* mlp_flat = nullptr;  // 2*nbasis ones: weights of determinants without a row
   int64_t att_bound = -1;            // bound of the next cycle's attempts (-1: unknown)
   bool keys_ready = false;           // the spawning pass made this cycle's sort keys
+  int est_blocks = 0;                // k_det_pass blocks whose partials k_finish adds (0: none)
   int new_src = 0;                   // the sort's idle buffers after this cycle's passes
   int64_t run_tiles = 0;             // run tiles of this cycle's spawned list (a bound of it while captured)
   int64_t mlp_tab_rows = 0;
@@ -404,7 +404,7 @@ struct fq_engine {
   int64_t* pop[2] = {nullptr, nullptr};
   double* kii[2] = {nullptr, nullptr};
   int64_t* pop_new = nullptr;   // S*cap, populations after death
-  int64_t* nat = nullptr;       // S*cap attempts per (det, space), then scanned
+  int32_t* nat = nullptr;       // S*cap attempts per (det, space)
   int64_t* att_off = nullptr;   // S*cap+1
   int64_t* flags = nullptr;     // cap parent initiator flags
   uint64_t* mrank[2] = {nullptr, nullptr};  // sort_kw*cap: the entries' sort values (ranks), as the list's buffers
@@ -416,13 +416,14 @@ struct fq_engine {
   int64_t* mdraw_off = nullptr;
   double* part_d = nullptr;     // 4 * (cap/256+1) block partials
   int64_t* part_i = nullptr;    // 2 * (cap/256+1)
+  int64_t* blk_att = nullptr;   // cap/256+2: attempts of k_det_pass's blocks
+  int64_t* blk_off = nullptr;   // their exclusive prefix (lists of more than kPrefixMax blocks)
   // spawning-attempt staging (one slot per attempt of a batch)
   int64_t bcap = 0;
   uint64_t* st_det = nullptr;   // W*bcap
   int64_t* st_pop = nullptr;    // bcap
   int64_t* st_ent = nullptr;    // bcap
-  int64_t* tile_cnt = nullptr;  // successes per spawning tile (bcap / kSpawnTile + 2)
-  int64_t* tile_off = nullptr;  // their exclusive prefix
+  int32_t* tile_cnt = nullptr;  // successes per spawning tile (bcap / kSmallTile + 2)
   int64_t* tile_win = nullptr;  // parents of each tile's first and last attempt
   // spawned list
   int64_t scap = 0;
@@ -468,6 +469,7 @@ struct fq_engine {
   int64_t rng_cap = 0, rng_pos = 0, rng_end = 0;
   // per-cycle
   Stats* d_stats = nullptr;
+  Stats* h_pin = nullptr;  // pinned: the cycle's finished stats (k_finish)
   Stats h_stats{};
   uint64_t cycle_index = 0;
   hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
@@ -602,25 +604,54 @@ __device__ __forceinline__ void load_det(const uint64_t* det, int64_t cap, int W
   for (int w = 0; w < FQ_MAX_WORDS; ++w) f[w] = w < W ? det[w * cap + i] : 0;
 }
 
+static_assert(sizeof(Stats) % sizeof(int64_t) == 0, "Stats is cleared and copied as int64 words");
+// A cycle's first kernel clears its counters (no later kernel runs beside it).
+__device__ __forceinline__ void clear_stats(Stats* st) {
+  if (blockIdx.x == 0 && threadIdx.x < sizeof(Stats) / sizeof(int64_t)) reinterpret_cast<int64_t*>(st)[threadIdx.x] = 0;
+}
+// Tree sums of NQ arrays of kBlock values in LDS (value t plus value t + h for
+// h = 128, 64, ..., 1) into their first elements; the last six levels within
+// the first wavefront.  Every thread of the block calls it, after a barrier.
+template <int NQ>
+__device__ __forceinline__ void block_tree_sum(double (&sh)[NQ][kBlock], int tid) {
+#pragma unroll
+  for (int h = kBlock / 2; h >= 64; h >>= 1) {
+    if (tid < h)
+      for (int q = 0; q < NQ; ++q) sh[q][tid] += sh[q][tid + h];
+    __syncthreads();
+  }
+  if (tid < 64) {
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      double x = sh[q][tid];
+#pragma unroll
+      for (int h = 32; h > 0; h >>= 1) x += __shfl_down(x, h, 64);  // lanes past 64 - h add their own value: unused
+      if (tid == 0) sh[q][0] = x;
+    }
+  }
+}
+
 // Production: per determinant (loop body of src/fciqmc.f90:315-374 minus the
 // spawning attempts).  Block partial sums (projected energy, reference
-// population, deaths) are reduced in a fixed order by k_sum_partials, so the
+// population, deaths) are reduced in a fixed order by k_finish, so the
 // estimators are deterministic and no global atomics are issued.  A
 // semi-stochastic core determinant (set_determ_info) records its population
 // and position for the projection, is flagged an initiator with kCoreFlag,
-// and skips death.
+// and skips death.  Each block also sums its attempts (blk_att, for k_att_scan).
 __global__ __launch_bounds__(kBlock) void k_det_pass(Sys s, int64_t n, int64_t cap, const uint64_t* __restrict__ det,
                                                      const int64_t* __restrict__ pop, const double* __restrict__ kii,
-                                                     int64_t* __restrict__ pop_new, int64_t* __restrict__ nat,
+                                                     int64_t* __restrict__ pop_new, int32_t* __restrict__ nat,
                                                      int64_t* __restrict__ flags, double tau, double sh0, double sh1,
                                                      double e0, double e1, uint64_t seed, uint32_t cyc,
                                                      double* __restrict__ part_d, int64_t* __restrict__ part_i,
-                                                     double* __restrict__ dvec, int64_t* __restrict__ dpos) {
+                                                     double* __restrict__ dvec, int64_t* __restrict__ dpos,
+                                                     int64_t* __restrict__ blk_att, Stats* __restrict__ st) {
   __shared__ double sh_d[2 * FQ_MAX_SPACES][kBlock];
-  __shared__ int64_t sh_death[kBlock];
+  __shared__ int64_t wsh[kBlock / 64];
+  clear_stats(st);
   const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
   double proj[FQ_MAX_SPACES] = {0.0, 0.0}, d0[FQ_MAX_SPACES] = {0.0, 0.0};
-  int64_t ndeath = 0;
+  int64_t ndeath = 0, att = 0;
   if (i < n) {
     uint64_t f[FQ_MAX_WORDS];
     load_det(det, cap, s.W, i, f);
@@ -641,7 +672,9 @@ __global__ __launch_bounds__(kBlock) void k_det_pass(Sys s, int64_t n, int64_t c
       fqd::proj_energy_term(s, f, rp[sp], proj[sp], d0[sp]);
       const uint32_t hi = static_cast<uint32_t>(i >> 32) ^ (static_cast<uint32_t>(sp) << 28);
       fqd::Philox rng(seed, static_cast<uint32_t>(i), hi, cyc ^ (fqd::kDrawNattempts << 24));
-      nat[i * s.S + sp] = fqd::decide_nattempts(rng, rp[sp]);
+      const int32_t na = fqd::decide_nattempts(rng, rp[sp]);
+      nat[i * s.S + sp] = na;
+      att += na;
       int64_t q = p[sp];
       if (ci < 0) {
         fqd::Philox rd(seed, static_cast<uint32_t>(i), hi, cyc ^ (fqd::kDrawDeath << 24));
@@ -654,68 +687,89 @@ __global__ __launch_bounds__(kBlock) void k_det_pass(Sys s, int64_t n, int64_t c
     sh_d[2 * sp][threadIdx.x] = proj[sp];
     sh_d[2 * sp + 1][threadIdx.x] = d0[sp];
   }
-  sh_death[threadIdx.x] = ndeath;
-  __syncthreads();
-  for (int k = kBlock / 2; k > 0; k >>= 1) {
-    if (threadIdx.x < k) {
-      for (int q = 0; q < 2 * FQ_MAX_SPACES; ++q) sh_d[q][threadIdx.x] += sh_d[q][threadIdx.x + k];
-      sh_death[threadIdx.x] += sh_death[threadIdx.x + k];
-    }
-    __syncthreads();
-  }
+  ndeath = block_sum(ndeath, wsh);  // its barriers publish sh_d
+  att = block_sum(att, wsh);
+  block_tree_sum<2 * FQ_MAX_SPACES>(sh_d, threadIdx.x);
   if (threadIdx.x == 0) {
     for (int q = 0; q < 2 * FQ_MAX_SPACES; ++q) part_d[q * gridDim.x + blockIdx.x] = sh_d[q][0];
-    part_i[blockIdx.x] = sh_death[0];
+    part_i[blockIdx.x] = ndeath;
+    blk_att[blockIdx.x] = att;
   }
 }
 
-// Fixed-order reduction of the k_det_pass block partials: thread t sums
-// blocks t, t+256, ... in order, then a tree in LDS.
-__global__ __launch_bounds__(kBlock) void k_sum_partials(const double* __restrict__ part_d,
+// End of a cycle, one block: the k_det_pass block partials (nb of them; 0: the
+// estimators are already in the stats) in a fixed order -- thread t of the first
+// 256 adds blocks t, t + 256, ..., then a tree -- while the other threads add
+// the insertion's |N| block sums (exact integers: any order gives the same
+// totals); the finished stats go to pinned host memory from here, so no copy
+// follows.
+constexpr int kFinishBlock = 1024;
+template <int S>
+__global__ __launch_bounds__(kFinishBlock) void k_finish(const double* __restrict__ part_d,
                                                          const int64_t* __restrict__ part_i, int nb,
-                                                         Stats* __restrict__ st) {
-  __shared__ double sh[2 * FQ_MAX_SPACES][kBlock];
-  __shared__ int64_t shi[kBlock];
-  double acc[2 * FQ_MAX_SPACES] = {0.0, 0.0, 0.0, 0.0};
-  int64_t ai = 0;
-  // blocks t, t + 256, ... added in that order; eight are loaded ahead at a time
-  constexpr int kAhead = 8;
-  for (int b0 = threadIdx.x; b0 < nb; b0 += kAhead * kBlock) {
-    double v[kAhead][2 * FQ_MAX_SPACES];
-    int64_t vi[kAhead];
+                                                         const int64_t* __restrict__ abs_part, int64_t ld,
+                                                         int64_t nabs, Stats* __restrict__ st,
+                                                         Stats* __restrict__ host) {
+  constexpr int NQ = 2 * S;
+  __shared__ double sh[NQ][kBlock];
+  __shared__ int64_t wi[1 + S][kFinishBlock / 64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  double acc[NQ];
 #pragma unroll
-    for (int k = 0; k < kAhead; ++k) {
-      const int b = b0 + k * kBlock;
+  for (int q = 0; q < NQ; ++q) acc[q] = 0.0;
+  int64_t ai = 0, ap[FQ_MAX_SPACES] = {0, 0};
+  if (tid < kBlock) {
+    // blocks t, t + 256, ... added in that order; sixteen are loaded ahead at a time
+    constexpr int kAhead = 16;
+    for (int b0 = tid; b0 < nb; b0 += kAhead * kBlock) {
+      double v[kAhead][NQ];
+      int64_t vi[kAhead];
 #pragma unroll
-      for (int q = 0; q < 2 * FQ_MAX_SPACES; ++q) v[k][q] = b < nb ? part_d[q * nb + b] : 0.0;
-      vi[k] = b < nb ? part_i[b] : 0;
-    }
+      for (int k = 0; k < kAhead; ++k) {
+        const int b = b0 + k * kBlock;
 #pragma unroll
-    for (int k = 0; k < kAhead; ++k) {
-      if (b0 + k * kBlock < nb) {
+        for (int q = 0; q < NQ; ++q) v[k][q] = b < nb ? part_d[q * nb + b] : 0.0;
+        vi[k] = b < nb ? part_i[b] : 0;
+      }
 #pragma unroll
-        for (int q = 0; q < 2 * FQ_MAX_SPACES; ++q) acc[q] = acc[q] + v[k][q];
-        ai += vi[k];
+      for (int k = 0; k < kAhead; ++k) {
+        if (b0 + k * kBlock < nb) {
+#pragma unroll
+          for (int q = 0; q < NQ; ++q) acc[q] = acc[q] + v[k][q];
+          ai += vi[k];
+        }
       }
     }
+    for (int q = 0; q < NQ; ++q) sh[q][tid] = acc[q];
+  } else {
+    for (int sp = 0; sp < S; ++sp)
+#pragma unroll 4
+      for (int64_t b = tid - kBlock; b < nabs; b += kFinishBlock - kBlock) ap[sp] += abs_part[sp * ld + b];
   }
-  for (int q = 0; q < 2 * FQ_MAX_SPACES; ++q) sh[q][threadIdx.x] = acc[q];
-  shi[threadIdx.x] = ai;
+  ai = wave_sum(ai);
+  for (int sp = 0; sp < S; ++sp) ap[sp] = wave_sum(ap[sp]);
+  if (lane == 0) {
+    wi[0][wave] = ai;
+    for (int sp = 0; sp < S; ++sp) wi[1 + sp][wave] = ap[sp];
+  }
   __syncthreads();
-  for (int k = kBlock / 2; k > 0; k >>= 1) {
-    if (threadIdx.x < k) {
-      for (int q = 0; q < 2 * FQ_MAX_SPACES; ++q) sh[q][threadIdx.x] += sh[q][threadIdx.x + k];
-      shi[threadIdx.x] += shi[threadIdx.x + k];
+  block_tree_sum<NQ>(sh, tid);
+  if (tid == 0) {
+    int64_t t[1 + FQ_MAX_SPACES] = {0, 0, 0};
+    for (int w = 0; w < kFinishBlock / 64; ++w)
+      for (int q = 0; q < 1 + S; ++q) t[q] += wi[q][w];
+    if (nb > 0) {
+      for (int sp = 0; sp < S; ++sp) {
+        st->proj[sp] = sh[2 * sp][0];
+        st->d0[sp] = sh[2 * sp + 1][0];
+      }
+      st->ndeath = t[0];
     }
-    __syncthreads();
+    for (int sp = 0; sp < S; ++sp) st->abs_pop[sp] = static_cast<unsigned long long>(t[1 + sp]);
   }
-  if (threadIdx.x == 0) {
-    for (int sp = 0; sp < FQ_MAX_SPACES; ++sp) {
-      st->proj[sp] = sh[2 * sp][0];
-      st->d0[sp] = sh[2 * sp + 1][0];
-    }
-    st->ndeath = shi[0];
-  }
+  __syncthreads();
+  if (tid < static_cast<int>(sizeof(Stats) / sizeof(int64_t)))
+    reinterpret_cast<int64_t*>(host)[tid] = reinterpret_cast<const volatile int64_t*>(st)[tid];
 }
 
 // Last entry e in [lo, hi] with att_off[e] <= t.
@@ -730,7 +784,94 @@ __device__ __forceinline__ int64_t parent_of(const int64_t* __restrict__ att_off
   return lo;
 }
 
-constexpr int kSpawnTile = 4 * kBlock;  // attempts per block tile
+// Attempts per spawning tile: kSpawnTile, or kSmallTile for cycles whose
+// attempts would not fill the chip with tiles of 1024 (a tile's four rounds run
+// one after the other in its block: 39 us for 10^4 attempts on 26 orbitals, 16
+// with four times the blocks; 195 and 105 us for 3.4e5 of the heat-bath generator).
+constexpr int kSpawnTile = 4 * kBlock, kSmallTile = kBlock;
+constexpr int64_t kSmallTileMax = 512 * kSpawnTile;  // attempts up to which the small tile is used
+
+// Attempt offsets: exclusive scan of the attempts of the nent (det, space)
+// entries, kScanTile entries a block, out[nent] = total.  part: the sums of
+// k_det_pass's blocks (`per` entries each, nblk of them), added up by every
+// block for its offset; poff, when given, is their exclusive prefix (lists of
+// more than kPrefixMax blocks).  The block that holds the first or last attempt
+// of a spawning tile (1 << tile_bits attempts, the first ntile tiles) looks its
+// parent up among the starts it keeps in LDS and notes it as that end of the
+// tile's parent window, so no search precedes the spawning kernel.  (2.8e6
+// entries, 1.1e7 attempts, the densest of them in the first blocks: 34 us;
+// tile sums, scan and a search of the offsets per tile took 46, in four
+// launches.)
+__global__ __launch_bounds__(kBlock) void k_att_scan(const int32_t* __restrict__ in, int64_t nent,
+                                                     const int64_t* __restrict__ part, int64_t nblk, int per,
+                                                     const int64_t* __restrict__ poff, int64_t* __restrict__ out,
+                                                     int64_t* __restrict__ tile_win, int64_t ntile, int tile_bits) {
+  __shared__ int64_t wsh[kBlock / 64];
+  __shared__ int64_t start[kScanTile + 1];  // first attempt of each entry of the block; then the end
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t b0 = static_cast<int64_t>(blockIdx.x) * (kScanTile / per);
+  int64_t off, total;
+  if (poff) {
+    off = poff[b0 < nblk ? b0 : nblk];
+    total = poff[nblk];
+  } else {
+    int64_t pre = 0, all = 0;
+#pragma unroll 4
+    for (int64_t k = threadIdx.x; k < nblk; k += kBlock) {
+      const int64_t v = part[k];
+      all += v;
+      pre += k < b0 ? v : 0;
+    }
+    off = block_sum(pre, wsh);
+    total = block_sum(all, wsh);
+  }
+  // a wavefront's 64 x kScanItems entries, 64 consecutive ones a round (coalesced)
+  const int64_t base = static_cast<int64_t>(blockIdx.x) * kScanTile + wave * (64 * kScanItems) + lane;
+  int32_t v[kScanItems];
+  int64_t local = 0;
+#pragma unroll
+  for (int k = 0; k < kScanItems; ++k) {
+    const int64_t i = base + 64 * k;
+    v[k] = i < nent ? in[i] : 0;
+    local += v[k];
+  }
+  local = wave_sum(local);
+  if (lane == 0) wsh[wave] = local;
+  __syncthreads();
+  int64_t carry = off;  // attempts before the wavefront's round
+#pragma unroll
+  for (int w = 0; w < kBlock / 64; ++w) carry += w < wave ? wsh[w] : 0;
+#pragma unroll
+  for (int k = 0; k < kScanItems; ++k) {
+    const int64_t i = base + 64 * k;
+    const int64_t end = carry + wave_inclusive_scan(static_cast<int64_t>(v[k]), lane), run = end - v[k];
+    if (i < nent) out[i] = run;
+    start[(wave * kScanItems + k) * 64 + lane] = run;
+    carry = __shfl(end, 63, 64);
+  }
+  if (threadIdx.x == kBlock - 1) start[kScanTile] = carry;  // the block's last wavefront, lane 63
+  __syncthreads();
+  // entry of attempt x of this block: the last one starting at or before it (it has attempts)
+  auto entry_of = [&](int64_t x) {
+    int lo = 0, hi = static_cast<int>(kScanTile) - 1;
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (start[mid] <= x)
+        lo = mid;
+      else
+        hi = mid - 1;
+    }
+    return static_cast<int64_t>(blockIdx.x) * kScanTile + lo;
+  };
+  const int64_t beg = off, fin = start[kScanTile];
+  for (int64_t t = (beg >> tile_bits) + threadIdx.x; (t << tile_bits) < fin && t < ntile; t += kBlock) {
+    const int64_t t0 = t << tile_bits, t1 = t0 + (int64_t{1} << tile_bits), last = (t1 < total ? t1 : total) - 1;
+    if (t0 >= beg) tile_win[2 * t] = entry_of(t0);
+    if (last < fin) tile_win[2 * t + 1] = entry_of(last);
+  }
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) out[nent] = total;
+}
+
 // Philox blocks of an attempt's stream generated before its generator runs
 // (two draws each: the single/double choice, the orbital choices with their
 // first rejection redraws, the spawn rounding).  On mol26 (renormalised
@@ -739,23 +880,16 @@ constexpr int kSpawnTile = 4 * kBlock;  // attempts per block tile
 constexpr int kSpawnPre = 4;
 constexpr int kRecipN = 4096;  // entries of the host-made reciprocal table
 
-// Parents of each spawning tile's first and last attempt (one thread per
-// tile, so the searches' latencies overlap instead of opening every block).
-// Parent windows of the tiles of the batch [t_begin, t_end), t_end clamped to
-// the attempt total att_off[nent] (the host may only know a bound of it);
-// tiles of the grid past the total get a zero count.
+// Parent windows of the tiles of the batch [t_begin, t_end) (kSpawnTile
+// attempts each; one thread per tile), for cycles whose attempts take more than
+// one batch; t_end is clamped to the attempt total att_off[nent].
 __global__ void k_tile_bounds(int64_t nent, const int64_t* __restrict__ att_off, int64_t t_begin, int64_t t_end,
-                              int64_t* __restrict__ tile_win, int64_t* __restrict__ tile_cnt) {
-  const int64_t nt_batch = (t_end - t_begin + kSpawnTile - 1) / kSpawnTile;  // tiles the host sized for
+                              int64_t* __restrict__ tile_win) {
   const int64_t tot = att_off[nent];
   t_end = t_end < tot ? t_end : tot;
-  const int64_t ntiles = t_end > t_begin ? (t_end - t_begin + kSpawnTile - 1) / kSpawnTile : 0;
   const int64_t tile = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (tile >= ntiles) {
-    if (tile < nt_batch) tile_cnt[tile] = 0;
-    return;
-  }
   const int64_t t0 = t_begin + tile * kSpawnTile;
+  if (t0 >= t_end) return;
   const int64_t t1 = (t0 + kSpawnTile < t_end) ? t0 + kSpawnTile : t_end;
   const int64_t p0 = parent_of(att_off, t0, 0, nent - 1);
   tile_win[2 * tile] = p0;
@@ -822,20 +956,20 @@ __device__ __forceinline__ void make_key(const KeyPlan& kp, const uint64_t* f, i
 }
 
 // Production: one thread per spawning attempt.  Each block takes tiles of
-// kSpawnTile consecutive attempts of the batch [t_begin, t_end); the parents
+// T consecutive attempts of the batch [t_begin, t_end); the parents
 // of a tile's first and last attempts bound a short window of the attempt
 // prefix sum (n*S (det, space) entries, det-major) in which each thread
 // searches its own parent.  The successful attempts of a tile are ranked in
 // attempt order (wavefront ballots plus per-wave totals) and written
 // contiguously from the tile's first staging slot, with the tile's count in
 // tile_cnt; k_pack_tiles then copies the tiles, in order, into the spawned list.
-template <int G, bool B>
+template <int G, bool B, int T>
 __global__ __launch_bounds__(kBlock) void k_spawn(const Sys* __restrict__ sdev, int64_t nent, int64_t cap, int64_t t_begin, int64_t t_end,
                                                   const int64_t* __restrict__ att_off,
                                                   const uint64_t* __restrict__ det, const int64_t* __restrict__ pop,
                                                   double tau, uint64_t seed, uint32_t cyc, int64_t bcap,
                                                   uint64_t* __restrict__ st_det, int64_t* __restrict__ st_pop,
-                                                  int64_t* __restrict__ st_ent, int64_t* __restrict__ tile_cnt,
+                                                  int64_t* __restrict__ st_ent, int32_t* __restrict__ tile_cnt,
                                                   const int64_t* __restrict__ tile_win,
                                                   const int64_t* __restrict__ pflags,
                                                   const Sys* __restrict__ sys_arr, const int64_t* __restrict__ iatt,
@@ -861,18 +995,18 @@ __global__ __launch_bounds__(kBlock) void k_spawn(const Sys* __restrict__ sdev, 
   // wavefront seldom runs both paths; successes are still compacted in
   // attempt order.
   constexpr bool kPart = (G == fqd::kGenMolRenorm || G == fqd::kGenLearned) && !B;
-  __shared__ int16_t order[kPart ? kSpawnTile : 1];   // processing slot -> attempt in tile
-  __shared__ int64_t rpop[kPart ? kSpawnTile : 1];    // results by attempt in tile
-  __shared__ int32_t rent[kPart ? kSpawnTile : 1];    // parent entry - lo
+  __shared__ int16_t order[kPart ? T : 1];   // processing slot -> attempt in tile
+  __shared__ int64_t rpop[kPart ? T : 1];    // results by attempt in tile
+  __shared__ int32_t rent[kPart ? T : 1];    // parent entry - lo
   __shared__ int32_t wcs[kBlock / 64];
-  uint64_t* rdet = nullptr;                            // [w * kSpawnTile + r], dynamic LDS
+  uint64_t* rdet = nullptr;                            // [w * T + r], dynamic LDS
   const float* aff_lds = nullptr;  // learned: affinity table then flat row, after rdet
   const float* flat_lds = nullptr;
   if constexpr (kPart) {
     extern __shared__ uint64_t part_lds[];
     rdet = part_lds;
     if constexpr (G == fqd::kGenLearned) {
-      float* a = reinterpret_cast<float*>(part_lds + s.W * kSpawnTile);
+      float* a = reinterpret_cast<float*>(part_lds + s.W * T);
       const int na = s.nbasis * s.nbasis;
       for (int k = threadIdx.x; k < na + 2 * s.nbasis; k += kBlock)
         a[k] = k < na ? s.mlp_aff[k] : s.mlp_flat[k - na];
@@ -883,11 +1017,15 @@ __global__ __launch_bounds__(kBlock) void k_spawn(const Sys* __restrict__ sdev, 
   }
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const unsigned long long below = (1ull << lane) - 1;
+  const int64_t ntiles = (t_end - t_begin + T - 1) / T;  // tiles the host sized for
   if (const int64_t tot = att_off[nent]; tot < t_end) t_end = tot;  // the host may pass a bound
-  const int64_t ntiles = t_end > t_begin ? (t_end - t_begin + kSpawnTile - 1) / kSpawnTile : 0;
   for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    const int64_t t0 = t_begin + tile * kSpawnTile;
-    const int64_t t1 = (t0 + kSpawnTile < t_end) ? t0 + kSpawnTile : t_end;
+    const int64_t t0 = t_begin + tile * T;
+    if (t0 >= t_end) {  // past the total (block-uniform)
+      if (threadIdx.x == 0) tile_cnt[tile] = 0;
+      continue;
+    }
+    const int64_t t1 = (t0 + T < t_end) ? t0 + T : t_end;
     const int tn = static_cast<int>(t1 - t0);
     const int64_t lo = tile_win[2 * tile], hi = tile_win[2 * tile + 1];
     const bool staged = hi - lo < kSpawnWin;
@@ -939,7 +1077,7 @@ __global__ __launch_bounds__(kBlock) void k_spawn(const Sys* __restrict__ sdev, 
     if constexpr (kPart) {
       // processing order: doubles from the front, singles from the back
       int32_t nd = 0, ns = 0;
-      for (int k = 0; k < kSpawnTile / kBlock; ++k) {
+      for (int k = 0; k < T / kBlock; ++k) {
         const int r = k * kBlock + threadIdx.x;
         bool single = false;
         if (r < tn) {
@@ -966,14 +1104,14 @@ __global__ __launch_bounds__(kBlock) void k_spawn(const Sys* __restrict__ sdev, 
         if (r < tn) order[single ? tn - 1 - ps : pd] = static_cast<int16_t>(r);
         __syncthreads();
       }
-      for (int k = 0; k < kSpawnTile / kBlock; ++k) {
+      for (int k = 0; k < T / kBlock; ++k) {
         const int q = k * kBlock + threadIdx.x;
         if (q < tn) {
           const int r = order[q];
           int64_t e = 0, nspawn = 0;
           uint64_t child[FQ_MAX_WORDS] = {0, 0};
           attempt(t0 + r, r, e, nspawn, child);
-          FQ_FOR_WORDS(w, s.W) rdet[w * kSpawnTile + r] = child[w];
+          FQ_FOR_WORDS(w, s.W) rdet[w * T + r] = child[w];
           rpop[r] = nspawn;
           rent[r] = static_cast<int32_t>(e - lo);
         }
@@ -981,7 +1119,7 @@ __global__ __launch_bounds__(kBlock) void k_spawn(const Sys* __restrict__ sdev, 
       __syncthreads();
     }
     int32_t run = 0;  // successes of this tile so far (all threads hold the same value)
-    for (int k = 0; k < kSpawnTile / kBlock; ++k) {
+    for (int k = 0; k < T / kBlock; ++k) {
       const int r = k * kBlock + threadIdx.x;
       const bool valid = r < tn;
       int64_t e = 0, nspawn = 0;
@@ -990,7 +1128,7 @@ __global__ __launch_bounds__(kBlock) void k_spawn(const Sys* __restrict__ sdev, 
         if constexpr (kPart) {
           nspawn = rpop[r];
           e = lo + rent[r];
-          FQ_FOR_WORDS(w, s.W) child[w] = rdet[w * kSpawnTile + r];
+          FQ_FOR_WORDS(w, s.W) child[w] = rdet[w * T + r];
         } else {
           attempt(t0 + r, r, e, nspawn, child);
         }
@@ -1021,32 +1159,52 @@ __global__ __launch_bounds__(kBlock) void k_spawn(const Sys* __restrict__ sdev, 
   }
 }
 
-// Pack each tile's compacted successes into the spawned list after the entries
-// of earlier batches (st->nspawn), in attempt order, as sort keys (made here,
-// the binomial table staged in LDS) and payload (the population in its
-// space's word, 0 in the other); blocks loop over tiles.  st_ent holds the
-// spawning space and, from bit 8, the parent's initiator flags.
-__global__ __launch_bounds__(kBlock) void k_pack_tiles(int W, int S, int64_t ntiles,
-                                                       const int64_t* __restrict__ tile_cnt,
-                                                       const int64_t* __restrict__ tile_off,
+// Pack each tile's compacted successes into the spawned list in attempt order,
+// as sort keys (made here, the binomial table staged in LDS) and payload (the
+// population in its space's word, 0 in the other).  A block takes a contiguous
+// range of tiles and adds the counts of the tiles before it for its place.
+// first: the cycle's only batch -- the list starts empty and block 0 records
+// its length and the attempt total (*ptot; more than tlim >= 0 of them: some
+// were not made); else the entries follow those of earlier batches (st->nspawn).
+// st_ent holds the spawning space and, from bit 8, the parent's initiator flags.
+__global__ __launch_bounds__(kBlock) void k_pack_tiles(int W, int S, int64_t ntiles, int tile_size,
+                                                       const int32_t* __restrict__ tile_cnt,
                                                        const uint64_t* __restrict__ st_det,
                                                        const int64_t* __restrict__ st_pop,
                                                        const int64_t* __restrict__ st_ent, int64_t bcap,
                                                        int64_t scap, KeyPlan kp, uint64_t* __restrict__ keys,
-                                                       int64_t* __restrict__ pay, Stats* __restrict__ st) {
+                                                       int64_t* __restrict__ pay, Stats* __restrict__ st, int first,
+                                                       const int64_t* __restrict__ ptot, int64_t tlim) {
   extern __shared__ uint64_t binom_lds[];
+  __shared__ int64_t wsh[kBlock / 64];
   if (kp.rank && kp.binom_lds) {  // blocks loop over tiles, so each stages the table once
     const int nw = 2 * kp.nbasis * kp.nel;
     for (int k = threadIdx.x; k < nw; k += kBlock) binom_lds[k] = kp.binom[k];
-    __syncthreads();
     kp.binom = binom_lds;
   }
-  const int64_t nspawn0 = st->nspawn;
-  for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+  const int64_t per = (ntiles + gridDim.x - 1) / gridDim.x;
+  const int64_t tile0 = blockIdx.x * per, tile1 = tile0 + per < ntiles ? tile0 + per : ntiles;
+  int64_t base = first ? 0 : st->nspawn;
+  {
+    const int64_t upto = blockIdx.x == 0 ? ntiles : (tile0 < ntiles ? tile0 : ntiles);
+    int64_t x = 0;
+#pragma unroll 4
+    for (int64_t k = threadIdx.x; k < upto; k += kBlock) x += tile_cnt[k];
+    x = block_sum(x, wsh);  // its barriers also publish the table
+    if (blockIdx.x == 0) {  // the batch's length
+      if (first && threadIdx.x == 0) {
+        st->nspawn = x;
+        st->total_attempts = *ptot;
+        if (tlim >= 0 && *ptot > tlim) st->spawn_overflow = 1;  // attempts past the launch's bound were not made
+      }
+    } else {
+      base += x;
+    }
+  }
+  for (int64_t tile = tile0; tile < tile1; ++tile) {
     const int64_t cnt = tile_cnt[tile];
-    const int64_t base = nspawn0 + tile_off[tile];
     for (int64_t j = threadIdx.x; j < cnt; j += kBlock) {
-      const int64_t u = tile * kSpawnTile + j;
+      const int64_t u = tile * tile_size + j;
       const int64_t slot = base + j;
       if (slot >= scap) {
         st->spawn_overflow = 1;
@@ -1062,14 +1220,21 @@ __global__ __launch_bounds__(kBlock) void k_pack_tiles(int W, int S, int64_t nti
       make_key(kp, f, W, static_cast<uint64_t>(e) >> 8, k);
       for (int w = 0; w < kp.kw; ++w) keys[w * scap + slot] = k[w];
     }
+    base += cnt;
   }
 }
 
-__global__ void k_add_spawned(const int64_t* __restrict__ pos, int64_t nb, const int64_t* __restrict__ ptot,
-                              Stats* __restrict__ st, int64_t tlim) {
-  st->nspawn += pos[nb];
-  st->total_attempts = *ptot;
-  if (tlim >= 0 && *ptot > tlim) st->spawn_overflow = 1;  // attempts past the launches' bound were not made
+// After a batch that is not the cycle's only one: its entries join the length.
+__global__ __launch_bounds__(kBlock) void k_add_spawned(const int32_t* __restrict__ tile_cnt, int64_t ntiles,
+                                                        const int64_t* __restrict__ ptot, Stats* __restrict__ st) {
+  __shared__ int64_t wsh[kBlock / 64];
+  int64_t x = 0;
+  for (int64_t k = threadIdx.x; k < ntiles; k += kBlock) x += tile_cnt[k];
+  x = block_sum(x, wsh);
+  if (threadIdx.x == 0) {
+    st->nspawn += x;
+    st->total_attempts = *ptot;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1106,51 +1271,58 @@ __global__ __launch_bounds__(kBlock) void k_det_pass_batch(Sys s, const Sys* __r
                                                            int64_t cap, const uint64_t* __restrict__ det,
                                                            const int64_t* __restrict__ pop,
                                                            const double* __restrict__ kii,
-                                                           int64_t* __restrict__ pop_new, int64_t* __restrict__ nat,
+                                                           int64_t* __restrict__ pop_new, int32_t* __restrict__ nat,
                                                            int64_t* __restrict__ flags, uint64_t seed, uint32_t cyc,
                                                            double* __restrict__ cterm,
                                                            int64_t* __restrict__ cdeath,
                                                            const int64_t* __restrict__ pn,
-                                                           const uint32_t* __restrict__ pcyc) {
+                                                           const uint32_t* __restrict__ pcyc,
+                                                           int64_t* __restrict__ blk_att, Stats* __restrict__ st) {
+  __shared__ int64_t wsh[kBlock / 64];
+  clear_stats(st);
   const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
-  if (i >= n) return;
-  if (i >= list_len(pn, n)) {  // past the list in a launch sized by a bound: no attempts
+  int64_t att = 0;
+  if (i < list_len(pn, n)) {
+    cyc = cycle_of(pcyc, cyc);
+    uint64_t f[FQ_MAX_WORDS];
+    load_det(det, cap, s.W, i, f);
+    const int inst = static_cast<int>(f[0] >> kInstShift);
+    f[0] &= kOrbMask;
+    const Sys& si = sys_arr[inst];
+    const int64_t irel = i - bound[inst];
+    const double tau = ipar[inst];
+    double rp[FQ_MAX_SPACES] = {0.0, 0.0};
+    int64_t p[FQ_MAX_SPACES] = {0, 0};
+    for (int sp = 0; sp < s.S; ++sp) {
+      p[sp] = pop[sp * cap + i];
+      rp[sp] = static_cast<double>(p[sp]) / static_cast<double>(s.rf);
+    }
+    flags[i] = fqd::parent_flag(s, rp);
+    const double K = kii[i];
+    int64_t ndeath = 0;
+    for (int sp = 0; sp < s.S; ++sp) {
+      double proj = 0.0, d0 = 0.0;
+      fqd::proj_energy_term(si, f, rp[sp], proj, d0);
+      cterm[(2 * sp) * cap + i] = proj;
+      cterm[(2 * sp + 1) * cap + i] = d0;
+      const uint32_t hi = static_cast<uint32_t>(irel >> 32) ^ (static_cast<uint32_t>(sp) << 28);
+      const uint64_t key = seed + static_cast<uint64_t>(inst);
+      fqd::Philox rng(key, static_cast<uint32_t>(irel), hi, cyc ^ (fqd::kDrawNattempts << 24));
+      const int32_t na = fqd::decide_nattempts(rng, rp[sp]);
+      nat[i * s.S + sp] = na;
+      att += na;
+      fqd::Philox rd(key, static_cast<uint32_t>(irel), hi, cyc ^ (fqd::kDrawDeath << 24));
+      int64_t q = p[sp];
+      const double sh = ipar[ninst + sp * ninst + inst], eo = ipar[(1 + s.S) * ninst + sp * ninst + inst];
+      ndeath += fqd::death(rd, tau, K, sh, eo, q);
+      pop_new[sp * cap + i] = q;
+    }
+    cdeath[i] = ndeath;
+  } else if (i < n) {  // past the list in a launch sized by a bound: no attempts
     for (int sp = 0; sp < s.S; ++sp) nat[i * s.S + sp] = 0;
-    return;
   }
-  cyc = cycle_of(pcyc, cyc);
-  uint64_t f[FQ_MAX_WORDS];
-  load_det(det, cap, s.W, i, f);
-  const int inst = static_cast<int>(f[0] >> kInstShift);
-  f[0] &= kOrbMask;
-  const Sys& si = sys_arr[inst];
-  const int64_t irel = i - bound[inst];
-  const double tau = ipar[inst];
-  double rp[FQ_MAX_SPACES] = {0.0, 0.0};
-  int64_t p[FQ_MAX_SPACES] = {0, 0};
-  for (int sp = 0; sp < s.S; ++sp) {
-    p[sp] = pop[sp * cap + i];
-    rp[sp] = static_cast<double>(p[sp]) / static_cast<double>(s.rf);
-  }
-  flags[i] = fqd::parent_flag(s, rp);
-  const double K = kii[i];
-  int64_t ndeath = 0;
-  for (int sp = 0; sp < s.S; ++sp) {
-    double proj = 0.0, d0 = 0.0;
-    fqd::proj_energy_term(si, f, rp[sp], proj, d0);
-    cterm[(2 * sp) * cap + i] = proj;
-    cterm[(2 * sp + 1) * cap + i] = d0;
-    const uint32_t hi = static_cast<uint32_t>(irel >> 32) ^ (static_cast<uint32_t>(sp) << 28);
-    const uint64_t key = seed + static_cast<uint64_t>(inst);
-    fqd::Philox rng(key, static_cast<uint32_t>(irel), hi, cyc ^ (fqd::kDrawNattempts << 24));
-    nat[i * s.S + sp] = fqd::decide_nattempts(rng, rp[sp]);
-    fqd::Philox rd(key, static_cast<uint32_t>(irel), hi, cyc ^ (fqd::kDrawDeath << 24));
-    int64_t q = p[sp];
-    const double sh = ipar[ninst + sp * ninst + inst], eo = ipar[(1 + s.S) * ninst + sp * ninst + inst];
-    ndeath += fqd::death(rd, tau, K, sh, eo, q);
-    pop_new[sp * cap + i] = q;
-  }
-  cdeath[i] = ndeath;
+  att = block_sum(att, wsh);
+  if (threadIdx.x == 0) blk_att[blockIdx.x] = att;
 }
 
 // First attempt index of each instance: attempts are numbered over the
@@ -2804,27 +2976,6 @@ __global__ __launch_bounds__(kBlock) void k_scatter_new(InsertArgs g, KeyPlan kp
   }
 }
 
-// Sum |N| over the new list from the insertion's block sums (exact integers:
-// any order gives the same totals).
-constexpr int kFinishBlock = 1024;
-__global__ __launch_bounds__(kFinishBlock) void k_sum_abs(const int64_t* __restrict__ part, int64_t ld, int64_t nb, int S,
-                                                          Stats* __restrict__ st) {
-  __shared__ int64_t sh[kFinishBlock / 64];
-  for (int sp = 0; sp < S; ++sp) {
-    int64_t x = 0;
-#pragma unroll 4
-    for (int64_t b = threadIdx.x; b < nb; b += kFinishBlock) x += part[sp * ld + b];
-    x = wave_sum(x);
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = x;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      for (int w = 1; w < kFinishBlock / 64; ++w) x += sh[w];
-      st->abs_pop[sp] = static_cast<unsigned long long>(x);
-    }
-    __syncthreads();
-  }
-}
-
 // Sort values of the main list (a loaded list; the insertion keeps them up).
 __global__ void k_rank_list(KeyPlan kp, int W, int64_t n, int64_t cap, const uint64_t* __restrict__ det,
                             uint64_t* __restrict__ rank) {
@@ -2988,6 +3139,12 @@ int sort_pass_db(fq_engine* e, int src, int64_t ns, const int64_t* pns, int shif
   return db == 9 ? sort_pass<KW, S, 9>(e, src, ns, pns, shift) : sort_pass<KW, S, 8>(e, src, ns, pns, shift);
 }
 
+// Spawned lists bounded by this many entries run the whole annihilation in
+// launches sized by the bound, reading the length on the device: the blocks past
+// the length (the bound is the attempts, two to ten times the spawned entries)
+// cost less than a stop of the host for the exact length (~20 us).
+constexpr int64_t kNoWaitMax = int64_t{1} << 21;
+
 // The main list's sort values in buffer c.
 const uint64_t* main_values(const fq_engine* e, int c) { return e->rank_words ? e->mrank[c] : e->det[c]; }
 constexpr int64_t kNewBlocks = 1024;  // most blocks of the new determinants' insertion
@@ -3028,7 +3185,7 @@ int sort_and_reduce(fq_engine* e, int64_t ns, const int64_t* pns, bool replay, u
       }
     }
   }
-  if (pns && !e->capturing) {  // the passes are queued: now the exact length (copied before them)
+  if (pns && !e->capturing && ns > kNoWaitMax) {  // the passes are queued: now the exact length (copied before them)
     FQ_HIP(hipEventSynchronize(e->ev_len));
     // the attempts cannot exceed the bound the spawning launches covered (every
     // entry makes at most floor(|N|) + 1 of them, |N| for integer populations)
@@ -3217,10 +3374,12 @@ int annihilate(fq_engine* e, int64_t ns, const int64_t* pns, bool replay, uint32
     nblk += nb;
   }
   mark(e, e->pev[8]);
-  hipLaunchKernelGGL(k_sum_abs, dim3(1), dim3(kFinishBlock), 0, st, e->abs_part, g.abs_ld, nblk, e->S, e->d_stats);
+  hipLaunchKernelGGL(e->S == 1 ? k_finish<1> : k_finish<2>, dim3(1), dim3(kFinishBlock), 0, st, e->part_d, e->part_i,
+                     e->est_blocks, e->abs_part, g.abs_ld, nblk, e->d_stats, e->h_pin);
+  e->est_blocks = 0;
   if (e->capturing) return FQ_OK;  // the caller reads the stats when the graph has run
-  rc = sync_stats(e);
-  if (rc != FQ_OK) return rc;
+  FQ_HIP(hipStreamSynchronize(st));
+  e->h_stats = *e->h_pin;
   e->cur = o;
   e->n = e->h_stats.new_n;
   e->att_bound = -1;
@@ -3457,7 +3616,7 @@ int setup_learned(fq_engine* e) {
 
 // Determinants with at least min_att spawning attempts this cycle get a
 // network row; mlp_gather lists them in order.
-__global__ void k_mlp_mark(int64_t n, int S, const int64_t* __restrict__ nat, int64_t min_att,
+__global__ void k_mlp_mark(int64_t n, int S, const int32_t* __restrict__ nat, int64_t min_att,
                            int64_t* __restrict__ on) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= n) return;
@@ -3510,7 +3669,7 @@ size_t hb_lds_bytes(int nel) { return static_cast<size_t>(nel) * kBlock * sizeof
 bool hb_lds_fits(int device, int nel) {
   hipFuncAttributes fa;
   int maxlds = 0;
-  if (hipFuncGetAttributes(&fa, reinterpret_cast<const void*>(&k_spawn<fqd::kGenHeatBath, false>)) != hipSuccess ||
+  if (hipFuncGetAttributes(&fa, reinterpret_cast<const void*>(&k_spawn<fqd::kGenHeatBath, false, kSpawnTile>)) != hipSuccess ||
       hipDeviceGetAttribute(&maxlds, hipDeviceAttributeMaxSharedMemoryPerBlock, device) != hipSuccess)
     return false;
   return fa.sharedSizeBytes + hb_lds_bytes(nel) <= static_cast<size_t>(maxlds);
@@ -3518,35 +3677,65 @@ bool hb_lds_fits(int device, int nel) {
 
 // Dynamic LDS of the learned spawning kernel: the tile's parked child
 // determinants, the affinity table and the flat weight row.
-size_t learned_lds_bytes(int W, int nbasis) {
+size_t learned_lds_bytes(int W, int nbasis, int tile = kSpawnTile) {
   const size_t nb = static_cast<size_t>(nbasis);
-  return sizeof(uint64_t) * W * kSpawnTile + sizeof(float) * (nb * nb + 2 * nb);
+  return sizeof(uint64_t) * W * tile + sizeof(float) * (nb * nb + 2 * nb);
 }
 bool learned_lds_fits(int device, int W, int nbasis) {
   hipFuncAttributes fa;
   int maxlds = 0;
-  if (hipFuncGetAttributes(&fa, reinterpret_cast<const void*>(&k_spawn<fqd::kGenLearned, false>)) != hipSuccess ||
+  if (hipFuncGetAttributes(&fa, reinterpret_cast<const void*>(&k_spawn<fqd::kGenLearned, false, kSpawnTile>)) != hipSuccess ||
       hipDeviceGetAttribute(&maxlds, hipDeviceAttributeMaxSharedMemoryPerBlock, device) != hipSuccess)
     return false;
   return fa.sharedSizeBytes + learned_lds_bytes(W, nbasis) <= static_cast<size_t>(maxlds);
 }
 
-// Spawned entries of a batch of nbt attempts starting at t_begin: scan the
-// per-tile success counts, pack the tiles in order, advance the spawned count.
-// ptot: the attempt total on the device (recorded in the stats).
-int pack_spawned(fq_engine* e, int64_t nbt, int64_t t_begin, const int64_t* ptot, int64_t tlim = -1) {
-  const int64_t nt = ceil_div(nbt, kSpawnTile);
-  int rc = scan_exclusive(e, e->tile_cnt, e->tile_off, nt);
-  if (rc != FQ_OK) return rc;
-  (void)t_begin;
+// Attempt offsets of the nent entries from k_det_pass's attempts, and the parent
+// windows of the spawning tiles of the first `attempts` attempts.
+int scan_attempts(fq_engine* e, int64_t nent, int64_t attempts, int tile) {
+  if (nent == 0) {
+    hipLaunchKernelGGL(k_set_zero_total, dim3(1), dim3(1), 0, e->stream, e->att_off);
+    return FQ_OK;
+  }
+  const int64_t nblk = ceil_div(nent, static_cast<int64_t>(kBlock) * e->S);
+  const bool prefix = nblk <= kPrefixMax;
+  if (!prefix) {
+    const int rc = scan_exclusive(e, e->blk_att, e->blk_off, nblk);
+    if (rc != FQ_OK) return rc;
+  }
+  hipLaunchKernelGGL(k_att_scan, dim3(grid_for(nent, kScanTile)), dim3(kBlock), 0, e->stream, e->nat, nent, e->blk_att,
+                     nblk, kBlock * e->S, prefix ? nullptr : e->blk_off, e->att_off, e->tile_win,
+                     ceil_div(attempts, tile), 31 - __builtin_clz(static_cast<unsigned>(tile)));
+  return FQ_OK;
+}
+
+// Pack the spawned entries of a batch of nbt attempts (tiles of `tile`); first:
+// the cycle's only batch.  ptot: the attempt total on the device (recorded in
+// the stats); tlim as in k_pack_tiles.
+void pack_spawned(fq_engine* e, int64_t nbt, int tile, bool first, const int64_t* ptot, int64_t tlim = -1) {
+  const int64_t nt = ceil_div(nbt, tile);
   KeyPlan kp = key_plan(e);
   const size_t tab = binom_bytes(e);
   kp.binom_lds = tab > 0 && tab <= kBinomLdsMax;
   hipLaunchKernelGGL(k_pack_tiles, dim3(static_cast<unsigned>(std::min<int64_t>(nt, 2048))), dim3(kBlock),
-                     kp.binom_lds ? tab : 0, e->stream, e->W, e->S, nt, e->tile_cnt, e->tile_off, e->st_det,
-                     e->st_pop, e->st_ent, e->bcap, e->scap, kp, e->kbuf[0], e->pbuf[0], e->d_stats);
-  hipLaunchKernelGGL(k_add_spawned, dim3(1), dim3(1), 0, e->stream, e->tile_off, nt, ptot, e->d_stats, tlim);
-  return FQ_OK;
+                     kp.binom_lds ? tab : 0, e->stream, e->W, e->S, nt, tile, e->tile_cnt, e->st_det, e->st_pop,
+                     e->st_ent, e->bcap, e->scap, kp, e->kbuf[0], e->pbuf[0], e->d_stats, first ? 1 : 0, ptot, tlim);
+  if (!first)
+    hipLaunchKernelGGL(k_add_spawned, dim3(1), dim3(kBlock), 0, e->stream, e->tile_cnt, nt, ptot, e->d_stats);
+}
+
+// Attempts per tile of a cycle with at most `attempts` attempts.
+int spawn_tile(int64_t attempts) { return attempts <= kSmallTileMax ? kSmallTile : kSpawnTile; }
+template <bool B, int T>
+auto spawn_kernel(int gen) {
+  if constexpr (B) {
+    return gen == fqd::kGenHubK ? k_spawn<fqd::kGenHubK, true, T> : k_spawn<fqd::kGenMolRenorm, true, T>;
+  } else {
+    return gen == fqd::kGenHubK       ? k_spawn<fqd::kGenHubK, false, T>
+           : gen == fqd::kGenHeatBath ? k_spawn<fqd::kGenHeatBath, false, T>
+           : gen == fqd::kGenLearned  ? k_spawn<fqd::kGenLearned, false, T>
+                                      : k_spawn<fqd::kGenMolRenorm, false, T>;
+  }
 }
 
 int alloc_engine(fq_engine* e) {
@@ -3580,9 +3769,10 @@ int alloc_engine(fq_engine* e) {
   rc |= dalloc(&e->st_det, W * e->bcap);
   rc |= dalloc(&e->st_pop, e->bcap);
   rc |= dalloc(&e->st_ent, e->bcap);
-  rc |= dalloc(&e->tile_cnt, e->bcap / kSpawnTile + 2);
-  rc |= dalloc(&e->tile_off, e->bcap / kSpawnTile + 2);
-  rc |= dalloc(&e->tile_win, 2 * (e->bcap / kSpawnTile + 2));
+  rc |= dalloc(&e->tile_cnt, e->bcap / kSmallTile + 2);
+  rc |= dalloc(&e->tile_win, 2 * (e->bcap / kSmallTile + 2));
+  rc |= dalloc(&e->blk_att, cap / kBlock + 2);
+  rc |= dalloc(&e->blk_off, cap / kBlock + 2);
   rc |= dalloc(&e->d_sysp, 1);
   if (replay) {
     rc |= dalloc(&e->ndraw, scap / kRunTile + 2);
@@ -3764,6 +3954,8 @@ int fq_create(const fq_system* sys, const fq_params* params, fq_engine** out) {
     if (hipEventCreate(&e->sev[k]) != hipSuccess) rc = FQ_ERR_DEVICE;
   if (rc == FQ_OK && hipEventCreateWithFlags(&e->ev_len, hipEventDisableTiming) != hipSuccess) rc = FQ_ERR_DEVICE;
   if (rc == FQ_OK && hipHostMalloc(reinterpret_cast<void**>(&e->h_len), 4 * sizeof(int64_t)) != hipSuccess)
+    rc = FQ_ERR_NOMEM;
+  if (rc == FQ_OK && hipHostMalloc(reinterpret_cast<void**>(&e->h_pin), sizeof(Stats)) != hipSuccess)
     rc = FQ_ERR_NOMEM;
   if (rc != FQ_OK) {
     fq_destroy(e);
@@ -3955,10 +4147,9 @@ static int cycle_body(fq_engine* e, const double* shift, const double* eproj_old
   hipStream_t st = e->stream;
   const uint32_t cyc = static_cast<uint32_t>(e->cycle_index++);
   const double sh1 = e->S > 1 ? shift[1] : 0.0, e1 = e->S > 1 ? eproj_old[1] : 0.0;
-  // per-cycle counters cleared by a kernel (no memset node in the stream)
-  static_assert(sizeof(Stats) % sizeof(int64_t) == 0, "Stats is cleared as int64 words");
-  hipLaunchKernelGGL(k_zero, dim3(1), dim3(kBlock), 0, st, reinterpret_cast<int64_t*>(e->d_stats),
-                     static_cast<int64_t>(sizeof(Stats) / sizeof(int64_t)));
+  if (replay)  // production: the determinant pass clears the counters
+    hipLaunchKernelGGL(k_zero, dim3(1), dim3(kBlock), 0, st, reinterpret_cast<int64_t*>(e->d_stats),
+                       static_cast<int64_t>(sizeof(Stats) / sizeof(int64_t)));
   FQ_HIP(hipEventRecord(e->ev[0], st));
   FQ_HIP(hipEventRecord(e->pev[0], st));
   int64_t rng_pos = e->rng_pos;
@@ -3990,12 +4181,10 @@ static int cycle_body(fq_engine* e, const double* shift, const double* eproj_old
       ++e->online_runs;
     }
     const unsigned nb = grid_for(n);
-    if (n > 0)
-      hipLaunchKernelGGL(k_det_pass, dim3(nb), dim3(kBlock), 0, st, e->sys, n, cap, e->det[c], e->pop[c], e->kii[c],
-                         e->pop_new, e->nat, e->flags, tau, shift[0], sh1, eproj_old[0], e1, e->par.philox_seed, cyc,
-                         e->part_d, e->part_i, e->d_dvec, e->d_dpos);
-    hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(kBlock), 0, st, e->part_d, e->part_i,
-                       n > 0 ? static_cast<int>(nb) : 0, e->d_stats);
+    hipLaunchKernelGGL(k_det_pass, dim3(nb), dim3(kBlock), 0, st, e->sys, n, cap, e->det[c], e->pop[c], e->kii[c],
+                       e->pop_new, e->nat, e->flags, tau, shift[0], sh1, eproj_old[0], e1, e->par.philox_seed, cyc,
+                       e->part_d, e->part_i, e->d_dvec, e->d_dpos, e->blk_att, e->d_stats);
+    e->est_blocks = static_cast<int>(nb);
     FQ_HIP(hipEventRecord(e->pev[1], st));
     if (e->par.excit_gen == FQ_EXCIT_LEARNED && n > 0) {
       hipLaunchKernelGGL(k_mlp_mark, dim3(grid_for(n)), dim3(kBlock), 0, st, n, e->S, e->nat,
@@ -4022,14 +4211,15 @@ static int cycle_body(fq_engine* e, const double* shift, const double* eproj_old
     }
     // Attempt offsets over the n*S (det, space) entries.
     const int64_t nent = e->S * n;
-    int rc = scan_exclusive(e, e->nat, e->att_off, nent);
-    if (rc != FQ_OK) return rc;
     // The spawning launches cover attempts [0, bound): after a production
     // cycle the host holds a bound of this cycle's total (every entry makes at
     // most floor(|N|) + 1 attempts, |N| for integer populations), so it need
     // not wait for the prefix sum; otherwise it reads the total.  The kernels
     // clamp to the total on the device.
     int64_t bound = e->att_bound;
+    const int tile = bound > 0 && bound <= e->bcap ? spawn_tile(bound) : kSpawnTile;  // batches: k_tile_bounds' tiles
+    int rc = scan_attempts(e, nent, bound > 0 ? std::min(bound, e->bcap) : e->bcap, tile);
+    if (rc != FQ_OK) return rc;
     if (bound <= 0) {  // unknown (or an empty list): the exact total
       FQ_HIP(hipMemcpyAsync(&bound, e->att_off + nent, sizeof(int64_t), hipMemcpyDeviceToHost, st));
       FQ_HIP(hipStreamSynchronize(st));
@@ -4037,36 +4227,28 @@ static int cycle_body(fq_engine* e, const double* shift, const double* eproj_old
     FQ_HIP(hipEventRecord(e->pev[2], st));
     e->spawn_launches = 0;
     if (int rs = sync_sysp(e); rs != FQ_OK) return rs;
-    auto spawn_range = [&](int64_t from, int64_t to) -> int {
-      for (int64_t tb = from; tb < to;) {
-        const int64_t te = std::min(to, tb + e->bcap);
-        const int64_t nbt = te - tb;
-        const unsigned g = static_cast<unsigned>(std::min<int64_t>(ceil_div(nbt, kSpawnTile), 1 << 20));
-        const int li = e->spawn_launches++;
-        hipLaunchKernelGGL(k_tile_bounds, dim3(grid_for(ceil_div(nbt, kSpawnTile))), dim3(kBlock), 0, st, nent,
-                           e->att_off, tb, te, e->tile_win, e->tile_cnt);
-        if (li < fq_engine::kSpawnEvents) FQ_HIP(hipEventRecord(e->sev[2 * li], st));
-        const int gen = fqd::gen_of(e->sys.system, e->sys.excit_gen);
-        auto kern = gen == fqd::kGenHubK       ? k_spawn<fqd::kGenHubK, false>
-                    : gen == fqd::kGenHeatBath ? k_spawn<fqd::kGenHeatBath, false>
-                    : gen == fqd::kGenLearned  ? k_spawn<fqd::kGenLearned, false>
-                                               : k_spawn<fqd::kGenMolRenorm, false>;
-        const size_t lds = gen == fqd::kGenHeatBath    ? hb_lds_bytes(e->sys.nel)
-                           : gen == fqd::kGenMolRenorm ? sizeof(uint64_t) * e->W * kSpawnTile
-                           : gen == fqd::kGenLearned   ? learned_lds_bytes(e->W, e->sys.nbasis)
-                                                       : 0;
-        hipLaunchKernelGGL(kern, dim3(g), dim3(kBlock), lds, st, e->d_sysp, nent, cap, tb, te, e->att_off,
-                           e->det[c], e->pop[c], tau, e->par.philox_seed, cyc, e->bcap, e->st_det, e->st_pop,
-                           e->st_ent, e->tile_cnt, e->tile_win, e->flags, nullptr, nullptr, nullptr, nullptr);
-        if (li < fq_engine::kSpawnEvents) FQ_HIP(hipEventRecord(e->sev[2 * li + 1], st));
-        const int prc = pack_spawned(e, nbt, tb, e->att_off + nent);
-        if (prc != FQ_OK) return prc;
-        tb = te;
-      }
-      return FQ_OK;
-    };
-    rc = spawn_range(0, bound);
-    if (rc != FQ_OK) return rc;
+    const bool one_batch = bound <= e->bcap;
+    const int gen = fqd::gen_of(e->sys.system, e->sys.excit_gen);
+    auto kern = tile == kSmallTile ? spawn_kernel<false, kSmallTile>(gen) : spawn_kernel<false, kSpawnTile>(gen);
+    const size_t lds = gen == fqd::kGenHeatBath    ? hb_lds_bytes(e->sys.nel)
+                       : gen == fqd::kGenMolRenorm ? sizeof(uint64_t) * e->W * tile
+                       : gen == fqd::kGenLearned   ? learned_lds_bytes(e->W, e->sys.nbasis, tile)
+                                                   : 0;
+    for (int64_t tb = 0; tb < bound; tb += e->bcap) {
+      const int64_t te = std::min(bound, tb + e->bcap);
+      const int64_t nt = ceil_div(te - tb, tile);
+      const int li = e->spawn_launches++;
+      if (!one_batch)
+        hipLaunchKernelGGL(k_tile_bounds, dim3(grid_for(nt)), dim3(kBlock), 0, st, nent, e->att_off, tb, te,
+                           e->tile_win);
+      if (li < fq_engine::kSpawnEvents) FQ_HIP(hipEventRecord(e->sev[2 * li], st));
+      hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(std::min<int64_t>(nt, 1 << 20))), dim3(kBlock), lds, st,
+                         e->d_sysp, nent, cap, tb, te, e->att_off, e->det[c], e->pop[c], tau, e->par.philox_seed, cyc,
+                         e->bcap, e->st_det, e->st_pop, e->st_ent, e->tile_cnt, e->tile_win, e->flags, nullptr,
+                         nullptr, nullptr, nullptr);
+      if (li < fq_engine::kSpawnEvents) FQ_HIP(hipEventRecord(e->sev[2 * li + 1], st));
+      pack_spawned(e, te - tb, tile, one_batch, e->att_off + nent);
+    }
     int64_t ndet_entries = 0;  // the deterministic projection's spawned entries (combined annihilation)
     if (e->ndeterm > 0) {
       const int64_t m = e->ndeterm * e->S;
@@ -4084,9 +4266,12 @@ static int cycle_body(fq_engine* e, const double* shift, const double* eproj_old
     // memory behind the spawning kernels; the radix passes read the length on
     // the device (their grids sized by a bound: successes <= attempts <=
     // bound), so the host waits for the copy only once they are queued, and
-    // the device does not idle meanwhile.
-    FQ_HIP(hipMemcpyAsync(e->h_len, &e->d_stats->nspawn, 3 * sizeof(int64_t), hipMemcpyDeviceToHost, st));
-    FQ_HIP(hipEventRecord(e->ev_len, st));
+    // the device does not idle meanwhile.  Lists bounded by kNoWaitMax are not
+    // waited for at all.
+    if (bound + ndet_entries > kNoWaitMax) {
+      FQ_HIP(hipMemcpyAsync(e->h_len, &e->d_stats->nspawn, 3 * sizeof(int64_t), hipMemcpyDeviceToHost, st));
+      FQ_HIP(hipEventRecord(e->ev_len, st));
+    }
     e->spawn_bound = bound;
     ns = std::min<int64_t>(bound + ndet_entries, e->scap);
   }
@@ -4095,6 +4280,8 @@ static int cycle_body(fq_engine* e, const double* shift, const double* eproj_old
   if (rc != FQ_OK) return rc;
   FQ_HIP(hipEventRecord(e->ev[2], st));
   FQ_HIP(hipEventSynchronize(e->ev[2]));
+  // the attempts cannot exceed the bound the spawning launches covered (see sort_and_reduce)
+  if (!replay && e->h_stats.total_attempts > e->spawn_bound) return FQ_ERR_DEVICE;
   ns = std::min<int64_t>(e->h_stats.nspawn, e->scap);
   if (!replay) {  // next cycle's attempts <= sum floor(|N|) (+1 per entry with real amplitudes)
     unsigned long long sum = 0;
@@ -4506,30 +4693,27 @@ static int enqueue_graph_cycle(fq_engine* e, int64_t nb, int64_t tb) {
   const uint32_t* dcyc = reinterpret_cast<const uint32_t*>(e->d_in + 8);
   const double* par = reinterpret_cast<const double*>(e->d_in + 16);
   FQ_HIP(hipMemcpyAsync(e->d_in, e->h_in, graph_in_bytes(e), hipMemcpyHostToDevice, st));
-  hipLaunchKernelGGL(k_zero, dim3(1), dim3(kBlock), 0, st, reinterpret_cast<int64_t*>(e->d_stats),
-                     static_cast<int64_t>(sizeof(Stats) / sizeof(int64_t)));
   int64_t* ob = e->d_ibound;
   int64_t* nbd = e->d_ibound + (ninst + 1);
   hipLaunchKernelGGL(k_inst_bounds, dim3(grid_for(ninst + 1)), dim3(kBlock), 0, st, e->det[c], nb, ninst, kInstShift,
                      ob, dn);
   hipLaunchKernelGGL(k_det_pass_batch, dim3(grid_for(nb)), dim3(kBlock), 0, st, e->sys, e->d_sys_arr, ob, par, ninst,
                      nb, cap, e->det[c], e->pop[c], e->kii[c], e->pop_new, e->nat, e->flags, e->par.philox_seed, 0u,
-                     e->d_cterm, e->d_cdeath, dn, dcyc);
+                     e->d_cterm, e->d_cdeath, dn, dcyc, e->blk_att, e->d_stats);
   // entries past the list have no attempts, so att_off[S nb] is the total
   const int64_t nent = S * nb;
-  int rc = scan_exclusive(e, e->nat, e->att_off, nent);
+  const int tile = spawn_tile(tb);
+  int rc = scan_attempts(e, nent, tb, tile);
   if (rc != FQ_OK) return rc;
   hipLaunchKernelGGL(k_inst_att, dim3(grid_for(ninst)), dim3(kBlock), 0, st, ninst, S, ob, e->att_off, e->d_iatt);
   const unsigned g = static_cast<unsigned>(std::min<int64_t>(
-      ceil_div(tb, kSpawnTile), e->spawn_blocks > 0 ? e->spawn_blocks : int64_t{1} << 20));
-  hipLaunchKernelGGL(k_tile_bounds, dim3(grid_for(ceil_div(tb, kSpawnTile))), dim3(kBlock), 0, st, nent, e->att_off,
-                     int64_t{0}, tb, e->tile_win, e->tile_cnt);
-  auto kern = e->sys.system == FQ_SYS_HUB_K ? k_spawn<fqd::kGenHubK, true> : k_spawn<fqd::kGenMolRenorm, true>;
+      ceil_div(tb, tile), e->spawn_blocks > 0 ? e->spawn_blocks : int64_t{1} << 20));
+  const int gen = fqd::gen_of(e->sys.system, e->sys.excit_gen);
+  auto kern = tile == kSmallTile ? spawn_kernel<true, kSmallTile>(gen) : spawn_kernel<true, kSpawnTile>(gen);
   hipLaunchKernelGGL(kern, dim3(g), dim3(kBlock), 0, st, e->d_sysp, nent, cap, int64_t{0}, tb, e->att_off, e->det[c],
                      e->pop[c], 0.0, e->par.philox_seed, 0u, e->bcap, e->st_det, e->st_pop, e->st_ent, e->tile_cnt,
                      e->tile_win, e->flags, e->d_sys_arr, e->d_iatt, par, dcyc);
-  rc = pack_spawned(e, tb, 0, e->att_off + nent, tb);
-  if (rc != FQ_OK) return rc;
+  pack_spawned(e, tb, tile, true, e->att_off + nent, tb);
   e->keys_ready = true;
   const int64_t nsb = std::min<int64_t>(tb, e->scap);
   const int64_t* pns = &e->d_stats->nspawn;
@@ -4543,7 +4727,6 @@ static int enqueue_graph_cycle(fq_engine* e, int64_t nb, int64_t tb) {
                      std::min<int64_t>(nb + nsb, cap), ninst, kInstShift, nbd, &e->d_stats->new_n);
   rc = inst_stats(e, ob, nbd, nb, std::min<int64_t>(nb + nsb, cap), e->pop[o]);
   if (rc != FQ_OK) return rc;
-  FQ_HIP(hipMemcpyAsync(e->h_gstats, e->d_stats, sizeof(Stats), hipMemcpyDeviceToHost, st));
   FQ_HIP(hipMemcpyAsync(e->h_god, e->d_iout_d, sizeof(double) * 2 * S * ninst, hipMemcpyDeviceToHost, st));
   FQ_HIP(hipMemcpyAsync(e->h_goi, e->d_iout_i, sizeof(int64_t) * (4 + S) * ninst, hipMemcpyDeviceToHost, st));
   return FQ_OK;
@@ -4648,7 +4831,7 @@ static int graph_cycle(fq_engine* e, const double* shift, const double* eproj_ol
       e->sched[oct] = best;
     }
   }
-  e->h_stats = *e->h_gstats;
+  e->h_stats = *e->h_pin;
   if (e->h_stats.spawn_overflow && e->h_stats.total_attempts > tb) return FQ_ERR_DEVICE;  // the bound was wrong
   e->cur = 1 - e->cur;
   e->n = e->h_stats.new_n;
@@ -4673,7 +4856,6 @@ int fq_batch_graph(fq_engine* e, int32_t enable) {
   if (enable && !e->h_in) {
     const size_t nin = graph_in_bytes(e);
     if (hipHostMalloc(reinterpret_cast<void**>(&e->h_in), nin) != hipSuccess ||
-        hipHostMalloc(reinterpret_cast<void**>(&e->h_gstats), sizeof(Stats)) != hipSuccess ||
         hipHostMalloc(reinterpret_cast<void**>(&e->h_god), sizeof(double) * 2 * e->S * e->ninst) != hipSuccess ||
         hipHostMalloc(reinterpret_cast<void**>(&e->h_goi), sizeof(int64_t) * (4 + e->S) * e->ninst) != hipSuccess)
       return FQ_ERR_NOMEM;
@@ -4738,21 +4920,18 @@ int fq_cycle_batch(fq_engine* e, const double* shift, const double* eproj_old, c
     }
   }
   FQ_HIP(hipMemcpyAsync(e->d_ipar, par.data(), sizeof(double) * par.size(), hipMemcpyHostToDevice, st));
-  hipLaunchKernelGGL(k_zero, dim3(1), dim3(kBlock), 0, st, reinterpret_cast<int64_t*>(e->d_stats),
-                     static_cast<int64_t>(sizeof(Stats) / sizeof(int64_t)));
   FQ_HIP(hipEventRecord(e->ev[0], st));
   FQ_HIP(hipEventRecord(e->pev[0], st));
   int64_t* ob = e->d_ibound;
   int64_t* nbd = e->d_ibound + (ninst + 1);
   hipLaunchKernelGGL(k_inst_bounds, dim3(grid_for(ninst + 1)), dim3(kBlock), 0, st, e->det[c], n, ninst, kInstShift, ob,
                      nullptr);
-  if (n > 0)
-    hipLaunchKernelGGL(k_det_pass_batch, dim3(grid_for(n)), dim3(kBlock), 0, st, e->sys, e->d_sys_arr, ob, e->d_ipar,
-                       ninst, n, cap, e->det[c], e->pop[c], e->kii[c], e->pop_new, e->nat, e->flags,
-                       e->par.philox_seed, cyc, e->d_cterm, e->d_cdeath, nullptr, nullptr);
+  hipLaunchKernelGGL(k_det_pass_batch, dim3(grid_for(n)), dim3(kBlock), 0, st, e->sys, e->d_sys_arr, ob, e->d_ipar,
+                     ninst, n, cap, e->det[c], e->pop[c], e->kii[c], e->pop_new, e->nat, e->flags, e->par.philox_seed,
+                     cyc, e->d_cterm, e->d_cdeath, nullptr, nullptr, e->blk_att, e->d_stats);
   FQ_HIP(hipEventRecord(e->pev[1], st));
   const int64_t nent = S * n;
-  int rc = scan_exclusive(e, e->nat, e->att_off, nent);
+  int rc = scan_attempts(e, nent, e->bcap, kSpawnTile);
   if (rc != FQ_OK) return rc;
   hipLaunchKernelGGL(k_inst_att, dim3(grid_for(ninst)), dim3(kBlock), 0, st, ninst, S, ob, e->att_off, e->d_iatt);
   int64_t total = 0;
@@ -4761,21 +4940,22 @@ int fq_cycle_batch(fq_engine* e, const double* shift, const double* eproj_old, c
   FQ_HIP(hipEventRecord(e->pev[2], st));
   e->spawn_launches = 0;
   if (int rs = sync_sysp(e); rs != FQ_OK) return rs;
+  const bool one_batch = total <= e->bcap;
+  auto kern = spawn_kernel<true, kSpawnTile>(fqd::gen_of(e->sys.system, e->sys.excit_gen));
   for (int64_t tb = 0; tb < total; tb += e->bcap) {
     const int64_t te = std::min(total, tb + e->bcap);
-    const int64_t nbt = te - tb;
-    const unsigned g = static_cast<unsigned>(std::min<int64_t>(ceil_div(nbt, kSpawnTile), 1 << 20));
+    const int64_t nt = ceil_div(te - tb, kSpawnTile);
     const int li = e->spawn_launches++;
-    hipLaunchKernelGGL(k_tile_bounds, dim3(grid_for(ceil_div(nbt, kSpawnTile))), dim3(kBlock), 0, st, nent,
-                       e->att_off, tb, te, e->tile_win, e->tile_cnt);
+    if (!one_batch)
+      hipLaunchKernelGGL(k_tile_bounds, dim3(grid_for(nt)), dim3(kBlock), 0, st, nent, e->att_off, tb, te,
+                         e->tile_win);
     if (li < fq_engine::kSpawnEvents) FQ_HIP(hipEventRecord(e->sev[2 * li], st));
-    auto kern = e->sys.system == FQ_SYS_HUB_K ? k_spawn<fqd::kGenHubK, true> : k_spawn<fqd::kGenMolRenorm, true>;
-    hipLaunchKernelGGL(kern, dim3(g), dim3(kBlock), 0, st, e->d_sysp, nent, cap, tb, te, e->att_off, e->det[c],
-                       e->pop[c], 0.0, e->par.philox_seed, cyc, e->bcap, e->st_det, e->st_pop, e->st_ent,
-                       e->tile_cnt, e->tile_win, e->flags, e->d_sys_arr, e->d_iatt, e->d_ipar, nullptr);
+    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(std::min<int64_t>(nt, 1 << 20))), dim3(kBlock), 0, st,
+                       e->d_sysp, nent, cap, tb, te, e->att_off, e->det[c], e->pop[c], 0.0, e->par.philox_seed, cyc,
+                       e->bcap, e->st_det, e->st_pop, e->st_ent, e->tile_cnt, e->tile_win, e->flags, e->d_sys_arr,
+                       e->d_iatt, e->d_ipar, nullptr);
     if (li < fq_engine::kSpawnEvents) FQ_HIP(hipEventRecord(e->sev[2 * li + 1], st));
-    rc = pack_spawned(e, nbt, tb, e->att_off + nent);
-    if (rc != FQ_OK) return rc;
+    pack_spawned(e, te - tb, kSpawnTile, one_batch, e->att_off + nent);
   }
   FQ_HIP(hipEventRecord(e->pev[3], st));
   e->keys_ready = true;  // the packing kernels wrote the sort keys
@@ -5072,7 +5252,8 @@ void fq_destroy(fq_engine* e) {
   dfree(e->st_pop);
   dfree(e->st_ent);
   dfree(e->tile_cnt);
-  dfree(e->tile_off);
+  dfree(e->blk_att);
+  dfree(e->blk_off);
   dfree(e->tile_win);
   e->sdet = nullptr;  // aliases of kbuf[1], pbuf[1]
   e->srec = nullptr;
@@ -5147,11 +5328,11 @@ void fq_destroy(fq_engine* e) {
     if (e->sev[k]) (void)hipEventDestroy(e->sev[k]);
   if (e->ev_len) (void)hipEventDestroy(e->ev_len);
   if (e->h_len) (void)hipHostFree(e->h_len);
+  if (e->h_pin) (void)hipHostFree(e->h_pin);
   for (auto& g : e->graphs) (void)hipGraphExecDestroy(g.exec);
   for (int k = 0; k < 2; ++k)
     if (e->gev[k]) (void)hipEventDestroy(e->gev[k]);
   if (e->h_in) (void)hipHostFree(e->h_in);
-  if (e->h_gstats) (void)hipHostFree(e->h_gstats);
   if (e->h_god) (void)hipHostFree(e->h_god);
   if (e->h_goi) (void)hipHostFree(e->h_goi);
   dfree(e->d_in);
