@@ -21,7 +21,7 @@ run contains only cycles of the measured shape.
 Prints one JSON line (rank 0).  Extra fields:
   roofline      the spawning-attempt kernel (the largest device-time share):
                 algorithmic HBM bytes per launch / its average launch time
-                (HIP event pair around each launch on the engine's stream)
+                (the device clock at the start of the launch and of the next kernel)
                 vs the 8 TB/s HBM3E peak;
   cpu_baseline  the CPU oracle (a serial restatement of the reference loop)
                 timed on the same walker state: one instance per host core on

@@ -41,6 +41,7 @@
 #include <algorithm>
 #include <cmath>
 #include <climits>
+#include <cstddef>
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
@@ -110,6 +111,11 @@ inline unsigned grid_for(int64_t n, int64_t per_block = kBlock) {
   return static_cast<unsigned>(g);
 }
 
+// Times of a cycle's phases: block 0 of a phase's first kernel notes the device's
+// constant-rate clock as it starts, so the phases are timed without event packets
+// between the kernels (a record costs the queue 2-4 us; a cycle took 16).
+enum Stamp { kStBegin, kStProposal, kStScan, kStSpawn, kStSort, kStRuns, kStRound, kStFinish, kStEnd, kStamps };
+
 // Per-cycle device counters.
 struct Stats {
   double proj[FQ_MAX_SPACES];
@@ -126,6 +132,8 @@ struct Stats {
   int64_t rng_pos;
   int64_t rng_failed;
   unsigned long long abs_pop[FQ_MAX_SPACES];  // sum |pop| after annihilation (encoded)
+  int64_t spawn_begin, spawn_ticks;           // start of the last spawning launch; time of them all
+  int64_t stamp[kStamps];                     // device clock at the start of the phases
 };
 
 // The semi-stochastic core as the projection kernels see it: CSR rows of the
@@ -158,6 +166,10 @@ constexpr int64_t kScanTile = static_cast<int64_t>(kBlock) * kScanItems;
 constexpr int kSmallBlock = 1024, kSmallItems = 8;
 constexpr int64_t kSmallScanMax = kSmallBlock * kSmallItems;  // one chunk: a single block is latency-bound
 constexpr int64_t kPrefixTiles = 2048;
+
+__device__ __forceinline__ void stamp(Stats* st, int which) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) st->stamp[which] = wall_clock64();
+}
 
 // Inclusive scan of x over the 64 lanes of a wavefront.
 __device__ __forceinline__ int64_t wave_inclusive_scan(int64_t x, int lane) {
@@ -472,7 +484,6 @@ struct fq_engine {
   Stats* h_pin = nullptr;  // pinned: the cycle's finished stats (k_finish)
   Stats h_stats{};
   uint64_t cycle_index = 0;
-  hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
   // the spawned-list length, spawn overflow and attempt total, copied behind
   // the spawning kernels into pinned memory (h_len) and marked by ev_len
   int64_t* h_len = nullptr;
@@ -491,12 +502,7 @@ struct fq_engine {
   double* d_dvec = nullptr;
   int64_t* d_dpos = nullptr;
   float t_spawn = 0, t_annih = 0, t_total = 0;
-  // phase events: 0 cycle start, 1 det pass end, 2 spawn start, 3 spawn end,
-  // 4 sort start, 5 sort end, 6 reduce end, 7 merge start, 8 merge end
-  hipEvent_t pev[9] = {};
-  // an event pair around each spawning-kernel launch of a cycle (the first kSpawnEvents)
-  static constexpr int kSpawnEvents = 16;
-  hipEvent_t sev[2 * kSpawnEvents] = {};
+  double ms_per_tick = 1e-5;  // of the device clock
   int spawn_launches = 0;
   fq_profile_out prof{};
   int radix_passes = 0;
@@ -605,9 +611,12 @@ __device__ __forceinline__ void load_det(const uint64_t* det, int64_t cap, int W
 }
 
 static_assert(sizeof(Stats) % sizeof(int64_t) == 0, "Stats is cleared and copied as int64 words");
-// A cycle's first kernel clears its counters (no later kernel runs beside it).
+// A cycle's first kernel clears its counters (no later kernel runs beside it) and notes its start.
 __device__ __forceinline__ void clear_stats(Stats* st) {
-  if (blockIdx.x == 0 && threadIdx.x < sizeof(Stats) / sizeof(int64_t)) reinterpret_cast<int64_t*>(st)[threadIdx.x] = 0;
+  if (blockIdx.x == 0 && threadIdx.x < sizeof(Stats) / sizeof(int64_t)) {
+    constexpr unsigned begin = offsetof(Stats, stamp) / sizeof(int64_t) + kStBegin;
+    reinterpret_cast<int64_t*>(st)[threadIdx.x] = threadIdx.x == begin ? static_cast<int64_t>(wall_clock64()) : 0;
+  }
 }
 // Tree sums of NQ arrays of kBlock values in LDS (value t plus value t + h for
 // h = 128, 64, ..., 1) into their first elements; the last six levels within
@@ -714,6 +723,7 @@ __global__ __launch_bounds__(kFinishBlock) void k_finish(const double* __restric
   __shared__ double sh[NQ][kBlock];
   __shared__ int64_t wi[1 + S][kFinishBlock / 64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  stamp(st, kStFinish);
   double acc[NQ];
 #pragma unroll
   for (int q = 0; q < NQ; ++q) acc[q] = 0.0;
@@ -766,6 +776,7 @@ __global__ __launch_bounds__(kFinishBlock) void k_finish(const double* __restric
       st->ndeath = t[0];
     }
     for (int sp = 0; sp < S; ++sp) st->abs_pop[sp] = static_cast<unsigned long long>(t[1 + sp]);
+    st->stamp[kStEnd] = wall_clock64();
   }
   __syncthreads();
   if (tid < static_cast<int>(sizeof(Stats) / sizeof(int64_t)))
@@ -805,8 +816,10 @@ constexpr int64_t kSmallTileMax = 512 * kSpawnTile;  // attempts up to which the
 __global__ __launch_bounds__(kBlock) void k_att_scan(const int32_t* __restrict__ in, int64_t nent,
                                                      const int64_t* __restrict__ part, int64_t nblk, int per,
                                                      const int64_t* __restrict__ poff, int64_t* __restrict__ out,
-                                                     int64_t* __restrict__ tile_win, int64_t ntile, int tile_bits) {
+                                                     int64_t* __restrict__ tile_win, int64_t ntile, int tile_bits,
+                                                     Stats* __restrict__ st) {
   __shared__ int64_t wsh[kBlock / 64];
+  stamp(st, kStScan);
   __shared__ int64_t start[kScanTile + 1];  // first attempt of each entry of the block; then the end
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t b0 = static_cast<int64_t>(blockIdx.x) * (kScanTile / per);
@@ -973,7 +986,12 @@ __global__ __launch_bounds__(kBlock) void k_spawn(const Sys* __restrict__ sdev, 
                                                   const int64_t* __restrict__ tile_win,
                                                   const int64_t* __restrict__ pflags,
                                                   const Sys* __restrict__ sys_arr, const int64_t* __restrict__ iatt,
-                                                  const double* __restrict__ itau, const uint32_t* __restrict__ pcyc) {
+                                                  const double* __restrict__ itau, const uint32_t* __restrict__ pcyc,
+                                                  Stats* __restrict__ st) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    st->spawn_begin = wall_clock64();
+    if (t_begin == 0) st->stamp[kStSpawn] = st->spawn_begin;
+  }
   cyc = cycle_of(pcyc, cyc);
   // the system descriptor is read from device memory (scalar loads on use)
   // rather than passed by value: its many table pointers would otherwise sit
@@ -1177,6 +1195,7 @@ __global__ __launch_bounds__(kBlock) void k_pack_tiles(int W, int S, int64_t nti
                                                        const int64_t* __restrict__ ptot, int64_t tlim) {
   extern __shared__ uint64_t binom_lds[];
   __shared__ int64_t wsh[kBlock / 64];
+  if (blockIdx.x == 0 && threadIdx.x == 0) st->spawn_ticks += wall_clock64() - st->spawn_begin;
   if (kp.rank && kp.binom_lds) {  // blocks loop over tiles, so each stages the table once
     const int nw = 2 * kp.nbasis * kp.nel;
     for (int k = threadIdx.x; k < nw; k += kBlock) binom_lds[k] = kp.binom[k];
@@ -1481,6 +1500,7 @@ __global__ void k_replay_walk(Sys s, int64_t n, int64_t cap, const uint64_t* __r
                               uint64_t* __restrict__ sdet, int64_t* __restrict__ srec, Stats* __restrict__ st,
                               DetermDev dd) {
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
+  stamp(st, kStBegin);
   fqd::ReplayRng rng{rbuf, rpos, rend, false};
   double proj[FQ_MAX_SPACES] = {0.0, 0.0}, d0[FQ_MAX_SPACES] = {0.0, 0.0};
   int64_t ndeath = 0, nspawn_total = 0, attempts = 0;
@@ -1564,6 +1584,7 @@ __global__ void k_replay_walk(Sys s, int64_t n, int64_t cap, const uint64_t* __r
   st->total_attempts = attempts;
   st->rng_pos = rng.pos;
   st->rng_failed = rng.failed ? 1 : 0;
+  stamp(st, kStScan);
 }
 
 // ---------------------------------------------------------------------------
@@ -1646,9 +1667,11 @@ __device__ __forceinline__ uint32_t block_exclusive_u32(uint32_t x, uint32_t* ws
 template <int KW, int S, int DB>
 __global__ __launch_bounds__(kBlock) void k_pass_count(const uint64_t* __restrict__ keys,
                                                        const int64_t* __restrict__ pn, int64_t nb, int64_t stride,
-                                                       int shift, int64_t* __restrict__ cnt) {
+                                                       int shift, int64_t* __restrict__ cnt,
+                                                       Stats* __restrict__ st) {
   constexpr int NB = 1 << DB, R = sort_items(KW, S), T = kBlock * R;
   __shared__ uint32_t h[NB];
+  if (st) stamp(st, kStSort);  // the first pass
   for (int d = threadIdx.x; d < NB; d += kBlock) h[d] = 0;
   __syncthreads();
   const int64_t n = list_len(pn, nb);
@@ -1844,8 +1867,9 @@ __global__ void k_make_keys(KeyPlan kp, int S, const uint64_t* __restrict__ sdet
 // Replay: the reference's quicksort (src/sort.f90:213-396) on an index array,
 // one thread; comparisons read the spawned bit strings.
 __global__ void k_replay_qsort(const uint64_t* __restrict__ sdet, int64_t ns, int W, int64_t scap,
-                               uint32_t* __restrict__ idx) {
+                               uint32_t* __restrict__ idx, Stats* __restrict__ st) {
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
+  stamp(st, kStSort);
   for (int64_t i = 0; i < ns; ++i) idx[i] = static_cast<uint32_t>(i);
   auto gt = [&](uint32_t a, uint32_t b) { return key_cmp(sdet, scap, W, a, b) > 0; };
   auto ge = [&](uint32_t a, uint32_t b) { return key_cmp(sdet, scap, W, a, b) >= 0; };
@@ -2048,8 +2072,10 @@ __global__ __launch_bounds__(kBlock) void k_run_count(const uint64_t* __restrict
                                                       const uint64_t* __restrict__ mrank, int64_t n, int64_t cap,
                                                       const int64_t* __restrict__ pmain, int64_t ntiles,
                                                       int32_t* __restrict__ tcnt, int32_t* __restrict__ tfirst,
-                                                      int64_t* __restrict__ tpre, int64_t* __restrict__ win) {
+                                                      int64_t* __restrict__ tpre, int64_t* __restrict__ win,
+                                                      Stats* __restrict__ st) {
   constexpr int R = kRunTile / kBlock, NV = 3 * S;
+  stamp(st, kStRuns);
   const int64_t ns = list_len(pn, nsb);
   __shared__ int64_t wsh[kBlock / 64];
   __shared__ int32_t wfirst[kBlock / 64];
@@ -2691,6 +2717,7 @@ __global__ __launch_bounds__(kBlock) void k_round(RoundArgs g) {
   __shared__ int32_t wc[R * NW];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int S = g.s.S;
+  stamp(g.st, kStRound);
   if (blockIdx.x >= g.mtiles) {
     const int64_t b = blockIdx.x - g.mtiles;
     const int32_t cnt = g.ncnt[b];
@@ -3015,11 +3042,6 @@ int reserve_rng(fq_engine* e, int64_t extra) {
   return FQ_OK;
 }
 
-// Profiling event, recorded when the cycle is not being captured into a graph.
-void mark(fq_engine* e, hipEvent_t ev) {
-  if (!e->capturing) (void)hipEventRecord(ev, e->stream);
-}
-
 int sync_stats(fq_engine* e) {
   FQ_HIP(hipMemcpyAsync(&e->h_stats, e->d_stats, sizeof(Stats), hipMemcpyDeviceToHost, e->stream));
   FQ_HIP(hipStreamSynchronize(e->stream));
@@ -3126,7 +3148,7 @@ int sort_pass(fq_engine* e, int src, int64_t ns, const int64_t* pns, int shift) 
   constexpr int T = kBlock * sort_items(KW, S);
   const int64_t nb = std::min<int64_t>(ceil_div(ns, T), kSortBlocks);
   hipLaunchKernelGGL((k_pass_count<KW, S, DB>), dim3(static_cast<unsigned>(nb)), dim3(kBlock), 0, e->stream,
-                     e->kbuf[src], pns, ns, e->scap, shift, e->pass_cnt);
+                     e->kbuf[src], pns, ns, e->scap, shift, e->pass_cnt, e->radix_passes == 0 ? e->d_stats : nullptr);
   hipLaunchKernelGGL(k_pass_rowscan, dim3(1u << DB), dim3(kSortBlocks), 0, e->stream, static_cast<int>(nb),
                      e->pass_cnt, e->pass_off);
   hipLaunchKernelGGL((k_pass_scatter<KW, S, DB>), dim3(static_cast<unsigned>(nb)), dim3(kBlock), 0, e->stream,
@@ -3163,10 +3185,9 @@ int sort_and_reduce(fq_engine* e, int64_t ns, const int64_t* pns, bool replay, u
   hipStream_t st = e->stream;
   int src = 0;
   e->radix_passes = 0;
-  mark(e, e->pev[4]);
   if (ns > 0) {
     if (replay) {
-      hipLaunchKernelGGL(k_replay_qsort, dim3(1), dim3(1), 0, st, e->sdet, ns, e->W, scap, e->perm);
+      hipLaunchKernelGGL(k_replay_qsort, dim3(1), dim3(1), 0, st, e->sdet, ns, e->W, scap, e->perm, e->d_stats);
       launch_make_keys(e, ns, e->perm);
     } else {
       if (!keys_ready) launch_make_keys(e, ns, nullptr);
@@ -3193,7 +3214,6 @@ int sort_and_reduce(fq_engine* e, int64_t ns, const int64_t* pns, bool replay, u
     ns = std::min<int64_t>(e->h_len[0], e->scap);
     pns = nullptr;
   }
-  mark(e, e->pev[5]);
   // Runs: totals, merge with the main list, the tiles' new determinants.
   const int64_t nt = ceil_div(ns, kRunTile);
   e->run_tiles = nt;
@@ -3205,7 +3225,7 @@ int sort_and_reduce(fq_engine* e, int64_t ns, const int64_t* pns, bool replay, u
                        : (S == 1 ? k_run_count<2, 1> : k_run_count<2, 2>);
     hipLaunchKernelGGL(cnt, dim3(static_cast<unsigned>(nt)), dim3(kBlock), 0, st, e->kbuf[src], e->pbuf[src], pns, ns,
                        scap, e->flag_bits, mrank, e->n, e->cap, dn, nt, e->run_tcnt, e->run_tfirst, e->run_tpre,
-                       e->run_win);
+                       e->run_win, e->d_stats);
     if (nt > kPrefixMax) {
       const int rc = scan_exclusive(e, e->run_tcnt, e->run_toff, nt);
       if (rc != FQ_OK) return rc;
@@ -3243,7 +3263,6 @@ int sort_and_reduce(fq_engine* e, int64_t ns, const int64_t* pns, bool replay, u
     auto kern = kw == 1 ? (S == 1 ? k_runs<1, 1> : k_runs<1, 2>) : (S == 1 ? k_runs<2, 1> : k_runs<2, 2>);
     hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(nt)), dim3(kBlock), 0, st, g);
   }
-  mark(e, e->pev[6]);
   return FQ_OK;
 }
 
@@ -3261,7 +3280,6 @@ int annihilate(fq_engine* e, int64_t ns, const int64_t* pns, bool replay, uint32
   hipStream_t st = e->stream;
   uint64_t* nval = e->kbuf[e->new_src];
   int64_t* npop = e->pbuf[e->new_src];
-  mark(e, e->pev[7]);
   // Rounding draws (replay: main list first, then new candidates, in order).
   int64_t main_draws = 0, new_draws = 0;
   if (replay) {
@@ -3373,7 +3391,6 @@ int annihilate(fq_engine* e, int64_t ns, const int64_t* pns, bool replay, uint32
                        use_jk ? 1 : 0);
     nblk += nb;
   }
-  mark(e, e->pev[8]);
   hipLaunchKernelGGL(e->S == 1 ? k_finish<1> : k_finish<2>, dim3(1), dim3(kFinishBlock), 0, st, e->part_d, e->part_i,
                      e->est_blocks, e->abs_part, g.abs_ld, nblk, e->d_stats, e->h_pin);
   e->est_blocks = 0;
@@ -3384,6 +3401,37 @@ int annihilate(fq_engine* e, int64_t ns, const int64_t* pns, bool replay, uint32
   e->n = e->h_stats.new_n;
   e->att_bound = -1;
   return FQ_OK;
+}
+
+// The cycle's times from its stamps (a phase without kernels: none) and its
+// sizes: n determinants before it, ns spawned entries.
+void fill_profile(fq_engine* e, int64_t n, int64_t ns) {
+  int64_t t[kStamps];
+  int64_t later = e->h_stats.stamp[kStEnd];
+  for (int k = kStamps - 1; k >= 0; --k) {  // a phase that did not run starts where the next one does
+    if (e->h_stats.stamp[k] != 0) later = e->h_stats.stamp[k];
+    t[k] = later;
+  }
+  auto ms = [&](int from, int to) { return static_cast<double>(t[to] - t[from]) * e->ms_per_tick; };
+  e->t_spawn = static_cast<float>(ms(kStBegin, kStSort));
+  e->t_annih = static_cast<float>(ms(kStSort, kStEnd));
+  e->t_total = static_cast<float>(ms(kStBegin, kStEnd));
+  fq_profile_out& pr = e->prof;
+  pr.det_pass_ms = ms(kStBegin, kStProposal);
+  pr.proposal_ms = e->par.excit_gen == FQ_EXCIT_LEARNED ? ms(kStProposal, kStSpawn) : 0.0;
+  pr.spawn_ms = ms(kStSpawn, kStSort);
+  pr.sort_ms = ms(kStSort, kStRuns);
+  pr.reduce_ms = ms(kStRuns, kStRound);
+  pr.merge_ms = ms(kStRound, kStFinish);
+  pr.total_ms = ms(kStBegin, kStFinish);
+  pr.spawn_kernel_ms = static_cast<double>(e->h_stats.spawn_ticks) * e->ms_per_tick;
+  pr.spawn_launches = e->spawn_launches;
+  pr.nstates_in = n;
+  pr.nattempts = e->h_stats.total_attempts;
+  pr.nspawned = ns;
+  pr.nruns = e->h_stats.nruns;
+  pr.nstates_out = e->n;
+  pr.radix_passes = e->radix_passes;
 }
 
 void fill_out(fq_engine* e, fq_cycle_out* out, int64_t rng_used) {
@@ -3617,7 +3665,8 @@ int setup_learned(fq_engine* e) {
 // Determinants with at least min_att spawning attempts this cycle get a
 // network row; mlp_gather lists them in order.
 __global__ void k_mlp_mark(int64_t n, int S, const int32_t* __restrict__ nat, int64_t min_att,
-                           int64_t* __restrict__ on) {
+                           int64_t* __restrict__ on, Stats* __restrict__ st) {
+  stamp(st, kStProposal);
   const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= n) return;
   int64_t a = 0;
@@ -3705,7 +3754,7 @@ int scan_attempts(fq_engine* e, int64_t nent, int64_t attempts, int tile) {
   }
   hipLaunchKernelGGL(k_att_scan, dim3(grid_for(nent, kScanTile)), dim3(kBlock), 0, e->stream, e->nat, nent, e->blk_att,
                      nblk, kBlock * e->S, prefix ? nullptr : e->blk_off, e->att_off, e->tile_win,
-                     ceil_div(attempts, tile), 31 - __builtin_clz(static_cast<unsigned>(tile)));
+                     ceil_div(attempts, tile), 31 - __builtin_clz(static_cast<unsigned>(tile)), e->d_stats);
   return FQ_OK;
 }
 
@@ -3946,12 +3995,9 @@ int fq_create(const fq_system* sys, const fq_params* params, fq_engine** out) {
   if (rc == FQ_OK && params->excit_gen == FQ_EXCIT_LEARNED) rc = setup_learned(e);
   if (rc == FQ_OK) rc = alloc_engine(e);
   if (rc == FQ_OK) rc = setup_sort(e);
-  for (int k = 0; k < 4 && rc == FQ_OK; ++k)
-    if (hipEventCreate(&e->ev[k]) != hipSuccess) rc = FQ_ERR_DEVICE;
-  for (int k = 0; k < 9 && rc == FQ_OK; ++k)
-    if (hipEventCreate(&e->pev[k]) != hipSuccess) rc = FQ_ERR_DEVICE;
-  for (int k = 0; k < 2 * fq_engine::kSpawnEvents && rc == FQ_OK; ++k)
-    if (hipEventCreate(&e->sev[k]) != hipSuccess) rc = FQ_ERR_DEVICE;
+  if (int khz = 0; rc == FQ_OK && hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, e->device) == hipSuccess &&
+                   khz > 0)
+    e->ms_per_tick = 1.0 / khz;
   if (rc == FQ_OK && hipEventCreateWithFlags(&e->ev_len, hipEventDisableTiming) != hipSuccess) rc = FQ_ERR_DEVICE;
   if (rc == FQ_OK && hipHostMalloc(reinterpret_cast<void**>(&e->h_len), 4 * sizeof(int64_t)) != hipSuccess)
     rc = FQ_ERR_NOMEM;
@@ -4150,17 +4196,12 @@ static int cycle_body(fq_engine* e, const double* shift, const double* eproj_old
   if (replay)  // production: the determinant pass clears the counters
     hipLaunchKernelGGL(k_zero, dim3(1), dim3(kBlock), 0, st, reinterpret_cast<int64_t*>(e->d_stats),
                        static_cast<int64_t>(sizeof(Stats) / sizeof(int64_t)));
-  FQ_HIP(hipEventRecord(e->ev[0], st));
-  FQ_HIP(hipEventRecord(e->pev[0], st));
   int64_t rng_pos = e->rng_pos;
   int64_t ns = 0;
   if (replay) {
     hipLaunchKernelGGL(k_replay_walk, dim3(1), dim3(1), 0, st, e->sys, n, cap, e->det[c], e->pop[c], e->kii[c],
                        e->pop_new, tau, shift[0], sh1, eproj_old[0], e1, e->rng_buf, e->rng_pos, e->rng_end, e->scap,
                        e->sdet, e->srec, e->d_stats, determ_dev(e));
-    FQ_HIP(hipEventRecord(e->pev[1], st));
-    FQ_HIP(hipEventRecord(e->pev[2], st));
-    FQ_HIP(hipEventRecord(e->pev[3], st));
     int rc = sync_stats(e);
     if (rc != FQ_OK) return rc;
     if (e->h_stats.rng_failed) return FQ_ERR_RNG_EXHAUSTED;
@@ -4185,10 +4226,9 @@ static int cycle_body(fq_engine* e, const double* shift, const double* eproj_old
                        e->pop_new, e->nat, e->flags, tau, shift[0], sh1, eproj_old[0], e1, e->par.philox_seed, cyc,
                        e->part_d, e->part_i, e->d_dvec, e->d_dpos, e->blk_att, e->d_stats);
     e->est_blocks = static_cast<int>(nb);
-    FQ_HIP(hipEventRecord(e->pev[1], st));
     if (e->par.excit_gen == FQ_EXCIT_LEARNED && n > 0) {
       hipLaunchKernelGGL(k_mlp_mark, dim3(grid_for(n)), dim3(kBlock), 0, st, n, e->S, e->nat,
-                         static_cast<int64_t>(e->par.proposal_min_attempts), e->mlp_on);
+                         static_cast<int64_t>(e->par.proposal_min_attempts), e->mlp_on, e->d_stats);
       int mrc = scan_exclusive(e, e->mlp_on, e->mlp_row, n);
       if (mrc != FQ_OK) return mrc;
       hipLaunchKernelGGL(k_mlp_gather, dim3(grid_for(n)), dim3(kBlock), 0, st, n, e->mlp_on, e->mlp_row,
@@ -4224,7 +4264,6 @@ static int cycle_body(fq_engine* e, const double* shift, const double* eproj_old
       FQ_HIP(hipMemcpyAsync(&bound, e->att_off + nent, sizeof(int64_t), hipMemcpyDeviceToHost, st));
       FQ_HIP(hipStreamSynchronize(st));
     }
-    FQ_HIP(hipEventRecord(e->pev[2], st));
     e->spawn_launches = 0;
     if (int rs = sync_sysp(e); rs != FQ_OK) return rs;
     const bool one_batch = bound <= e->bcap;
@@ -4237,16 +4276,14 @@ static int cycle_body(fq_engine* e, const double* shift, const double* eproj_old
     for (int64_t tb = 0; tb < bound; tb += e->bcap) {
       const int64_t te = std::min(bound, tb + e->bcap);
       const int64_t nt = ceil_div(te - tb, tile);
-      const int li = e->spawn_launches++;
+      ++e->spawn_launches;
       if (!one_batch)
         hipLaunchKernelGGL(k_tile_bounds, dim3(grid_for(nt)), dim3(kBlock), 0, st, nent, e->att_off, tb, te,
                            e->tile_win);
-      if (li < fq_engine::kSpawnEvents) FQ_HIP(hipEventRecord(e->sev[2 * li], st));
       hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(std::min<int64_t>(nt, 1 << 20))), dim3(kBlock), lds, st,
                          e->d_sysp, nent, cap, tb, te, e->att_off, e->det[c], e->pop[c], tau, e->par.philox_seed, cyc,
                          e->bcap, e->st_det, e->st_pop, e->st_ent, e->tile_cnt, e->tile_win, e->flags, nullptr,
-                         nullptr, nullptr, nullptr);
-      if (li < fq_engine::kSpawnEvents) FQ_HIP(hipEventRecord(e->sev[2 * li + 1], st));
+                         nullptr, nullptr, nullptr, e->d_stats);
       pack_spawned(e, te - tb, tile, one_batch, e->att_off + nent);
     }
     int64_t ndet_entries = 0;  // the deterministic projection's spawned entries (combined annihilation)
@@ -4260,7 +4297,6 @@ static int cycle_body(fq_engine* e, const double* shift, const double* eproj_old
         ndet_entries = m;
       }
     }
-    FQ_HIP(hipEventRecord(e->pev[3], st));
     e->keys_ready = true;  // the packing kernels wrote the sort keys
     // The spawned-list length and the attempt total are copied to pinned host
     // memory behind the spawning kernels; the radix passes read the length on
@@ -4275,11 +4311,8 @@ static int cycle_body(fq_engine* e, const double* shift, const double* eproj_old
     e->spawn_bound = bound;
     ns = std::min<int64_t>(bound + ndet_entries, e->scap);
   }
-  FQ_HIP(hipEventRecord(e->ev[1], st));
   int rc = annihilate(e, ns, replay ? nullptr : &e->d_stats->nspawn, replay, cyc, rng_pos);
   if (rc != FQ_OK) return rc;
-  FQ_HIP(hipEventRecord(e->ev[2], st));
-  FQ_HIP(hipEventSynchronize(e->ev[2]));
   // the attempts cannot exceed the bound the spawning launches covered (see sort_and_reduce)
   if (!replay && e->h_stats.total_attempts > e->spawn_bound) return FQ_ERR_DEVICE;
   ns = std::min<int64_t>(e->h_stats.nspawn, e->scap);
@@ -4291,42 +4324,9 @@ static int cycle_body(fq_engine* e, const double* shift, const double* eproj_old
   }
   const int64_t used = rng_pos - e->rng_pos;
   e->rng_pos = rng_pos;
-  (void)hipEventElapsedTime(&e->t_spawn, e->ev[0], e->ev[1]);
-  (void)hipEventElapsedTime(&e->t_annih, e->ev[1], e->ev[2]);
-  (void)hipEventElapsedTime(&e->t_total, e->ev[0], e->ev[2]);
-  {
-    float t[6] = {0, 0, 0, 0, 0, 0};
-    (void)hipEventElapsedTime(&t[0], e->pev[0], e->pev[1]);
-    (void)hipEventElapsedTime(&t[1], e->pev[2], e->pev[3]);
-    (void)hipEventElapsedTime(&t[2], e->pev[4], e->pev[5]);
-    (void)hipEventElapsedTime(&t[3], e->pev[5], e->pev[6]);
-    (void)hipEventElapsedTime(&t[4], e->pev[7], e->pev[8]);
-    (void)hipEventElapsedTime(&t[5], e->pev[0], e->pev[8]);
-    fq_profile_out& pr = e->prof;
-    pr.det_pass_ms = t[0];
-    pr.spawn_ms = t[1];
-    pr.sort_ms = t[2];
-    pr.reduce_ms = t[3];
-    pr.merge_ms = t[4];
-    pr.total_ms = t[5];
-    float tp = 0.0f;
-    if (!replay) (void)hipEventElapsedTime(&tp, e->pev[1], e->pev[2]);
-    pr.proposal_ms = e->par.excit_gen == FQ_EXCIT_LEARNED ? tp : 0.0;
-    if (e->par.excit_gen != FQ_EXCIT_LEARNED || n == 0) pr.proposal_rows = 0;
-    pr.nstates_in = n;
-    pr.nattempts = e->h_stats.total_attempts;
-    pr.nspawned = ns;
-    pr.nruns = e->h_stats.nruns;
-    pr.nstates_out = e->n;
-    pr.radix_passes = e->radix_passes;
-    pr.spawn_launches = replay ? 0 : std::min(e->spawn_launches, fq_engine::kSpawnEvents);
-    pr.spawn_kernel_ms = 0.0;
-    for (int li = 0; li < pr.spawn_launches; ++li) {
-      float ms = 0.0f;
-      (void)hipEventElapsedTime(&ms, e->sev[2 * li], e->sev[2 * li + 1]);
-      pr.spawn_kernel_ms += ms;
-    }
-  }
+  fill_profile(e, n, ns);
+  if (e->par.excit_gen != FQ_EXCIT_LEARNED || n == 0) e->prof.proposal_rows = 0;
+  if (replay) e->prof.spawn_launches = 0;
   fill_out(e, out, used);
   return FQ_OK;
 }
@@ -4712,7 +4712,7 @@ static int enqueue_graph_cycle(fq_engine* e, int64_t nb, int64_t tb) {
   auto kern = tile == kSmallTile ? spawn_kernel<true, kSmallTile>(gen) : spawn_kernel<true, kSpawnTile>(gen);
   hipLaunchKernelGGL(kern, dim3(g), dim3(kBlock), 0, st, e->d_sysp, nent, cap, int64_t{0}, tb, e->att_off, e->det[c],
                      e->pop[c], 0.0, e->par.philox_seed, 0u, e->bcap, e->st_det, e->st_pop, e->st_ent, e->tile_cnt,
-                     e->tile_win, e->flags, e->d_sys_arr, e->d_iatt, par, dcyc);
+                     e->tile_win, e->flags, e->d_sys_arr, e->d_iatt, par, dcyc, e->d_stats);
   pack_spawned(e, tb, tile, true, e->att_off + nent, tb);
   e->keys_ready = true;
   const int64_t nsb = std::min<int64_t>(tb, e->scap);
@@ -4920,8 +4920,6 @@ int fq_cycle_batch(fq_engine* e, const double* shift, const double* eproj_old, c
     }
   }
   FQ_HIP(hipMemcpyAsync(e->d_ipar, par.data(), sizeof(double) * par.size(), hipMemcpyHostToDevice, st));
-  FQ_HIP(hipEventRecord(e->ev[0], st));
-  FQ_HIP(hipEventRecord(e->pev[0], st));
   int64_t* ob = e->d_ibound;
   int64_t* nbd = e->d_ibound + (ninst + 1);
   hipLaunchKernelGGL(k_inst_bounds, dim3(grid_for(ninst + 1)), dim3(kBlock), 0, st, e->det[c], n, ninst, kInstShift, ob,
@@ -4929,7 +4927,6 @@ int fq_cycle_batch(fq_engine* e, const double* shift, const double* eproj_old, c
   hipLaunchKernelGGL(k_det_pass_batch, dim3(grid_for(n)), dim3(kBlock), 0, st, e->sys, e->d_sys_arr, ob, e->d_ipar,
                      ninst, n, cap, e->det[c], e->pop[c], e->kii[c], e->pop_new, e->nat, e->flags, e->par.philox_seed,
                      cyc, e->d_cterm, e->d_cdeath, nullptr, nullptr, e->blk_att, e->d_stats);
-  FQ_HIP(hipEventRecord(e->pev[1], st));
   const int64_t nent = S * n;
   int rc = scan_attempts(e, nent, e->bcap, kSpawnTile);
   if (rc != FQ_OK) return rc;
@@ -4937,7 +4934,6 @@ int fq_cycle_batch(fq_engine* e, const double* shift, const double* eproj_old, c
   int64_t total = 0;
   FQ_HIP(hipMemcpyAsync(&total, e->att_off + nent, sizeof(int64_t), hipMemcpyDeviceToHost, st));
   FQ_HIP(hipStreamSynchronize(st));
-  FQ_HIP(hipEventRecord(e->pev[2], st));
   e->spawn_launches = 0;
   if (int rs = sync_sysp(e); rs != FQ_OK) return rs;
   const bool one_batch = total <= e->bcap;
@@ -4945,19 +4941,16 @@ int fq_cycle_batch(fq_engine* e, const double* shift, const double* eproj_old, c
   for (int64_t tb = 0; tb < total; tb += e->bcap) {
     const int64_t te = std::min(total, tb + e->bcap);
     const int64_t nt = ceil_div(te - tb, kSpawnTile);
-    const int li = e->spawn_launches++;
+    ++e->spawn_launches;
     if (!one_batch)
       hipLaunchKernelGGL(k_tile_bounds, dim3(grid_for(nt)), dim3(kBlock), 0, st, nent, e->att_off, tb, te,
                          e->tile_win);
-    if (li < fq_engine::kSpawnEvents) FQ_HIP(hipEventRecord(e->sev[2 * li], st));
     hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(std::min<int64_t>(nt, 1 << 20))), dim3(kBlock), 0, st,
                        e->d_sysp, nent, cap, tb, te, e->att_off, e->det[c], e->pop[c], 0.0, e->par.philox_seed, cyc,
                        e->bcap, e->st_det, e->st_pop, e->st_ent, e->tile_cnt, e->tile_win, e->flags, e->d_sys_arr,
-                       e->d_iatt, e->d_ipar, nullptr);
-    if (li < fq_engine::kSpawnEvents) FQ_HIP(hipEventRecord(e->sev[2 * li + 1], st));
+                       e->d_iatt, e->d_ipar, nullptr, e->d_stats);
     pack_spawned(e, te - tb, kSpawnTile, one_batch, e->att_off + nent);
   }
-  FQ_HIP(hipEventRecord(e->pev[3], st));
   e->keys_ready = true;  // the packing kernels wrote the sort keys
   rc = sync_stats(e);
   if (rc != FQ_OK) return rc;
@@ -4978,38 +4971,8 @@ int fq_cycle_batch(fq_engine* e, const double* shift, const double* eproj_old, c
   std::vector<int64_t> oi(static_cast<size_t>((4 + S) * ninst));
   FQ_HIP(hipMemcpyAsync(od.data(), e->d_iout_d, sizeof(double) * od.size(), hipMemcpyDeviceToHost, st));
   FQ_HIP(hipMemcpyAsync(oi.data(), e->d_iout_i, sizeof(int64_t) * oi.size(), hipMemcpyDeviceToHost, st));
-  FQ_HIP(hipEventRecord(e->ev[2], st));
   FQ_HIP(hipStreamSynchronize(st));
-  (void)hipEventElapsedTime(&e->t_total, e->ev[0], e->ev[2]);
-  {
-    fq_profile_out& pr = e->prof;
-    float t[6] = {0, 0, 0, 0, 0, 0};
-    (void)hipEventElapsedTime(&t[0], e->pev[0], e->pev[1]);
-    (void)hipEventElapsedTime(&t[1], e->pev[2], e->pev[3]);
-    (void)hipEventElapsedTime(&t[2], e->pev[4], e->pev[5]);
-    (void)hipEventElapsedTime(&t[3], e->pev[5], e->pev[6]);
-    (void)hipEventElapsedTime(&t[4], e->pev[7], e->pev[8]);
-    (void)hipEventElapsedTime(&t[5], e->pev[0], e->pev[8]);
-    pr.det_pass_ms = t[0];
-    pr.spawn_ms = t[1];
-    pr.sort_ms = t[2];
-    pr.reduce_ms = t[3];
-    pr.merge_ms = t[4];
-    pr.total_ms = t[5];
-    pr.nstates_in = n;
-    pr.nattempts = total;
-    pr.nspawned = ns;
-    pr.nruns = e->h_stats.nruns;
-    pr.nstates_out = e->n;
-    pr.radix_passes = e->radix_passes;
-    pr.spawn_launches = std::min(e->spawn_launches, fq_engine::kSpawnEvents);
-    pr.spawn_kernel_ms = 0.0;
-    for (int li = 0; li < pr.spawn_launches; ++li) {
-      float ms = 0.0f;
-      (void)hipEventElapsedTime(&ms, e->sev[2 * li], e->sev[2 * li + 1]);
-      pr.spawn_kernel_ms += ms;
-    }
-  }
+  fill_profile(e, n, ns);
   batch_outputs(e, keep.spawn_overflow != 0, e->h_stats.main_overflow != 0, od.data(), oi.data(), out);
   // the next cycle's attempt total: sum |N| over the new list (integer populations)
   unsigned long long sum = 0;
@@ -5320,12 +5283,6 @@ void fq_destroy(fq_engine* e) {
   dfree(e->d_iout_i);
   for (fq_engine* sub : e->subs) fq_destroy(sub);
   e->subs.clear();
-  for (int k = 0; k < 4; ++k)
-    if (e->ev[k]) (void)hipEventDestroy(e->ev[k]);
-  for (int k = 0; k < 9; ++k)
-    if (e->pev[k]) (void)hipEventDestroy(e->pev[k]);
-  for (int k = 0; k < 2 * fq_engine::kSpawnEvents; ++k)
-    if (e->sev[k]) (void)hipEventDestroy(e->sev[k]);
   if (e->ev_len) (void)hipEventDestroy(e->ev_len);
   if (e->h_len) (void)hipHostFree(e->h_len);
   if (e->h_pin) (void)hipHostFree(e->h_pin);

@@ -224,8 +224,8 @@ int fq_download(fq_engine *e, uint64_t *states, int64_t *pops, double *dat, int6
 /* Device-side timing of the last cycle's kernels (milliseconds). */
 int fq_last_timing(fq_engine *e, double *spawn_ms, double *annihilate_ms, double *total_ms);
 
-/* Per-phase device times of the last fq_cycle, from HIP events recorded on
- * the engine's stream around each phase, and the sizes that phase handled. */
+/* Per-phase device times of the last fq_cycle, from the device clock as each
+ * phase's first kernel starts, and the sizes that phase handled. */
 typedef struct fq_profile_out {
   double det_pass_ms;    /* per-determinant pass: estimators, nattempts, death */
   double spawn_ms;       /* spawning-attempt kernel */
@@ -240,7 +240,7 @@ typedef struct fq_profile_out {
   int64_t nstates_out;   /* occupied determinants after annihilation */
   int32_t radix_passes;  /* 8-bit digit passes of the sort */
   int32_t spawn_launches;    /* launches of the spawning-attempt kernel this cycle */
-  double spawn_kernel_ms;    /* summed device time of those launches (event pair around each) */
+  double spawn_kernel_ms;    /* summed device time of those launches (device clock) */
   double proposal_ms;        /* learned proposal: network marking, inference and attempt offsets */
   int64_t proposal_rows;     /* learned proposal: determinants the network ran on */
 } fq_profile_out;
