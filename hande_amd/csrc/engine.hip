@@ -132,6 +132,8 @@ struct Stats {
   int64_t rng_pos;
   int64_t rng_failed;
   unsigned long long abs_pop[FQ_MAX_SPACES];  // sum |pop| after annihilation (encoded)
+  int64_t sorted;                             // entries k_sort_small sorted
+  int64_t resort;                             // 1: the list was too long for it (nothing downstream ran)
   int64_t spawn_begin, spawn_ticks;           // start of the last spawning launch; time of them all
   int64_t stamp[kStamps];                     // device clock at the start of the phases
 };
@@ -402,6 +404,7 @@ struct fq_engine {
   float* mlp_flat = nullptr;  // 2*nbasis ones: weights of determinants without a row
   int64_t att_bound = -1;            // bound of the next cycle's attempts (-1: unknown)
   bool keys_ready = false;           // the spawning pass made this cycle's sort keys
+  int64_t last_ns = -1;              // spawned entries of the last cycle (-1: none run on this list)
   int est_blocks = 0;                // k_det_pass blocks whose partials k_finish adds (0: none)
   int new_src = 0;                   // the sort's idle buffers after this cycle's passes
   int64_t run_tiles = 0;             // run tiles of this cycle's spawned list (a bound of it while captured)
@@ -1846,6 +1849,121 @@ __global__ __launch_bounds__(kBlock) void k_pass_scatter(const uint64_t* __restr
   }
 }
 
+// A short spawned list sorted by one block in LDS: (value, index) packed in one
+// word per entry, idx_bits of index, stable LSD passes of 9-bit digits over the
+// value; keys and payload are then gathered by index.  Wavefront w keeps a
+// contiguous 1/16 of the entries, 64 at a time, in registers between the passes.
+// One launch for the three per digit of the passes over memory, which for short
+// lists are launch after launch of 3-11 us: 3800 entries of 34-bit values take
+// 39 us instead of 76, 150 entries of 18 bits 10 instead of 29.  A pass costs
+// 2.4 us and 1.9 more for every 1024 entries past the first, against ~20 for a
+// pass over memory: 8192 entries are where the two are still clear of each other.
+// st->sorted receives the length; a list longer than limit (the host may have
+// gone by the last cycle's length) is left alone and st->resort set.
+constexpr int kSmallSort = 8192, kSmallSortBlock = 1024, kSmallSortBits = 9;
+template <int S>
+__global__ __launch_bounds__(kSmallSortBlock) void k_sort_small(const uint64_t* __restrict__ kin,
+                                                                const int64_t* __restrict__ pin,
+                                                                uint64_t* __restrict__ kout,
+                                                                int64_t* __restrict__ pout,
+                                                                const int64_t* __restrict__ pn, int64_t nb,
+                                                                int64_t stride, int fb, int vb, int idx_bits,
+                                                                int limit, Stats* __restrict__ st) {
+  constexpr int NB = 1 << kSmallSortBits, NW = kSmallSortBlock / 64, R = kSmallSort / kSmallSortBlock;
+  __shared__ uint64_t sk[kSmallSort];
+  __shared__ uint16_t wc[NW][NB];  // per-wave running digit counts, then the first place of each wave's keys
+  __shared__ uint32_t wsh[NW];
+  stamp(st, kStSort);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int64_t len = list_len(pn, nb);
+  if (len > limit) {  // block-uniform
+    if (tid == 0) st->resort = 1;
+    return;
+  }
+  const int n = static_cast<int>(len);
+  const int rounds = (n + kSmallSortBlock - 1) / kSmallSortBlock, e0 = wave * rounds * 64 + lane;
+  const uint64_t imask = (uint64_t{1} << idx_bits) - 1;
+  uint64_t key[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int e = e0 + r * 64;
+    key[r] = r < rounds && e < n ? ((kin[e] >> fb) << idx_bits) | static_cast<uint64_t>(e) : 0;
+  }
+  for (int shift = idx_bits; shift < idx_bits + vb; shift += kSmallSortBits) {
+    for (int k = tid; k < NW * NB / 2; k += kSmallSortBlock) reinterpret_cast<uint32_t*>(&wc[0][0])[k] = 0;
+    __syncthreads();  // also: the previous pass's reads of sk are done
+    // the ballots of all rounds first: only the counts form a chain from round to round
+    unsigned long long peers[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      if (r < rounds)  // block-uniform
+        peers[r] = match_digit<kSmallSortBits>(static_cast<uint32_t>(key[r] >> shift) & (NB - 1), e0 + r * 64 < n);
+    uint16_t rank[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      if (r < rounds) {
+        const bool valid = e0 + r * 64 < n;
+        const uint32_t d = static_cast<uint32_t>(key[r] >> shift) & (NB - 1);
+        const uint32_t below = static_cast<uint32_t>(__popcll(peers[r] & ((1ull << lane) - 1)));
+        const uint32_t old = valid ? wc[wave][d] : 0;
+        __builtin_amdgcn_wave_barrier();
+        if (valid && below == 0) wc[wave][d] = static_cast<uint16_t>(old + __popcll(peers[r]));
+        __builtin_amdgcn_wave_barrier();
+        rank[r] = static_cast<uint16_t>(old + below);
+      }
+    __syncthreads();
+    // thread d: digit d's keys in each wave, then the digits before d
+    uint32_t x[NW], c = 0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) x[w] = wc[w][tid & (NB - 1)];
+#pragma unroll
+    for (int w = 0; w < NW; ++w) c += x[w];
+    if (tid >= NB) c = 0;
+    uint32_t inc = c;
+#pragma unroll
+    for (int h = 1; h < 64; h <<= 1) {
+      const uint32_t y = __shfl_up(inc, h, 64);
+      if (lane >= h) inc += y;
+    }
+    if (lane == 63) wsh[wave] = inc;
+    __syncthreads();
+    uint32_t before = inc - c;
+#pragma unroll
+    for (int w = 0; w < NB / 64; ++w) before += w < wave ? wsh[w] : 0;
+    if (tid < NB) {
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        wc[w][tid] = static_cast<uint16_t>(before);
+        before += x[w];
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      if (r >= rounds) break;
+      if (e0 + r * 64 < n) sk[wc[wave][static_cast<uint32_t>(key[r] >> shift) & (NB - 1)] + rank[r]] = key[r];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      if (r >= rounds) break;
+      if (e0 + r * 64 < n) key[r] = sk[e0 + r * 64];
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    if (r >= rounds) break;
+    const int e = e0 + r * 64;
+    if (e < n) {
+      const int64_t i = static_cast<int64_t>(key[r] & imask);
+      kout[e] = kin[i];
+#pragma unroll
+      for (int q = 0; q < S; ++q) pout[q * stride + e] = pin[q * stride + i];
+    }
+  }
+  if (tid == 0) st->sorted = n;
+}
+
 // Sort keys and payload from the spawned list (determinant words, records of
 // populations and flag): entry i gets those of entry perm[i] (perm may be
 // null: the identity).
@@ -2717,6 +2835,7 @@ __global__ __launch_bounds__(kBlock) void k_round(RoundArgs g) {
   __shared__ int32_t wc[R * NW];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int S = g.s.S;
+  if (g.st->resort) return;  // the list has yet to be sorted
   stamp(g.st, kStRound);
   if (blockIdx.x >= g.mtiles) {
     const int64_t b = blockIdx.x - g.mtiles;
@@ -2838,6 +2957,7 @@ __global__ __launch_bounds__(kBlock) void k_scatter_main(InsertArgs g) {
   __shared__ int32_t win[kInsWin];
   __shared__ int64_t wsh[NW], bounds[2];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  if (g.st->resort) return;
   const int64_t n = list_len(g.pn, g.n), tile = blockIdx.x, t0 = tile * kMainTile;
   const int64_t nnew = g.st->nnew;
   // survivors before the tile, and of the whole list
@@ -3172,18 +3292,26 @@ const uint64_t* main_values(const fq_engine* e, int c) { return e->rank_words ? 
 constexpr int64_t kNewBlocks = 1024;  // most blocks of the new determinants' insertion
 constexpr size_t kInsertLdsMax = 60 * 1024;  // their tables, beside the kernel's own LDS in the default 64 KB
 
+// Index bits of k_sort_small beside the value, and the list length it takes (0: none).
+int small_sort_idx_bits(const fq_engine* e) { return std::min(13, 64 - e->value_bits); }
+int small_sort_limit(const fq_engine* e) {
+  static_assert(kSmallSort == 1 << 13, "indexes of 13 bits");
+  return e->sort_kw == 1 && small_sort_idx_bits(e) >= 8 ? 1 << small_sort_idx_bits(e) : 0;
+}
+
 // Sort the spawned list, reduce its runs and merge them with the main list;
 // leaves the tiles' new determinants in the sort's idle buffers (new_src) and
 // the number of run tiles in run_tiles.  The list holds ns entries, or, when
 // pns is given (production, no host wait for the length), *pns entries with ns
-// a bound of them.
-int sort_and_reduce(fq_engine* e, int64_t ns, const int64_t* pns, bool replay, uint32_t cyc) {
+// a bound of them.  no_small: not by k_sort_small unless the bound is short.
+int sort_and_reduce(fq_engine* e, int64_t ns, const int64_t* pns, bool replay, uint32_t cyc, bool no_small) {
   const bool keys_ready = e->keys_ready;  // made by the spawning pass for this spawned list
   e->keys_ready = false;
   const int64_t scap = e->scap;
   const int kw = e->sort_kw, S = e->S;
   hipStream_t st = e->stream;
   int src = 0;
+  bool small = false;
   e->radix_passes = 0;
   if (ns > 0) {
     if (replay) {
@@ -3192,7 +3320,19 @@ int sort_and_reduce(fq_engine* e, int64_t ns, const int64_t* pns, bool replay, u
     } else {
       if (!keys_ready) launch_make_keys(e, ns, nullptr);
       const DigitPlan dp = digit_plan(e);
-      for (int p = 0; p < dp.np; ++p) {
+      const int limit = small_sort_limit(e);
+      // in LDS when the list is short, by its bound or, if not, by the last cycle's length
+      small = ns <= limit || (pns && !e->capturing && ns <= kNoWaitMax && !no_small && e->last_ns >= 0 &&
+                              e->last_ns + e->last_ns / 4 + 256 <= limit);
+      if (small) {
+        hipLaunchKernelGGL(S == 1 ? k_sort_small<1> : k_sort_small<2>, dim3(1), dim3(kSmallSortBlock), 0, st,
+                           e->kbuf[0], e->pbuf[0], e->kbuf[1], e->pbuf[1], pns, ns, scap, e->flag_bits, e->value_bits,
+                           small_sort_idx_bits(e), limit, e->d_stats);
+        src = 1;
+        e->radix_passes = ceil_div(e->value_bits, kSmallSortBits);
+        pns = &e->d_stats->sorted;
+      }
+      for (int p = 0; p < dp.np && !small; ++p) {
         int rc;
         if (kw == 1)
           rc = S == 1 ? sort_pass_db<1, 1>(e, src, ns, pns, dp.shift[p], dp.bits[p])
@@ -3206,7 +3346,7 @@ int sort_and_reduce(fq_engine* e, int64_t ns, const int64_t* pns, bool replay, u
       }
     }
   }
-  if (pns && !e->capturing && ns > kNoWaitMax) {  // the passes are queued: now the exact length (copied before them)
+  if (pns && !e->capturing && !small && ns > kNoWaitMax) {  // the passes are queued: now the exact length (copied before them)
     FQ_HIP(hipEventSynchronize(e->ev_len));
     // the attempts cannot exceed the bound the spawning launches covered (every
     // entry makes at most floor(|N|) + 1 of them, |N| for integer populations)
@@ -3268,8 +3408,9 @@ int sort_and_reduce(fq_engine* e, int64_t ns, const int64_t* pns, bool replay, u
 
 // Annihilation proper: merge runs, round, compact, insert.  ns spawned
 // entries are in the spawned list; pop_new holds the post-death populations.
-int annihilate(fq_engine* e, int64_t ns, const int64_t* pns, bool replay, uint32_t cyc, int64_t& rng_pos) {
-  int rc = sort_and_reduce(e, ns, pns, replay, cyc);
+int annihilate(fq_engine* e, int64_t ns, const int64_t* pns, bool replay, uint32_t cyc, int64_t& rng_pos,
+               bool no_small = false) {
+  int rc = sort_and_reduce(e, ns, pns, replay, cyc, no_small);
   if (rc != FQ_OK) return rc;
   const int64_t ntiles = e->run_tiles;
   // a graph-captured cycle: n is a bound of the list's length, read on the device from dn
@@ -3393,10 +3534,16 @@ int annihilate(fq_engine* e, int64_t ns, const int64_t* pns, bool replay, uint32
   }
   hipLaunchKernelGGL(e->S == 1 ? k_finish<1> : k_finish<2>, dim3(1), dim3(kFinishBlock), 0, st, e->part_d, e->part_i,
                      e->est_blocks, e->abs_part, g.abs_ld, nblk, e->d_stats, e->h_pin);
-  e->est_blocks = 0;
   if (e->capturing) return FQ_OK;  // the caller reads the stats when the graph has run
   FQ_HIP(hipStreamSynchronize(st));
   e->h_stats = *e->h_pin;
+  if (e->h_stats.resort) {  // longer than k_sort_small takes: its keys and the populations are as they were
+    hipLaunchKernelGGL(k_zero, dim3(1), dim3(kBlock), 0, st, &e->d_stats->resort, int64_t{1});
+    e->keys_ready = true;
+    return annihilate(e, std::min<int64_t>(e->h_stats.nspawn, scap), nullptr, replay, cyc, rng_pos, true);
+  }
+  e->est_blocks = 0;
+  e->last_ns = ns > 0 ? std::min<int64_t>(e->h_stats.nspawn, scap) : 0;
   e->cur = o;
   e->n = e->h_stats.new_n;
   e->att_bound = -1;
@@ -4056,6 +4203,7 @@ int fq_load(fq_engine* e, const uint64_t* states, const int64_t* pops, const dou
   FQ_HIP(hipStreamSynchronize(e->stream));
   e->n = n;
   e->att_bound = -1;
+  e->last_ns = -1;
   release_determ(e);  // a new list: no semi-stochastic core until fq_semi_stoch_init
   return FQ_OK;
 }

@@ -104,6 +104,68 @@ def test_annihilate_replay_matches_oracle(hub, initiator, real, seed):
     assert _run(lib, orc, hub, st, p, main, pops, sk, sp, sf, stable=False) > 0
 
 
+@pytest.mark.parametrize("nspawn", [1, 63, 64, 65, 1023, 1024, 1025, 4097, 8191, 8192, 8193])
+def test_annihilate_one_block_sort_edges(nspawn):
+    """Lengths around the wavefront, round and capacity edges of the sort that
+    takes short lists in one block, and the first length past it."""
+    lib, orc = N.lib(), oracle()
+    ring = api.hubbard_k(electrons=14, lattice=[[14]], ms=0, sym=1, U=1)
+    st, p = _mk(ring, True, True, "philox")
+    rf = 1 << p.pop_bit_shift
+    rng = np.random.default_rng(nspawn)
+    main, pops, sk, sp, sf = _random_state(rng, ring, 300, nspawn, rf, True, big=True)
+    assert _run(lib, orc, ring, st, p, main, pops, sk, sp, sf, stable=True) > 0
+
+
+def test_cycle_after_a_short_list_sorts_a_long_one():
+    """A cycle whose list outgrows the one-block sort that the last one's
+    length called for runs the passes instead: the same walkers as an engine
+    that never saw the short list."""
+    lib = N.lib()
+    ring = api.hubbard_k(electrons=14, lattice=[[14]], ms=0, sym=1, U=2)
+    st, p = _mk(ring, True, True, "philox")
+    p.main_capacity = p.spawn_capacity = 1 << 18
+    ptr = lambda a, t: a.ctypes.data_as(C.POINTER(t))
+
+    def start():
+        eng = C.c_void_p()
+        N.check(lib.fq_create(ring.view, C.byref(p), C.byref(eng)), "fq_create")
+        pop = np.array([20000 << p.pop_bit_shift], dtype=np.int64)
+        f0 = ring.f0()
+        N.check(lib.fq_load(eng, ptr(f0, C.c_uint64), ptr(pop, C.c_int64), ptr(np.zeros(1), C.c_double), 1), "load")
+        return eng
+
+    def lists(eng):
+        n, got = C.c_int64(), C.c_int64()
+        N.check(lib.fq_nstates(eng, C.byref(n)), "fq_nstates")
+        a = [np.zeros(n.value, np.uint64), np.zeros(n.value, np.int64), np.zeros(n.value)]
+        N.check(lib.fq_download(eng, ptr(a[0], C.c_uint64), ptr(a[1], C.c_int64), ptr(a[2], C.c_double), n.value,
+                                C.byref(got)), "download")
+        return a
+
+    out, sh = N.FqCycleOut(), (C.c_double * 2)()
+    none, empty = np.zeros(1, np.uint64), np.zeros(1, np.int64)
+    one, two = start(), start()
+    for eng in (one, two):  # cycles 0 and 1: 20000 attempts, then a list of no spawned entries
+        N.check(lib.fq_cycle(eng, sh, sh, 0.01, C.byref(out)), "fq_cycle")
+        N.check(lib.fq_annihilate(eng, ptr(none, C.c_uint64), ptr(empty, C.c_int64), ptr(empty, C.c_int64), 0,
+                                  C.byref(out)), "fq_annihilate")
+    st_, po, da = lists(two)
+    N.check(lib.fq_load(two, ptr(st_, C.c_uint64), ptr(po, C.c_int64), ptr(da, C.c_double), len(da)), "load")
+    for _ in range(3):
+        o1, o2 = N.FqCycleOut(), N.FqCycleOut()
+        N.check(lib.fq_cycle(one, sh, sh, 0.01, C.byref(o1)), "fq_cycle")
+        N.check(lib.fq_cycle(two, sh, sh, 0.01, C.byref(o2)), "fq_cycle")
+        assert o1.nspawn_events > 8192
+        assert (o1.nspawn_events, o1.nstates, o1.ndeath, o1.nattempts) == \
+               (o2.nspawn_events, o2.nstates, o2.ndeath, o2.nattempts)
+        assert o1.proj_energy[0] == o2.proj_energy[0] and o1.nparticles[0] == o2.nparticles[0]
+        for x, y in zip(lists(one), lists(two)):
+            assert np.array_equal(x, y)
+    lib.fq_destroy(one)
+    lib.fq_destroy(two)
+
+
 @pytest.mark.parametrize("initiator", [False, True])
 @pytest.mark.parametrize("seed", [4, 5])
 def test_annihilate_production_matches_stable_oracle(hub, initiator, seed):
