@@ -153,8 +153,8 @@ struct DetermDev {
 };
 // A determinant-pass flag bit above the initiator flags: the parent is a core
 // determinant (its spawns onto the core are the deterministic projection's).
-constexpr int64_t kCoreFlag = int64_t{1} << 40;
-constexpr int64_t kInitFlagMask = 0xff;
+constexpr uint8_t kCoreFlag = 0x80;
+constexpr uint8_t kInitFlagMask = 0x7f;
 
 // ---------------------------------------------------------------------------
 // Prefix sums.  Up to kSmallScanMax entries: one 1024-thread block (one
@@ -421,7 +421,7 @@ struct fq_engine {
   int64_t* pop_new = nullptr;   // S*cap, populations after death
   int32_t* nat = nullptr;       // S*cap attempts per (det, space)
   int64_t* att_off = nullptr;   // S*cap+1
-  int64_t* flags = nullptr;     // cap parent initiator flags
+  uint8_t* flags = nullptr;     // cap parent initiator flags
   uint64_t* mrank[2] = {nullptr, nullptr};  // sort_kw*cap: the entries' sort values (ranks), as the list's buffers
   uint64_t* mmask = nullptr;    // surviving main entries, one bit each, by tiles of kMainTile
   uint16_t* mpre = nullptr;     // per word of mmask: survivors of its tile before it
@@ -437,7 +437,7 @@ struct fq_engine {
   int64_t bcap = 0;
   uint64_t* st_det = nullptr;   // W*bcap
   int64_t* st_pop = nullptr;    // bcap
-  int64_t* st_ent = nullptr;    // bcap
+  uint16_t* st_ent = nullptr;   // bcap: spawning space, parent's initiator flags from bit 8
   int32_t* tile_cnt = nullptr;  // successes per spawning tile (bcap / kSmallTile + 2)
   int64_t* tile_win = nullptr;  // parents of each tile's first and last attempt
   // spawned list
@@ -650,15 +650,16 @@ __device__ __forceinline__ void block_tree_sum(double (&sh)[NQ][kBlock], int tid
 // semi-stochastic core determinant (set_determ_info) records its population
 // and position for the projection, is flagged an initiator with kCoreFlag,
 // and skips death.  Each block also sums its attempts (blk_att, for k_att_scan).
+template <int S>
 __global__ __launch_bounds__(kBlock) void k_det_pass(Sys s, int64_t n, int64_t cap, const uint64_t* __restrict__ det,
                                                      const int64_t* __restrict__ pop, const double* __restrict__ kii,
                                                      int64_t* __restrict__ pop_new, int32_t* __restrict__ nat,
-                                                     int64_t* __restrict__ flags, double tau, double sh0, double sh1,
+                                                     uint8_t* __restrict__ flags, double tau, double sh0, double sh1,
                                                      double e0, double e1, uint64_t seed, uint32_t cyc,
                                                      double* __restrict__ part_d, int64_t* __restrict__ part_i,
                                                      double* __restrict__ dvec, int64_t* __restrict__ dpos,
                                                      int64_t* __restrict__ blk_att, Stats* __restrict__ st) {
-  __shared__ double sh_d[2 * FQ_MAX_SPACES][kBlock];
+  __shared__ double sh_d[2 * S][kBlock];
   __shared__ int64_t wsh[kBlock / 64];
   clear_stats(st);
   const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
@@ -669,23 +670,23 @@ __global__ __launch_bounds__(kBlock) void k_det_pass(Sys s, int64_t n, int64_t c
     load_det(det, cap, s.W, i, f);
     double rp[FQ_MAX_SPACES] = {0.0, 0.0};
     int64_t p[FQ_MAX_SPACES] = {0, 0};
-    for (int sp = 0; sp < s.S; ++sp) {
+    for (int sp = 0; sp < S; ++sp) {
       p[sp] = pop[sp * cap + i];
       rp[sp] = static_cast<double>(p[sp]) / static_cast<double>(s.rf);
     }
     const int64_t ci = s.ndeterm > 0 ? fqd::core_index(s, f) : -1;
     if (ci >= 0) {
-      for (int sp = 0; sp < s.S; ++sp) dvec[ci * s.S + sp] = rp[sp];
+      for (int sp = 0; sp < S; ++sp) dvec[ci * S + sp] = rp[sp];
       dpos[ci] = i;
     }
-    flags[i] = ci >= 0 ? kCoreFlag : fqd::parent_flag(s, rp);
+    flags[i] = ci >= 0 ? kCoreFlag : static_cast<uint8_t>(fqd::parent_flag(s, rp));
     const double K = kii[i];
-    for (int sp = 0; sp < s.S; ++sp) {
+    for (int sp = 0; sp < S; ++sp) {
       fqd::proj_energy_term(s, f, rp[sp], proj[sp], d0[sp]);
       const uint32_t hi = static_cast<uint32_t>(i >> 32) ^ (static_cast<uint32_t>(sp) << 28);
       fqd::Philox rng(seed, static_cast<uint32_t>(i), hi, cyc ^ (fqd::kDrawNattempts << 24));
       const int32_t na = fqd::decide_nattempts(rng, rp[sp]);
-      nat[i * s.S + sp] = na;
+      nat[i * S + sp] = na;
       att += na;
       int64_t q = p[sp];
       if (ci < 0) {
@@ -695,15 +696,15 @@ __global__ __launch_bounds__(kBlock) void k_det_pass(Sys s, int64_t n, int64_t c
       pop_new[sp * cap + i] = q;
     }
   }
-  for (int sp = 0; sp < FQ_MAX_SPACES; ++sp) {
+  for (int sp = 0; sp < S; ++sp) {
     sh_d[2 * sp][threadIdx.x] = proj[sp];
     sh_d[2 * sp + 1][threadIdx.x] = d0[sp];
   }
   ndeath = block_sum(ndeath, wsh);  // its barriers publish sh_d
   att = block_sum(att, wsh);
-  block_tree_sum<2 * FQ_MAX_SPACES>(sh_d, threadIdx.x);
+  block_tree_sum<2 * S>(sh_d, threadIdx.x);
   if (threadIdx.x == 0) {
-    for (int q = 0; q < 2 * FQ_MAX_SPACES; ++q) part_d[q * gridDim.x + blockIdx.x] = sh_d[q][0];
+    for (int q = 0; q < 2 * S; ++q) part_d[q * gridDim.x + blockIdx.x] = sh_d[q][0];
     part_i[blockIdx.x] = ndeath;
     blk_att[blockIdx.x] = att;
   }
@@ -950,25 +951,41 @@ struct DigitPlan {
 __host__ __device__ constexpr int sort_items(int kw, int S) { return kw + S <= 2 ? 16 : 8; }
 constexpr int kSortBlocks = 512;  // blocks of a radix pass (each owns a contiguous range of tiles)
 
+// STRIDE: words per entry of the table (2: low and high; 1: low words only).
+// One-word keys need the sums modulo 2^64 only, so the high words are left out.
+template <int KW, int STRIDE>
 __device__ __forceinline__ void make_key(const KeyPlan& kp, const uint64_t* f, int W, uint64_t flags, uint64_t* key) {
-  unsigned __int128 v = 0;
+  using V = typename std::conditional<KW == 1, uint64_t, unsigned __int128>::type;
+  static_assert(KW == 1 || STRIDE == 2, "two-word keys read both words");
+  V v = 0;
   if (kp.rank) {
     int k = 0;
     FQ_FOR_WORDS(w, W) {
       for (uint64_t x = f[w]; x && k < kp.nel; x &= x - 1) {
         const int p = (w << 6) + __builtin_ctzll(x);
         if (p >= kp.nbasis) break;  // not a determinant of this system (caller-supplied list)
-        const uint64_t* c = kp.binom + 2 * (static_cast<int64_t>(p) * kp.nel + k);
-        v += (static_cast<unsigned __int128>(c[1]) << 64) | c[0];
+        const uint64_t* c = kp.binom + STRIDE * (p * kp.nel + k);
+        if constexpr (KW == 1)
+          v += c[0];
+        else
+          v += (static_cast<unsigned __int128>(c[1]) << 64) | c[0];
         ++k;
       }
     }
   } else {
     v = f[0];
   }
-  const unsigned __int128 k = (v << kp.flag_bits) | (flags & ((uint64_t{1} << kp.flag_bits) - 1));
+  const V k = (v << kp.flag_bits) | (flags & ((uint64_t{1} << kp.flag_bits) - 1));
   key[0] = static_cast<uint64_t>(k);
-  key[1] = static_cast<uint64_t>(k >> 64);
+  if constexpr (KW == 2) key[1] = static_cast<uint64_t>(k >> 64);
+}
+// The same, the table in global memory, key words chosen at run time.
+__device__ __forceinline__ void make_key_any(const KeyPlan& kp, const uint64_t* f, int W, uint64_t flags,
+                                             uint64_t* key) {
+  if (kp.kw == 1)
+    make_key<1, 2>(kp, f, W, flags, key);
+  else
+    make_key<2, 2>(kp, f, W, flags, key);
 }
 
 // Production: one thread per spawning attempt.  Each block takes tiles of
@@ -985,9 +1002,9 @@ __global__ __launch_bounds__(kBlock) void k_spawn(const Sys* __restrict__ sdev, 
                                                   const uint64_t* __restrict__ det, const int64_t* __restrict__ pop,
                                                   double tau, uint64_t seed, uint32_t cyc, int64_t bcap,
                                                   uint64_t* __restrict__ st_det, int64_t* __restrict__ st_pop,
-                                                  int64_t* __restrict__ st_ent, int32_t* __restrict__ tile_cnt,
+                                                  uint16_t* __restrict__ st_ent, int32_t* __restrict__ tile_cnt,
                                                   const int64_t* __restrict__ tile_win,
-                                                  const int64_t* __restrict__ pflags,
+                                                  const uint8_t* __restrict__ pflags,
                                                   const Sys* __restrict__ sys_arr, const int64_t* __restrict__ iatt,
                                                   const double* __restrict__ itau, const uint32_t* __restrict__ pcyc,
                                                   Stats* __restrict__ st) {
@@ -1170,7 +1187,7 @@ __global__ __launch_bounds__(kBlock) void k_spawn(const Sys* __restrict__ sdev, 
         FQ_FOR_WORDS(w, s.W) st_det[w * bcap + u] = child[w];
         st_pop[u] = nspawn;
         // the spawning space and the parent's initiator flags (the sort key's flag bits)
-        st_ent[u] = (e % s.S) | (s.initiator ? (pflags[e / s.S] & kInitFlagMask) << 8 : 0);
+        st_ent[u] = static_cast<uint16_t>((e % s.S) | (s.initiator ? (pflags[e / s.S] & kInitFlagMask) << 8 : 0));
       }
       run += round_total;
       __syncthreads();
@@ -1188,11 +1205,12 @@ __global__ __launch_bounds__(kBlock) void k_spawn(const Sys* __restrict__ sdev, 
 // its length and the attempt total (*ptot; more than tlim >= 0 of them: some
 // were not made); else the entries follow those of earlier batches (st->nspawn).
 // st_ent holds the spawning space and, from bit 8, the parent's initiator flags.
+template <int KW>
 __global__ __launch_bounds__(kBlock) void k_pack_tiles(int W, int S, int64_t ntiles, int tile_size,
                                                        const int32_t* __restrict__ tile_cnt,
                                                        const uint64_t* __restrict__ st_det,
                                                        const int64_t* __restrict__ st_pop,
-                                                       const int64_t* __restrict__ st_ent, int64_t bcap,
+                                                       const uint16_t* __restrict__ st_ent, int64_t bcap,
                                                        int64_t scap, KeyPlan kp, uint64_t* __restrict__ keys,
                                                        int64_t* __restrict__ pay, Stats* __restrict__ st, int first,
                                                        const int64_t* __restrict__ ptot, int64_t tlim) {
@@ -1200,9 +1218,8 @@ __global__ __launch_bounds__(kBlock) void k_pack_tiles(int W, int S, int64_t nti
   __shared__ int64_t wsh[kBlock / 64];
   if (blockIdx.x == 0 && threadIdx.x == 0) st->spawn_ticks += wall_clock64() - st->spawn_begin;
   if (kp.rank && kp.binom_lds) {  // blocks loop over tiles, so each stages the table once
-    const int nw = 2 * kp.nbasis * kp.nel;
-    for (int k = threadIdx.x; k < nw; k += kBlock) binom_lds[k] = kp.binom[k];
-    kp.binom = binom_lds;
+    const int nw = KW * kp.nbasis * kp.nel;
+    for (int k = threadIdx.x; k < nw; k += kBlock) binom_lds[k] = kp.binom[KW == 1 ? 2 * k : k];
   }
   const int64_t per = (ntiles + gridDim.x - 1) / gridDim.x;
   const int64_t tile0 = blockIdx.x * per, tile1 = tile0 + per < ntiles ? tile0 + per : ntiles;
@@ -1232,15 +1249,21 @@ __global__ __launch_bounds__(kBlock) void k_pack_tiles(int W, int S, int64_t nti
         st->spawn_overflow = 1;
         continue;
       }
-      const int64_t e = st_ent[u];
-      const int sp = static_cast<int>(e & 0xff);
+      const int e = st_ent[u], sp = e & 0xff;
       uint64_t f[FQ_MAX_WORDS] = {0, 0};
       FQ_FOR_WORDS(w, W) f[w] = st_det[w * bcap + u];
       const int64_t v = st_pop[u];
       for (int q = 0; q < S; ++q) pay[q * scap + slot] = (q == sp) ? v : 0;
-      uint64_t k[2];
-      make_key(kp, f, W, static_cast<uint64_t>(e) >> 8, k);
-      for (int w = 0; w < kp.kw; ++w) keys[w * scap + slot] = k[w];
+      uint64_t k[KW];
+      if (kp.binom_lds) {
+        KeyPlan lp = kp;
+        lp.binom = binom_lds;
+        make_key<KW, KW>(lp, f, W, static_cast<uint64_t>(e >> 8), k);
+      } else {
+        make_key<KW, 2>(kp, f, W, static_cast<uint64_t>(e >> 8), k);
+      }
+#pragma unroll
+      for (int w = 0; w < KW; ++w) keys[w * scap + slot] = k[w];
     }
     base += cnt;
   }
@@ -1294,7 +1317,7 @@ __global__ __launch_bounds__(kBlock) void k_det_pass_batch(Sys s, const Sys* __r
                                                            const int64_t* __restrict__ pop,
                                                            const double* __restrict__ kii,
                                                            int64_t* __restrict__ pop_new, int32_t* __restrict__ nat,
-                                                           int64_t* __restrict__ flags, uint64_t seed, uint32_t cyc,
+                                                           uint8_t* __restrict__ flags, uint64_t seed, uint32_t cyc,
                                                            double* __restrict__ cterm,
                                                            int64_t* __restrict__ cdeath,
                                                            const int64_t* __restrict__ pn,
@@ -1319,7 +1342,7 @@ __global__ __launch_bounds__(kBlock) void k_det_pass_batch(Sys s, const Sys* __r
       p[sp] = pop[sp * cap + i];
       rp[sp] = static_cast<double>(p[sp]) / static_cast<double>(s.rf);
     }
-    flags[i] = fqd::parent_flag(s, rp);
+    flags[i] = static_cast<uint8_t>(fqd::parent_flag(s, rp));
     const double K = kii[i];
     int64_t ndeath = 0;
     for (int sp = 0; sp < s.S; ++sp) {
@@ -1977,7 +2000,7 @@ __global__ void k_make_keys(KeyPlan kp, int S, const uint64_t* __restrict__ sdet
   FQ_FOR_WORDS(w, W) f[w] = sdet[w * scap + src];
   const int64_t* rec = srec + src * rec_stride(S);
   uint64_t k[2];
-  make_key(kp, f, W, static_cast<uint64_t>(rec[S]), k);
+  make_key_any(kp, f, W, static_cast<uint64_t>(rec[S]), k);
   for (int w = 0; w < kp.kw; ++w) keys[w * scap + i] = k[w];
   for (int q = 0; q < S; ++q) pay[q * scap + i] = rec[q];
 }
@@ -2696,7 +2719,7 @@ __global__ __launch_bounds__(kBlock) void k_determ_proj(Sys s, KeyPlan kp, Deter
 #pragma unroll
   for (int w = 0; w < FQ_MAX_WORDS; ++w) f[w] = w < s.W ? s.determ[w * dd.nd + row] : 0;
   uint64_t key[2];
-  make_key(kp, f, s.W, 0, key);
+  make_key_any(kp, f, s.W, 0, key);
   for (int w = 0; w < kp.kw; ++w) keys[w * scap + slot] = key[w];
 }
 __global__ void k_add_nspawn(Stats* __restrict__ st, int64_t m) { st->nspawn += m; }
@@ -3131,7 +3154,7 @@ __global__ void k_rank_list(KeyPlan kp, int W, int64_t n, int64_t cap, const uin
   uint64_t f[FQ_MAX_WORDS] = {0, 0}, key[2];
   FQ_FOR_WORDS(w, W) f[w] = det[w * cap + i];
   kp.flag_bits = 0;
-  make_key(kp, f, W, 0, key);
+  make_key_any(kp, f, W, 0, key);
   for (int w = 0; w < kp.kw; ++w) rank[w * cap + i] = key[w];
 }
 
@@ -3911,9 +3934,9 @@ int scan_attempts(fq_engine* e, int64_t nent, int64_t attempts, int tile) {
 void pack_spawned(fq_engine* e, int64_t nbt, int tile, bool first, const int64_t* ptot, int64_t tlim = -1) {
   const int64_t nt = ceil_div(nbt, tile);
   KeyPlan kp = key_plan(e);
-  const size_t tab = binom_bytes(e);
+  const size_t tab = binom_bytes(e) / (e->sort_kw == 1 ? 2 : 1);
   kp.binom_lds = tab > 0 && tab <= kBinomLdsMax;
-  hipLaunchKernelGGL(k_pack_tiles, dim3(static_cast<unsigned>(std::min<int64_t>(nt, 2048))), dim3(kBlock),
+  hipLaunchKernelGGL(e->sort_kw == 1 ? k_pack_tiles<1> : k_pack_tiles<2>, dim3(static_cast<unsigned>(std::min<int64_t>(nt, 2048))), dim3(kBlock),
                      kp.binom_lds ? tab : 0, e->stream, e->W, e->S, nt, tile, e->tile_cnt, e->st_det, e->st_pop,
                      e->st_ent, e->bcap, e->scap, kp, e->kbuf[0], e->pbuf[0], e->d_stats, first ? 1 : 0, ptot, tlim);
   if (!first)
@@ -4370,7 +4393,7 @@ static int cycle_body(fq_engine* e, const double* shift, const double* eproj_old
       ++e->online_runs;
     }
     const unsigned nb = grid_for(n);
-    hipLaunchKernelGGL(k_det_pass, dim3(nb), dim3(kBlock), 0, st, e->sys, n, cap, e->det[c], e->pop[c], e->kii[c],
+    hipLaunchKernelGGL(e->S == 1 ? k_det_pass<1> : k_det_pass<2>, dim3(nb), dim3(kBlock), 0, st, e->sys, n, cap, e->det[c], e->pop[c], e->kii[c],
                        e->pop_new, e->nat, e->flags, tau, shift[0], sh1, eproj_old[0], e1, e->par.philox_seed, cyc,
                        e->part_d, e->part_i, e->d_dvec, e->d_dpos, e->blk_att, e->d_stats);
     e->est_blocks = static_cast<int>(nb);
