@@ -37,6 +37,9 @@ struct Sys {
   int nsym;
   const int* sym_table;
   const int* inv_sym;
+  // Hubbard-k: label of k_c - k_p (the wavevector that completes k_p to k_c), at
+  // [(c - 1) * nsym + p - 1]: one byte, one lookup for sym_table of inv_sym
+  const uint8_t* sym_diff;
   const double* sp_eigv;
   int norb, nsym_pg, max_sym_spin;
   const int* orb_sym;
@@ -211,6 +214,17 @@ struct PhiloxPre {
         left(2 * K), failed(false) {
 #pragma unroll
     for (int q = 0; q < K; ++q) gen(w + 4 * q);
+  }
+  // The first block (words x, y) generated before.
+  __device__ PhiloxPre(uint64_t key, uint32_t a, uint32_t b, uint32_t c, uint64_t x, uint64_t y)
+      : k0(static_cast<uint32_t>(key)), k1(static_cast<uint32_t>(key >> 32)), c0(a), c1(b), c2(c), block(1),
+        left(2 * K), failed(false) {
+    w[0] = static_cast<uint32_t>(x);
+    w[1] = static_cast<uint32_t>(x >> 32);
+    w[2] = static_cast<uint32_t>(y);
+    w[3] = static_cast<uint32_t>(y >> 32);
+#pragma unroll
+    for (int q = 1; q < K; ++q) gen(w + 4 * q);
   }
   __device__ double next() {
     if (left == 0) {
@@ -706,10 +720,11 @@ __device__ inline int64_t spawn_hub_k(const Sys& s, Rng& rng, const uint64_t* f,
   conn.to[0] = conn.to[1] = 0;
   conn.perm = false;
   double pgen, absh;
+  const uint8_t* diff = s.sym_diff + (ij_sym - 1) * s.nsym;  // partner of orbital a: 2 diff[(a + 1) / 2 - 1]
   if (s.excit_gen == FQ_EXCIT_NO_RENORM) {
     const int rr = static_cast<int>(rng.next() * s.nvirt_alpha) + 1;
     const int a = select_orb(unoa, s.W, rr - 1);
-    const int b = 2 * st(s, ij_sym, s.inv_sym[(a + 1) / 2 - 1]);
+    const int b = 2 * diff[(a + 1) / 2 - 1];
     conn.to[0] = a;
     conn.to[1] = b;
     if (!btest(f, b)) {
@@ -720,14 +735,21 @@ __device__ inline int64_t spawn_hub_k(const Sys& s, Rng& rng, const uint64_t* f,
       absh = 0.0;
     }
   } else {
+    // unoccupied alpha orbitals whose partner is occupied, four lookups in flight
     int forbidden = 0;
     FQ_FOR_WORDS(w, s.W) {
       uint64_t x = unoa[w];
       while (x) {
-        const int a = (w << 6) + __builtin_ctzll(x) + 1;
-        x &= x - 1;
-        const int b = 2 * st(s, ij_sym, s.inv_sym[(a + 1) / 2 - 1]);
-        if (btest(f, b)) ++forbidden;
+        int b[4];
+        bool in[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          in[q] = x != 0;
+          b[q] = 2 * diff[in[q] ? (w << 5) + (__builtin_ctzll(x) >> 1) : 0];
+          x &= x - 1;  // 0 stays 0
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) forbidden += in[q] && btest(f, b[q]) ? 1 : 0;
       }
     }
     pgen = 1.0 / static_cast<double>(s.nalpha * s.nbeta * (s.nvirt_alpha - forbidden));
@@ -736,12 +758,11 @@ __device__ inline int64_t spawn_hub_k(const Sys& s, Rng& rng, const uint64_t* f,
   int64_t nspawn = stoch_round_spawn(s, rng, static_cast<double>(s.rf) * tau * absh / pgen);
   if (nspawn != 0) {
     if (s.excit_gen != FQ_EXCIT_NO_RENORM) {
-      const int sym2 = st(s, (conn.from[0] + 1) / 2, (conn.from[1] + 1) / 2);
       int a = 0, b = 0;
       for (int tries = 0; tries < kMaxRejection; ++tries) {
         const int rr = static_cast<int>(rng.next() * s.nvirt_alpha) + 1;
         a = select_orb(unoa, s.W, rr - 1);
-        b = 2 * st(s, sym2, s.inv_sym[(a + 1) / 2 - 1]);
+        b = 2 * diff[(a + 1) / 2 - 1];
         if (!btest(f, b) || rng.failed) break;
       }
       conn.to[0] = a;

@@ -329,6 +329,7 @@ struct fq_engine {
   fq_params par{};
   int W = 1, S = 1;
   // device tables
+  uint8_t* d_sym_diff = nullptr;
   int *d_sym_table = nullptr, *d_inv_sym = nullptr, *d_orb_sym = nullptr, *d_nbss = nullptr, *d_ssbf = nullptr;
   double *d_sp_eigv = nullptr, *d_h1 = nullptr, *d_eri = nullptr, *d_jmat = nullptr, *d_kmat = nullptr;
   double *d_s1j = nullptr, *d_s1k = nullptr;
@@ -893,8 +894,12 @@ __global__ __launch_bounds__(kBlock) void k_att_scan(const int32_t* __restrict__
 // (two draws each: the single/double choice, the orbital choices with their
 // first rejection redraws, the spawn rounding).  On mol26 (renormalised
 // generator) k_spawn took 474, 465, 454 and 425 us with 0, 2, 3 and 4 blocks;
-// 4 keeps its 80 VGPRs (6 waves per SIMD).
-constexpr int kSpawnPre = 4;
+// 4 keeps its 80 VGPRs (6 waves per SIMD).  A Hubbard attempt draws the pair and
+// the rounding, and more only if it spawns: one block (114 -> 112 us for 1.5e6
+// attempts on an 18-site ring; with the one-byte partner table, 104).
+constexpr int spawn_pre(int g) { return g == fqd::kGenHubK ? 1 : 4; }
+// Wavefronts per SIMD the registers are held to.
+constexpr int spawn_waves(int g, bool batched) { return g == fqd::kGenMolRenorm && !batched ? 6 : 4; }
 constexpr int kRecipN = 4096;  // entries of the host-made reciprocal table
 
 // Parent windows of the tiles of the batch [t_begin, t_end) (kSpawnTile
@@ -997,7 +1002,7 @@ __device__ __forceinline__ void make_key_any(const KeyPlan& kp, const uint64_t* 
 // contiguously from the tile's first staging slot, with the tile's count in
 // tile_cnt; k_pack_tiles then copies the tiles, in order, into the spawned list.
 template <int G, bool B, int T>
-__global__ __launch_bounds__(kBlock) void k_spawn(const Sys* __restrict__ sdev, int64_t nent, int64_t cap, int64_t t_begin, int64_t t_end,
+__global__ __launch_bounds__(kBlock, spawn_waves(G, B)) void k_spawn(const Sys* __restrict__ sdev, int64_t nent, int64_t cap, int64_t t_begin, int64_t t_end,
                                                   const int64_t* __restrict__ att_off,
                                                   const uint64_t* __restrict__ det, const int64_t* __restrict__ pop,
                                                   double tau, uint64_t seed, uint32_t cyc, int64_t bcap,
@@ -1095,17 +1100,31 @@ __global__ __launch_bounds__(kBlock) void k_spawn(const Sys* __restrict__ sdev, 
       load_det(det, cap, s.W, i, f);
       const int64_t parent = pop[sp * cap + i];
       if constexpr (B) {
-        // batched instances: the instance's tables, time step, key and attempt numbering
-        const int inst = static_cast<int>(f[0] >> kInstShift);
+        // batched instances: the instance's tables, time step, key and attempt
+        // numbering.  Attempts are numbered instance by instance, so a wavefront
+        // seldom holds two: its instances are taken one after the other, the
+        // descriptor in scalar registers
+        const int mine = static_cast<int>(f[0] >> kInstShift);
         f[0] &= kOrbMask;
-        const int64_t trel = t - iatt[inst];
-        fqd::PhiloxPre<kSpawnPre> rng(seed + static_cast<uint64_t>(inst), static_cast<uint32_t>(trel),
-                                      static_cast<uint32_t>(trel >> 32), cyc ^ (fqd::kDrawAttempt << 24));
-        nspawn = fqd::spawn_attempt<G>(sys_arr[inst], rng, f, nullptr, parent, itau[inst], child);
-        if (nspawn != 0) child[0] |= static_cast<uint64_t>(inst) << kInstShift;
+        bool todo = true;
+        while (todo) {
+          const int inst = __builtin_amdgcn_readfirstlane(mine);
+          if (inst == mine) {
+            const int64_t trel = t - iatt[inst];
+            fqd::PhiloxPre<spawn_pre(G)> rng(seed + static_cast<uint64_t>(inst), static_cast<uint32_t>(trel),
+                                             static_cast<uint32_t>(trel >> 32), cyc ^ (fqd::kDrawAttempt << 24));
+            nspawn = fqd::spawn_attempt<G>(sys_arr[inst], rng, f, nullptr, parent, itau[inst], child);
+            if (nspawn != 0) child[0] |= static_cast<uint64_t>(inst) << kInstShift;
+            todo = false;
+          }
+        }
       } else {
-        fqd::PhiloxPre<kSpawnPre> rng(seed, static_cast<uint32_t>(t), static_cast<uint32_t>(t >> 32),
-                                      cyc ^ (fqd::kDrawAttempt << 24));
+        const uint32_t t_lo = static_cast<uint32_t>(t), t_hi = static_cast<uint32_t>(t >> 32);
+        const uint32_t purpose = cyc ^ (fqd::kDrawAttempt << 24);
+        using Rng = fqd::PhiloxPre<spawn_pre(G)>;
+        // partitioned tiles: the attempt's first block is parked in its result slots
+        Rng rng = kPart ? Rng(seed, t_lo, t_hi, purpose, static_cast<uint64_t>(rpop[kPart ? r : 0]), rdet[kPart ? r : 0])
+                        : Rng(seed, t_lo, t_hi, purpose);
         const float* wrow = (G == fqd::kGenLearned && s.mlp_on[i]) ? s.mlp_tab + s.mlp_row[i] * s.mlp_ld : nullptr;
         nspawn = fqd::spawn_attempt<G>(s, rng, f, wrow, parent, tau, child, hb, aff_lds, flat_lds);
         // a core parent's spawn onto the core is the deterministic projection's
@@ -1123,6 +1142,9 @@ __global__ __launch_bounds__(kBlock) void k_spawn(const Sys* __restrict__ sdev, 
           fqd::Philox rng(seed, static_cast<uint32_t>(t), static_cast<uint32_t>(t >> 32),
                           cyc ^ (fqd::kDrawAttempt << 24));
           single = rng.next() < s.psingle;
+          // the block stays in the attempt's result slots until the attempt is made
+          rpop[r] = static_cast<int64_t>(static_cast<uint64_t>(rng.o1) << 32 | rng.o0);
+          rdet[r] = static_cast<uint64_t>(rng.o3) << 32 | rng.o2;
         }
         const unsigned long long bd = __ballot(r < tn && !single), bs = __ballot(r < tn && single);
         if (lane == 0) {
@@ -3943,8 +3965,17 @@ void pack_spawned(fq_engine* e, int64_t nbt, int tile, bool first, const int64_t
     hipLaunchKernelGGL(k_add_spawned, dim3(1), dim3(kBlock), 0, e->stream, e->tile_cnt, nt, ptot, e->d_stats);
 }
 
-// Attempts per tile of a cycle with at most `attempts` attempts.
-int spawn_tile(int64_t attempts) { return attempts <= kSmallTileMax ? kSmallTile : kSpawnTile; }
+// Attempts per tile of a cycle with at most `attempts` attempts of generator
+// gen.  The learned generator's affinity table leaves LDS for two blocks of
+// 1024-attempt tiles on a CU, four of 256-attempt ones, and its attempts are
+// chains of table reads that need the wavefronts (9.5e5 attempts on 40 orbitals:
+// 486 -> 322 us).
+int spawn_tile(int gen, int64_t attempts) {
+  return attempts <= kSmallTileMax || gen == fqd::kGenLearned ? kSmallTile : kSpawnTile;
+}
+// Most blocks of a spawning launch: as many as are resident for the learned
+// generator, whose blocks each stage the affinity table once, else one per tile.
+int64_t spawn_grid(int gen, int64_t tiles) { return std::min<int64_t>(tiles, gen == fqd::kGenLearned ? 1024 : 1 << 20); }
 template <bool B, int T>
 auto spawn_kernel(int gen) {
   if constexpr (B) {
@@ -4100,6 +4131,18 @@ int fq_create(const fq_system* sys, const fq_params* params, fq_engine** out) {
   if (sys->system == FQ_SYS_HUB_K) {
     rc |= upload(&e->d_sym_table, sys->sym_table, static_cast<int64_t>(sys->nsym) * sys->nsym, e->stream);
     rc |= upload(&e->d_inv_sym, sys->inv_sym, sys->nsym, e->stream);
+    std::vector<uint8_t> diff;
+    if (sys->nsym <= 255 && sys->sym_table && sys->inv_sym) {  // labels in a byte: at most 64 of them
+      diff.resize(static_cast<size_t>(sys->nsym) * sys->nsym);
+      for (int c = 0; c < sys->nsym; ++c)
+        for (int p = 0; p < sys->nsym; ++p) {
+          const int inv = sys->inv_sym[p];
+          diff[c * sys->nsym + p] =
+              inv >= 1 && inv <= sys->nsym ? static_cast<uint8_t>(sys->sym_table[c * sys->nsym + inv - 1]) : 0;
+        }
+    }
+    if (rc == FQ_OK) rc = upload(&e->d_sym_diff, diff.data(), static_cast<int64_t>(diff.size()), e->stream);
+    if (rc == FQ_OK) FQ_HIP(hipStreamSynchronize(e->stream));
   } else {
     rc |= upload(&e->d_orb_sym, sys->orb_sym, sys->nbasis, e->stream);
     rc |= upload(&e->d_nbss, sys->nbasis_sym_spin, 2 * sys->nsym_pg, e->stream);
@@ -4147,6 +4190,7 @@ int fq_create(const fq_system* sys, const fq_params* params, fq_engine** out) {
   s.sp_eigv = e->d_sp_eigv;
   s.sym_table = e->d_sym_table;
   s.inv_sym = e->d_inv_sym;
+  s.sym_diff = e->d_sym_diff;
   s.orb_sym = e->d_orb_sym;
   s.nbss = e->d_nbss;
   s.ssbf = e->d_ssbf;
@@ -4428,7 +4472,8 @@ static int cycle_body(fq_engine* e, const double* shift, const double* eproj_old
     // not wait for the prefix sum; otherwise it reads the total.  The kernels
     // clamp to the total on the device.
     int64_t bound = e->att_bound;
-    const int tile = bound > 0 && bound <= e->bcap ? spawn_tile(bound) : kSpawnTile;  // batches: k_tile_bounds' tiles
+    const int gen = fqd::gen_of(e->sys.system, e->sys.excit_gen);
+    const int tile = bound > 0 && bound <= e->bcap ? spawn_tile(gen, bound) : kSpawnTile;  // batches: k_tile_bounds' tiles
     int rc = scan_attempts(e, nent, bound > 0 ? std::min(bound, e->bcap) : e->bcap, tile);
     if (rc != FQ_OK) return rc;
     if (bound <= 0) {  // unknown (or an empty list): the exact total
@@ -4438,7 +4483,6 @@ static int cycle_body(fq_engine* e, const double* shift, const double* eproj_old
     e->spawn_launches = 0;
     if (int rs = sync_sysp(e); rs != FQ_OK) return rs;
     const bool one_batch = bound <= e->bcap;
-    const int gen = fqd::gen_of(e->sys.system, e->sys.excit_gen);
     auto kern = tile == kSmallTile ? spawn_kernel<false, kSmallTile>(gen) : spawn_kernel<false, kSpawnTile>(gen);
     const size_t lds = gen == fqd::kGenHeatBath    ? hb_lds_bytes(e->sys.nel)
                        : gen == fqd::kGenMolRenorm ? sizeof(uint64_t) * e->W * tile
@@ -4451,7 +4495,7 @@ static int cycle_body(fq_engine* e, const double* shift, const double* eproj_old
       if (!one_batch)
         hipLaunchKernelGGL(k_tile_bounds, dim3(grid_for(nt)), dim3(kBlock), 0, st, nent, e->att_off, tb, te,
                            e->tile_win);
-      hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(std::min<int64_t>(nt, 1 << 20))), dim3(kBlock), lds, st,
+      hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(spawn_grid(gen, nt))), dim3(kBlock), lds, st,
                          e->d_sysp, nent, cap, tb, te, e->att_off, e->det[c], e->pop[c], tau, e->par.philox_seed, cyc,
                          e->bcap, e->st_det, e->st_pop, e->st_ent, e->tile_cnt, e->tile_win, e->flags, nullptr,
                          nullptr, nullptr, nullptr, e->d_stats);
@@ -4873,13 +4917,13 @@ static int enqueue_graph_cycle(fq_engine* e, int64_t nb, int64_t tb) {
                      e->d_cterm, e->d_cdeath, dn, dcyc, e->blk_att, e->d_stats);
   // entries past the list have no attempts, so att_off[S nb] is the total
   const int64_t nent = S * nb;
-  const int tile = spawn_tile(tb);
+  const int gen = fqd::gen_of(e->sys.system, e->sys.excit_gen);
+  const int tile = spawn_tile(gen, tb);
   int rc = scan_attempts(e, nent, tb, tile);
   if (rc != FQ_OK) return rc;
   hipLaunchKernelGGL(k_inst_att, dim3(grid_for(ninst)), dim3(kBlock), 0, st, ninst, S, ob, e->att_off, e->d_iatt);
   const unsigned g = static_cast<unsigned>(std::min<int64_t>(
       ceil_div(tb, tile), e->spawn_blocks > 0 ? e->spawn_blocks : int64_t{1} << 20));
-  const int gen = fqd::gen_of(e->sys.system, e->sys.excit_gen);
   auto kern = tile == kSmallTile ? spawn_kernel<true, kSmallTile>(gen) : spawn_kernel<true, kSpawnTile>(gen);
   hipLaunchKernelGGL(kern, dim3(g), dim3(kBlock), 0, st, e->d_sysp, nent, cap, int64_t{0}, tb, e->att_off, e->det[c],
                      e->pop[c], 0.0, e->par.philox_seed, 0u, e->bcap, e->st_det, e->st_pop, e->st_ent, e->tile_cnt,
@@ -5409,6 +5453,7 @@ void fq_destroy(fq_engine* e) {
   dfree(e->d_sp_eigv);
   dfree(e->d_sym_table);
   dfree(e->d_inv_sym);
+  dfree(e->d_sym_diff);
   dfree(e->d_orb_sym);
   dfree(e->d_nbss);
   dfree(e->d_ssbf);
