@@ -48,6 +48,7 @@
 #include <functional>
 #include <mutex>
 #include <queue>
+#include <thread>
 #include <type_traits>
 #include <vector>
 
@@ -91,6 +92,7 @@ constexpr int kMainTile = 4 * kBlock;  // main-list entries per rounding and ins
 // (its threads add the counts before its tile: 16384 counts are 64 KB from L2);
 // longer ones are scanned first.
 constexpr int64_t kPrefixMax = 16384;
+constexpr int64_t kListSlotBytes = int64_t{1} << 20;  // a pinned slot of fq_download
 // Words per spawned-list record (populations, flag), padded to 16-byte
 // alignment so one record is one aligned read after the sort's permutation.
 __host__ __device__ constexpr int rec_stride(int S) { return S == 1 ? 2 : 4; }
@@ -488,6 +490,13 @@ struct fq_engine {
   Stats* h_pin = nullptr;  // pinned: the cycle's finished stats (k_finish)
   Stats h_stats{};
   uint64_t cycle_index = 0;
+  // fq_download's pinned slots (one block of them, made on first use), their
+  // events, and the streams they share with the engine's (a stream takes ~1 ms to make)
+  static constexpr int kListSlots = 6, kListStreams = 3;
+  hipStream_t list_stream[kListStreams] = {};
+  uint64_t* list_buf = nullptr;
+  int list_slots = 0;
+  hipEvent_t list_ev[kListSlots] = {};
   // the spawned-list length, spawn overflow and attempt total, copied behind
   // the spawning kernels into pinned memory (h_len) and marked by ev_len
   int64_t* h_len = nullptr;
@@ -734,8 +743,8 @@ __global__ __launch_bounds__(kFinishBlock) void k_finish(const double* __restric
   for (int q = 0; q < NQ; ++q) acc[q] = 0.0;
   int64_t ai = 0, ap[FQ_MAX_SPACES] = {0, 0};
   if (tid < kBlock) {
-    // blocks t, t + 256, ... added in that order; sixteen are loaded ahead at a time
-    constexpr int kAhead = 16;
+    // blocks t, t + 256, ... added in that order; 16 (pairs: 8, within the registers) are loaded ahead at a time
+    constexpr int kAhead = 16 / S;
     for (int b0 = tid; b0 < nb; b0 += kAhead * kBlock) {
       double v[kAhead][NQ];
       int64_t vi[kAhead];
@@ -3335,7 +3344,7 @@ constexpr int64_t kNoWaitMax = int64_t{1} << 21;
 // The main list's sort values in buffer c.
 const uint64_t* main_values(const fq_engine* e, int c) { return e->rank_words ? e->mrank[c] : e->det[c]; }
 constexpr int64_t kNewBlocks = 1024;  // most blocks of the new determinants' insertion
-constexpr size_t kInsertLdsMax = 60 * 1024;  // their tables, beside the kernel's own LDS in the default 64 KB
+constexpr size_t kInsertLdsMax = 120 * 1024;  // LDS of their tables (set_insert_lds raises the default 64 KB)
 
 // Index bits of k_sort_small beside the value, and the list length it takes (0: none).
 int small_sort_idx_bits(const fq_engine* e) { return std::min(13, 64 - e->value_bits); }
@@ -3563,11 +3572,12 @@ int annihilate(fq_engine* e, int64_t ns, const int64_t* pns, bool replay, uint32
   hipLaunchKernelGGL(k_scatter_main, dim3(static_cast<unsigned>(mtiles)), dim3(kBlock), 0, st, g);
   int64_t nblk = mtiles;
   if (ns > 0) {
-    // dense pair tables in LDS for the diagonal when they fit in 32 KB, the binomial table when it fits beside them
+    // dense pair tables in LDS for the diagonal (up to 64 orbitals: 64 KB), the binomial table when it fits beside
+    // them: both are read in chains (60 orbitals, 20 electrons in pairs: 78 us from L2, 59 from LDS)
     const size_t jk = e->sys.system == FQ_SYS_READ_IN && !e->batched
                           ? 2 * sizeof(double) * static_cast<size_t>(e->sys.norb) * e->sys.norb
                           : 0;
-    const bool use_jk = jk > 0 && jk <= 32768;
+    const bool use_jk = jk > 0 && jk <= 65536;
     KeyPlan kp = key_plan(e);
     const size_t tab = binom_bytes(e) / (kw == 1 ? 2 : 1);
     kp.binom_lds = tab > 0 && tab + (use_jk ? jk : 0) <= kInsertLdsMax;
@@ -3851,6 +3861,14 @@ int setup_learned(fq_engine* e) {
   s.mlp_on = e->mlp_on;
   s.mlp_row = e->mlp_row;
   s.mix = e->par.proposal_mix > 0.0 ? e->par.proposal_mix : 0.1;
+  return FQ_OK;
+}
+
+// The insertion's dynamic LDS limit on the current device.
+int set_insert_lds() {
+  for (const void* f : {reinterpret_cast<const void*>(&k_scatter_new<false>),
+                        reinterpret_cast<const void*>(&k_scatter_new<true>)})
+    FQ_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kInsertLdsMax)));
   return FQ_OK;
 }
 
@@ -4207,6 +4225,7 @@ int fq_create(const fq_system* sys, const fq_params* params, fq_engine** out) {
   if (rc == FQ_OK && (params->excit_gen == FQ_EXCIT_HEAT_BATH || params->excit_gen == FQ_EXCIT_LEARNED))
     rc = build_heat_bath(e);
   if (rc == FQ_OK && params->excit_gen == FQ_EXCIT_LEARNED) rc = setup_learned(e);
+  if (rc == FQ_OK) rc = set_insert_lds();
   if (rc == FQ_OK) rc = alloc_engine(e);
   if (rc == FQ_OK) rc = setup_sort(e);
   if (int khz = 0; rc == FQ_OK && hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, e->device) == hipSuccess &&
@@ -4705,6 +4724,56 @@ int fq_nstates(fq_engine* e, int64_t* n) {
   return FQ_OK;
 }
 
+// Rows [r0, r1) of the list to the caller's arrays by way of one pinned slot,
+// as many rows at a time as it holds.
+static hipError_t copy_rows(fq_engine* e, int slot, int64_t r0, int64_t r1, uint64_t* states, int64_t* pops,
+                            double* dat) {
+  if (hipError_t err = hipSetDevice(e->device); err != hipSuccess) return err;
+  const int W = e->W, S = e->S, c = e->cur;
+  const int64_t rows = kListSlotBytes / (8 * (W + S + 1));
+  uint64_t* buf = e->list_buf + slot * (kListSlotBytes / 8);
+  const int q3 = slot % fq_engine::kListStreams;
+  hipStream_t st = q3 == 0 ? e->stream : e->list_stream[q3];  // shared: each thread waits for its own copies only
+  for (int64_t i = r0; i < r1; i += rows) {
+    const int64_t m = std::min(rows, r1 - i);
+    uint64_t* q = buf;
+    auto fetch = [&](const void* from) {
+      const hipError_t err = hipMemcpyAsync(q, from, 8 * m, hipMemcpyDeviceToHost, st);
+      q += m;
+      return err;
+    };
+    hipError_t err = hipSuccess;
+    if (states)
+      for (int w = 0; w < W && err == hipSuccess; ++w) err = fetch(e->det[c] + w * e->cap + i);
+    if (pops)
+      for (int sp = 0; sp < S && err == hipSuccess; ++sp) err = fetch(e->pop[c] + sp * e->cap + i);
+    if (dat && err == hipSuccess) err = fetch(e->kii[c] + i);
+    if (err == hipSuccess) err = hipEventRecord(e->list_ev[slot], st);
+    if (err == hipSuccess) err = hipEventSynchronize(e->list_ev[slot]);
+    if (err != hipSuccess) return err;
+    q = buf;
+    auto place = [&](void* to, int n) {  // n arrays of m words, interleaved
+      if (n == 1) {
+        std::memcpy(static_cast<uint64_t*>(to) + i, q, 8 * m);
+      } else {
+        uint64_t* d = static_cast<uint64_t*>(to) + n * i;
+        for (int64_t k = 0; k < m; ++k)
+          for (int w = 0; w < n; ++w) d[n * k + w] = q[w * m + k];
+      }
+      q += n * m;
+    };
+    if (states) place(states, W);
+    if (pops) place(pops, S);
+    if (dat) place(dat, 1);
+  }
+  return hipSuccess;
+}
+
+// The list leaves through pinned slots, one per thread: each thread copies its
+// part of the rows a slot at a time, so one thread's transfer runs while the
+// others move theirs to the caller's (pageable) arrays.  (Copies to pageable
+// temporaries and a second pass over them took 15.8 ms for 2.7e6 one-word
+// entries and 8.4 ms for 1.0e6 two-word pairs; 2.3 and 1.7 ms now.)
 int fq_download(fq_engine* e, uint64_t* states, int64_t* pops, double* dat, int64_t capacity, int64_t* nout) {
   if (!e || !nout) return FQ_ERR_ARG;
   const int64_t n = e->n;
@@ -4712,22 +4781,41 @@ int fq_download(fq_engine* e, uint64_t* states, int64_t* pops, double* dat, int6
   if (capacity < n) return FQ_ERR_CAPACITY;
   if (n == 0) return FQ_OK;
   FQ_HIP(hipSetDevice(e->device));
-  const int W = e->W, S = e->S;
-  std::vector<uint64_t> dw(static_cast<size_t>(W) * n);
-  std::vector<int64_t> dp(static_cast<size_t>(S) * n);
-  const int c = e->cur;
-  for (int w = 0; w < W; ++w)
-    FQ_HIP(hipMemcpyAsync(dw.data() + w * n, e->det[c] + w * e->cap, 8 * n, hipMemcpyDeviceToHost, e->stream));
-  for (int s = 0; s < S; ++s)
-    FQ_HIP(hipMemcpyAsync(dp.data() + s * n, e->pop[c] + s * e->cap, 8 * n, hipMemcpyDeviceToHost, e->stream));
-  if (dat) FQ_HIP(hipMemcpyAsync(dat, e->kii[c], 8 * n, hipMemcpyDeviceToHost, e->stream));
   FQ_HIP(hipStreamSynchronize(e->stream));
-  for (int64_t i = 0; i < n; ++i) {
-    if (states)
-      for (int w = 0; w < W; ++w) states[i * W + w] = dw[w * n + i];
-    if (pops)
-      for (int s = 0; s < S; ++s) pops[i * S + s] = dp[s * n + i];
+  const int64_t bytes = 8 * n * (e->W + e->S + 1);
+  const int nt = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(fq_engine::kListSlots, bytes / kListSlotBytes)));
+  if (e->list_slots < nt) {
+    if (e->list_buf) (void)hipHostFree(e->list_buf);
+    e->list_buf = nullptr;
+    e->list_slots = nt == 1 ? 1 : fq_engine::kListSlots;
+    if (hipHostMalloc(reinterpret_cast<void**>(&e->list_buf), e->list_slots * kListSlotBytes) != hipSuccess) {
+      e->list_buf = nullptr;
+      e->list_slots = 0;
+      return FQ_ERR_NOMEM;
+    }
   }
+  for (int t = 0; t < nt; ++t) {
+    if (!e->list_ev[t]) FQ_HIP(hipEventCreateWithFlags(&e->list_ev[t], hipEventDisableTiming));
+    const int q = t % fq_engine::kListStreams;
+    if (q > 0 && !e->list_stream[q]) FQ_HIP(hipStreamCreateWithFlags(&e->list_stream[q], hipStreamNonBlocking));
+  }
+  hipError_t err[fq_engine::kListSlots] = {};
+  std::thread th[fq_engine::kListSlots];
+  auto part = [&](int t) { err[t] = copy_rows(e, t, n * t / nt, n * (t + 1) / nt, states, pops, dat); };
+  for (int t = 1; t < nt; ++t) {
+    try {
+      th[t] = std::thread(part, t);
+    } catch (const std::exception&) {  // no thread to be had: this one does the part below
+    }
+  }
+  part(0);
+  for (int t = 1; t < nt; ++t) {
+    if (th[t].joinable())
+      th[t].join();
+    else
+      part(t);
+  }
+  for (int t = 0; t < nt; ++t) FQ_HIP(err[t]);
   return FQ_OK;
 }
 
@@ -5502,6 +5590,11 @@ void fq_destroy(fq_engine* e) {
   if (e->ev_len) (void)hipEventDestroy(e->ev_len);
   if (e->h_len) (void)hipHostFree(e->h_len);
   if (e->h_pin) (void)hipHostFree(e->h_pin);
+  if (e->list_buf) (void)hipHostFree(e->list_buf);
+  for (hipEvent_t ev : e->list_ev)
+    if (ev) (void)hipEventDestroy(ev);
+  for (hipStream_t q : e->list_stream)
+    if (q) (void)hipStreamDestroy(q);
   for (auto& g : e->graphs) (void)hipGraphExecDestroy(g.exec);
   for (int k = 0; k < 2; ++k)
     if (e->gev[k]) (void)hipEventDestroy(e->gev[k]);
