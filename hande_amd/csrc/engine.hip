@@ -961,8 +961,12 @@ struct DigitPlan {
   int shift[kMaxPasses];   // first key bit of each pass's digit
   int bits[kMaxPasses];    // digit width (8 or 9)
 };
-// Keys per thread of a sort tile: the tile's keys and payload sit in LDS.
+// Keys per thread of a sort tile: the tile's keys and payload sit in LDS.  Lists
+// that tiles of kSmallSortItems keys a thread spread over at most kSortBlocks
+// blocks take those: with the large tiles 2e5 keys ran on 49 of the 256 CUs
+// (count and scatter of a 9-bit pass 10 and 13.5 us; 7.4 and 9.2 now).
 __host__ __device__ constexpr int sort_items(int kw, int S) { return kw + S <= 2 ? 16 : 8; }
+constexpr int kSmallSortItems = 4;
 constexpr int kSortBlocks = 512;  // blocks of a radix pass (each owns a contiguous range of tiles)
 
 // STRIDE: words per entry of the table (2: low and high; 1: low words only).
@@ -1721,12 +1725,12 @@ __device__ __forceinline__ uint32_t block_exclusive_u32(uint32_t x, uint32_t* ws
 // k_pass_scatter walks its tiles in order, ranks each tile's keys by digit in
 // input order (stable), and writes keys and payload (S population words) to
 // their sorted positions.  No block waits on another.
-template <int KW, int S, int DB>
+template <int KW, int S, int DB, int R>
 __global__ __launch_bounds__(kBlock) void k_pass_count(const uint64_t* __restrict__ keys,
                                                        const int64_t* __restrict__ pn, int64_t nb, int64_t stride,
                                                        int shift, int64_t* __restrict__ cnt,
                                                        Stats* __restrict__ st) {
-  constexpr int NB = 1 << DB, R = sort_items(KW, S), T = kBlock * R;
+  constexpr int NB = 1 << DB, T = kBlock * R;
   __shared__ uint32_t h[NB];
   if (st) stamp(st, kStSort);  // the first pass
   for (int d = threadIdx.x; d < NB; d += kBlock) h[d] = 0;
@@ -1778,14 +1782,14 @@ __global__ __launch_bounds__(kSortBlocks) void k_pass_rowscan(int nb, int64_t* _
   if (b == 0) tot[d] = t;
 }
 
-template <int KW, int S, int DB>
+template <int KW, int S, int DB, int R>
 __global__ __launch_bounds__(kBlock) void k_pass_scatter(const uint64_t* __restrict__ kin,
                                                          const int64_t* __restrict__ pin, uint64_t* __restrict__ kout,
                                                          int64_t* __restrict__ pout, const int64_t* __restrict__ pn,
                                                          int64_t nb, int64_t stride, int shift,
                                                          const int64_t* __restrict__ off,
                                                          const int64_t* __restrict__ dtot) {
-  constexpr int NB = 1 << DB, R = sort_items(KW, S), T = kBlock * R, NW = kBlock / 64;
+  constexpr int NB = 1 << DB, T = kBlock * R, NW = kBlock / 64;
   const int64_t n = list_len(pn, nb);
   const int64_t tpb = ((n + T - 1) / T + gridDim.x - 1) / gridDim.x;
   constexpr uint32_t MASK = NB - 1;
@@ -3317,22 +3321,25 @@ void launch_make_keys(fq_engine* e, int64_t ns, const uint32_t* perm) {
 
 // One radix pass from buffer `src` to the other.
 // ns: the list length, or a bound of it when pns (the device count) is given.
-template <int KW, int S, int DB>
+template <int KW, int S, int DB, int R>
 int sort_pass(fq_engine* e, int src, int64_t ns, const int64_t* pns, int shift) {
-  constexpr int T = kBlock * sort_items(KW, S);
+  constexpr int T = kBlock * R;
   const int64_t nb = std::min<int64_t>(ceil_div(ns, T), kSortBlocks);
-  hipLaunchKernelGGL((k_pass_count<KW, S, DB>), dim3(static_cast<unsigned>(nb)), dim3(kBlock), 0, e->stream,
+  hipLaunchKernelGGL((k_pass_count<KW, S, DB, R>), dim3(static_cast<unsigned>(nb)), dim3(kBlock), 0, e->stream,
                      e->kbuf[src], pns, ns, e->scap, shift, e->pass_cnt, e->radix_passes == 0 ? e->d_stats : nullptr);
   hipLaunchKernelGGL(k_pass_rowscan, dim3(1u << DB), dim3(kSortBlocks), 0, e->stream, static_cast<int>(nb),
                      e->pass_cnt, e->pass_off);
-  hipLaunchKernelGGL((k_pass_scatter<KW, S, DB>), dim3(static_cast<unsigned>(nb)), dim3(kBlock), 0, e->stream,
+  hipLaunchKernelGGL((k_pass_scatter<KW, S, DB, R>), dim3(static_cast<unsigned>(nb)), dim3(kBlock), 0, e->stream,
                      e->kbuf[src], e->pbuf[src], e->kbuf[1 - src], e->pbuf[1 - src], pns, ns, e->scap, shift,
                      e->pass_cnt, e->pass_off);
   return FQ_OK;
 }
 template <int KW, int S>
-int sort_pass_db(fq_engine* e, int src, int64_t ns, const int64_t* pns, int shift, int db) {
-  return db == 9 ? sort_pass<KW, S, 9>(e, src, ns, pns, shift) : sort_pass<KW, S, 8>(e, src, ns, pns, shift);
+int sort_pass_db(fq_engine* e, int src, int64_t ns, const int64_t* pns, int shift, int db, bool small) {
+  constexpr int R = sort_items(KW, S), Q = kSmallSortItems;
+  if (small)
+    return db == 9 ? sort_pass<KW, S, 9, Q>(e, src, ns, pns, shift) : sort_pass<KW, S, 8, Q>(e, src, ns, pns, shift);
+  return db == 9 ? sort_pass<KW, S, 9, R>(e, src, ns, pns, shift) : sort_pass<KW, S, 8, R>(e, src, ns, pns, shift);
 }
 
 // Spawned lists bounded by this many entries run the whole annihilation in
@@ -3386,14 +3393,17 @@ int sort_and_reduce(fq_engine* e, int64_t ns, const int64_t* pns, bool replay, u
         e->radix_passes = ceil_div(e->value_bits, kSmallSortBits);
         pns = &e->d_stats->sorted;
       }
+      // tile size by the last cycle's length where this one's is only bounded
+      const int64_t like = pns && !e->capturing && e->last_ns >= 0 ? std::min(e->last_ns, ns) : ns;
+      const bool st_small = like <= int64_t{kSortBlocks} * kBlock * kSmallSortItems;
       for (int p = 0; p < dp.np && !small; ++p) {
         int rc;
         if (kw == 1)
-          rc = S == 1 ? sort_pass_db<1, 1>(e, src, ns, pns, dp.shift[p], dp.bits[p])
-                      : sort_pass_db<1, 2>(e, src, ns, pns, dp.shift[p], dp.bits[p]);
+          rc = S == 1 ? sort_pass_db<1, 1>(e, src, ns, pns, dp.shift[p], dp.bits[p], st_small)
+                      : sort_pass_db<1, 2>(e, src, ns, pns, dp.shift[p], dp.bits[p], st_small);
         else
-          rc = S == 1 ? sort_pass_db<2, 1>(e, src, ns, pns, dp.shift[p], dp.bits[p])
-                      : sort_pass_db<2, 2>(e, src, ns, pns, dp.shift[p], dp.bits[p]);
+          rc = S == 1 ? sort_pass_db<2, 1>(e, src, ns, pns, dp.shift[p], dp.bits[p], st_small)
+                      : sort_pass_db<2, 2>(e, src, ns, pns, dp.shift[p], dp.bits[p], st_small);
         if (rc != FQ_OK) return rc;
         src = 1 - src;
         ++e->radix_passes;
