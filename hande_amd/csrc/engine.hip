@@ -134,6 +134,7 @@ struct Stats {
   int64_t rng_pos;
   int64_t rng_failed;
   unsigned long long abs_pop[FQ_MAX_SPACES];  // sum |pop| after annihilation (encoded)
+  int64_t mlp_rows;                           // determinants the network runs on
   int64_t sorted;                             // entries k_sort_small sorted
   int64_t resort;                             // 1: the list was too long for it (nothing downstream ran)
   int64_t spawn_begin, spawn_ticks;           // start of the last spawning launch; time of them all
@@ -412,8 +413,8 @@ struct fq_engine {
   int new_src = 0;                   // the sort's idle buffers after this cycle's passes
   int64_t run_tiles = 0;             // run tiles of this cycle's spawned list (a bound of it while captured)
   int64_t mlp_tab_rows = 0;
-  int64_t* mlp_on = nullptr;   // [cap] network runs on this determinant this cycle
-  int64_t* mlp_row = nullptr;  // [cap + 1] exclusive prefix of mlp_on
+  int cls_sorted = 0;          // the spin/irrep classes list their orbitals in ascending order
+  int32_t* mlp_row = nullptr;  // [cap] this cycle's row of the weight table (-1: none)
   int64_t* mlp_idx = nullptr;  // [cap] determinants the network runs on
   // main list (double-buffered)
   int64_t cap = 0, n = 0;
@@ -1138,7 +1139,11 @@ __global__ __launch_bounds__(kBlock, spawn_waves(G, B)) void k_spawn(const Sys* 
         // partitioned tiles: the attempt's first block is parked in its result slots
         Rng rng = kPart ? Rng(seed, t_lo, t_hi, purpose, static_cast<uint64_t>(rpop[kPart ? r : 0]), rdet[kPart ? r : 0])
                         : Rng(seed, t_lo, t_hi, purpose);
-        const float* wrow = (G == fqd::kGenLearned && s.mlp_on[i]) ? s.mlp_tab + s.mlp_row[i] * s.mlp_ld : nullptr;
+        const float* wrow = nullptr;
+        if constexpr (G == fqd::kGenLearned) {
+          const int32_t row = s.mlp_row[i];
+          if (row >= 0) wrow = s.mlp_tab + row * s.mlp_ld;
+        }
         nspawn = fqd::spawn_attempt<G>(s, rng, f, wrow, parent, tau, child, hb, aff_lds, flat_lds);
         // a core parent's spawn onto the core is the deterministic projection's
         if (s.ndeterm > 0 && nspawn != 0 && (pflags[i] & kCoreFlag) && fqd::core_index(s, child) >= 0) nspawn = 0;
@@ -3859,8 +3864,8 @@ int setup_learned(fq_engine* e) {
   rc = fqm::mlp_init(e->mlp, e->par.philox_seed, e->stream);
   if (rc != FQ_OK) return rc;
   e->mlp_tab_rows = std::min<int64_t>(e->cap, int64_t{1} << 16);
-  if (dalloc(&e->mlp_tab, e->mlp_tab_rows * e->mlp.d_out) != FQ_OK || dalloc(&e->mlp_on, e->cap) != FQ_OK ||
-      dalloc(&e->mlp_row, e->cap + 1) != FQ_OK || dalloc(&e->mlp_idx, e->cap) != FQ_OK)
+  if (dalloc(&e->mlp_tab, e->mlp_tab_rows * e->mlp.d_out) != FQ_OK || dalloc(&e->mlp_row, e->cap) != FQ_OK ||
+      dalloc(&e->mlp_idx, e->cap) != FQ_OK)
     return FQ_ERR_NOMEM;
   s.mlp_tab = e->mlp_tab;
   s.mlp_aff = e->mlp.aff;
@@ -3878,9 +3883,9 @@ int setup_learned(fq_engine* e) {
   }
   s.mlp_flat = e->mlp_flat;
   s.mlp_ld = e->mlp.d_out;
-  s.mlp_on = e->mlp_on;
   s.mlp_row = e->mlp_row;
   s.mix = e->par.proposal_mix > 0.0 ? e->par.proposal_mix : 0.1;
+  s.cls_sorted = e->cls_sorted;
   return FQ_OK;
 }
 
@@ -3893,20 +3898,49 @@ int set_insert_lds() {
 }
 
 // Determinants with at least min_att spawning attempts this cycle get a
-// network row; mlp_gather lists them in order.
-__global__ void k_mlp_mark(int64_t n, int S, const int32_t* __restrict__ nat, int64_t min_att,
-                           int64_t* __restrict__ on, Stats* __restrict__ st) {
-  stamp(st, kStProposal);
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+// network row: k_mlp_mark counts them per tile of kMainTile entries, k_mlp_rows
+// numbers them in list order (row[i], -1: none) and lists them (idx), adding up
+// the counts of the tiles before its own (off, when given, holds them); the
+// number of rows goes to the stats, where the inference reads it.  No row is
+// numbered lim or above (lim: a bound of their number).
+constexpr int64_t kProposalTable = int64_t{1} << 30;  // bytes
+__device__ __forceinline__ bool gets_row(const int32_t* __restrict__ nat, int S, int64_t i, int64_t min_att) {
   int64_t a = 0;
   for (int sp = 0; sp < S; ++sp) a += nat[i * S + sp];
-  on[i] = a >= min_att ? 1 : 0;
+  return a >= min_att;
 }
-__global__ void k_mlp_gather(int64_t n, const int64_t* __restrict__ on, const int64_t* __restrict__ row,
-                             int64_t* __restrict__ idx) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i < n && on[i]) idx[row[i]] = i;
+__global__ __launch_bounds__(kBlock) void k_mlp_mark(int64_t n, int S, const int32_t* __restrict__ nat,
+                                                     int64_t min_att, int32_t* __restrict__ cnt,
+                                                     Stats* __restrict__ st) {
+  __shared__ int64_t wsh[kBlock / 64];
+  stamp(st, kStProposal);
+  int64_t c = 0;
+  for (int r = 0; r < kMainTile / kBlock; ++r) {
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * kMainTile + r * kBlock + threadIdx.x;
+    c += i < n && gets_row(nat, S, i, min_att) ? 1 : 0;
+  }
+  c = block_sum(c, wsh);
+  if (threadIdx.x == 0) cnt[blockIdx.x] = static_cast<int32_t>(c);
+}
+__global__ __launch_bounds__(kBlock) void k_mlp_rows(int64_t n, int S, const int32_t* __restrict__ nat,
+                                                     int64_t min_att, int64_t lim, const int32_t* __restrict__ cnt,
+                                                     const int64_t* __restrict__ off, int32_t* __restrict__ row,
+                                                     int64_t* __restrict__ idx, Stats* __restrict__ st) {
+  __shared__ int64_t wsh[kBlock / 64];
+  __shared__ uint32_t wsh32[kBlock / 64];
+  const int64_t before = tiles_before(cnt, off, blockIdx.x, wsh);
+  uint32_t at = static_cast<uint32_t>(before);
+  for (int r = 0; r < kMainTile / kBlock; ++r) {
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * kMainTile + r * kBlock + threadIdx.x;
+    bool on = i < n && gets_row(nat, S, i, min_att);
+    uint32_t all;
+    const uint32_t k = at + block_exclusive_u32(on ? 1u : 0u, wsh32, all);
+    on = on && k < lim;
+    if (i < n) row[i] = on ? static_cast<int32_t>(k) : -1;
+    if (on) idx[k] = i;
+    at += all;
+  }
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) st->mlp_rows = at < lim ? at : lim;
 }
 
 int scan_cb(void* ctx, const int64_t* in, int64_t* out, int64_t n) {
@@ -4185,6 +4219,11 @@ int fq_create(const fq_system* sys, const fq_params* params, fq_engine** out) {
     rc |= upload(&e->d_orb_sym, sys->orb_sym, sys->nbasis, e->stream);
     rc |= upload(&e->d_nbss, sys->nbasis_sym_spin, 2 * sys->nsym_pg, e->stream);
     rc |= upload(&e->d_ssbf, sys->sym_spin_basis_fns, 2 * sys->nsym_pg * sys->max_sym_spin, e->stream);
+    e->cls_sorted = sys->sym_spin_basis_fns && sys->nbasis_sym_spin ? 1 : 0;
+    for (int c = 0; e->cls_sorted && c < 2 * sys->nsym_pg; ++c)
+      for (int k = 1; k < sys->nbasis_sym_spin[c]; ++k)
+        if (sys->sym_spin_basis_fns[c * sys->max_sym_spin + k] <= sys->sym_spin_basis_fns[c * sys->max_sym_spin + k - 1])
+          e->cls_sorted = 0;
     rc |= upload(&e->d_h1, sys->h1, static_cast<int64_t>(sys->norb) * sys->norb, e->stream);
     rc |= upload(&e->d_eri, sys->eri, sys->n_eri, e->stream);
     // Dense Coulomb/exchange pair tables for the diagonal rule: entries copied
@@ -4481,26 +4520,44 @@ static int cycle_body(fq_engine* e, const double* shift, const double* eproj_old
                        e->part_d, e->part_i, e->d_dvec, e->d_dpos, e->blk_att, e->d_stats);
     e->est_blocks = static_cast<int>(nb);
     if (e->par.excit_gen == FQ_EXCIT_LEARNED && n > 0) {
-      hipLaunchKernelGGL(k_mlp_mark, dim3(grid_for(n)), dim3(kBlock), 0, st, n, e->S, e->nat,
-                         static_cast<int64_t>(e->par.proposal_min_attempts), e->mlp_on, e->d_stats);
-      int mrc = scan_exclusive(e, e->mlp_on, e->mlp_row, n);
-      if (mrc != FQ_OK) return mrc;
-      hipLaunchKernelGGL(k_mlp_gather, dim3(grid_for(n)), dim3(kBlock), 0, st, n, e->mlp_on, e->mlp_row,
-                         e->mlp_idx);
-      int64_t ninf = 0;
-      FQ_HIP(hipMemcpyAsync(&ninf, e->mlp_row + n, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-      FQ_HIP(hipStreamSynchronize(st));
-      e->prof.proposal_rows = ninf;
-      if (ninf > e->mlp_tab_rows) {  // grow the weight table (rare: rows follow the inferred determinants)
-        const int64_t rows = std::min<int64_t>(e->cap, std::max<int64_t>(ninf, 2 * e->mlp_tab_rows));
+      const int64_t min_att = e->par.proposal_min_attempts, mt = ceil_div(n, kMainTile);
+      // A bound of the rows: every determinant without a threshold; else at most
+      // one per min_att of the attempts, where these are bounded (see the
+      // spawning below), so that the host need not wait for the count (the
+      // wait and the three kernels of its scan took 50 us of a cycle with 1e6
+      // walkers, the two kernels here take 10).  It waits where the attempts are
+      // unknown or the table would grow past kProposalTable for the bound alone.
+      int64_t rows = n;
+      bool count = false;
+      if (min_att > 0) {
+        if (e->att_bound > 0) rows = std::min(n, e->att_bound / min_att);
+        count = e->att_bound <= 0 ||
+                (rows > e->mlp_tab_rows && rows > kProposalTable / (static_cast<int64_t>(sizeof(float)) * e->mlp.d_out));
+      }
+      hipLaunchKernelGGL(k_mlp_mark, dim3(static_cast<unsigned>(mt)), dim3(kBlock), 0, st, n, e->S, e->nat, min_att,
+                         e->mcnt, e->d_stats);
+      if (mt > kPrefixMax) {
+        const int mrc = scan_exclusive(e, e->mcnt, e->moff, mt);
+        if (mrc != FQ_OK) return mrc;
+      }
+      hipLaunchKernelGGL(k_mlp_rows, dim3(static_cast<unsigned>(mt)), dim3(kBlock), 0, st, n, e->S, e->nat, min_att,
+                         rows, e->mcnt, mt > kPrefixMax ? e->moff : nullptr, e->mlp_row, e->mlp_idx, e->d_stats);
+      if (count) {
+        FQ_HIP(hipMemcpyAsync(&rows, &e->d_stats->mlp_rows, sizeof(int64_t), hipMemcpyDeviceToHost, st));
+        FQ_HIP(hipStreamSynchronize(st));
+      }
+      if (rows > e->mlp_tab_rows) {  // grow the weight table (rare: rows follow the inferred determinants)
+        const int64_t more = std::min<int64_t>(e->cap, std::max<int64_t>(rows, 2 * e->mlp_tab_rows));
+        FQ_HIP(hipStreamSynchronize(st));
         dfree(e->mlp_tab);
         e->mlp_tab_rows = 0;
-        if (dalloc(&e->mlp_tab, rows * e->mlp.d_out) != FQ_OK) return FQ_ERR_NOMEM;
-        e->mlp_tab_rows = rows;
+        if (dalloc(&e->mlp_tab, more * e->mlp.d_out) != FQ_OK) return FQ_ERR_NOMEM;
+        e->mlp_tab_rows = more;
         e->sys.mlp_tab = e->mlp_tab;
         e->sys_dirty = true;
       }
-      mrc = fqm::mlp_infer(e->mlp, e->sys, e->det[c], cap, ninf, e->mlp_tab, st, e->mlp_idx);
+      const int mrc = fqm::mlp_infer(e->mlp, e->sys, e->det[c], cap, rows, e->mlp_tab, st, e->mlp_idx,
+                                     &e->d_stats->mlp_rows, e->prof.proposal_rows);
       if (mrc != FQ_OK) return mrc;
     }
     // Attempt offsets over the n*S (det, space) entries.
@@ -4579,7 +4636,7 @@ static int cycle_body(fq_engine* e, const double* shift, const double* eproj_old
   const int64_t used = rng_pos - e->rng_pos;
   e->rng_pos = rng_pos;
   fill_profile(e, n, ns);
-  if (e->par.excit_gen != FQ_EXCIT_LEARNED || n == 0) e->prof.proposal_rows = 0;
+  e->prof.proposal_rows = e->par.excit_gen == FQ_EXCIT_LEARNED && !replay ? e->h_stats.mlp_rows : 0;
   if (replay) e->prof.spawn_launches = 0;
   fill_out(e, out, used);
   return FQ_OK;
@@ -5587,7 +5644,6 @@ void fq_destroy(fq_engine* e) {
   fqm::mlp_free(e->mlp);
   dfree(e->mlp_tab);
   dfree(e->mlp_flat);
-  dfree(e->mlp_on);
   dfree(e->mlp_row);
   dfree(e->mlp_idx);
   dfree(e->d_binom);

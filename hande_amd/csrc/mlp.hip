@@ -94,10 +94,13 @@ __global__ __launch_bounds__(kBlock) void k_mlp_infer(int nb, int k1, int n3, in
                                                       const uint16_t* __restrict__ w1t, const float* __restrict__ b1,
                                                       const uint16_t* __restrict__ w2t, const float* __restrict__ b2,
                                                       const uint16_t* __restrict__ w3t, const float* __restrict__ b3,
-                                                      float* __restrict__ tab, int64_t ld) {
+                                                      float* __restrict__ tab, int64_t ld,
+                                                      const int64_t* __restrict__ pn) {
   constexpr int R = 16 * RT;
   __shared__ __attribute__((aligned(16))) uint16_t act[R * kActLd];
   const int64_t row0 = static_cast<int64_t>(blockIdx.x) * R;
+  if (pn) n = *pn < n ? *pn : n;  // n is a bound
+  if (row0 >= n) return;
   for (int el = threadIdx.x; el < R * k1; el += blockDim.x) {
     const int r = el / k1, c = el - r * k1;
     const int64_t d = row0 + r;
@@ -934,12 +937,12 @@ int mlp_init(Mlp& m, uint64_t seed, hipStream_t st) {
 }
 
 int mlp_infer(const Mlp& m, const fqd::Sys& s, const uint64_t* det, int64_t cap, int64_t n, float* tab,
-              hipStream_t st, const int64_t* idx) {
+              hipStream_t st, const int64_t* idx, const int64_t* pn, int64_t like) {
   if (n <= 0) return FQ_OK;
-  const int rt = n <= kFewRows ? 1 : 4;
+  const int rt = (pn ? std::min(like, n) : n) <= kFewRows ? 1 : 4;
   hipLaunchKernelGGL(rt == 1 ? k_mlp_infer<1> : k_mlp_infer<4>, dim3(static_cast<unsigned>(ceil_div(n, 16 * rt))),
                      dim3(kBlock), 0, st, m.nb, m.k1, m.n3, m.d_out, det, cap, n, idx, s.sp_eigv, m.w1t, m.p + m.o_b1,
-                     m.w2t, m.p + m.o_b2, m.w3t, m.p + m.o_b3, tab, static_cast<int64_t>(m.d_out));
+                     m.w2t, m.p + m.o_b2, m.w3t, m.p + m.o_b3, tab, static_cast<int64_t>(m.d_out), pn);
   MLP_HIP(hipGetLastError());
   return FQ_OK;
 }

@@ -83,8 +83,9 @@ int mlp_set(Mlp& m, const float* host, hipStream_t st);
 int mlp_refresh(Mlp& m, hipStream_t st);
 // Proposal weights of determinants [0, n) of a structure-of-arrays list (row
 // r of tab for determinant r), or of determinants idx[0..n) when idx is given.
+// pn: the number of rows on the device, n a bound of it and like a guess.
 int mlp_infer(const Mlp& m, const fqd::Sys& s, const uint64_t* det, int64_t cap, int64_t n, float* tab,
-              hipStream_t st, const int64_t* idx = nullptr);
+              hipStream_t st, const int64_t* idx = nullptr, const int64_t* pn = nullptr, int64_t like = 0);
 // Forward/backward over the first ns stored samples (sdet/sexc/sw): fills g,
 // leaves sum(w) and the weighted loss in dsum.  apply: one Adam step (lr).
 int mlp_train_step(Mlp& m, const fqd::Sys& s, int64_t ns, double lr, bool apply, hipStream_t st);

@@ -1,0 +1,95 @@
+"""Sizes at which the learned proposal's kernels change shape: rows of the
+inference (16 or 64 to a block), samples of the training products (chunks of
+four slabs), list lengths around the tiles that number the network's rows."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from hande_amd import _native as N
+from test_gpu_learned import M, P, _engine, _forward, _orb_info, _random_dets, _random_samples, _set_params, _system
+
+pytestmark = pytest.mark.gpu
+
+
+def test_inference_rows_do_not_depend_on_the_list(tmp_path):
+    """Every list gives the first rows of the longest one, bit for bit; those
+    agree with the oracle within the bounds of the inference test."""
+    system = _system(tmp_path, 8, 4, 308)
+    nb, eps, _ = _orb_info(system)
+    lib, eng = _engine(system)
+    try:
+        params = M.init_params(nb, 17)
+        _set_params(lib, eng, params)
+        dets, _ = _random_dets(nb, 4, 8257, np.random.default_rng(5))
+        full = _forward(lib, eng, dets, nb)
+        ref = np.clip(M.forward(params, M.occupations(dets, nb), eps, bf16_inference=True), -M.CLIP, M.CLIP)
+        err = np.abs(np.log(full.astype(np.float64)) - ref)
+        assert err.max() < 3e-2 and err.mean() < 2e-3
+        for n in (1, 15, 16, 17, 63, 64, 65, 8191, 8192, 8193):
+            assert np.array_equal(_forward(lib, eng, dets[:n], nb), full[:n]), n
+    finally:
+        lib.fq_destroy(eng)
+
+
+@pytest.mark.parametrize("ns", [1, 15, 16, 17, 63, 64, 65, 127, 129, 257, 1030])
+def test_gradient_at_sample_counts(tmp_path, ns):
+    system = _system(tmp_path, 8, 4, 808)
+    nb, eps, orb_sym = _orb_info(system)
+    lib, eng = _engine(system)
+    try:
+        params = M.init_params(nb, 23)
+        _set_params(lib, eng, params)
+        dets, _occs, exc, w = _random_samples(nb, 4, orb_sym, ns, np.random.default_rng(ns))
+        w[0] = 1.0
+        flat = np.zeros(ns, dtype=np.int32)
+        loss = C.c_double()
+        grad = np.zeros(len(params), dtype=np.float32)
+        N.check(lib.fq_mlp_loss_grad(eng, np.ascontiguousarray(dets).ctypes.data_as(P(C.c_uint64)),
+                                     exc.ctypes.data_as(P(C.c_int32)), w.ctypes.data_as(P(C.c_double)),
+                                     flat.ctypes.data_as(P(C.c_int32)), ns, C.byref(loss),
+                                     grad.ctypes.data_as(P(C.c_float))), "fq_mlp_loss_grad")
+        ref_loss, ref_grad = M.loss_and_grad(params.astype(np.float64), M.occupations(dets, nb), eps, orb_sym,
+                                             [tuple(int(x) for x in e) for e in exc], w, flat.astype(bool))
+        assert abs(loss.value - ref_loss) < 1e-5 * abs(ref_loss)
+        for name, (o, cnt) in M.sizes(nb)[2].items():
+            g, r = grad[o:o + cnt].astype(np.float64), ref_grad[o:o + cnt]
+            assert np.abs(g - r).max() <= 2e-4 * np.abs(r).max() + 1e-9, name
+    finally:
+        lib.fq_destroy(eng)
+
+
+@pytest.mark.parametrize("min_attempts", [0, 1, 4])
+@pytest.mark.parametrize("n", [1, 255, 1023, 1024, 1025, 2500])
+def test_network_rows_are_the_determinants_with_enough_attempts(tmp_path, n, min_attempts):
+    """Integer populations make |N| attempts.  The first cycle of a loaded list
+    counts the rows, the second has them bounded by the first one's list."""
+    system = _system(tmp_path, 10, 6, 1010)
+    nb, _eps, _sym = _orb_info(system)
+    lib = N.lib()
+    p = N.FqParams()
+    p.nspaces, p.excit_gen, p.rng_mode, p.philox_seed = 1, N.FQ_EXCIT_LEARNED, N.FQ_RNG_PHILOX, 7
+    p.main_capacity = p.spawn_capacity = 1 << 15
+    p.proposal_mix, p.proposal_min_attempts = 0.1, min_attempts
+    eng = C.c_void_p()
+    N.check(lib.fq_create(system.view, C.byref(p), C.byref(eng)), "fq_create")
+    try:
+        rng = np.random.default_rng(n)
+        dets = np.unique(_random_dets(nb, 6, 2 * n + 8, rng)[0][:, 0])
+        dets = np.sort(rng.permutation(dets)[:n])
+        pops = rng.choice([-1, 1], n) * rng.integers(1, 7, n)
+        N.check(lib.fq_load(eng, dets.ctypes.data_as(P(C.c_uint64)), pops.ctypes.data_as(P(C.c_int64)),
+                            np.zeros(n).ctypes.data_as(P(C.c_double)), n), "fq_load")
+        for _ in range(3):
+            o, pr = N.FqCycleOut(), N.FqProfileOut()
+            N.check(lib.fq_cycle(eng, (C.c_double * 2)(0.0, 0.0), (C.c_double * 2)(0.0, 0.0), 0.01, C.byref(o)),
+                    "fq_cycle")
+            N.check(lib.fq_last_profile(eng, C.byref(pr)), "fq_last_profile")
+            assert o.nattempts == np.abs(pops).sum()
+            assert pr.proposal_rows == (np.abs(pops) >= min_attempts).sum()
+            pops = np.zeros(o.nstates, dtype=np.int64)
+            got = C.c_int64()
+            N.check(lib.fq_download(eng, None, pops.ctypes.data_as(P(C.c_int64)), None, o.nstates, C.byref(got)),
+                    "fq_download")
+    finally:
+        lib.fq_destroy(eng)
