@@ -2351,9 +2351,13 @@ __device__ __forceinline__ int64_t tiles_before(const int32_t* __restrict__ cnt,
   return block_sum(x, wsh);
 }
 
-// Runs longer than this are reduced by the whole block (a queue in LDS), so a
+// Runs longer than this are reduced by a wavefront each (a queue in LDS), so a
 // determinant spawned onto thousands of times does not hold one lane while
-// its wavefront idles; shorter ones by one thread each.
+// its wavefront idles; shorter ones by one thread each.  16 measured the same
+// for one space and 40 us against 35 for pairs (7e5 two-word keys).  (One
+// such run after the other by the whole block, with loads waited for one by
+// one: k_runs 24 us against 17 with 9e4 walkers on a 14-site ring, 87 against
+// 76 for 4.3e6 keys.)
 constexpr int kShortRun = 32;
 
 // Inputs and outputs of k_runs.
@@ -2394,7 +2398,7 @@ constexpr int kRunWin = 2048;  // main-list values a tile stages in LDS (two-wor
 // one block per tile of kRunTile keys.  The tile's run heads are listed in
 // order (wavefront ballots); thread h takes run h and sums its entries' shares
 // (entry_share), so every lane has a run whatever the run lengths.  Runs longer
-// than kShortRun are queued and reduced by the whole block afterwards.  The
+// than kShortRun are queued and reduced by the wavefronts afterwards.  The
 // tile's last run adds the head-free prefixes of the following tiles
 // (k_run_count) up to the next head.  The run's first entry is its first in
 // sorted order: the reference's quicksort order in replay mode, the earliest
@@ -2407,15 +2411,15 @@ constexpr int kRunWin = 2048;  // main-list values a tile stages in LDS (two-wor
 // determinants that are inserted are ever unranked, by the insertion.
 // (Before, every run was unranked and written as a record that three further
 // kernels read: 253 us for 4.3e6 keys on 2.8e6 determinants (k_runs 165,
-// search bounds 26, merge 39, rounding of new 18, their list 5), 88 us now and
+// search bounds 26, merge 39, rounding of new 18, their list 5), 76 us now and
 // 20 for the ranks k_scatter_main moves and the unranking of the inserted.)
 template <int KW, int S>
 __global__ __launch_bounds__(kBlock) void k_runs(RunArgs g) {
   using V = SortValue<KW>;
-  constexpr int R = kRunTile / kBlock, NV = 3 * S, NW = kBlock / 64, WIN = kRunWin / KW;
+  constexpr int R = kRunTile / kBlock, NV = 3 * S, NW = kBlock / 64, WIN = kRunWin / KW, kAhead = 4;
   __shared__ int32_t wcount[R][NW];
   __shared__ int32_t hpos[kRunTile + 1];  // tile-relative index of each head, in order; then the tile length
-  __shared__ int16_t longq[kRunTile];     // runs (by h) left to the whole block
+  __shared__ int16_t longq[kRunTile];     // runs (by h) left to a whole wavefront
   __shared__ uint8_t rflag[kRunTile];     // a run's flags, bit 7: some population is not zero
   __shared__ int64_t rtot[S][kRunTile];   // a run's populations
   __shared__ V wval[WIN];                 // the main-list values between the tile's bounds when they fit
@@ -2480,13 +2484,24 @@ __global__ __launch_bounds__(kBlock) void k_runs(RunArgs g) {
   __syncthreads();
   // the shares of run h's entries [a, b) of the tile, from index `from` (stride `step`)
   auto shares = [&](int a, int b, int from, int step, int64_t* acc) {
-    for (int j = from; j < b; j += step) {
-      int64_t pop[S], cv[NV];
+    for (int j = from; j < b; j += kAhead * step) {
+      uint64_t key[kAhead];
+      int64_t pop[kAhead][S];
 #pragma unroll
-      for (int q = 0; q < S; ++q) pop[q] = g.pay[q * stride + t0 + j];
-      entry_share<S>(static_cast<int64_t>(g.keys[t0 + j] & fmask), pop, j == a, cv);
+      for (int u = 0; u < kAhead; ++u) {  // loads of kAhead entries in flight
+        const int64_t i = t0 + (j + u * step < b ? j + u * step : j);
+        key[u] = g.keys[i];
 #pragma unroll
-      for (int k = 0; k < NV; ++k) acc[k] += cv[k];
+        for (int q = 0; q < S; ++q) pop[u][q] = g.pay[q * stride + i];
+      }
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        if (j + u * step >= b) break;
+        int64_t cv[NV];
+        entry_share<S>(static_cast<int64_t>(key[u] & fmask), pop[u], j + u * step == a, cv);
+#pragma unroll
+        for (int k = 0; k < NV; ++k) acc[k] += cv[k];
+      }
     }
   };
   // run h's totals complete: the continuation of the tile's last run and the initiator rules
@@ -2525,16 +2540,16 @@ __global__ __launch_bounds__(kBlock) void k_runs(RunArgs g) {
   }
   __syncthreads();
   const int nq = nlong;
-  for (int q = 0; q < nq; ++q) {  // block-uniform
+  for (int q = wave; q < nq; q += NW) {
     const int h = longq[q];
     const int a = hpos[h], b = hpos[h + 1];
     int64_t acc[NV];
 #pragma unroll
     for (int k = 0; k < NV; ++k) acc[k] = 0;
-    shares(a, b, a + tid, kBlock, acc);
+    shares(a, b, a + lane, 64, acc);
 #pragma unroll
-    for (int k = 0; k < NV; ++k) acc[k] = block_sum(acc[k], wsh);
-    if (tid == 0) finish(h, acc);
+    for (int k = 0; k < NV; ++k) acc[k] = wave_sum(acc[k]);
+    if (lane == 0) finish(h, acc);
   }
   __syncthreads();
   // merge with the main list and list the new determinants, kBlock runs at a time in order

@@ -327,3 +327,23 @@ def test_annihilate_production_two_word_rank_keys():
     finally:
         lib.fq_destroy(eng)
         orc.orc_destroy(h)
+
+
+@pytest.mark.parametrize("mode", ["philox", "replay"])
+def test_annihilate_runs_at_the_lane_and_wavefront_edges(hub, mode):
+    """Runs of 1 to 6 entries (a lane's loads are taken four at a time), around
+    32 (the longest a lane adds up) and around one, four and eight wavefronts'
+    shares, in random order and several to a tile."""
+    lib, orc = N.lib(), oracle()
+    rng = np.random.default_rng(91)
+    st, p = _mk(hub, True, True, mode)
+    p.spawn_capacity = 1 << 16
+    rf = 1 << p.pop_bit_shift
+    main, pops, sk, _, _ = _random_state(rng, hub, 300, 3000, rf, True, big=True)
+    lengths = [1, 2, 3, 4, 5, 6, 31, 32, 33, 34, 36, 63, 64, 65, 255, 256, 257, 511, 513] * 3
+    sk = np.repeat(rng.choice(np.unique(sk), len(lengths), replace=False), rng.permutation(lengths))
+    ns = len(sk)
+    sk = rng.permutation(sk)
+    sp = (rng.integers(1, 4, ns) * rng.choice([-1, 1], ns) * (3 * rf // 2)).astype(np.int64)
+    sf = rng.integers(0, 2, ns).astype(np.int64)
+    assert _run(lib, orc, hub, st, p, main, pops, sk, sp, sf, stable=(mode == "philox")) > 0
