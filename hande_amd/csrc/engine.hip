@@ -13,10 +13,11 @@
 //                         replay: k_replay_walk, one thread walking the list
 //                         in the reference's order and consuming the uploaded
 //                         dSFMT stream exactly as get_rand_close_open does.
-//   sort                  production: LSD radix sort (8-bit digits, stable
-//                         per-round wavefront ranking) of the spawned list's
-//                         combinatorial ranks, which order determinants as
-//                         their bit strings do in fewer bits.
+//   sort                  production: LSD radix sort (8- or 9-bit digits, stable;
+//                         short lists by one block in LDS) of the spawned list's
+//                         sort values: combinatorial ranks, which order
+//                         determinants as their bit strings do in fewer bits, or
+//                         the bit strings where that saves no pass.
 //                         replay: the reference's quicksort (src/sort.f90:213-396)
 //                         on one thread, so equal keys keep its order.
 //   self-annihilation,    k_run_count / k_runs: one thread per run of equal keys,
