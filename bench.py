@@ -201,20 +201,19 @@ def compulsory_bytes(prof, W=1, S=1):
 def phase_bytes(prof, W=1, S=1, kw=1):
     """Algorithmic HBM bytes of each phase of one cycle as the kernels move
     them; kw: words of the sort key."""
-    nd, ns, nr, nout = prof.nstates_in, prof.nspawned, prof.nruns, prof.nstates_out
+    nd, ns, nout = prof.nstates_in, prof.nspawned, prof.nstates_out
     bm, bs = entry_bytes(W, S)
     return {
         # read det/pop/K_ii, write post-death pops, attempt counts, flags
-        "det_pass": nd * (bm + 8 * S + 8 * S + 8),
+        "det_pass": nd * (bm + 8 * S + 4 * S + 1),
         # parents (det, pop, flag) and attempt offsets once, spawned entries and their sort keys written
-        "spawn": nd * (8 * W + 8 * S + 8 + 8 * S) + ns * (bs + 8 * kw),
-        # one read of the keys for every pass's digit counts; each pass reads and writes them once
-        "sort": ns * 8 * kw + prof.radix_passes * ns * 2 * 8 * kw,
-        # sorted keys read (and each key's neighbour), each entry's populations
-        # and flag gathered by slot, each run's determinant gathered, runs written
-        "reduce": ns * (2 * 8 * kw + 8 * S + 8) + nr * (8 * W) + nr * (8 * W + 8 * S + 8 + 8),
-        # main list read twice (merge search ~ touched lines ignored) and written once, runs read
-        "merge": nd * (2 * bm + 3 * 8) + nout * bm + nr * (8 * W + 8 * S + 8 + 8 * 3),
+        "spawn": nd * (8 * W + 8 * S + 1 + 8 * S) + ns * (bs + 8 * kw),
+        # each pass reads the keys for its counts, then reads and writes keys and populations
+        "sort": prof.radix_passes * ns * (8 * kw + 2 * (8 * kw + 8 * S)),
+        # sorted keys read for the run heads, then with the populations; the main list's sort values once
+        "reduce": ns * (2 * 8 * kw + 8 * S) + nd * 8 * kw,
+        # post-death populations rounded; main list and sort values read and written once
+        "merge": nd * (8 * S + bm + 8 * kw) + nout * (bm + 8 * kw),
     }
 
 
