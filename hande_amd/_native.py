@@ -163,6 +163,8 @@ def _declare(lib):
         "fq_mlp_train": (C.c_int, [vp, i64, i32, f64, u64, P(f64)]),
         "fq_probe_excitations": (C.c_int, [vp, P(u64), i64, u64, P(i32), P(f64), P(f64)]),
         "fq_destroy": (None, [vp]),
+        # for the tests (engine.hip, after fq_destroy)
+        "fqt_tile_windows": (C.c_int, [vp, P(i64), i64]),
     }
     for name, (res, args) in sig.items():
         if hasattr(lib, name):

@@ -896,7 +896,8 @@ __global__ __launch_bounds__(kBlock) void k_att_scan(const int32_t* __restrict__
   for (int64_t t = (beg >> tile_bits) + threadIdx.x; (t << tile_bits) < fin && t < ntile; t += kBlock) {
     const int64_t t0 = t << tile_bits, t1 = t0 + (int64_t{1} << tile_bits), last = (t1 < total ? t1 : total) - 1;
     if (t0 >= beg) tile_win[2 * t] = entry_of(t0);
-    if (last < fin) tile_win[2 * t + 1] = entry_of(last);
+    // (a block without attempts, past the total, must not take the last tile's end)
+    if (last >= beg && last < fin) tile_win[2 * t + 1] = entry_of(last);
   }
   if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) out[nent] = total;
 }
@@ -5696,6 +5697,17 @@ void fq_destroy(fq_engine* e) {
   dfree(e->d_in);
   if (e->stream) (void)hipStreamDestroy(e->stream);
   delete e;
+}
+
+// ---- for the tests; not part of the interface in include/fqmc.h ----------------
+// The parents (det-major (det, space) entries) of the first and last attempt of
+// the last cycle's first ntiles spawning tiles.
+int fqt_tile_windows(fq_engine* e, int64_t* out, int64_t ntiles) {
+  if (!e || !out || ntiles < 1 || ntiles > e->bcap / kSmallTile + 2) return FQ_ERR_ARG;
+  FQ_HIP(hipSetDevice(e->device));
+  FQ_HIP(hipMemcpyAsync(out, e->tile_win, sizeof(int64_t) * 2 * ntiles, hipMemcpyDeviceToHost, e->stream));
+  FQ_HIP(hipStreamSynchronize(e->stream));
+  return FQ_OK;
 }
 
 }  // extern "C"
