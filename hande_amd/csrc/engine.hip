@@ -566,7 +566,8 @@ int64_t* fixed_scratch_address(int device) {
 
 // Scratch buffer `slot` of at least `need` elements (grown on demand; inside
 // fq_cycle_noalloc, the slot's region of the fixed array, or null when the
-// request exceeds it).
+// request exceeds it).  Captured graphs hold the buffer's address, so from
+// fq_batch_graph on, which sizes it for the engine's longest scan, it stays.
 int64_t* scan_scratch(fq_engine* e, int slot, int64_t need) {
   if (e->noalloc) {
     if (slot >= kScratchSlots || need > kScratchSlotElems[slot]) {
@@ -580,6 +581,7 @@ int64_t* scan_scratch(fq_engine* e, int slot, int64_t need) {
     e->scan_tmp_cap.push_back(0);
   }
   if (e->scan_tmp_cap[slot] < need) {
+    if (e->h_in) return nullptr;
     dfree(e->scan_tmp[slot]);
     if (dalloc(&e->scan_tmp[slot], need) != FQ_OK) {
       e->scan_tmp_cap[slot] = 0;
@@ -5136,13 +5138,6 @@ static int graph_for(fq_engine* e, int64_t nb, int64_t tb, int sched, hipGraphEx
       *out = g.exec;
       return FQ_OK;
     }
-  // no allocation may happen inside the capture: size the scan scratch for
-  // the longest scan of the cycle first
-  const int64_t longest = std::max<int64_t>(e->S * nb, tb);
-  if (longest > kSmallScanMax) {
-    const int64_t ntile = ceil_div(longest, kScanTile);
-    if (!scan_scratch(e, 0, ntile) || !scan_scratch(e, 1, ntile + 1)) return FQ_ERR_NOMEM;
-  }
   e->digit8 = kSchedDigit8[sched];
   e->spawn_blocks = kSchedSpawnBlocks[sched];
   const int64_t n_keep = e->n;
@@ -5251,6 +5246,11 @@ int fq_batch_graph(fq_engine* e, int32_t enable) {
   if (!e || !e->batched) return FQ_ERR_ARG;
   FQ_HIP(hipSetDevice(e->device));
   if (enable && !e->h_in) {
+    // scan scratch for the longest list of counts a cycle of this engine can
+    // scan: the determinant pass's blocks, the run and main tiles, the instances
+    const int64_t longest = std::max({ceil_div(e->cap, kBlock), ceil_div(e->scap, kRunTile), int64_t{e->ninst}});
+    const int64_t ntile = ceil_div(longest, kScanTile);
+    if (!scan_scratch(e, 0, ntile) || !scan_scratch(e, 1, ntile + 1)) return FQ_ERR_NOMEM;
     const size_t nin = graph_in_bytes(e);
     if (hipHostMalloc(reinterpret_cast<void**>(&e->h_in), nin) != hipSuccess ||
         hipHostMalloc(reinterpret_cast<void**>(&e->h_god), sizeof(double) * 2 * e->S * e->ninst) != hipSuccess ||
@@ -5707,6 +5707,15 @@ int fqt_tile_windows(fq_engine* e, int64_t* out, int64_t ntiles) {
   FQ_HIP(hipSetDevice(e->device));
   FQ_HIP(hipMemcpyAsync(out, e->tile_win, sizeof(int64_t) * 2 * ntiles, hipMemcpyDeviceToHost, e->stream));
   FQ_HIP(hipStreamSynchronize(e->stream));
+  return FQ_OK;
+}
+
+// Address and elements of a scan scratch buffer (0 and 0: none).
+int fqt_scan_scratch(fq_engine* e, int slot, int64_t* address, int64_t* elements) {
+  if (!e || slot < 0 || !address || !elements) return FQ_ERR_ARG;
+  const bool have = slot < static_cast<int>(e->scan_tmp.size());
+  *address = have ? reinterpret_cast<intptr_t>(e->scan_tmp[slot]) : 0;
+  *elements = have ? e->scan_tmp_cap[slot] : 0;
   return FQ_OK;
 }
 

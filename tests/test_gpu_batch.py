@@ -171,3 +171,51 @@ def test_graph_cycles_match_ordinary_cycles():
     finally:
         for eng in engs:
             lib.fq_destroy(eng)
+
+
+def test_graph_scratch_keeps_its_address():
+    """Captured graphs hold the scan scratch's address: it is there from
+    fq_batch_graph on, large enough for the engine's longest list of counts, and
+    stays while the launch bounds grow and shrink and new graphs are captured."""
+    lib = N.lib()
+    systems = [api.hubbard_k(**d) for d in DECKS]
+    K = len(systems)
+    arr = (N.FqSystem * K)(*[s.view for s in systems])
+    p = _params(98, cap=1 << 20)
+    p.main_capacity = 1 << 23
+    eng = C.c_void_p()
+    N.check(lib.fq_create_batch(arr, K, C.byref(p), C.byref(eng)), "fq_create_batch")
+
+    def scratch():
+        out = []
+        for slot in (0, 1):
+            address, elements = C.c_int64(), C.c_int64()
+            N.check(lib.fqt_scan_scratch(eng, slot, C.byref(address), C.byref(elements)), "fqt_scan_scratch")
+            out.append((address.value, elements.value))
+        return out
+
+    try:
+        N.check(lib.fq_batch_graph(eng, 1), "fq_batch_graph")
+        first = scratch()
+        tiles = (1 << 23) // 256 // 4096  # 256 determinants a count, 4096 counts a scan tile
+        assert first[0][0] and first[0][1] >= tiles and first[1][0] and first[1][1] >= tiles + 1
+        inst = np.arange(K, dtype=np.int32)
+        f0 = np.array([int(s.f0()[0]) for s in systems], dtype=np.uint64)
+        taus, eolds = np.full(K, 0.02), np.zeros(K)
+        outs = (N.FqCycleOut * K)()
+        graphs = []
+        for scale in (1, 40, 1):  # a list, a far longer one, the first again
+            pops = np.array([1200, 800, 2000, 500, 1000], dtype=np.int64) * scale
+            N.check(lib.fq_load_batch(eng, inst.ctypes.data_as(P(C.c_int32)), f0.ctypes.data_as(P(C.c_uint64)),
+                                      pops.ctypes.data_as(P(C.c_int64)), np.zeros(K).ctypes.data_as(P(C.c_double)),
+                                      K), "load")
+            for _ in range(8):
+                N.check(lib.fq_cycle_batch(eng, eolds.ctypes.data_as(P(C.c_double)), eolds.ctypes.data_as(P(C.c_double)),
+                                           taus.ctypes.data_as(P(C.c_double)), outs), "fq_cycle_batch")
+                assert scratch() == first
+            info = N.FqScheduleOut()
+            N.check(lib.fq_batch_schedule(eng, C.byref(info)), "fq_batch_schedule")
+            graphs.append(info.graphs)
+        assert graphs[0] < graphs[1]
+    finally:
+        lib.fq_destroy(eng)
