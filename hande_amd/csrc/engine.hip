@@ -409,7 +409,8 @@ struct fq_engine {
   float* mlp_flat = nullptr;  // 2*nbasis ones: weights of determinants without a row
   int64_t att_bound = -1;            // bound of the next cycle's attempts (-1: unknown)
   bool keys_ready = false;           // the spawning pass made this cycle's sort keys
-  int64_t last_ns = -1;              // spawned entries of the last cycle (-1: none run on this list)
+  int64_t last_ns = -1;              // spawned entries last annihilated (-1: none on this list)
+  int64_t resorts = 0;               // lists that outgrew the one-block sort they were given to
   int est_blocks = 0;                // k_det_pass blocks whose partials k_finish adds (0: none)
   int new_src = 0;                   // the sort's idle buffers after this cycle's passes
   int64_t run_tiles = 0;             // run tiles of this cycle's spawned list (a bound of it while captured)
@@ -3639,10 +3640,11 @@ int annihilate(fq_engine* e, int64_t ns, const int64_t* pns, bool replay, uint32
   if (e->h_stats.resort) {  // longer than k_sort_small takes: its keys and the populations are as they were
     hipLaunchKernelGGL(k_zero, dim3(1), dim3(kBlock), 0, st, &e->d_stats->resort, int64_t{1});
     e->keys_ready = true;
+    ++e->resorts;
     return annihilate(e, std::min<int64_t>(e->h_stats.nspawn, scap), nullptr, replay, cyc, rng_pos, true);
   }
   e->est_blocks = 0;
-  e->last_ns = ns > 0 ? std::min<int64_t>(e->h_stats.nspawn, scap) : 0;
+  e->last_ns = pns ? std::min<int64_t>(e->h_stats.nspawn, scap) : ns;  // a caller's list is not counted on the device
   e->cur = o;
   e->n = e->h_stats.new_n;
   e->att_bound = -1;
@@ -5709,6 +5711,9 @@ int fqt_tile_windows(fq_engine* e, int64_t* out, int64_t ntiles) {
   FQ_HIP(hipStreamSynchronize(e->stream));
   return FQ_OK;
 }
+
+// Spawned lists so far that were sorted again because the one-block sort could not take them.
+int64_t fqt_resorts(fq_engine* e) { return e ? e->resorts : -1; }
 
 // Address and elements of a scan scratch buffer (0 and 0: none).
 int fqt_scan_scratch(fq_engine* e, int slot, int64_t* address, int64_t* elements) {

@@ -152,6 +152,7 @@ def test_cycle_after_a_short_list_sorts_a_long_one():
                                   C.byref(out)), "fq_annihilate")
     st_, po, da = lists(two)
     N.check(lib.fq_load(two, ptr(st_, C.c_uint64), ptr(po, C.c_int64), ptr(da, C.c_double), len(da)), "load")
+    assert lib.fqt_resorts(one) == lib.fqt_resorts(two) == 0
     for _ in range(3):
         o1, o2 = N.FqCycleOut(), N.FqCycleOut()
         N.check(lib.fq_cycle(one, sh, sh, 0.01, C.byref(o1)), "fq_cycle")
@@ -162,8 +163,34 @@ def test_cycle_after_a_short_list_sorts_a_long_one():
         assert o1.proj_energy[0] == o2.proj_energy[0] and o1.nparticles[0] == o2.nparticles[0]
         for x, y in zip(lists(one), lists(two)):
             assert np.array_equal(x, y)
+        assert lib.fqt_resorts(one) == 1 and lib.fqt_resorts(two) == 0
     lib.fq_destroy(one)
     lib.fq_destroy(two)
+
+
+def test_cycle_after_a_long_annihilated_list_sorts_once():
+    """A caller's list of 20000 entries is the length the next cycle goes by: its
+    list, past the one-block sort, is sorted by the passes and once."""
+    lib = N.lib()
+    ring = api.hubbard_k(electrons=14, lattice=[[14]], ms=0, sym=1, U=2)
+    st, p = _mk(ring, True, True, "philox")
+    p.main_capacity = p.spawn_capacity = 1 << 18
+    rf = 1 << p.pop_bit_shift
+    main, pops, sk, sp, sf = _random_state(np.random.default_rng(3), ring, 3000, 20000, rf, True, big=True)
+    ptr = lambda a, t: a.ctypes.data_as(C.POINTER(t))
+    eng = C.c_void_p()
+    N.check(lib.fq_create(ring.view, C.byref(p), C.byref(eng)), "fq_create")
+    try:
+        N.check(lib.fq_load(eng, ptr(main, C.c_uint64), ptr(pops, C.c_int64), ptr(np.zeros(len(main)), C.c_double),
+                            len(main)), "load")
+        out, sh = N.FqCycleOut(), (C.c_double * 2)()
+        N.check(lib.fq_annihilate(eng, ptr(sk, C.c_uint64), ptr(sp, C.c_int64), ptr(sf, C.c_int64), len(sk),
+                                  C.byref(out)), "fq_annihilate")
+        N.check(lib.fq_cycle(eng, sh, sh, 0.05, C.byref(out)), "fq_cycle")
+        assert out.nspawn_events > 8192
+        assert lib.fqt_resorts(eng) == 0
+    finally:
+        lib.fq_destroy(eng)
 
 
 @pytest.mark.parametrize("initiator", [False, True])
