@@ -532,6 +532,7 @@ int dalloc(T** p, int64_t count) {
   if (count <= 0) count = 1;
   if (hipMalloc(reinterpret_cast<void**>(p), sizeof(T) * static_cast<size_t>(count)) != hipSuccess) {
     *p = nullptr;
+    (void)hipGetLastError();  // the caller may do without it
     return FQ_ERR_NOMEM;
   }
   return FQ_OK;
@@ -3924,7 +3925,7 @@ int set_insert_lds() {
 // the counts of the tiles before its own (off, when given, holds them); the
 // number of rows goes to the stats, where the inference reads it.  No row is
 // numbered lim or above (lim: a bound of their number).
-constexpr int64_t kProposalTable = int64_t{1} << 30;  // bytes
+constexpr int64_t kProposalTable = int64_t{1} << 28;  // bytes the weight table may take for a bound of its rows
 __device__ __forceinline__ bool gets_row(const int32_t* __restrict__ nat, int S, int64_t i, int64_t min_att) {
   int64_t a = 0;
   for (int sp = 0; sp < S; ++sp) a += nat[i * S + sp];
@@ -3962,6 +3963,25 @@ __global__ __launch_bounds__(kBlock) void k_mlp_rows(int64_t n, int S, const int
     at += all;
   }
   if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) st->mlp_rows = at < lim ? at : lim;
+}
+
+// A weight table of `rows` rows (the list's capacity at most).  keep: the old one
+// stays where there is no memory for the new one beside it.
+int grow_proposal_table(fq_engine* e, int64_t rows, bool keep) {
+  rows = std::min(e->cap, rows);
+  FQ_HIP(hipStreamSynchronize(e->stream));
+  if (!keep) {
+    dfree(e->mlp_tab);
+    e->mlp_tab_rows = 0;
+  }
+  float* tab = nullptr;
+  if (dalloc(&tab, rows * e->mlp.d_out) != FQ_OK) return FQ_ERR_NOMEM;
+  dfree(e->mlp_tab);
+  e->mlp_tab = tab;
+  e->mlp_tab_rows = rows;
+  e->sys.mlp_tab = tab;
+  e->sys_dirty = true;
+  return FQ_OK;
 }
 
 int scan_cb(void* ctx, const int64_t* in, int64_t* out, int64_t n) {
@@ -4547,13 +4567,14 @@ static int cycle_body(fq_engine* e, const double* shift, const double* eproj_old
       // spawning below), so that the host need not wait for the count (the
       // wait and the three kernels of its scan took 50 us of a cycle with 1e6
       // walkers, the two kernels here take 10).  It waits where the attempts are
-      // unknown or the table would grow past kProposalTable for the bound alone.
+      // unknown, or the table would have to grow past kProposalTable for the
+      // bound alone or finds no memory to: then it follows the rows present.
+      const int64_t bound_rows = kProposalTable / (static_cast<int64_t>(sizeof(float)) * e->mlp.d_out);
       int64_t rows = n;
       bool count = false;
       if (min_att > 0) {
         if (e->att_bound > 0) rows = std::min(n, e->att_bound / min_att);
-        count = e->att_bound <= 0 ||
-                (rows > e->mlp_tab_rows && rows > kProposalTable / (static_cast<int64_t>(sizeof(float)) * e->mlp.d_out));
+        count = e->att_bound <= 0 || (rows > e->mlp_tab_rows && rows > bound_rows);
       }
       hipLaunchKernelGGL(k_mlp_mark, dim3(static_cast<unsigned>(mt)), dim3(kBlock), 0, st, n, e->S, e->nat, min_att,
                          e->mcnt, e->d_stats);
@@ -4563,19 +4584,15 @@ static int cycle_body(fq_engine* e, const double* shift, const double* eproj_old
       }
       hipLaunchKernelGGL(k_mlp_rows, dim3(static_cast<unsigned>(mt)), dim3(kBlock), 0, st, n, e->S, e->nat, min_att,
                          rows, e->mcnt, mt > kPrefixMax ? e->moff : nullptr, e->mlp_row, e->mlp_idx, e->d_stats);
+      if (min_att > 0 && !count && rows > e->mlp_tab_rows)
+        count = grow_proposal_table(e, std::max(rows, std::min(2 * e->mlp_tab_rows, bound_rows)), true) != FQ_OK;
       if (count) {
         FQ_HIP(hipMemcpyAsync(&rows, &e->d_stats->mlp_rows, sizeof(int64_t), hipMemcpyDeviceToHost, st));
         FQ_HIP(hipStreamSynchronize(st));
       }
-      if (rows > e->mlp_tab_rows) {  // grow the weight table (rare: rows follow the inferred determinants)
-        const int64_t more = std::min<int64_t>(e->cap, std::max<int64_t>(rows, 2 * e->mlp_tab_rows));
-        FQ_HIP(hipStreamSynchronize(st));
-        dfree(e->mlp_tab);
-        e->mlp_tab_rows = 0;
-        if (dalloc(&e->mlp_tab, more * e->mlp.d_out) != FQ_OK) return FQ_ERR_NOMEM;
-        e->mlp_tab_rows = more;
-        e->sys.mlp_tab = e->mlp_tab;
-        e->sys_dirty = true;
+      if (rows > e->mlp_tab_rows) {  // rare: rows follow the inferred determinants
+        const int grc = grow_proposal_table(e, std::max(rows, 2 * e->mlp_tab_rows), false);
+        if (grc != FQ_OK) return grc;
       }
       const int mrc = fqm::mlp_infer(e->mlp, e->sys, e->det[c], cap, rows, e->mlp_tab, st, e->mlp_idx,
                                      &e->d_stats->mlp_rows, e->prof.proposal_rows);

@@ -2,11 +2,13 @@
 inference (16 or 64 to a block), samples of the training products (chunks of
 four slabs), list lengths around the tiles that number the network's rows."""
 import ctypes as C
+import itertools
 
 import numpy as np
 import pytest
 
 from hande_amd import _native as N
+from helpers import download
 from test_gpu_learned import M, P, _engine, _forward, _orb_info, _random_dets, _random_samples, _set_params, _system
 
 pytestmark = pytest.mark.gpu
@@ -93,3 +95,62 @@ def test_network_rows_are_the_determinants_with_enough_attempts(tmp_path, n, min
                     "fq_download")
     finally:
         lib.fq_destroy(eng)
+
+
+def _many_dets(norb, nel, n):
+    """n determinants of nel/2 alpha and nel/2 beta electrons in list order."""
+    half = np.array([sum(1 << (2 * o) for o in c) for c in itertools.combinations(range(norb), nel // 2)], dtype=np.uint64)
+    beta = half[:-(-n // len(half))] << np.uint64(1)
+    return np.sort((half[:, None] | beta[None, :]).reshape(-1))[:n]
+
+
+def test_rows_follow_the_list_where_their_bound_has_no_memory(tmp_path):
+    """1e6 determinants, nearly all with one walker, at a threshold of two: the
+    attempts bound the rows by 5e5 (160 MB of weights), a few thousand are there.
+    With 100 MB of the card left the cycle runs as it does with all of it."""
+    norb, nel, n = 20, 8, 1000000
+    system = _system(tmp_path, norb, nel, 2008)
+    lib = N.lib()
+    p = N.FqParams()
+    p.nspaces, p.excit_gen, p.rng_mode, p.philox_seed = 1, N.FQ_EXCIT_LEARNED, N.FQ_RNG_PHILOX, 9
+    p.main_capacity = p.spawn_capacity = 1 << 22
+    p.proposal_mix, p.proposal_min_attempts = 0.1, 2
+    dets = _many_dets(norb, nel, n)
+    pops = np.ones(n, dtype=np.int64)
+    pops[::500] = 5
+    engs, results, hog = [], [], []
+    sh = (C.c_double * 2)(0.0, 0.0)
+    hip = C.CDLL("libamdhip64.so.7")  # the engine's own runtime, loaded with it
+
+    def free_memory():
+        free, total = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return free.value
+
+    try:
+        for _ in range(2):
+            eng = C.c_void_p()
+            N.check(lib.fq_create(system.view, C.byref(p), C.byref(eng)), "fq_create")
+            engs.append(eng)
+            N.check(lib.fq_load(eng, dets.ctypes.data_as(P(C.c_uint64)), pops.ctypes.data_as(P(C.c_int64)),
+                                np.zeros(n).ctypes.data_as(P(C.c_double)), n), "fq_load")
+            N.check(lib.fq_cycle(eng, sh, sh, 1e-3, C.byref(N.FqCycleOut())), "fq_cycle")
+        for full, eng in ((True, engs[0]), (False, engs[1])):
+            while full and free_memory() > 100 << 20:
+                take = free_memory() - (1 << 30) if free_memory() > 2 << 30 else 64 << 20
+                hog.append(C.c_void_p())
+                assert hip.hipMalloc(C.byref(hog[-1]), C.c_size_t(take)) == 0
+            out, prof = N.FqCycleOut(), N.FqProfileOut()
+            N.check(lib.fq_cycle(eng, sh, sh, 1e-3, C.byref(out)), "fq_cycle")
+            N.check(lib.fq_last_profile(eng, C.byref(prof)), "fq_last_profile")
+            while hog:
+                hip.hipFree(hog.pop())
+            assert out.nattempts > 8e5 and 1000 < prof.proposal_rows < 65536
+            results.append((out.nstates, out.nspawn_events, out.nattempts, out.ndeath, out.nparticles[0],
+                            prof.proposal_rows, *[x.tobytes() for x in download(lib, eng, 1, 1)]))
+        assert results[0] == results[1]
+    finally:
+        for x in hog:
+            hip.hipFree(x)
+        for eng in engs:
+            lib.fq_destroy(eng)
