@@ -107,7 +107,7 @@ def _many_dets(norb, nel, n):
 def test_rows_follow_the_list_where_their_bound_has_no_memory(tmp_path):
     """1e6 determinants, nearly all with one walker, at a threshold of two: the
     attempts bound the rows by 5e5 (160 MB of weights), a few thousand are there.
-    With 100 MB of the card left the cycle runs as it does with all of it."""
+    Where the card has no 128 MB left the cycle runs as it does with all of it."""
     norb, nel, n = 20, 8, 1000000
     system = _system(tmp_path, norb, nel, 2008)
     lib = N.lib()
@@ -121,12 +121,6 @@ def test_rows_follow_the_list_where_their_bound_has_no_memory(tmp_path):
     engs, results, hog = [], [], []
     sh = (C.c_double * 2)(0.0, 0.0)
     hip = C.CDLL("libamdhip64.so.7")  # the engine's own runtime, loaded with it
-
-    def free_memory():
-        free, total = C.c_size_t(), C.c_size_t()
-        assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
-        return free.value
-
     try:
         for _ in range(2):
             eng = C.c_void_p()
@@ -136,10 +130,10 @@ def test_rows_follow_the_list_where_their_bound_has_no_memory(tmp_path):
                                 np.zeros(n).ctypes.data_as(P(C.c_double)), n), "fq_load")
             N.check(lib.fq_cycle(eng, sh, sh, 1e-3, C.byref(N.FqCycleOut())), "fq_cycle")
         for full, eng in ((True, engs[0]), (False, engs[1])):
-            while full and free_memory() > 100 << 20:
-                take = free_memory() - (1 << 30) if free_memory() > 2 << 30 else 64 << 20
-                hog.append(C.c_void_p())
-                assert hip.hipMalloc(C.byref(hog[-1]), C.c_size_t(take)) == 0
+            for size in (1 << 33, 128 << 20) if full else ():  # until the card has no 128 MB to give
+                while hip.hipMalloc(C.byref(block := C.c_void_p()), C.c_size_t(size)) == 0:
+                    hog.append(block)
+                hip.hipGetLastError()
             out, prof = N.FqCycleOut(), N.FqProfileOut()
             N.check(lib.fq_cycle(eng, sh, sh, 1e-3, C.byref(out)), "fq_cycle")
             N.check(lib.fq_last_profile(eng, C.byref(prof)), "fq_last_profile")
