@@ -418,17 +418,17 @@ struct fq_engine {
   int cls_sorted = 0;          // the spin/irrep classes list their orbitals in ascending order
   int32_t* mlp_row = nullptr;  // [cap] this cycle's row of the weight table (-1: none)
   int64_t* mlp_idx = nullptr;  // [cap] determinants the network runs on
-  // main list (double-buffered)
+  // main list: determinants, K_ii and sort values in buffer cur, the insertion
+  // writing the other; populations in pop, which the cycle has done with when
+  // the insertion writes them from pop_new
   int64_t cap = 0, n = 0;
   int cur = 0;
   uint64_t* det[2] = {nullptr, nullptr};
-  int64_t* pop[2] = {nullptr, nullptr};
+  int64_t* pop = nullptr;       // S*cap
   double* kii[2] = {nullptr, nullptr};
   int64_t* pop_new = nullptr;   // S*cap, populations after death
-  int32_t* nat = nullptr;       // S*cap attempts per (det, space)
-  int64_t* att_off = nullptr;   // S*cap+1
-  uint8_t* flags = nullptr;     // cap parent initiator flags
-  uint64_t* mrank[2] = {nullptr, nullptr};  // sort_kw*cap: the entries' sort values (ranks), as the list's buffers
+  int64_t* att_off = nullptr;   // S*cap+1 attempt offsets (null: see att_offsets)
+  uint64_t* mrank[2] = {nullptr, nullptr};  // sort_kw*cap + 1: the entries' sort values (ranks), as the list's buffers
   uint64_t* mmask = nullptr;    // surviving main entries, one bit each, by tiles of kMainTile
   uint16_t* mpre = nullptr;     // per word of mmask: survivors of its tile before it
   int32_t* mcnt = nullptr;      // survivors per tile
@@ -541,6 +541,18 @@ template <class T>
 void dfree(T*& p) {
   if (p) (void)hipFree(p);
   p = nullptr;
+}
+
+// What a cycle needs of its determinants until their spawns are packed lies in
+// the list's idle buffer, which the insertion writes after that: the attempts
+// per (det, space) entry (4 S <= 8 bytes) with the K_ii, the parents' initiator
+// flags (one byte) with the determinants, and, where the sort values are two
+// words, the attempt offsets (8 S <= 16 bytes) with those.  So a slot of the
+// main list takes no more memory with its sort values kept than without.
+int32_t* att_counts(const fq_engine* e) { return reinterpret_cast<int32_t*>(e->kii[1 - e->cur]); }
+uint8_t* parent_flags(const fq_engine* e) { return reinterpret_cast<uint8_t*>(e->det[1 - e->cur]); }
+int64_t* att_offsets(const fq_engine* e) {
+  return e->att_off ? e->att_off : reinterpret_cast<int64_t*>(e->mrank[1 - e->cur]);
 }
 
 // Device address of the fixed scratch array on `device` (current), looked up
@@ -3344,7 +3356,9 @@ int setup_sort(fq_engine* e) {
   if (new_kw || !e->rank_words)
     for (int b = 0; b < 2; ++b) dfree(e->mrank[b]);
   for (int b = 0; b < 2 && e->rank_words; ++b)
-    if (!e->mrank[b]) rc |= dalloc(&e->mrank[b], kw * e->cap);
+    if (!e->mrank[b]) rc |= dalloc(&e->mrank[b], kw * e->cap + 1);
+  // (batched instances, whose sort values are one word, read them to the cycle's end)
+  if (!e->att_off && !(kw == 2 && e->rank_words)) rc |= dalloc(&e->att_off, e->S * e->cap + 1);
   return rc == FQ_OK ? FQ_OK : FQ_ERR_NOMEM;
 }
 
@@ -3611,7 +3625,7 @@ int annihilate(fq_engine* e, int64_t ns, const int64_t* pns, bool replay, uint32
   g.st = e->d_stats;
   g.det_out = e->det[o];
   g.rank_out = e->mrank[o];
-  g.pop_out = e->pop[o];
+  g.pop_out = e->pop;
   g.kii_out = e->kii[o];
   g.abs_part = e->abs_part;
   g.abs_ld = cap / kMainTile + 2 + kNewBlocks;
@@ -4048,7 +4062,7 @@ bool learned_lds_fits(int device, int W, int nbasis) {
 // windows of the spawning tiles of the first `attempts` attempts.
 int scan_attempts(fq_engine* e, int64_t nent, int64_t attempts, int tile) {
   if (nent == 0) {
-    hipLaunchKernelGGL(k_set_zero_total, dim3(1), dim3(1), 0, e->stream, e->att_off);
+    hipLaunchKernelGGL(k_set_zero_total, dim3(1), dim3(1), 0, e->stream, att_offsets(e));
     return FQ_OK;
   }
   const int64_t nblk = ceil_div(nent, static_cast<int64_t>(kBlock) * e->S);
@@ -4057,8 +4071,8 @@ int scan_attempts(fq_engine* e, int64_t nent, int64_t attempts, int tile) {
     const int rc = scan_exclusive(e, e->blk_att, e->blk_off, nblk);
     if (rc != FQ_OK) return rc;
   }
-  hipLaunchKernelGGL(k_att_scan, dim3(grid_for(nent, kScanTile)), dim3(kBlock), 0, e->stream, e->nat, nent, e->blk_att,
-                     nblk, kBlock * e->S, prefix ? nullptr : e->blk_off, e->att_off, e->tile_win,
+  hipLaunchKernelGGL(k_att_scan, dim3(grid_for(nent, kScanTile)), dim3(kBlock), 0, e->stream, att_counts(e), nent, e->blk_att,
+                     nblk, kBlock * e->S, prefix ? nullptr : e->blk_off, att_offsets(e), e->tile_win,
                      ceil_div(attempts, tile), 31 - __builtin_clz(static_cast<unsigned>(tile)), e->d_stats);
   return FQ_OK;
 }
@@ -4107,13 +4121,10 @@ int alloc_engine(fq_engine* e) {
   int rc = FQ_OK;
   for (int b = 0; b < 2; ++b) {
     rc |= dalloc(&e->det[b], W * cap);
-    rc |= dalloc(&e->pop[b], S * cap);
     rc |= dalloc(&e->kii[b], cap);
   }
+  rc |= dalloc(&e->pop, S * cap);
   rc |= dalloc(&e->pop_new, S * cap);
-  rc |= dalloc(&e->nat, S * cap + 1);  // det-major (det, space) entries
-  rc |= dalloc(&e->att_off, S * cap + 1);
-  rc |= dalloc(&e->flags, cap);
   const int64_t mtiles = cap / kMainTile + 2;
   rc |= dalloc(&e->mmask, mtiles * (kMainTile / 64));
   rc |= dalloc(&e->mpre, mtiles * (kMainTile / 64));
@@ -4381,7 +4392,7 @@ int fq_load(fq_engine* e, const uint64_t* states, const int64_t* pops, const dou
   for (int w = 0; w < W && n > 0; ++w)
     FQ_HIP(hipMemcpyAsync(e->det[0] + w * e->cap, dw.data() + w * n, 8 * n, hipMemcpyHostToDevice, e->stream));
   for (int s = 0; s < S && n > 0; ++s)
-    FQ_HIP(hipMemcpyAsync(e->pop[0] + s * e->cap, dp.data() + s * n, 8 * n, hipMemcpyHostToDevice, e->stream));
+    FQ_HIP(hipMemcpyAsync(e->pop + s * e->cap, dp.data() + s * n, 8 * n, hipMemcpyHostToDevice, e->stream));
   if (n > 0) FQ_HIP(hipMemcpyAsync(e->kii[0], dat, 8 * n, hipMemcpyHostToDevice, e->stream));
   if (n > 0 && e->rank_words)
     hipLaunchKernelGGL(k_rank_list, dim3(grid_for(n)), dim3(kBlock), 0, e->stream, key_plan(e), W, n, e->cap,
@@ -4416,7 +4427,7 @@ int fq_semi_stoch_init(fq_engine* e, int64_t target_size, int separate) {
   std::vector<int64_t> pw(static_cast<size_t>(S) * n);
   std::vector<uint64_t> dw(static_cast<size_t>(W) * n);
   for (int sp = 0; sp < S; ++sp)
-    FQ_HIP(hipMemcpyAsync(pw.data() + sp * n, e->pop[c] + sp * e->cap, 8 * n, hipMemcpyDeviceToHost, st));
+    FQ_HIP(hipMemcpyAsync(pw.data() + sp * n, e->pop + sp * e->cap, 8 * n, hipMemcpyDeviceToHost, st));
   for (int w = 0; w < W; ++w)
     FQ_HIP(hipMemcpyAsync(dw.data() + w * n, e->det[c] + w * e->cap, 8 * n, hipMemcpyDeviceToHost, st));
   FQ_HIP(hipStreamSynchronize(st));
@@ -4533,7 +4544,7 @@ static int cycle_body(fq_engine* e, const double* shift, const double* eproj_old
   int64_t rng_pos = e->rng_pos;
   int64_t ns = 0;
   if (replay) {
-    hipLaunchKernelGGL(k_replay_walk, dim3(1), dim3(1), 0, st, e->sys, n, cap, e->det[c], e->pop[c], e->kii[c],
+    hipLaunchKernelGGL(k_replay_walk, dim3(1), dim3(1), 0, st, e->sys, n, cap, e->det[c], e->pop, e->kii[c],
                        e->pop_new, tau, shift[0], sh1, eproj_old[0], e1, e->rng_buf, e->rng_pos, e->rng_end, e->scap,
                        e->sdet, e->srec, e->d_stats, determ_dev(e));
     int rc = sync_stats(e);
@@ -4546,7 +4557,7 @@ static int cycle_body(fq_engine* e, const double* shift, const double* eproj_old
       // online training from the current list: this cycle already uses the update
       fqm::Mlp& m = e->mlp;
       for (int32_t k = 0; k < e->online_steps; ++k) {
-        int trc = fqm::mlp_sample(m, e->sys, e->det[c], e->pop[c], cap, n, e->online_batch,
+        int trc = fqm::mlp_sample(m, e->sys, e->det[c], e->pop, cap, n, e->online_batch,
                                   static_cast<int64_t>(e->par.proposal_min_attempts),
                                   e->par.philox_seed ^ 0x6a09e667f3bcc908ull, static_cast<uint32_t>(m.adam_t), st,
                                   scan_cb, e);
@@ -4556,8 +4567,8 @@ static int cycle_body(fq_engine* e, const double* shift, const double* eproj_old
       ++e->online_runs;
     }
     const unsigned nb = grid_for(n);
-    hipLaunchKernelGGL(e->S == 1 ? k_det_pass<1> : k_det_pass<2>, dim3(nb), dim3(kBlock), 0, st, e->sys, n, cap, e->det[c], e->pop[c], e->kii[c],
-                       e->pop_new, e->nat, e->flags, tau, shift[0], sh1, eproj_old[0], e1, e->par.philox_seed, cyc,
+    hipLaunchKernelGGL(e->S == 1 ? k_det_pass<1> : k_det_pass<2>, dim3(nb), dim3(kBlock), 0, st, e->sys, n, cap, e->det[c], e->pop, e->kii[c],
+                       e->pop_new, att_counts(e), parent_flags(e), tau, shift[0], sh1, eproj_old[0], e1, e->par.philox_seed, cyc,
                        e->part_d, e->part_i, e->d_dvec, e->d_dpos, e->blk_att, e->d_stats);
     e->est_blocks = static_cast<int>(nb);
     if (e->par.excit_gen == FQ_EXCIT_LEARNED && n > 0) {
@@ -4576,13 +4587,13 @@ static int cycle_body(fq_engine* e, const double* shift, const double* eproj_old
         if (e->att_bound > 0) rows = std::min(n, e->att_bound / min_att);
         count = e->att_bound <= 0 || (rows > e->mlp_tab_rows && rows > bound_rows);
       }
-      hipLaunchKernelGGL(k_mlp_mark, dim3(static_cast<unsigned>(mt)), dim3(kBlock), 0, st, n, e->S, e->nat, min_att,
+      hipLaunchKernelGGL(k_mlp_mark, dim3(static_cast<unsigned>(mt)), dim3(kBlock), 0, st, n, e->S, att_counts(e), min_att,
                          e->mcnt, e->d_stats);
       if (mt > kPrefixMax) {
         const int mrc = scan_exclusive(e, e->mcnt, e->moff, mt);
         if (mrc != FQ_OK) return mrc;
       }
-      hipLaunchKernelGGL(k_mlp_rows, dim3(static_cast<unsigned>(mt)), dim3(kBlock), 0, st, n, e->S, e->nat, min_att,
+      hipLaunchKernelGGL(k_mlp_rows, dim3(static_cast<unsigned>(mt)), dim3(kBlock), 0, st, n, e->S, att_counts(e), min_att,
                          rows, e->mcnt, mt > kPrefixMax ? e->moff : nullptr, e->mlp_row, e->mlp_idx, e->d_stats);
       if (min_att > 0 && !count && rows > e->mlp_tab_rows)
         count = grow_proposal_table(e, std::max(rows, std::min(2 * e->mlp_tab_rows, bound_rows)), true) != FQ_OK;
@@ -4611,7 +4622,7 @@ static int cycle_body(fq_engine* e, const double* shift, const double* eproj_old
     int rc = scan_attempts(e, nent, bound > 0 ? std::min(bound, e->bcap) : e->bcap, tile);
     if (rc != FQ_OK) return rc;
     if (bound <= 0) {  // unknown (or an empty list): the exact total
-      FQ_HIP(hipMemcpyAsync(&bound, e->att_off + nent, sizeof(int64_t), hipMemcpyDeviceToHost, st));
+      FQ_HIP(hipMemcpyAsync(&bound, att_offsets(e) + nent, sizeof(int64_t), hipMemcpyDeviceToHost, st));
       FQ_HIP(hipStreamSynchronize(st));
     }
     e->spawn_launches = 0;
@@ -4627,13 +4638,13 @@ static int cycle_body(fq_engine* e, const double* shift, const double* eproj_old
       const int64_t nt = ceil_div(te - tb, tile);
       ++e->spawn_launches;
       if (!one_batch)
-        hipLaunchKernelGGL(k_tile_bounds, dim3(grid_for(nt)), dim3(kBlock), 0, st, nent, e->att_off, tb, te,
+        hipLaunchKernelGGL(k_tile_bounds, dim3(grid_for(nt)), dim3(kBlock), 0, st, nent, att_offsets(e), tb, te,
                            e->tile_win);
       hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(spawn_grid(gen, nt))), dim3(kBlock), lds, st,
-                         e->d_sysp, nent, cap, tb, te, e->att_off, e->det[c], e->pop[c], tau, e->par.philox_seed, cyc,
-                         e->bcap, e->st_det, e->st_pop, e->st_ent, e->tile_cnt, e->tile_win, e->flags, nullptr,
+                         e->d_sysp, nent, cap, tb, te, att_offsets(e), e->det[c], e->pop, tau, e->par.philox_seed, cyc,
+                         e->bcap, e->st_det, e->st_pop, e->st_ent, e->tile_cnt, e->tile_win, parent_flags(e), nullptr,
                          nullptr, nullptr, nullptr, e->d_stats);
-      pack_spawned(e, te - tb, tile, one_batch, e->att_off + nent);
+      pack_spawned(e, te - tb, tile, one_batch, att_offsets(e) + nent);
     }
     int64_t ndet_entries = 0;  // the deterministic projection's spawned entries (combined annihilation)
     if (e->ndeterm > 0) {
@@ -4695,7 +4706,7 @@ int fq_cycle_spawn(fq_engine* e, const double* shift, const double* eproj_old, d
   const double sh1 = e->S > 1 ? shift[1] : 0.0, e1 = e->S > 1 ? eproj_old[1] : 0.0;
   hipLaunchKernelGGL(k_zero, dim3(1), dim3(kBlock), 0, st, reinterpret_cast<int64_t*>(e->d_stats),
                      static_cast<int64_t>(sizeof(Stats) / sizeof(int64_t)));
-  hipLaunchKernelGGL(k_replay_walk, dim3(1), dim3(1), 0, st, e->sys, e->n, e->cap, e->det[c], e->pop[c], e->kii[c],
+  hipLaunchKernelGGL(k_replay_walk, dim3(1), dim3(1), 0, st, e->sys, e->n, e->cap, e->det[c], e->pop, e->kii[c],
                      e->pop_new, tau, shift[0], sh1, eproj_old[0], e1, e->rng_buf, e->rng_pos, e->rng_end, e->scap,
                      e->sdet, e->srec, e->d_stats, determ_dev(e));
   int rc = sync_stats(e);
@@ -4819,7 +4830,7 @@ int fq_annihilate(fq_engine* e, const uint64_t* sstates, const int64_t* spops, c
   if (ns > 0) FQ_HIP(hipMemcpyAsync(e->srec, rec.data(), 8 * RS * ns, hipMemcpyHostToDevice, st));
   // post-death populations = current populations
   for (int s = 0; s < S && n > 0; ++s)
-    FQ_HIP(hipMemcpyAsync(e->pop_new + s * cap, e->pop[e->cur] + s * cap, 8 * n, hipMemcpyDeviceToDevice, st));
+    FQ_HIP(hipMemcpyAsync(e->pop_new + s * cap, e->pop + s * cap, 8 * n, hipMemcpyDeviceToDevice, st));
   FQ_HIP(hipMemsetAsync(e->d_stats, 0, sizeof(Stats), st));
   FQ_HIP(hipStreamSynchronize(st));
   const uint32_t cyc = static_cast<uint32_t>(e->cycle_index++);
@@ -4861,7 +4872,7 @@ static hipError_t copy_rows(fq_engine* e, int slot, int64_t r0, int64_t r1, uint
     if (states)
       for (int w = 0; w < W && err == hipSuccess; ++w) err = fetch(e->det[c] + w * e->cap + i);
     if (pops)
-      for (int sp = 0; sp < S && err == hipSuccess; ++sp) err = fetch(e->pop[c] + sp * e->cap + i);
+      for (int sp = 0; sp < S && err == hipSuccess; ++sp) err = fetch(e->pop + sp * e->cap + i);
     if (dat && err == hipSuccess) err = fetch(e->kii[c] + i);
     if (err == hipSuccess) err = hipEventRecord(e->list_ev[slot], st);
     if (err == hipSuccess) err = hipEventSynchronize(e->list_ev[slot]);
@@ -5053,7 +5064,7 @@ static int inst_stats(fq_engine* e, const int64_t* ob, const int64_t* nbd, int64
                      e->d_iblk_off, e->d_cterm, e->d_cdeath, nbd, e->d_nblk_off, pnew, e->ipb,
                      e->d_ipart_d, e->d_ipart_i);
   hipLaunchKernelGGL(k_inst_stats, dim3(ninst), dim3(kBlock), 0, st, ninst, S, ob, nbd, e->d_isb, e->d_iblk_off,
-                     e->d_nblk_off, e->ipb, e->d_ipart_d, e->d_ipart_i, e->att_off, e->d_iout_d, e->d_iout_i);
+                     e->d_nblk_off, e->ipb, e->d_ipart_d, e->d_ipart_i, att_offsets(e), e->d_iout_d, e->d_iout_i);
   return FQ_OK;
 }
 
@@ -5116,7 +5127,7 @@ static int enqueue_graph_cycle(fq_engine* e, int64_t nb, int64_t tb) {
   hipLaunchKernelGGL(k_inst_bounds, dim3(grid_for(ninst + 1)), dim3(kBlock), 0, st, e->det[c], nb, ninst, kInstShift,
                      ob, dn);
   hipLaunchKernelGGL(k_det_pass_batch, dim3(grid_for(nb)), dim3(kBlock), 0, st, e->sys, e->d_sys_arr, ob, par, ninst,
-                     nb, cap, e->det[c], e->pop[c], e->kii[c], e->pop_new, e->nat, e->flags, e->par.philox_seed, 0u,
+                     nb, cap, e->det[c], e->pop, e->kii[c], e->pop_new, att_counts(e), parent_flags(e), e->par.philox_seed, 0u,
                      e->d_cterm, e->d_cdeath, dn, dcyc, e->blk_att, e->d_stats);
   // entries past the list have no attempts, so att_off[S nb] is the total
   const int64_t nent = S * nb;
@@ -5124,14 +5135,14 @@ static int enqueue_graph_cycle(fq_engine* e, int64_t nb, int64_t tb) {
   const int tile = spawn_tile(gen, tb);
   int rc = scan_attempts(e, nent, tb, tile);
   if (rc != FQ_OK) return rc;
-  hipLaunchKernelGGL(k_inst_att, dim3(grid_for(ninst)), dim3(kBlock), 0, st, ninst, S, ob, e->att_off, e->d_iatt);
+  hipLaunchKernelGGL(k_inst_att, dim3(grid_for(ninst)), dim3(kBlock), 0, st, ninst, S, ob, att_offsets(e), e->d_iatt);
   const unsigned g = static_cast<unsigned>(std::min<int64_t>(
       ceil_div(tb, tile), e->spawn_blocks > 0 ? e->spawn_blocks : int64_t{1} << 20));
   auto kern = tile == kSmallTile ? spawn_kernel<true, kSmallTile>(gen) : spawn_kernel<true, kSpawnTile>(gen);
-  hipLaunchKernelGGL(kern, dim3(g), dim3(kBlock), 0, st, e->d_sysp, nent, cap, int64_t{0}, tb, e->att_off, e->det[c],
-                     e->pop[c], 0.0, e->par.philox_seed, 0u, e->bcap, e->st_det, e->st_pop, e->st_ent, e->tile_cnt,
-                     e->tile_win, e->flags, e->d_sys_arr, e->d_iatt, par, dcyc, e->d_stats);
-  pack_spawned(e, tb, tile, true, e->att_off + nent, tb);
+  hipLaunchKernelGGL(kern, dim3(g), dim3(kBlock), 0, st, e->d_sysp, nent, cap, int64_t{0}, tb, att_offsets(e), e->det[c],
+                     e->pop, 0.0, e->par.philox_seed, 0u, e->bcap, e->st_det, e->st_pop, e->st_ent, e->tile_cnt,
+                     e->tile_win, parent_flags(e), e->d_sys_arr, e->d_iatt, par, dcyc, e->d_stats);
+  pack_spawned(e, tb, tile, true, att_offsets(e) + nent, tb);
   e->keys_ready = true;
   const int64_t nsb = std::min<int64_t>(tb, e->scap);
   const int64_t* pns = &e->d_stats->nspawn;
@@ -5143,7 +5154,7 @@ static int enqueue_graph_cycle(fq_engine* e, int64_t nb, int64_t tb) {
   const int o = 1 - c;
   hipLaunchKernelGGL(k_inst_bounds, dim3(grid_for(ninst + 1)), dim3(kBlock), 0, st, e->det[o],
                      std::min<int64_t>(nb + nsb, cap), ninst, kInstShift, nbd, &e->d_stats->new_n);
-  rc = inst_stats(e, ob, nbd, nb, std::min<int64_t>(nb + nsb, cap), e->pop[o]);
+  rc = inst_stats(e, ob, nbd, nb, std::min<int64_t>(nb + nsb, cap), e->pop);
   if (rc != FQ_OK) return rc;
   FQ_HIP(hipMemcpyAsync(e->h_god, e->d_iout_d, sizeof(double) * 2 * S * ninst, hipMemcpyDeviceToHost, st));
   FQ_HIP(hipMemcpyAsync(e->h_goi, e->d_iout_i, sizeof(int64_t) * (4 + S) * ninst, hipMemcpyDeviceToHost, st));
@@ -5341,14 +5352,14 @@ int fq_cycle_batch(fq_engine* e, const double* shift, const double* eproj_old, c
   hipLaunchKernelGGL(k_inst_bounds, dim3(grid_for(ninst + 1)), dim3(kBlock), 0, st, e->det[c], n, ninst, kInstShift, ob,
                      nullptr);
   hipLaunchKernelGGL(k_det_pass_batch, dim3(grid_for(n)), dim3(kBlock), 0, st, e->sys, e->d_sys_arr, ob, e->d_ipar,
-                     ninst, n, cap, e->det[c], e->pop[c], e->kii[c], e->pop_new, e->nat, e->flags, e->par.philox_seed,
+                     ninst, n, cap, e->det[c], e->pop, e->kii[c], e->pop_new, att_counts(e), parent_flags(e), e->par.philox_seed,
                      cyc, e->d_cterm, e->d_cdeath, nullptr, nullptr, e->blk_att, e->d_stats);
   const int64_t nent = S * n;
   int rc = scan_attempts(e, nent, e->bcap, kSpawnTile);
   if (rc != FQ_OK) return rc;
-  hipLaunchKernelGGL(k_inst_att, dim3(grid_for(ninst)), dim3(kBlock), 0, st, ninst, S, ob, e->att_off, e->d_iatt);
+  hipLaunchKernelGGL(k_inst_att, dim3(grid_for(ninst)), dim3(kBlock), 0, st, ninst, S, ob, att_offsets(e), e->d_iatt);
   int64_t total = 0;
-  FQ_HIP(hipMemcpyAsync(&total, e->att_off + nent, sizeof(int64_t), hipMemcpyDeviceToHost, st));
+  FQ_HIP(hipMemcpyAsync(&total, att_offsets(e) + nent, sizeof(int64_t), hipMemcpyDeviceToHost, st));
   FQ_HIP(hipStreamSynchronize(st));
   e->spawn_launches = 0;
   if (int rs = sync_sysp(e); rs != FQ_OK) return rs;
@@ -5359,13 +5370,13 @@ int fq_cycle_batch(fq_engine* e, const double* shift, const double* eproj_old, c
     const int64_t nt = ceil_div(te - tb, kSpawnTile);
     ++e->spawn_launches;
     if (!one_batch)
-      hipLaunchKernelGGL(k_tile_bounds, dim3(grid_for(nt)), dim3(kBlock), 0, st, nent, e->att_off, tb, te,
+      hipLaunchKernelGGL(k_tile_bounds, dim3(grid_for(nt)), dim3(kBlock), 0, st, nent, att_offsets(e), tb, te,
                          e->tile_win);
     hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(std::min<int64_t>(nt, 1 << 20))), dim3(kBlock), 0, st,
-                       e->d_sysp, nent, cap, tb, te, e->att_off, e->det[c], e->pop[c], 0.0, e->par.philox_seed, cyc,
-                       e->bcap, e->st_det, e->st_pop, e->st_ent, e->tile_cnt, e->tile_win, e->flags, e->d_sys_arr,
+                       e->d_sysp, nent, cap, tb, te, att_offsets(e), e->det[c], e->pop, 0.0, e->par.philox_seed, cyc,
+                       e->bcap, e->st_det, e->st_pop, e->st_ent, e->tile_cnt, e->tile_win, parent_flags(e), e->d_sys_arr,
                        e->d_iatt, e->d_ipar, nullptr, e->d_stats);
-    pack_spawned(e, te - tb, kSpawnTile, one_batch, e->att_off + nent);
+    pack_spawned(e, te - tb, kSpawnTile, one_batch, att_offsets(e) + nent);
   }
   e->keys_ready = true;  // the packing kernels wrote the sort keys
   rc = sync_stats(e);
@@ -5381,7 +5392,7 @@ int fq_cycle_batch(fq_engine* e, const double* shift, const double* eproj_old, c
   const int o = e->cur;
   hipLaunchKernelGGL(k_inst_bounds, dim3(grid_for(ninst + 1)), dim3(kBlock), 0, st, e->det[o], e->n, ninst, kInstShift,
                      nbd, nullptr);
-  rc = inst_stats(e, ob, nbd, n, e->n, e->pop[o]);
+  rc = inst_stats(e, ob, nbd, n, e->n, e->pop);
   if (rc != FQ_OK) return rc;
   std::vector<double> od(static_cast<size_t>(2 * S * ninst));
   std::vector<int64_t> oi(static_cast<size_t>((4 + S) * ninst));
@@ -5529,7 +5540,7 @@ int fq_mlp_train(fq_engine* e, int64_t batch, int32_t steps, double lr, uint64_t
   hipStream_t st = e->stream;
   const int c = e->cur;
   for (int32_t k = 0; k < steps; ++k) {
-    int rc = fqm::mlp_sample(m, e->sys, e->det[c], e->pop[c], e->cap, e->n, batch,
+    int rc = fqm::mlp_sample(m, e->sys, e->det[c], e->pop, e->cap, e->n, batch,
                              static_cast<int64_t>(e->par.proposal_min_attempts), seed,
                              static_cast<uint32_t>(m.adam_t), st, scan_cb, e);
     if (rc != FQ_OK) return rc;
@@ -5602,16 +5613,14 @@ void fq_destroy(fq_engine* e) {
   if (e->stream) (void)hipStreamSynchronize(e->stream);
   for (int b = 0; b < 2; ++b) {
     dfree(e->det[b]);
-    dfree(e->pop[b]);
     dfree(e->kii[b]);
     dfree(e->kbuf[b]);
     dfree(e->mrank[b]);
     dfree(e->new_pos[b]);
   }
+  dfree(e->pop);
   dfree(e->pop_new);
-  dfree(e->nat);
   dfree(e->att_off);
-  dfree(e->flags);
   release_determ(e);
   dfree(e->mmask);
   dfree(e->mpre);
