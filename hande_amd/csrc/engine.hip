@@ -411,7 +411,6 @@ struct fq_engine {
   bool keys_ready = false;           // the spawning pass made this cycle's sort keys
   int64_t last_ns = -1;              // spawned entries last annihilated (-1: none on this list)
   int64_t resorts = 0;               // lists that outgrew the one-block sort they were given to
-  int est_blocks = 0;                // k_det_pass blocks whose partials k_finish adds (0: none)
   int new_src = 0;                   // the sort's idle buffers after this cycle's passes
   int64_t run_tiles = 0;             // run tiles of this cycle's spawned list (a bound of it while captured)
   int64_t mlp_tab_rows = 0;
@@ -3522,8 +3521,10 @@ int sort_and_reduce(fq_engine* e, int64_t ns, const int64_t* pns, bool replay, u
 
 // Annihilation proper: merge runs, round, compact, insert.  ns spawned
 // entries are in the spawned list; pop_new holds the post-death populations.
+// est_blocks: blocks of this cycle's k_det_pass, whose partials k_finish adds
+// (0: the estimators are in the stats, or there are none).
 int annihilate(fq_engine* e, int64_t ns, const int64_t* pns, bool replay, uint32_t cyc, int64_t& rng_pos,
-               bool no_small = false) {
+               int est_blocks = 0, bool no_small = false) {
   int rc = sort_and_reduce(e, ns, pns, replay, cyc, no_small);
   if (rc != FQ_OK) return rc;
   const int64_t ntiles = e->run_tiles;
@@ -3648,7 +3649,7 @@ int annihilate(fq_engine* e, int64_t ns, const int64_t* pns, bool replay, uint32
     nblk += nb;
   }
   hipLaunchKernelGGL(e->S == 1 ? k_finish<1> : k_finish<2>, dim3(1), dim3(kFinishBlock), 0, st, e->part_d, e->part_i,
-                     e->est_blocks, e->abs_part, g.abs_ld, nblk, e->d_stats, e->h_pin);
+                     est_blocks, e->abs_part, g.abs_ld, nblk, e->d_stats, e->h_pin);
   if (e->capturing) return FQ_OK;  // the caller reads the stats when the graph has run
   FQ_HIP(hipStreamSynchronize(st));
   e->h_stats = *e->h_pin;
@@ -3656,9 +3657,8 @@ int annihilate(fq_engine* e, int64_t ns, const int64_t* pns, bool replay, uint32
     hipLaunchKernelGGL(k_zero, dim3(1), dim3(kBlock), 0, st, &e->d_stats->resort, int64_t{1});
     e->keys_ready = true;
     ++e->resorts;
-    return annihilate(e, std::min<int64_t>(e->h_stats.nspawn, scap), nullptr, replay, cyc, rng_pos, true);
+    return annihilate(e, std::min<int64_t>(e->h_stats.nspawn, scap), nullptr, replay, cyc, rng_pos, est_blocks, true);
   }
-  e->est_blocks = 0;
   e->last_ns = pns ? std::min<int64_t>(e->h_stats.nspawn, scap) : ns;  // a caller's list is not counted on the device
   e->cur = o;
   e->n = e->h_stats.new_n;
@@ -4543,6 +4543,7 @@ static int cycle_body(fq_engine* e, const double* shift, const double* eproj_old
                        static_cast<int64_t>(sizeof(Stats) / sizeof(int64_t)));
   int64_t rng_pos = e->rng_pos;
   int64_t ns = 0;
+  int est_blocks = 0;
   if (replay) {
     hipLaunchKernelGGL(k_replay_walk, dim3(1), dim3(1), 0, st, e->sys, n, cap, e->det[c], e->pop, e->kii[c],
                        e->pop_new, tau, shift[0], sh1, eproj_old[0], e1, e->rng_buf, e->rng_pos, e->rng_end, e->scap,
@@ -4570,7 +4571,7 @@ static int cycle_body(fq_engine* e, const double* shift, const double* eproj_old
     hipLaunchKernelGGL(e->S == 1 ? k_det_pass<1> : k_det_pass<2>, dim3(nb), dim3(kBlock), 0, st, e->sys, n, cap, e->det[c], e->pop, e->kii[c],
                        e->pop_new, att_counts(e), parent_flags(e), tau, shift[0], sh1, eproj_old[0], e1, e->par.philox_seed, cyc,
                        e->part_d, e->part_i, e->d_dvec, e->d_dpos, e->blk_att, e->d_stats);
-    e->est_blocks = static_cast<int>(nb);
+    est_blocks = static_cast<int>(nb);
     if (e->par.excit_gen == FQ_EXCIT_LEARNED && n > 0) {
       const int64_t min_att = e->par.proposal_min_attempts, mt = ceil_div(n, kMainTile);
       // A bound of the rows: every determinant without a threshold; else at most
@@ -4671,7 +4672,7 @@ static int cycle_body(fq_engine* e, const double* shift, const double* eproj_old
     e->spawn_bound = bound;
     ns = std::min<int64_t>(bound + ndet_entries, e->scap);
   }
-  int rc = annihilate(e, ns, replay ? nullptr : &e->d_stats->nspawn, replay, cyc, rng_pos);
+  int rc = annihilate(e, ns, replay ? nullptr : &e->d_stats->nspawn, replay, cyc, rng_pos, est_blocks);
   if (rc != FQ_OK) return rc;
   // the attempts cannot exceed the bound the spawning launches covered (see sort_and_reduce)
   if (!replay && e->h_stats.total_attempts > e->spawn_bound) return FQ_ERR_DEVICE;

@@ -1,6 +1,7 @@
 """Sizes at which the learned proposal's kernels change shape: rows of the
 inference (16 or 64 to a block), samples of the training products (chunks of
 four slabs), list lengths around the tiles that number the network's rows."""
+import contextlib
 import ctypes as C
 import itertools
 
@@ -104,47 +105,89 @@ def _many_dets(norb, nel, n):
     return np.sort((half[:, None] | beta[None, :]).reshape(-1))[:n]
 
 
-def test_rows_follow_the_list_where_their_bound_has_no_memory(tmp_path):
-    """1e6 determinants, nearly all with one walker, at a threshold of two: the
-    attempts bound the rows by 5e5 (160 MB of weights), a few thousand are there.
-    Where the card has no 128 MB left the cycle runs as it does with all of it."""
-    norb, nel, n = 20, 8, 1000000
-    system = _system(tmp_path, norb, nel, 2008)
-    lib = N.lib()
+@contextlib.contextmanager
+def _no_memory_left():
+    """The card's memory taken until it has no 128 MB to give."""
+    hip, hog = C.CDLL("libamdhip64.so.7"), []  # the engine's own runtime, loaded with it
+    try:
+        for size in (1 << 33, 128 << 20):
+            while hip.hipMalloc(C.byref(block := C.c_void_p()), C.c_size_t(size)) == 0:
+                hog.append(block)
+            hip.hipGetLastError()
+        yield
+    finally:
+        for block in hog:
+            hip.hipFree(block)
+
+
+def _list_of_1e6(tmp_path, min_attempts):
+    """A system, its parameters and 1e6 determinants of one walker, every 500th of five."""
     p = N.FqParams()
     p.nspaces, p.excit_gen, p.rng_mode, p.philox_seed = 1, N.FQ_EXCIT_LEARNED, N.FQ_RNG_PHILOX, 9
     p.main_capacity = p.spawn_capacity = 1 << 22
-    p.proposal_mix, p.proposal_min_attempts = 0.1, 2
-    dets = _many_dets(norb, nel, n)
-    pops = np.ones(n, dtype=np.int64)
+    p.proposal_mix, p.proposal_min_attempts = 0.1, min_attempts
+    pops = np.ones(1000000, dtype=np.int64)
     pops[::500] = 5
-    engs, results, hog = [], [], []
+    return _system(tmp_path, 20, 8, 2008), p, _many_dets(20, 8, len(pops)), pops
+
+
+def _load(lib, eng, dets, pops):
+    N.check(lib.fq_load(eng, dets.ctypes.data_as(P(C.c_uint64)), pops.ctypes.data_as(P(C.c_int64)),
+                        np.zeros(len(pops)).ctypes.data_as(P(C.c_double)), len(pops)), "fq_load")
+
+
+def test_rows_follow_the_list_where_their_bound_has_no_memory(tmp_path):
+    """At a threshold of two the attempts bound the rows by 5e5 (160 MB of
+    weights), a few thousand are there.  Where the card has no 128 MB left the
+    cycle runs as it does with all of it."""
+    lib = N.lib()
+    system, p, dets, pops = _list_of_1e6(tmp_path, 2)
+    engs, results = [], []
     sh = (C.c_double * 2)(0.0, 0.0)
-    hip = C.CDLL("libamdhip64.so.7")  # the engine's own runtime, loaded with it
     try:
         for _ in range(2):
             eng = C.c_void_p()
             N.check(lib.fq_create(system.view, C.byref(p), C.byref(eng)), "fq_create")
             engs.append(eng)
-            N.check(lib.fq_load(eng, dets.ctypes.data_as(P(C.c_uint64)), pops.ctypes.data_as(P(C.c_int64)),
-                                np.zeros(n).ctypes.data_as(P(C.c_double)), n), "fq_load")
+            _load(lib, eng, dets, pops)
             N.check(lib.fq_cycle(eng, sh, sh, 1e-3, C.byref(N.FqCycleOut())), "fq_cycle")
-        for full, eng in ((True, engs[0]), (False, engs[1])):
-            for size in (1 << 33, 128 << 20) if full else ():  # until the card has no 128 MB to give
-                while hip.hipMalloc(C.byref(block := C.c_void_p()), C.c_size_t(size)) == 0:
-                    hog.append(block)
-                hip.hipGetLastError()
+        for eng, memory in ((engs[0], _no_memory_left()), (engs[1], contextlib.nullcontext())):
             out, prof = N.FqCycleOut(), N.FqProfileOut()
-            N.check(lib.fq_cycle(eng, sh, sh, 1e-3, C.byref(out)), "fq_cycle")
+            with memory:
+                N.check(lib.fq_cycle(eng, sh, sh, 1e-3, C.byref(out)), "fq_cycle")
             N.check(lib.fq_last_profile(eng, C.byref(prof)), "fq_last_profile")
-            while hog:
-                hip.hipFree(hog.pop())
             assert out.nattempts > 8e5 and 1000 < prof.proposal_rows < 65536
             results.append((out.nstates, out.nspawn_events, out.nattempts, out.ndeath, out.nparticles[0],
                             prof.proposal_rows, *[x.tobytes() for x in download(lib, eng, 1, 1)]))
         assert results[0] == results[1]
     finally:
-        for x in hog:
-            hip.hipFree(x)
         for eng in engs:
             lib.fq_destroy(eng)
+
+
+def test_a_cycle_without_memory_leaves_nothing_to_the_next_call(tmp_path):
+    """Without a threshold every determinant needs its row: 320 MB are not there.
+    The walkers stay, and the annihilation of an empty list after it reports no
+    estimators of the cycle that failed."""
+    lib = N.lib()
+    system, p, dets, pops = _list_of_1e6(tmp_path, 0)
+    dets[0], pops[0] = system.view.f0[0], 7  # the reference determinant, the list's first
+    assert dets[0] < dets[1]
+    eng, out = C.c_void_p(), N.FqCycleOut()
+    sh = (C.c_double * 2)(0.0, 0.0)
+    N.check(lib.fq_create(system.view, C.byref(p), C.byref(eng)), "fq_create")
+    try:
+        _load(lib, eng, dets, pops)
+        with _no_memory_left():
+            assert lib.fq_cycle(eng, sh, sh, 1e-3, C.byref(out)) == -2  # FQ_ERR_NOMEM
+        none, empty = np.zeros(1, np.uint64), np.zeros(1, np.int64)
+        N.check(lib.fq_annihilate(eng, none.ctypes.data_as(P(C.c_uint64)), empty.ctypes.data_as(P(C.c_int64)),
+                                  empty.ctypes.data_as(P(C.c_int64)), 0, C.byref(out)), "fq_annihilate")
+        assert (out.proj_energy[0], out.D0_population[0], out.ndeath, out.nattempts) == (0.0, 0.0, 0, 0)
+        assert out.nstates == len(dets) and out.nparticles[0] == np.abs(pops).sum()
+        got = download(lib, eng, 1, 1)
+        assert np.array_equal(got[0], dets) and np.array_equal(got[1], pops)
+        N.check(lib.fq_cycle(eng, sh, sh, 1e-3, C.byref(out)), "fq_cycle")
+        assert out.D0_population[0] == 7.0 and out.nattempts == np.abs(pops).sum()
+    finally:
+        lib.fq_destroy(eng)
