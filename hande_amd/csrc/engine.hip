@@ -496,6 +496,7 @@ struct fq_engine {
   // events, and the streams they share with the engine's (a stream takes ~1 ms to make)
   static constexpr int kListSlots = 6, kListStreams = 3;
   hipStream_t list_stream[kListStreams] = {};
+  std::mutex list_mutex;  // a download at a time: they share the slots
   uint64_t* list_buf = nullptr;
   int list_slots = 0;
   hipEvent_t list_ev[kListSlots] = {};
@@ -4907,6 +4908,7 @@ int fq_download(fq_engine* e, uint64_t* states, int64_t* pops, double* dat, int6
   *nout = n;
   if (capacity < n) return FQ_ERR_CAPACITY;
   if (n == 0) return FQ_OK;
+  std::lock_guard<std::mutex> lock(e->list_mutex);
   FQ_HIP(hipSetDevice(e->device));
   FQ_HIP(hipStreamSynchronize(e->stream));
   const int64_t bytes = 8 * n * (e->W + e->S + 1);
