@@ -165,6 +165,7 @@ def _declare(lib):
         "fq_destroy": (None, [vp]),
         # for the tests (engine.hip, after fq_destroy)
         "fqt_tile_windows": (C.c_int, [vp, P(i64), i64]),
+        "fqt_prefix_tiles": (C.c_int, [vp, i64, i64, i64]),
         "fqt_resorts": (i64, [vp]),
         "fqt_scan_scratch": (C.c_int, [vp, C.c_int, P(i64), P(i64)]),
     }

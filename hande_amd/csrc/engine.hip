@@ -89,10 +89,23 @@ constexpr uint64_t kOrbMask = (uint64_t{1} << kInstShift) - 1;
 constexpr int kMaxInst = 1 << 16;
 constexpr int kRunTile = 4 * kBlock;   // sorted entries per run tile
 constexpr int kMainTile = 4 * kBlock;  // main-list entries per rounding and insertion tile
-// Counts of up to this many tiles are prefixed by every block that needs them
-// (its threads add the counts before its tile: 16384 counts are 64 KB from L2);
-// longer ones are scanned first.
-constexpr int64_t kPrefixMax = 16384;
+// Counts of up to this many blocks or tiles are prefixed by every block that
+// needs them (its threads add the counts before its own, work that grows with the
+// square of the list); more of them are scanned first.  Both ways on an 18-site
+// ring, scan against sums, us:
+// * attempts of k_det_pass's blocks, with the scans of more than 8192 counts in
+//   two launches or three: 87 and 80 for the determinant pass and k_att_scan at
+//   16300 blocks (4.2e6 determinants), 104 and 104 at 21700, 167 and 194 at 42200;
+// * run heads and new determinants of the run tiles (k_runs, k_round), and the
+//   network's rows (k_mlp_rows): reduction 117 and 111, rounding and insertion 201
+//   and 204 at 3900 tiles; 160 and 155, 347 and 360 at 5650; 411 and 438, 868 and
+//   935 at 13800; rows 54 and 52 at 3900 tiles, 88 and 94 at 7800;
+// * survivors of the main tiles (k_scatter_main, whose blocks add the whole list's
+//   as well): rounding and insertion 42.7 and 41.4 at 2100 tiles, 55 and 57 at
+//   3000, 101 and 109 at 5400, 272 and 375 at 15500.
+constexpr int64_t kPrefixAttempts = 16384;
+constexpr int64_t kPrefixRuns = 4096;
+constexpr int64_t kPrefixMain = 2048;
 constexpr int64_t kListSlotBytes = int64_t{1} << 20;  // a pinned slot of fq_download
 // Words per spawned-list record (populations, flag), padded to 16-byte
 // alignment so one record is one aligned read after the sort's permutation.
@@ -412,6 +425,8 @@ struct fq_engine {
   int64_t last_ns = -1;              // spawned entries last annihilated (-1: none on this list)
   int64_t resorts = 0;               // lists that outgrew the one-block sort they were given to
   int new_src = 0;                   // the sort's idle buffers after this cycle's passes
+  // counts that the kernels that need their prefix add up themselves
+  int64_t prefix_attempts = kPrefixAttempts, prefix_runs = kPrefixRuns, prefix_main = kPrefixMain;
   int64_t run_tiles = 0;             // run tiles of this cycle's spawned list (a bound of it while captured)
   int64_t mlp_tab_rows = 0;
   int cls_sorted = 0;          // the spin/irrep classes list their orbitals in ascending order
@@ -437,7 +452,7 @@ struct fq_engine {
   double* part_d = nullptr;     // 4 * (cap/256+1) block partials
   int64_t* part_i = nullptr;    // 2 * (cap/256+1)
   int64_t* blk_att = nullptr;   // cap/256+2: attempts of k_det_pass's blocks
-  int64_t* blk_off = nullptr;   // their exclusive prefix (lists of more than kPrefixMax blocks)
+  int64_t* blk_off = nullptr;   // their exclusive prefix (more than kPrefixAttempts of them)
   // spawning-attempt staging (one slot per attempt of a batch)
   int64_t bcap = 0;
   uint64_t* st_det = nullptr;   // W*bcap
@@ -457,14 +472,14 @@ struct fq_engine {
   int64_t* pass_cnt = nullptr;             // 512 * kSortBlocks digit counts of a pass's blocks
   int64_t* pass_off = nullptr;             // their exclusive prefix (+ total)
   int32_t* run_tcnt = nullptr;             // run heads per run tile
-  int64_t* run_toff = nullptr;             // their exclusive prefix (lists of more than kPrefixMax tiles)
+  int64_t* run_toff = nullptr;             // their exclusive prefix (more than kPrefixRuns tiles)
   int32_t* run_tfirst = nullptr;           // first head of each run tile (-1: none)
   int64_t* run_tpre = nullptr;             // sums of each run tile's entries before its first head
   int64_t* run_win = nullptr;              // main-list position of each run tile's first value; then the end
   // new determinants: per run tile (values and populations in the sort's idle
   // buffers, positions in new_pos[0]), then in one list
   int32_t* new_cnt = nullptr;    // per run tile
-  int64_t* new_off = nullptr;    // their exclusive prefix (lists of more than kPrefixMax tiles)
+  int64_t* new_off = nullptr;    // their exclusive prefix (more than kPrefixRuns tiles)
   int32_t* new_pos[2] = {nullptr, nullptr};  // scap: insertion positions (non-decreasing): staged, listed
   uint64_t* new_val = nullptr;   // sort_kw*scap: sort values of the new determinants
   int64_t* new_pop = nullptr;    // S*scap: their populations
@@ -838,7 +853,7 @@ constexpr int64_t kSmallTileMax = 512 * kSpawnTile;  // attempts up to which the
 // entries, kScanTile entries a block, out[nent] = total.  part: the sums of
 // k_det_pass's blocks (`per` entries each, nblk of them), added up by every
 // block for its offset; poff, when given, is their exclusive prefix (lists of
-// more than kPrefixMax blocks).  The block that holds the first or last attempt
+// more than kPrefixAttempts blocks).  The block that holds the first or last attempt
 // of a spawning tile (1 << tile_bits attempts, the first ntile tiles) looks its
 // parent up among the starts it keeps in LDS and notes it as that end of the
 // tile's parent window, so no search precedes the spawning kernel.  (2.8e6
@@ -3480,7 +3495,7 @@ int sort_and_reduce(fq_engine* e, int64_t ns, const int64_t* pns, bool replay, u
     hipLaunchKernelGGL(cnt, dim3(static_cast<unsigned>(nt)), dim3(kBlock), 0, st, e->kbuf[src], e->pbuf[src], pns, ns,
                        scap, e->flag_bits, mrank, e->n, e->cap, dn, nt, e->run_tcnt, e->run_tfirst, e->run_tpre,
                        e->run_win, e->d_stats);
-    if (nt > kPrefixMax) {
+    if (nt > e->prefix_runs) {
       const int rc = scan_exclusive(e, e->run_tcnt, e->run_toff, nt);
       if (rc != FQ_OK) return rc;
     }
@@ -3492,7 +3507,7 @@ int sort_and_reduce(fq_engine* e, int64_t ns, const int64_t* pns, bool replay, u
     g.stride = scap;
     g.fb = e->flag_bits;
     g.tcnt = e->run_tcnt;
-    g.toff = nt > kPrefixMax ? e->run_toff : nullptr;
+    g.toff = nt > e->prefix_runs ? e->run_toff : nullptr;
     g.tfirst = e->run_tfirst;
     g.tpre = e->run_tpre;
     g.win = e->run_win;
@@ -3564,7 +3579,7 @@ int annihilate(fq_engine* e, int64_t ns, const int64_t* pns, bool replay, uint32
                          e->new_cnt, nval, npop, e->new_pos[0], scap, e->rng_buf, rng_pos + main_draws, e->ndraw_off);
   }
   const int64_t mtiles = std::max<int64_t>(1, ceil_div(n, kMainTile));
-  if (ntiles > kPrefixMax) {
+  if (ntiles > e->prefix_runs) {
     rc = scan_exclusive(e, e->new_cnt, e->new_off, ntiles);
     if (rc != FQ_OK) return rc;
   }
@@ -3590,7 +3605,7 @@ int annihilate(fq_engine* e, int64_t ns, const int64_t* pns, bool replay, uint32
   r.scap = scap;
   r.ntiles = ntiles;
   r.ncnt = e->new_cnt;
-  r.noff = ntiles > kPrefixMax ? e->new_off : nullptr;
+  r.noff = ntiles > e->prefix_runs ? e->new_off : nullptr;
   r.nval = nval;
   r.npop = npop;
   r.npos = e->new_pos[0];
@@ -3600,7 +3615,7 @@ int annihilate(fq_engine* e, int64_t ns, const int64_t* pns, bool replay, uint32
   r.st = e->d_stats;
   hipLaunchKernelGGL(k_round, dim3(static_cast<unsigned>(mtiles + ntiles)), dim3(kBlock), 0, st, r);
   rng_pos += main_draws + new_draws;
-  if (mtiles > kPrefixMax) {  // offsets first: every tile's block would add too many counts
+  if (mtiles > e->prefix_main) {  // offsets first: every tile's block would add too many counts
     rc = scan_exclusive(e, e->mcnt, e->moff, mtiles);
     if (rc != FQ_OK) return rc;
   }
@@ -3618,7 +3633,7 @@ int annihilate(fq_engine* e, int64_t ns, const int64_t* pns, bool replay, uint32
   g.mmask = e->mmask;
   g.mpre = e->mpre;
   g.mcnt = e->mcnt;
-  g.moff_in = mtiles > kPrefixMax ? e->moff : nullptr;
+  g.moff_in = mtiles > e->prefix_main ? e->moff : nullptr;
   g.moff = e->moff;
   g.lpos = e->new_pos[1];
   g.lval = e->new_val;
@@ -4067,7 +4082,7 @@ int scan_attempts(fq_engine* e, int64_t nent, int64_t attempts, int tile) {
     return FQ_OK;
   }
   const int64_t nblk = ceil_div(nent, static_cast<int64_t>(kBlock) * e->S);
-  const bool prefix = nblk <= kPrefixMax;
+  const bool prefix = nblk <= e->prefix_attempts;
   if (!prefix) {
     const int rc = scan_exclusive(e, e->blk_att, e->blk_off, nblk);
     if (rc != FQ_OK) return rc;
@@ -4591,12 +4606,12 @@ static int cycle_body(fq_engine* e, const double* shift, const double* eproj_old
       }
       hipLaunchKernelGGL(k_mlp_mark, dim3(static_cast<unsigned>(mt)), dim3(kBlock), 0, st, n, e->S, att_counts(e), min_att,
                          e->mcnt, e->d_stats);
-      if (mt > kPrefixMax) {
+      if (mt > e->prefix_runs) {
         const int mrc = scan_exclusive(e, e->mcnt, e->moff, mt);
         if (mrc != FQ_OK) return mrc;
       }
       hipLaunchKernelGGL(k_mlp_rows, dim3(static_cast<unsigned>(mt)), dim3(kBlock), 0, st, n, e->S, att_counts(e), min_att,
-                         rows, e->mcnt, mt > kPrefixMax ? e->moff : nullptr, e->mlp_row, e->mlp_idx, e->d_stats);
+                         rows, e->mcnt, mt > e->prefix_runs ? e->moff : nullptr, e->mlp_row, e->mlp_idx, e->d_stats);
       if (min_att > 0 && !count && rows > e->mlp_tab_rows)
         count = grow_proposal_table(e, std::max(rows, std::min(2 * e->mlp_tab_rows, bound_rows)), true) != FQ_OK;
       if (count) {
@@ -5738,6 +5753,17 @@ int fqt_tile_windows(fq_engine* e, int64_t* out, int64_t ntiles) {
   FQ_HIP(hipSetDevice(e->device));
   FQ_HIP(hipMemcpyAsync(out, e->tile_win, sizeof(int64_t) * 2 * ntiles, hipMemcpyDeviceToHost, e->stream));
   FQ_HIP(hipStreamSynchronize(e->stream));
+  return FQ_OK;
+}
+
+// The longest counts of the attempts' blocks, the run tiles and the main tiles
+// that no scan precedes (kPrefixAttempts, ...); results do not depend on them.
+// Before graph cycles only.
+int fqt_prefix_tiles(fq_engine* e, int64_t attempts, int64_t runs, int64_t main) {
+  if (!e || attempts < 0 || runs < 0 || main < 0 || !e->graphs.empty()) return FQ_ERR_ARG;
+  e->prefix_attempts = attempts;
+  e->prefix_runs = runs;
+  e->prefix_main = main;
   return FQ_OK;
 }
 

@@ -252,10 +252,11 @@ def _random_keys(rng, nbits, nel, count):
 
 @pytest.mark.parametrize("nmain,nspawn", [(600_000, 1_200_000), (600_000, 3_000)])
 def test_annihilate_production_large_lists(nmain, nspawn):
-    """Lists of 1e6 entries: every prefix sum spans many tiles and several
-    chunks of the tile-sum scan; radix sort over 32-bit keys in 4 passes.
-    With few spawns the main-list window of a merge block is too wide to stage
-    in LDS (searched in global memory); with many it is staged."""
+    """Lists of 1e6 entries: hundreds of run and main tiles, whose counts are
+    prefixed in the kernels that need them (test_gpu_prefix_tiles.py runs this
+    with scans); radix passes over 27-bit ranks or 32-bit words.  With few spawns
+    a run tile's window of the main list is too wide to stage in LDS (searched in
+    global memory); with many it is staged."""
     print(f"[annihilate] production, {nmain} main + {nspawn} spawned", flush=True)
     lib, orc = N.lib(), oracle()
     system = api.hubbard_k(electrons=10, lattice=[[4, 0], [0, 4]], ms=0, sym="tot_sym", U=4)

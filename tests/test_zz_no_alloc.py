@@ -3,10 +3,13 @@ array, no device allocation) against fq_cycle, bit for bit.
 
 Two engines with the same parameters and seed hold the same walker list; one
 cycles through fq_cycle, the other through fq_cycle_noalloc.  Cycle outputs
-and walker lists must be identical after each call: first on a list large
-enough for the multi-tile prefix sums and several radix-sort tiles, then, on
-the next call, on a smaller list loaded into both engines."""
+and walker lists must be identical after each call: first on a list of several
+radix-sort tiles, then, on the next call, on a smaller list loaded into both
+engines.  The scratch itself holds the tile sums of scans of more than 8192
+counts: a list of 2.2e6 determinants makes that many, and the second engine is
+told to scan them where the first adds them up."""
 import ctypes as C
+import itertools
 import os
 
 import numpy as np
@@ -107,7 +110,35 @@ def test_noalloc_cycle_matches_cycle(tmp_path, kind):
             print(f"  {label}: attempts={o1.nattempts} spawned={o1.nspawn_events} nstates={o1.nstates}", flush=True)
             _same(lib, ra, rb, W, o1, o2, label)
             if label == "large":
-                assert o1.nspawn_events > 2 * 2048 and o1.nattempts > 8192  # several sort tiles, tiled scans
+                assert o1.nspawn_events > 2 * 2048 and o1.nattempts > 8192  # several sort tiles
+    finally:
+        lib.fq_destroy(ra)
+        lib.fq_destroy(rb)
+
+
+def test_noalloc_scans_in_the_fixed_scratch():
+    lib = N.lib()
+    system = api.hubbard_k(electrons=18, lattice=[[18]], ms=0, sym=1, U=1.0, t=1.0)
+    n = 2200000  # 8594 blocks of 256 determinants, each with its count of attempts
+    half = np.array([sum(1 << (2 * o) for o in c) for c in itertools.combinations(range(18), 9)], dtype=np.uint64)
+    dets = np.sort((half[:, None] | half[None, :-(-n // len(half))] << np.uint64(1)).reshape(-1))[:n]
+    p = _params(214, real=False, initiator=False, cap=1 << 23)
+    ra, rb = C.c_void_p(), C.c_void_p()
+    N.check(lib.fq_create(system.view, C.byref(p), C.byref(ra)), "fq_create")
+    N.check(lib.fq_create(system.view, C.byref(p), C.byref(rb)), "fq_create")
+    try:
+        N.check(lib.fqt_prefix_tiles(rb, 0, 0, 0), "fqt_prefix_tiles")
+        sh = (C.c_double * 2)(0.0, 0.0)
+        for eng in (ra, rb):
+            _load(lib, eng, (dets, np.ones(n, dtype=np.int64), np.zeros(n)))
+        for cyc in range(3):
+            o1, o2 = N.FqCycleOut(), N.FqCycleOut()
+            N.check(lib.fq_cycle(ra, sh, sh, 0.002, C.byref(o1)), "fq_cycle")
+            N.check(lib.fq_cycle_noalloc(rb, sh, sh, 0.002, C.byref(o2)), "fq_cycle_noalloc")
+            _same(lib, ra, rb, 1, o1, o2, cyc)
+        address, elements = C.c_int64(), C.c_int64()  # the scans left the growing scratch alone
+        N.check(lib.fqt_scan_scratch(rb, 0, C.byref(address), C.byref(elements)), "fqt_scan_scratch")
+        assert (address.value, elements.value) == (0, 0)
     finally:
         lib.fq_destroy(ra)
         lib.fq_destroy(rb)
