@@ -202,6 +202,8 @@ def phase_bytes(prof, W=1, S=1, kw=1):
     """Algorithmic HBM bytes of each phase of one cycle as the kernels move
     them; kw: words of the sort key."""
     nd, ns, nout = prof.nstates_in, prof.nspawned, prof.nstates_out
+    # a list that one workgroup sorts (at most 8192 one-word keys) makes its passes in LDS
+    passes = 1 if kw == 1 and ns <= 8192 else prof.radix_passes
     bm, bs = entry_bytes(W, S)
     return {
         # read det/pop/K_ii, write post-death pops, attempt counts, flags
@@ -209,7 +211,7 @@ def phase_bytes(prof, W=1, S=1, kw=1):
         # parents (det, pop, flag) and attempt offsets once, spawned entries and their sort keys written
         "spawn": nd * (8 * W + 8 * S + 1 + 8 * S) + ns * (bs + 8 * kw),
         # each pass reads the keys for its counts, then reads and writes keys and populations
-        "sort": prof.radix_passes * ns * (8 * kw + 2 * (8 * kw + 8 * S)),
+        "sort": passes * ns * (8 * kw + 2 * (8 * kw + 8 * S)),
         # sorted keys read for the run heads, then with the populations; the main list's sort values once
         "reduce": ns * (2 * 8 * kw + 8 * S) + nd * 8 * kw,
         # post-death populations rounded; main list and sort values read and written once

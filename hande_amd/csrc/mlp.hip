@@ -368,17 +368,15 @@ __global__ __launch_bounds__(kBlock) void k_wgrad(WGrads w, int64_t ns, int64_t 
     if (wave == 0 && j0 + c < g.N) out[g.o_b + j0 + c] = (cs[c] + cs[64 + c]) + (cs[128 + c] + cs[192 + c]);
   }
 }
-// The gradient of parameter t: its chunks' partial sums in order.
-__device__ __forceinline__ float sum_splits(const float* __restrict__ part, int64_t t, int64_t stride, int nsplit) {
-  float acc = 0.0f;
-#pragma unroll 8
-  for (int z = 0; z < nsplit; ++z) acc += part[z * stride + t];
-  return acc;
-}
+// The gradient of each parameter: its chunks' partial sums in order.
 __global__ void k_sum_splits(int64_t n, int64_t stride, int nsplit, const float* __restrict__ part,
                              float* __restrict__ g) {
   const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t < n) g[t] = sum_splits(part, t, stride, nsplit);
+  if (t >= n) return;
+  float acc = 0.0f;
+#pragma unroll 8
+  for (int z = 0; z < nsplit; ++z) acc += part[z * stride + t];
+  g[t] = acc;
 }
 // Fixed-order sum of n doubles on one block (kSumBlock threads: 16384 values
 // are 16 loads a thread, all in flight; 16.6 us with 256 threads, 4.7 now).

@@ -137,7 +137,7 @@ typedef struct fq_engine fq_engine;
  * FQ_ERR_ARG for an inconsistent request, including the heat-bath or learned
  * generator on a system other than read_in or with more than 32 electrons,
  * spawned lists whose sort keys would not fit 128 bits (ceil(log2 C(nbasis, nel))
- * plus ceil(log2 spawn_capacity) above 128: half-filled systems near 128 spin orbitals),
+ * and a flag bit per space),
  * the heat-bath generator when its per-attempt weights (8 bytes per
  * electron per thread of a 256-thread workgroup) do not fit the device's
  * workgroup LDS, and the learned generator when its affinity table (4 nbasis^2
@@ -217,7 +217,8 @@ int fq_annihilate(fq_engine *e, const uint64_t *sstates, const int64_t *spops, c
                   int64_t ns, fq_cycle_out *out);
 
 /* Current walker count and a copy of the main list to the host (report /
- * restart boundaries only).  Arrays must hold capacity entries. */
+ * restart boundaries only).  Arrays must hold capacity entries; those not
+ * wanted may be NULL.  Downloads of one engine from several threads take turns. */
 int fq_nstates(fq_engine *e, int64_t *n);
 int fq_download(fq_engine *e, uint64_t *states, int64_t *pops, double *dat, int64_t capacity, int64_t *n);
 
@@ -228,17 +229,18 @@ int fq_last_timing(fq_engine *e, double *spawn_ms, double *annihilate_ms, double
  * phase's first kernel starts, and the sizes that phase handled. */
 typedef struct fq_profile_out {
   double det_pass_ms;    /* per-determinant pass: estimators, nattempts, death */
-  double spawn_ms;       /* spawning-attempt kernel */
+  double spawn_ms;       /* spawning attempts and the packing of the spawned list */
   double sort_ms;        /* radix sort (or reference quicksort) of the spawned list */
-  double reduce_ms;      /* run detection and self-annihilation */
-  double merge_ms;       /* merge with the main list, rounding, compaction, insertion */
-  double total_ms;       /* whole cycle, first to last kernel */
+  double reduce_ms;      /* runs: self-annihilation, merge with the main list, rounding of new determinants */
+  double merge_ms;       /* rounding and compaction of the main list, insertion */
+  double total_ms;       /* whole cycle, from the first kernel's start to the last one's */
   int64_t nstates_in;    /* occupied determinants at the start of the cycle */
   int64_t nattempts;     /* spawning attempts */
   int64_t nspawned;      /* spawned entries written */
   int64_t nruns;         /* unique spawned determinants */
   int64_t nstates_out;   /* occupied determinants after annihilation */
-  int32_t radix_passes;  /* 8-bit digit passes of the sort */
+  int32_t radix_passes;  /* digit passes of the sort (8 or 9 bits each), over the list in memory or, for a short
+                          * one, inside one workgroup */
   int32_t spawn_launches;    /* launches of the spawning-attempt kernel this cycle */
   double spawn_kernel_ms;    /* summed device time of those launches (device clock) */
   double proposal_ms;        /* learned proposal: network marking, inference and attempt offsets */
@@ -283,7 +285,7 @@ typedef struct fq_schedule_out {
   int32_t graph;          /* graph cycles enabled */
   int32_t tuned;          /* the tuner has chosen for the octave of the last graph cycle's attempt bound */
   int32_t digit_bits;     /* widest radix digit of the chosen schedule: 9 (8- and 9-bit digits) or 8 */
-  int32_t spawn_blocks;   /* spawning grid cap of the chosen schedule (0: one block per 1024-attempt tile) */
+  int32_t spawn_blocks;   /* spawning grid cap of the chosen schedule (0: one block per tile of attempts) */
   int32_t ncand;          /* candidate schedules */
   int32_t chosen;         /* index of the chosen one (-1 while tuning) */
   int32_t octave;         /* floor(log2) of the last graph cycle's attempt bound (-1: none yet) */
